@@ -114,7 +114,7 @@ template <int TY, bool LOCAL>
 __global__ __launch_bounds__(BTX *TY) __attribute__((amdgpu_waves_per_eu(2))) void kb_vanka(const BEntry *__restrict__ E, const int *__restrict__ pre, int n,
                                                      const unsigned char *__restrict__ on, int n_newton)
 {
-    __shared__ double eta_s[TY + 2][BTX + 2];
+    __shared__ VankaLDS<BTX, TY> L;
     tile_loop(pre[n], [&](int t) {
         const int e = find_entry(pre, n, t);
         const GlideLevel &A = E[e].L;
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(BTX *TY) __attribute__((amdgpu_waves_per_eu(2))) vo
         const int lt = t - pre[e], tx = cdiv(A.g.nx, BTX);
         __syncthreads();
         vanka_tile<BTX, TY, LOCAL>(A.g, to_params(A.p), A.U, A.f, A.bed, A.B, A.beta, A.gamma, A.active,
-                                   A.g.nx / RB + 1, n_newton, A.scratch, lt % tx, lt / tx, eta_s);
+                                   A.g.nx / RB + 1, n_newton, A.scratch, lt % tx, lt / tx, L);
     });
 }
 

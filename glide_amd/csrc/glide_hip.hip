@@ -157,11 +157,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                                               const double *__restrict__ gamma, const unsigned char *__restrict__ blk,
                                               int nbx, int n_newton, double *__restrict__ cd)
 {
-    __shared__ double eta_s[TY + 2][TX + 2];
+    __shared__ VankaLDS<TX, TY> L;
     const int tx = cdiv(g.nx, TX), total = tx * cdiv(g.ny, TY);
     tile_loop(total, [&](int t) {
-        __syncthreads();   // the previous tile's readers of eta_s are done
-        vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, t % tx, t / tx, eta_s);
+        __syncthreads();   // the previous tile's readers of L are done
+        vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, t % tx, t / tx, L);
     });
 }
 
@@ -173,10 +173,10 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1))) void k_
     const double *__restrict__ bed, const double *__restrict__ B, const double *__restrict__ beta,
     const double *__restrict__ gamma, const unsigned char *__restrict__ blk, int nbx, int n_newton)
 {
-    __shared__ double eta_s[TY + 2][TX + 2];
+    __shared__ VankaLDS<TX, TY> L;
     __shared__ double cd_s[5][TY][TX];
     vanka_halo_tile<TX, TY, LOCAL>(g, p, U, Uo, f, bed, B, beta, gamma, blk, nbx, n_newton, blockIdx.x, blockIdx.y,
-                                   eta_s, cd_s);
+                                   L, cd_s);
 }
 dim3 halo_grid(int ny, int nx) { return dim3(cdiv(nx, TX - 2), cdiv(ny, TY - 2)); }
 

@@ -8,7 +8,7 @@
 // shape, so every shape gives bitwise-identical results.
 #pragma once
 
-#include "vanka_device.h"
+#include "newton_device.h"
 
 namespace glide {
 
@@ -300,65 +300,150 @@ __device__ __forceinline__ CellNbhd load_nbhd(int i, int j, int ny, int nx, size
 }
 
 // ---------------------------------------------------------------------------
-// One cell's Vanka update: neighbourhood, damped Newton iterations, and the
-// per-cell deltas (glide/cuda/vanka.cu:56-439).
-// INTERIOR: the cell lies in [1, ny-2] x [1, nx-2].  Every boundary test of
-// the assembly compares a cell index in [i-1, i+1], or a face or vertex index
-// in [i, i+1] (likewise for j), with 0 and with ny (nx); all of them take the
-// interior branch for such a cell, as they do for the cell (1, 1) of a 3 x 3
-// grid.  Passing those constants lets the compiler drop the tests; the
-// arithmetic, and so every bit of the result, is unchanged.
+// What a Vanka sweep derives per cell from its input state, staged once for
+// the tile's cells and the ring around them: 2 eta and 2 eta H (0 outside the
+// domain), and H, surface and drag (those of the clamped cell outside it).
+// Each thread then reads its neighbours' values instead of evaluating four
+// neighbour sigmoids of its own.
 // ---------------------------------------------------------------------------
-template <bool INTERIOR, class EtaFn>
-__device__ __forceinline__ void vanka_cell_deltas(const GlideGeom &g, const Params &p, const double *__restrict__ u,
-                                                  const double *__restrict__ v, const double *__restrict__ H,
-                                                  const double *__restrict__ f, const double *__restrict__ bed,
-                                                  const double *__restrict__ beta, const double *__restrict__ gamma,
-                                                  int n_newton, int i, int j, const EtaFn &E, double d5[5])
+template <int TX, int TY>
+struct VankaLDS {
+    double e2[TY + 2][TX + 2];
+    double n[TY + 2][TX + 2];
+    double H[TY + 2][TX + 2];
+    double S[TY + 2][TX + 2];
+    double be[TY + 2][TX + 2];
+};
+
+// 2 eta of cell (i, j) (eta_cell, ssa_device.h): the factors of 1/2 of the
+// corner shear rates, their mean square and eta itself are exact and ride on
+// one constant; corners on the domain edge get the factor 0.
+__device__ __forceinline__ double eta2_cell(int i, int j, const double *__restrict__ u, const double *__restrict__ v,
+                                            double Bc, const Params &p, double glen_exp, double dxi, int ny, int nx)
 {
-    const int ny = g.ny, nx = g.nx;
-    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx), nc = n_c(ny, nx);
-    const double dx_inv = 1.0 / g.dx, dt = g.dt;
-    CellNbhd N = load_nbhd(i, j, ny, nx, nu, nv, u, v, H, f, bed, beta, E);
-    nbhd_grounding(N, p);
-    const double u_l0 = ld_u(u, i, j, ny, nx), u_r0 = ld_u(u, i, j + 1, ny, nx);
-    const double v_t0 = ld_v(v, i, j, ny, nx), v_b0 = ld_v(v, i + 1, j, ny, nx);
-    const double H_c0 = ld_c(H, i, j, ny, nx), th = ld_c(gamma, i, j, ny, nx);
-    double u_l = u_l0, u_r = u_r0, v_t = v_t0, v_b = v_b0, H_c = H_c0;
-    const int ai = INTERIOR ? 1 : i, aj = INTERIOR ? 1 : j, any = INTERIOR ? 3 : ny, anx = INTERIOR ? 3 : nx;
-    for (int k = 0; k < n_newton; k++) {
-        double J[25], r[5], d[5];
-        vanka_assemble<0>(N, p, ai, aj, any, anx, dx_inv, dt, u_l, u_r, v_t, v_b, H_c, th, false, J, r);
-        lu5_solve(J, r, d);
-        u_l -= 0.25 * d[0];
-        u_r -= 0.25 * d[1];
-        v_t -= 0.25 * d[2];
-        v_b -= 0.25 * d[3];
-        H_c -= 0.25 * d[4];
-        H_c = fmax(H_c, th);
-    }
-    d5[0] = 0.5 * (u_l - u_l0);
-    d5[1] = 0.5 * (u_r - u_r0);
-    d5[2] = 0.5 * (v_t - v_t0);
-    d5[3] = 0.5 * (v_b - v_b0);
-    d5[4] = H_c - H_c0;
+    const double u_l = ld_u(u, i, j, ny, nx), u_r = ld_u(u, i, j + 1, ny, nx);
+    const double v_t = ld_v(v, i, j, ny, nx), v_b = ld_v(v, i + 1, j, ny, nx);
+    const double dudx = (u_r - u_l) * dxi, dvdy = (v_t - v_b) * dxi;
+    const bool t = i > 0, b = i < ny - 1, l = j > 0, r = j < nx - 1;
+    const double V_tl = t && l ? dxi : 0.0, V_tr = t && r ? dxi : 0.0, V_bl = b && l ? dxi : 0.0, V_br = b && r ? dxi : 0.0;
+    const double e_tl = fma(ld_u(u, i - 1, j, ny, nx) - u_l, V_tl, (v_t - ld_v(v, i, j - 1, ny, nx)) * V_tl);
+    const double e_tr = fma(ld_u(u, i - 1, j + 1, ny, nx) - u_r, V_tr, (ld_v(v, i, j + 1, ny, nx) - v_t) * V_tr);
+    const double e_bl = fma(u_l - ld_u(u, i + 1, j, ny, nx), V_bl, (v_b - ld_v(v, i + 1, j - 1, ny, nx)) * V_bl);
+    const double e_br = fma(u_r - ld_u(u, i + 1, j + 1, ny, nx), V_br, (ld_v(v, i + 1, j + 1, ny, nx) - v_b) * V_br);
+    const double e2 = fma(e_br, e_br, fma(e_bl, e_bl, fma(e_tr, e_tr, e_tl * e_tl)));
+    const double eII = fma(0.0625, e2, fma(dudx, dvdy, fma(dvdy, dvdy, dudx * dudx))) + p.eps_reg;
+    return Bc * pow_pos(eII, glen_exp);
 }
 
-template <bool INTERIOR, class EtaFn>
-__device__ __forceinline__ void vanka_cell(const GlideGeom &g, const Params &p, const double *__restrict__ u,
-                                           const double *__restrict__ v, const double *__restrict__ H,
-                                           const double *__restrict__ f, const double *__restrict__ bed,
-                                           const double *__restrict__ beta, const double *__restrict__ gamma,
-                                           int n_newton, double *__restrict__ cd, int i, int j, const EtaFn &E)
+// cells [i0-1, i0+TY] x [j0-1, j0+TX]
+template <int TX, int TY>
+__device__ __forceinline__ void vanka_stage(VankaLDS<TX, TY> &L, int i0, int j0, const double *__restrict__ u,
+                                            const double *__restrict__ v, const double *__restrict__ H,
+                                            const double *__restrict__ bed, const double *__restrict__ B,
+                                            const double *__restrict__ beta, const Params &p, double dxi, int ny, int nx)
 {
-    double d5[5];
-    vanka_cell_deltas<INTERIOR>(g, p, u, v, H, f, bed, beta, gamma, n_newton, i, j, E, d5);
-    const size_t nc = n_c(g.ny, g.nx), ci = (size_t)i * g.nx + j;
-    cd[ci] = d5[0];
-    cd[nc + ci] = d5[1];
-    cd[2 * nc + ci] = d5[2];
-    cd[3 * nc + ci] = d5[3];
-    cd[4 * nc + ci] = d5[4];
+    const int tid = threadIdx.y * TX + threadIdx.x;
+    const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+    for (int k = tid; k < (TY + 2) * (TX + 2); k += TX * TY) {
+        const int a = k / (TX + 2), b = k - a * (TX + 2);
+        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
+        const int ic = clampi(ci, 0, ny - 1), jc = clampi(cj, 0, nx - 1);
+        const size_t kc = (size_t)ic * nx + jc;
+        const double h = H[kc], bd = bed[kc];
+        const double e2 = ic == ci && jc == cj ? eta2_cell(ci, cj, u, v, B[kc], p, glen_exp, dxi, ny, nx) : 0.0;
+        const double g = sigm_mid(fma(0.917, h, bd), p.gl_c);
+        L.e2[a][b] = e2;
+        L.n[a][b] = e2 * h;
+        L.H[a][b] = h;
+        L.S[a][b] = fmax(bd, -0.917 * h) + h;
+        L.be[a][b] = fma(g, beta[kc], (1.0 - g) * p.water_drag);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// One cell's Vanka update (glide/cuda/vanka.cu:56-439): its neighbourhood
+// (a, b index the staged arrays), n_newton damped Newton iterations
+// (newton_step) and the per-cell deltas.  INTERIOR: the cell lies in
+// [1, ny-2] x [1, nx-2], so no read is clamped and no term vanishes.
+// ---------------------------------------------------------------------------
+template <bool INTERIOR, int TX, int TY>
+__device__ __forceinline__ void vanka_cell_deltas(const GlideGeom &g, const Params &p, const NewtonK &K,
+                                                  const VankaLDS<TX, TY> &L, int a, int b,
+                                                  const double *__restrict__ u, const double *__restrict__ v,
+                                                  const double *__restrict__ f, const double *__restrict__ bed,
+                                                  const double *__restrict__ beta, const double *__restrict__ gamma,
+                                                  int n_newton, int i, int j, double d5[5])
+{
+    const int ny = g.ny, nx = g.nx;
+    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+    // offsets of the rows above, at and below, and of the columns around (clamped at the edge)
+    auto row = [&](int q, int hi) { return INTERIOR ? q : clampi(q, 0, hi); };
+    const double *u0 = u + (size_t)i * (nx + 1), *ut = u + (size_t)row(i - 1, ny - 1) * (nx + 1),
+                 *ub = u + (size_t)row(i + 1, ny - 1) * (nx + 1);
+    const double *v0 = v + (size_t)i * nx, *v1 = v + (size_t)(i + 1) * nx, *vt = v + (size_t)row(i - 1, ny) * nx,
+                 *vb = v + (size_t)row(i + 2, ny) * nx;
+    const int jl = row(j - 1, nx - 1), jr = row(j + 1, nx - 1), jrr = row(j + 2, nx);
+    NewtonX x;
+    x.u_l = u0[j];
+    x.u_r = u0[j + 1];
+    x.v_t = v0[j];
+    x.v_b = v1[j];
+    x.H = L.H[a][b];
+    const NewtonX x0 = x;
+    NewtonCell C;
+    C.u_ll = u0[row(j - 1, nx)];
+    C.u_rr = u0[jrr];
+    C.u_tl = ut[j];
+    C.u_tr = ut[j + 1];
+    C.u_bl = ub[j];
+    C.u_br = ub[j + 1];
+    C.v_lt = v0[jl];
+    C.v_lb = v1[jl];
+    C.v_rt = v0[jr];
+    C.v_rb = v1[jr];
+    C.v_tt = vt[j];
+    C.v_bb = vb[j];
+    const size_t ku = (size_t)i * (nx + 1) + j, kv = nu + (size_t)i * nx + j, kc = (size_t)i * nx + j;
+    C.f0 = f[ku];
+    C.f1 = f[ku + 1];
+    C.f2 = f[kv];
+    C.f3 = f[kv + nx];
+    C.f4 = f[kv + nv];
+    C.bed = bed[kc];
+    C.beta = beta[kc];
+    C.th = gamma[kc];
+    C.e2 = L.e2[a][b];
+    C.n_l = L.n[a][b - 1];
+    C.n_r = L.n[a][b + 1];
+    C.n_t = L.n[a - 1][b];
+    C.n_b = L.n[a + 1][b];
+    C.p_tl = (L.n[a - 1][b - 1] + C.n_t) + C.n_l;
+    C.p_tr = C.n_t + L.n[a - 1][b + 1];
+    C.n_bl = L.n[a + 1][b - 1];
+    C.n_br = L.n[a + 1][b + 1];
+    C.H_l = L.H[a][b - 1];
+    C.H_r = L.H[a][b + 1];
+    C.H_t = L.H[a - 1][b];
+    C.H_b = L.H[a + 1][b];
+    C.S_l = L.S[a][b - 1];
+    C.S_r = L.S[a][b + 1];
+    C.S_t = L.S[a - 1][b];
+    C.S_b = L.S[a + 1][b];
+    C.be_l = L.be[a][b - 1];
+    C.be_r = L.be[a][b + 1];
+    C.be_t = L.be[a - 1][b];
+    C.be_b = L.be[a + 1][b];
+    C.c_l = (C.v_lt - C.v_lb) * K.dxi;
+    C.c_r = (C.v_rt - C.v_rb) * K.dxi;
+    C.d_t = C.u_tr - C.u_tl;
+    C.d_b = C.u_br - C.u_bl;
+    newton_edges<INTERIOR>(C, K, i, j, ny, nx);
+    for (int k = 0; k < n_newton; k++) newton_step(C, K, p, x);
+    d5[0] = 0.5 * (x.u_l - x0.u_l);
+    d5[1] = 0.5 * (x.u_r - x0.u_r);
+    d5[2] = 0.5 * (x.v_t - x0.v_t);
+    d5[3] = 0.5 * (x.v_b - x0.v_b);
+    d5[4] = x.H - x0.H;
 }
 
 // ---------------------------------------------------------------------------
@@ -372,13 +457,14 @@ __device__ __forceinline__ void vanka_tile(const GlideGeom &g, const Params &p, 
                                            const double *__restrict__ B, const double *__restrict__ beta,
                                            const double *__restrict__ gamma, const unsigned char *__restrict__ blk,
                                            int nbx, int n_newton, double *__restrict__ cd, int bx, int by,
-                                           double (*eta_s)[TX + 2])
+                                           VankaLDS<TX, TY> &L)
 {
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx), nc = n_c(ny, nx);
     const double *u = U, *v = U + nu, *H = U + nu + nv;
     const int i0 = by * TY, j0 = bx * TX;
-    const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
+    const int a = threadIdx.y + 1, b = threadIdx.x + 1;
+    const int i = i0 - 1 + a, j = j0 - 1 + b;
     const bool mine = (i < ny && j < nx);
     // A local sweep smooths every cell of a tile that holds an active cell:
     // the apply pass reads only the active cells' updates, so the idle
@@ -388,18 +474,21 @@ __device__ __forceinline__ void vanka_tile(const GlideGeom &g, const Params &p, 
     if (LOCAL) {
         if (!__syncthreads_or(mine && blk[(i / RB) * nbx + j / RB])) return;   // uniform: the whole tile is idle
     }
-    fill_eta_tile<TX, TY>(eta_s, i0, j0, u, v, B, p, g.dx, ny, nx);
+    const NewtonK K = newton_constants(g.dx, g.dt);
+    vanka_stage<TX, TY>(L, i0, j0, u, v, H, bed, B, beta, p, K.dxi, ny, nx);
     __syncthreads();
     if (!mine) return;
-    auto E = [&](int ci, int cj) { return eta_s[ci - i0 + 1][cj - j0 + 1]; };
-    // A tile whose cells all lie in [1, ny-2] x [1, nx-2] runs the cell
-    // with its boundary tests resolved at compile time (same bits).  The
-    // whole per-cell body is instantiated twice so that no value is live
-    // across the branch.
+    // A tile whose cells all lie in [1, ny-2] x [1, nx-2] runs the interior
+    // form (same bits).  The whole per-cell body is instantiated twice so
+    // that no value is live across the branch.
+    double d5[5];
     if (i0 >= 1 && i0 + TY <= ny - 1 && j0 >= 1 && j0 + TX <= nx - 1)
-        vanka_cell<true>(g, p, u, v, H, f, bed, beta, gamma, n_newton, cd, i, j, E);
+        vanka_cell_deltas<true>(g, p, K, L, a, b, u, v, f, bed, beta, gamma, n_newton, i, j, d5);
     else
-        vanka_cell<false>(g, p, u, v, H, f, bed, beta, gamma, n_newton, cd, i, j, E);
+        vanka_cell_deltas<false>(g, p, K, L, a, b, u, v, f, bed, beta, gamma, n_newton, i, j, d5);
+    const size_t ci = (size_t)i * nx + j;
+#pragma unroll
+    for (int q = 0; q < 5; q++) cd[q * nc + ci] = d5[q];
 }
 
 // Gather the per-cell updates: U += 0.5 * delta (glide/grid.py:305-317)
@@ -450,7 +539,7 @@ __device__ __forceinline__ void vanka_halo_tile(const GlideGeom &g, const Params
                                                 const double *__restrict__ bed, const double *__restrict__ B,
                                                 const double *__restrict__ beta, const double *__restrict__ gamma,
                                                 const unsigned char *__restrict__ blk, int nbx, int n_newton, int bx,
-                                                int by, double (*eta_s)[TX + 2], double (*cd_s)[TY][TX])
+                                                int by, VankaLDS<TX, TY> &L, double (*cd_s)[TY][TX])
 {
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
@@ -464,16 +553,17 @@ __device__ __forceinline__ void vanka_halo_tile(const GlideGeom &g, const Params
     bool run = true;
     if (LOCAL) run = __syncthreads_or(in && act(i, j));   // uniform
     if (run) {
-        fill_eta_tile<TX, TY>(eta_s, i0 - 1, j0 - 1, u, v, B, p, g.dx, ny, nx);
+        const NewtonK K = newton_constants(g.dx, g.dt);
+        vanka_stage<TX, TY>(L, i0 - 1, j0 - 1, u, v, H, bed, B, beta, p, K.dxi, ny, nx);
         __syncthreads();
         const int ic = min(max(i, 0), ny - 1), jc = min(max(j, 0), nx - 1);
-        auto E = [&](int ci, int cj) { return eta_s[ci - i0 + 2][cj - j0 + 2]; };
+        const int la = ic - i0 + 2, lb = jc - j0 + 2;   // the cell in the staged arrays
         double d5[5];
-        // every run cell in [1, ny-2] x [1, nx-2]: the boundary tests resolved at compile time
+        // every run cell in [1, ny-2] x [1, nx-2]: the interior form
         if (i0 >= 2 && i0 + TY <= ny && j0 >= 2 && j0 + TX <= nx)
-            vanka_cell_deltas<true>(g, p, u, v, H, f, bed, beta, gamma, n_newton, ic, jc, E, d5);
+            vanka_cell_deltas<true>(g, p, K, L, la, lb, u, v, f, bed, beta, gamma, n_newton, ic, jc, d5);
         else
-            vanka_cell_deltas<false>(g, p, u, v, H, f, bed, beta, gamma, n_newton, ic, jc, E, d5);
+            vanka_cell_deltas<false>(g, p, K, L, la, lb, u, v, f, bed, beta, gamma, n_newton, ic, jc, d5);
 #pragma unroll
         for (int q = 0; q < 5; q++) cd_s[q][a][b] = d5[q];
         __syncthreads();

@@ -174,80 +174,175 @@ __global__ __launch_bounds__(256) void k_conv3x3(const bf16_t *__restrict__ xa, 
 
 // ---------------------------------------------------------------------------
 // Weight gradient: partial[z][t][co][ci] = sum over the z-th pixel chunk of
-// dz[p][co] * x[p + off_t][ci]; one block = 64 co x 64 ci of one tap.
+// dz[p][co] * x[p + off_t][ci]; one block = 32 co x 32 ci of all nine taps.
+//
+// A GEMM with K = pixels, whose operands lie channel-contiguous in memory: the
+// block stages WG_PX pixels of dz and of the three image rows of x around them
+// in LDS as they lie (16-byte stores), and ds_read_b64_tr_b16 hands each lane
+// the four consecutive pixels of its channel that a fragment needs.  A tap's
+// column shift is a row offset into the staged pixels, so x is read from
+// memory once for its nine taps.  Wave w takes the three taps of image row
+// w - 1: per 32 pixels it reads 2 dz and 6 x fragments for 12 MFMAs.  The
+// pitch of 96 bytes puts the four pixels that 16 lanes read in different
+// banks.  Every (tap, co, ci) sums its chunk in steps of 32 pixels in pixel
+// order, so the bits depend on neither the tile nor the grid.
+//
+// Bound by LDS reads (16 of 512 bytes per wave and step against 12 MFMAs of
+// 16 cycles).  One tap per block and 2-byte transposing stores took 5.0 ms of
+// a 16 x 256^2 training step for its 13 layers; this takes 1.1 ms.
 // ---------------------------------------------------------------------------
-constexpr int WG_K = 32;          // pixels per K step
-constexpr int WG_LD = WG_K + 8;   // LDS row pitch (bf16), breaks bank conflicts
+constexpr int WG_PX = 128;   // pixels per staged tile
+constexpr int WG_LD = 48;    // LDS pitch of a pixel's 32 channels (bf16)
 
-__global__ __launch_bounds__(256) void k_conv3x3_wgrad(const bf16_t *__restrict__ dz, int Cout,
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+
+// the 8 pixels [0, 8) from row t (pitch WG_LD) of channel `16-lane group's
+// first channel + r16`, in pixel order; t: the lane's row + 4-channel group
+__device__ __forceinline__ Frag tr_frag(const bf16_t *t)
+{
+    union {
+        s16x4 h[2];
+        Frag f;
+    } u;
+    u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)t);
+    u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(t + 4 * WG_LD));
+    return u.f;
+}
+
+__global__ __launch_bounds__(192) void k_conv3x3_wgrad(const bf16_t *__restrict__ dz, int Cout,
                                                        const bf16_t *__restrict__ xa, int CA,
                                                        const bf16_t *__restrict__ xb, int CB, int N, int H, int W,
                                                        long chunk, float *__restrict__ partial)
 {
-    __shared__ bf16_t sA[64][WG_LD];   // [co][pixel]
-    __shared__ bf16_t sB[64][WG_LD];   // [ci][pixel]
+    __shared__ bf16_t sD[WG_PX][WG_LD];          // dz of pixel p0 + k
+    __shared__ bf16_t sX[3][WG_PX + 2][WG_LD];   // x of pixel p0 - 1 + k, image row dy = -1, 0, 1
     const int Cin = CA + CB;
-    const int nco = (Cout + 63) / 64;
-    const int t = blockIdx.y / nco, cog = blockIdx.y % nco;
-    const int co0 = cog * 64, ci0 = blockIdx.x * 64;
-    const int dy = t / 3 - 1, dx = t % 3 - 1;
-    const long P = (long)N * H * W;
+    const int ci0 = blockIdx.x * 32, co0 = blockIdx.y * 32;
+    const long P = (long)N * H * W, HW = (long)H * W;
     const long p_lo = (long)blockIdx.z * chunk, p_hi = p_lo + chunk < P ? p_lo + chunk : P;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, dy = w - 1;
     const int r16 = lane & 15, kq = lane >> 4;
-    const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;   // wave's 32 x 32 sub-tile
-    f32x4 acc[2][2];
+    const bf16_t *xs = ci0 < CA ? xa + ci0 : xb + (ci0 - CA);
+    const int cs = ci0 < CA ? CA : CB;
+    constexpr int NX = ((WG_PX + 2) * 4 + 63) / 64;   // 16-byte pieces of the wave's x row per lane
+    constexpr int ND = (WG_PX * 4 + 191) / 192;       // ... and of dz per thread
+    uint4 rx[NX], rd[ND];
+    // position in its image of the staged x row's first pixel; its rows above
+    // (dy = -1) and below (dy = 1) the image are zero
+    long r0 = ((p_lo - 1 + (long)dy * W) % HW + HW) % HW;
+    const long bad_lo = dy < 0 ? HW - W : 0, bad_n = dy == 0 ? 0 : W;
+    auto load = [&](long p0) {
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+        for (int m = 0; m < NX; m++) {
+            const int s = (lane >> 2) + 16 * m;
+            const long q = p0 - 1 + (long)dy * W + s;
+            long r = r0 + s;
+            while (r >= HW) r -= HW;
+            const bool ok = s < WG_PX + 2 && q >= 0 && q < P && !(r >= bad_lo && r < bad_lo + bad_n);
+            rx[m] = ok ? *(const uint4 *)(xs + q * cs + 8 * (lane & 3)) : uint4{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
-        for (int b = 0; b < 2; b++) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // staging: thread -> (pixel row kk = tid / 8, 8-channel group g = tid % 8)
-    const int kk = tid >> 3, g = tid & 7;
-    for (long p0 = p_lo; p0 < p_hi; p0 += WG_K) {
-        const long p = p0 + kk;
-        uint4 va = uint4{0u, 0u, 0u, 0u}, vb = uint4{0u, 0u, 0u, 0u};
-        if (p < p_hi) {
-            if (co0 + 8 * g < Cout) va = *(const uint4 *)(dz + p * Cout + co0 + 8 * g);
-            const int x = (int)(p % W);
-            const long q = p / W;
-            const int y = (int)(q % H), n = (int)(q / H);
-            const int ys = y + dy, xs = x + dx;
-            const int c = ci0 + 8 * g;
-            if (ys >= 0 && ys < H && xs >= 0 && xs < W && c < Cin) {
-                const long s = ((long)n * H + ys) * W + xs;
-                vb = c < CA ? *(const uint4 *)(xa + s * CA + c) : *(const uint4 *)(xb + s * CB + (c - CA));
-            }
+        for (int m = 0; m < ND; m++) {
+            const int e = tid + 192 * m;
+            const long p = p0 + (e >> 2);
+            const bool ok = e < WG_PX * 4 && p < p_hi;
+            rd[m] = ok ? *(const uint4 *)(dz + p * Cout + co0 + 8 * (e & 3)) : uint4{0u, 0u, 0u, 0u};
+        }
+        r0 += WG_PX;
+        while (r0 >= HW) r0 -= HW;
+    };
+    f32x4 acc[3][2][2];
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int b = 0; b < 2; b++) acc[d][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // column of the lane's first pixel (8 kq past the step's first)
+    int col = (int)((p_lo + 8 * kq) % W);
+    const int cstep = 32 % W;
+    // the lane's corner of a fragment at step 0: pixel 8 kq + r16 / 4, channels 4 (r16 % 4)
+    const int fo = (8 * kq + (r16 >> 2)) * WG_LD + 4 * (r16 & 3);
+    load(p_lo);
+    for (long p0 = p_lo; p0 < p_hi; p0 += WG_PX) {
+        __syncthreads();   // the previous tile has been read
+#pragma unroll
+        for (int m = 0; m < NX; m++) {
+            const int s = (lane >> 2) + 16 * m;
+            if (s < WG_PX + 2) *(uint4 *)&sX[w][s][8 * (lane & 3)] = rx[m];
+        }
+#pragma unroll
+        for (int m = 0; m < ND; m++) {
+            const int e = tid + 192 * m;
+            if (e < WG_PX * 4) *(uint4 *)&sD[e >> 2][8 * (e & 3)] = rd[m];
         }
         __syncthreads();
-        const bf16_t *ea = (const bf16_t *)&va, *eb = (const bf16_t *)&vb;
+        if (p0 + WG_PX < p_hi) load(p0 + WG_PX);
+        // 8 consecutive pixels lie in one image row where W % 8 == 0 (chunks start at multiples of 8)
+        const bool plain = (W & 7) == 0 && p0 + WG_PX <= p_hi;
+#pragma unroll 1
+        for (int st = 0; st < WG_PX / 32; st++) {
+            if (p0 + 32 * st >= p_hi) break;
+            const int o = fo + 32 * st * WG_LD;
+            Frag A[2], B[3][2];
 #pragma unroll
-        for (int e = 0; e < 8; e++) {
-            sA[8 * g + e][kk] = ea[e];
-            sB[8 * g + e][kk] = eb[e];
-        }
-        __syncthreads();
+            for (int a = 0; a < 2; a++) A[a] = tr_frag(&sD[0][0] + o + 16 * a);
 #pragma unroll
-        for (int a = 0; a < 2; a++) {
-            Frag A;
-            A.raw = *(const uint4 *)&sA[wm + 16 * a + r16][8 * kq];
+            for (int d = 0; d < 3; d++)
 #pragma unroll
-            for (int b = 0; b < 2; b++) {
-                Frag B;
-                B.raw = *(const uint4 *)&sB[wn + 16 * b + r16][8 * kq];
-                acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A.v, B.v, acc[a][b], 0, 0, 0);
+                for (int b = 0; b < 2; b++) B[d][b] = tr_frag(&sX[w][0][0] + o + d * WG_LD + 16 * b);
+            // x is 0 left of column 0 (tap dx = -1) and right of column W - 1 (dx = 1)
+            if (plain) {
+                const uint32_t ml = col == 0 ? 0xffff0000u : 0xffffffffu, mr = col == W - 8 ? 0x0000ffffu : 0xffffffffu;
+#pragma unroll
+                for (int b = 0; b < 2; b++) {
+                    B[0][b].raw.x &= ml;
+                    B[2][b].raw.w &= mr;
+                }
+            } else {
+                uint32_t m[3][4] = {};
+                int c = col;
+#pragma unroll
+                for (int e = 0; e < 8; e++) {
+                    const uint32_t h = p0 + 32 * st + 8 * kq + e < p_hi ? 0xffffu << (16 * (e & 1)) : 0u;
+                    m[0][e >> 1] |= c > 0 ? h : 0u;
+                    m[1][e >> 1] |= h;
+                    m[2][e >> 1] |= c < W - 1 ? h : 0u;
+                    c = c + 1 == W ? 0 : c + 1;
+                }
+#pragma unroll
+                for (int d = 0; d < 3; d++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++) {
+                        B[d][b].raw.x &= m[d][0];
+                        B[d][b].raw.y &= m[d][1];
+                        B[d][b].raw.z &= m[d][2];
+                        B[d][b].raw.w &= m[d][3];
+                    }
             }
+            col += cstep;
+            col = col >= W ? col - W : col;
+#pragma unroll
+            for (int d = 0; d < 3; d++)
+#pragma unroll
+                for (int a = 0; a < 2; a++)
+#pragma unroll
+                    for (int b = 0; b < 2; b++)
+                        acc[d][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a].v, B[d][b].v, acc[d][a][b], 0, 0, 0);
         }
     }
-    float *dst = partial + ((long)blockIdx.z * 9 + t) * Cout * Cin;
 #pragma unroll
-    for (int a = 0; a < 2; a++)
+    for (int d = 0; d < 3; d++) {
+        float *dst = partial + ((long)blockIdx.z * 9 + 3 * w + d) * Cout * Cin;
 #pragma unroll
-        for (int b = 0; b < 2; b++)
+        for (int a = 0; a < 2; a++)
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int co = co0 + wm + 16 * a + 4 * kq + i, ci = ci0 + wn + 16 * b + r16;
-                if (co < Cout && ci < Cin) dst[(long)co * Cin + ci] = acc[a][b][i];
-            }
+            for (int b = 0; b < 2; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    dst[(long)(co0 + 16 * a + 4 * kq + i) * Cin + ci0 + 16 * b + r16] = acc[d][a][b][i];
+    }
 }
 
 // out[k] = sum_z partial[z][k] in z order
@@ -761,8 +856,8 @@ int glide_unet_conv3x3_wgrad(const uint16_t *dz, int Cout, const uint16_t *xa, i
     const long P = (long)N * H * W, chunk = 4096;
     const long nz = glide_unet_wgrad_chunks(N, H, W);
     const int Cin = CA + CB;
-    dim3 grid((Cin + 63) / 64, 9 * ((Cout + 63) / 64), (unsigned)nz);
-    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(256), 0, SS(stream), dz, Cout, xa, CA, xb, CB, N, H, W, chunk,
+    dim3 grid(Cin / 32, Cout / 32, (unsigned)nz);
+    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(192), 0, SS(stream), dz, Cout, xa, CA, xb, CB, N, H, W, chunk,
                        partial);
     const long n = 9L * Cout * Cin;
     hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(n)), dim3(256), 0, SS(stream), partial, n, (int)nz, dw);

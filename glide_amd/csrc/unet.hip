@@ -71,14 +71,169 @@ union Frag {
 //        x = concat(xa (CA ch), xb (CB ch)); act = ReLU when relu != 0.
 // MODE 1 (data gradient): the same sum without bias/act into FP32 outputs split
 //        by channel: co < SA -> ga[p][co] (+)= ..., else gb[p][co - SA] (+)= ...
-// Grid: x = pixel blocks of 256 (4 waves x 64), y = output-channel groups of 16*NJ.
+//
+// A workgroup of NW waves owns 2 NW rows x 32 columns of one image x 32 output
+// channels: it stages the (2 NW + 2) x 34 input pixels of every channel (NCH
+// chunks of 32) in LDS once (zero outside the image), so the nine taps read
+// memory once, and a wave takes 2 rows (4 MFMA blocks of 16 pixels).  An LDS
+// pixel is 32 channels at a pitch of 80 bytes, which puts the 16-byte reads of
+// 8 consecutive pixels in different banks.  Weight fragments come from the
+// caches, three steps ahead.  The weights are the MFMA's row operand, in an
+// order that leaves a lane with 8 consecutive output channels of its pixel:
+// one 16-byte store (two for FP32) instead of 8 of 2 bytes.  The K loop walks
+// the 9 taps x 32-channel chunks in that order whatever the tile, so the sums'
+// bits do not depend on it.
+//
+// Balance per step: a wave issues 4 LDS reads and 2 weight loads of 1 KB for 8
+// MFMAs of 16 cycles, about what LDS and L1 deliver to four waves in that
+// time.  Reading the pixels of every tap from the caches and storing 2 bytes
+// at a time took 30 us for 512^2 pixels of 32 -> 32 channels; this takes 13 us
+// (7 us at the rate of a large copy).
 // ---------------------------------------------------------------------------
+constexpr int CV_W = 32;      // tile columns
+constexpr int CV_LD = 40;     // LDS pitch of a pixel's 32 channels (bf16)
+
+// f2bf without the NaN case (a NaN becomes some other value)
+__device__ __forceinline__ uint32_t f2bf_num(float f)
+{
+    uint32_t u;
+    __builtin_memcpy(&u, &f, 4);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+
+template <int NW, int NCH, int MODE>
+__global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ xa, int CA,
+                                                     const bf16_t *__restrict__ xb, int H, int W, int tiles_x,
+                                                     int tiles, const bf16_t *__restrict__ Wt, int Cout,
+                                                     const float *__restrict__ bias, int relu,
+                                                     bf16_t *__restrict__ out, float *__restrict__ ga, int SA,
+                                                     int acc_a, float *__restrict__ gb, int acc_b)
+{
+    constexpr int PW = CV_W + 2, NPX = (2 * NW + 2) * PW, Cin = 32 * NCH;
+    __shared__ bf16_t sm[NCH * NPX * CV_LD];   // [chunk][pixel][CV_LD]
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, kq = lane >> 4;   // fragment row / k-quarter
+    const int n = blockIdx.x / tiles, tl = blockIdx.x - n * tiles;
+    const int y0 = (tl / tiles_x) * 2 * NW, x0 = (tl % tiles_x) * CV_W;
+    const int co0 = blockIdx.y * 32;
+    const long img = (long)n * H * W;
+
+    // weight fragments of step (t, c): row m of fragment j is channel co0 + 8 (m / 4) + 4 j + m % 4
+    const uint32_t wlane = ((co0 + 8 * (r16 >> 2) + (r16 & 3)) * Cin + 8 * kq) * 2u;
+    const long tap = (long)Cout * Cin * 2;
+    auto wload = [&](int t, int c, Frag(&B)[2]) {
+        const char *b = (const char *)Wt + t * tap + 64 * c;
+        B[0].raw = *(const uint4 *)(b + wlane);
+        B[1].raw = *(const uint4 *)(b + 8 * Cin + wlane);
+    };
+    Frag B[3][2];
+#pragma unroll
+    for (int s = 0; s < 3; s++) wload(s / NCH, s % NCH, B[s]);
+
+    // stage the input: 16-byte pieces, 4 per pixel and chunk
+    constexpr int NE = (NPX * 4 + 64 * NW - 1) / (64 * NW), NB = NCH > 2 ? 2 : 4;   // pieces per thread, in flight x NCH
+    const int CB = Cin - CA, ncha = CA / 32;
+#pragma unroll
+    for (int e0 = 0; e0 < NE; e0 += NB) {
+        uint4 v[NB][NCH];
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const int e = tid + 64 * NW * (e0 + k), px = e >> 2, q = e & 3;
+            const int ry = px / PW, rx = px - ry * PW;
+            const int y = y0 - 1 + ry, x = x0 - 1 + rx;
+            const bool ok = e < NPX * 4 && y >= 0 && y < H && x >= 0 && x < W;
+            const long p = img + (long)y * W + x;
+            const bf16_t *a = xa + p * CA + 8 * q, *b = xb + p * CB + 8 * q;
+#pragma unroll
+            for (int c = 0; c < NCH; c++)
+                v[k][c] = ok ? *(const uint4 *)(c < ncha ? a + 32 * c : b + 32 * (c - ncha)) : uint4{0u, 0u, 0u, 0u};
+        }
+#pragma unroll
+        for (int k = 0; k < NB; k++) {
+            const int e = tid + 64 * NW * (e0 + k);
+            if (e < NPX * 4) {
+#pragma unroll
+                for (int c = 0; c < NCH; c++) *(uint4 *)(sm + (c * NPX + (e >> 2)) * CV_LD + 8 * (e & 3)) = v[k][c];
+            }
+        }
+    }
+    __syncthreads();
+
+    f32x4 acc[4][2];
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int j = 0; j < 2; j++) acc[a][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // pixel block a: row 2 wave + a / 2, columns 16 (a % 2) + r16
+    const bf16_t *base = sm + (2 * wave * PW + r16) * CV_LD + 8 * kq;
+#pragma unroll 1
+    for (int dy = 0; dy < 3; dy++) {
+#pragma unroll
+        for (int s = 0; s < 3 * NCH; s++) {   // step 3 NCH dy + s: tap 3 dy + s / NCH, chunk s % NCH
+            const bf16_t *p = base + (s / NCH + s % NCH * NPX) * CV_LD;
+            Frag A[4];
+#pragma unroll
+            for (int a = 0; a < 4; a++) A[a].raw = *(const uint4 *)(p + ((a >> 1) * PW + 16 * (a & 1)) * CV_LD);
+#pragma unroll
+            for (int j = 0; j < 2; j++)
+#pragma unroll
+                for (int a = 0; a < 4; a++)
+                    acc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[s % 3][j].v, A[a].v, acc[a][j], 0, 0, 0);
+            const int q = s + 3;   // past the last step: the last tap again
+            const int t = 3 * dy + q / NCH;
+            wload(t < 9 ? t : 8, q % NCH, B[s % 3]);
+        }
+        base += PW * CV_LD;
+    }
+
+    // D fragment: row 4*kq + i of fragment j = channel co0 + 8*kq + 4*j + i, column r16 = pixel
+    const int co = co0 + 8 * kq;
+    float bs[8] = {};
+    if (MODE == 0) {
+        const float4 b0 = *(const float4 *)(bias + co), b1 = *(const float4 *)(bias + co + 4);
+        bs[0] = b0.x, bs[1] = b0.y, bs[2] = b0.z, bs[3] = b0.w, bs[4] = b1.x, bs[5] = b1.y, bs[6] = b1.z, bs[7] = b1.w;
+    }
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        const int y = y0 + 2 * wave + (a >> 1), x = x0 + 16 * (a & 1) + r16;
+        if (y >= H || x >= W) continue;
+        const long p = img + (long)y * W + x;
+        if (MODE == 0) {
+            uint32_t h[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float val = acc[a][i >> 2][i & 3] + bs[i];
+                h[i] = relu ? f2bf_num(fmaxf(val, 0.0f)) : (uint32_t)f2bf(val);   // fmaxf leaves no NaN
+            }
+            *(uint4 *)(out + p * Cout + co) =
+                uint4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+        } else {
+            const bool first = co0 < SA;   // 32-channel groups lie in one of the outputs
+            float4 *d = (float4 *)(first ? ga + p * SA + co : gb + p * (Cout - SA) + (co - SA));
+            float4 v0 = {acc[a][0][0], acc[a][0][1], acc[a][0][2], acc[a][0][3]};
+            float4 v1 = {acc[a][1][0], acc[a][1][1], acc[a][1][2], acc[a][1][3]};
+            if (first ? acc_a : acc_b) {
+                const float4 o0 = d[0], o1 = d[1];
+                v0 = float4{o0.x + v0.x, o0.y + v0.y, o0.z + v0.z, o0.w + v0.w};
+                v1 = float4{o1.x + v1.x, o1.y + v1.y, o1.z + v1.z, o1.w + v1.w};
+            }
+            d[0] = v0;
+            d[1] = v1;
+        }
+    }
+}
+
+// The same convolution reading every tap's pixels from the caches, for input
+// channel counts that k_conv3x3 has no instance for (160, and above 192, whose
+// halo tile outgrows its LDS): a wave owns 64 consecutive pixels x 16 NJ
+// channels.  Grid: x = pixel blocks of 256 (4
+// waves x 64), y = output-channel groups of 16 NJ.  The same sums, bit for bit.
 template <int NJ, int MODE>
-__global__ __launch_bounds__(256) void k_conv3x3(const bf16_t *__restrict__ xa, int CA, const bf16_t *__restrict__ xb,
-                                                 int CB, int N, int H, int W, const bf16_t *__restrict__ Wt, int Cout,
-                                                 const float *__restrict__ bias, int relu, bf16_t *__restrict__ out,
-                                                 float *__restrict__ ga, int SA, int acc_a, float *__restrict__ gb,
-                                                 int acc_b)
+__global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict__ xa, int CA, const bf16_t *__restrict__ xb,
+                                                        int CB, int N, int H, int W, const bf16_t *__restrict__ Wt, int Cout,
+                                                        const float *__restrict__ bias, int relu, bf16_t *__restrict__ out,
+                                                        float *__restrict__ ga, int SA, int acc_a, float *__restrict__ gb,
+                                                        int acc_b)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int Cin = CA + CB;
@@ -788,7 +943,8 @@ inline hipStream_t SS(void *s) { return (hipStream_t)s; }
 bool bad_ch(int c) { return c < 0 || c % 32 != 0 || c > 4096; }
 // 8-channel (16-byte) accesses apply: C % 8 == 0 and both tensors 16-byte aligned
 bool vec8(int C, const void *a, const void *b) { return C % 8 == 0 && (((uintptr_t)a | (uintptr_t)b) & 15) == 0; }
-// Output channels per wave (16 * NJ) of a 3x3 convolution over P pixels: the
+// Output channels per wave (16 * NJ) of the direct 3x3 convolution over P
+// pixels: the
 // widest of 64, 32 and 16 that still gives at least 2048 waves (two per
 // SIMD), else 16.  Small levels are bound by each wave's serial K loop, so
 // they take more, narrower waves; large ones keep the input fragments'
@@ -800,6 +956,74 @@ int conv_nj(long P, int C)
         if (C % (16 * nj) == 0 && pw * (C / (16 * nj)) >= 2048) return nj;
     return 1;
 }
+// LDS bytes of a workgroup of nw waves
+constexpr size_t conv_lds(int nw, int nch) { return (size_t)nch * (2 * nw + 2) * (CV_W + 2) * CV_LD * sizeof(bf16_t); }
+
+struct ConvArgs {
+    const bf16_t *xa;
+    int CA;
+    const bf16_t *xb;
+    int CB, N, H, W;
+    const bf16_t *Wt;
+    int Cout;
+    const float *bias;
+    int relu;
+    bf16_t *out;
+    float *ga;
+    int SA, acc_a;
+    float *gb;
+    int acc_b;
+};
+
+template <int NW, int NCH, int MODE>
+void conv_launch(const ConvArgs &c, hipStream_t st)
+{
+    const int tx = (c.W + CV_W - 1) / CV_W, tiles = tx * ((c.H + 2 * NW - 1) / (2 * NW));
+    hipLaunchKernelGGL((k_conv3x3<NW, NCH, MODE>), dim3((unsigned)((long)tiles * c.N), c.Cout / 32), dim3(64 * NW), 0,
+                       st, c.xa, c.CA, c.xb, c.H, c.W, tx, tiles, c.Wt, c.Cout, c.bias, c.relu, c.out, c.ga, c.SA,
+                       c.acc_a, c.gb, c.acc_b);
+}
+// Waves per workgroup (tile rows / 2): the tallest tile reads the fewest halo
+// rows, so 4 where that still gives a workgroup per CU and the input fits 64
+// KB of LDS, else 2, else 1.
+template <int NCH, int MODE>
+void conv_staged(const ConvArgs &c, hipStream_t st)
+{
+    auto wgs = [&](int nw) {
+        return (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * nw - 1) / (2 * nw)) * c.N * (c.Cout / 32);
+    };
+    if constexpr (conv_lds(4, NCH) <= 64 * 1024)
+        if (wgs(4) >= 256) return conv_launch<4, NCH, MODE>(c, st);
+    if constexpr (conv_lds(2, NCH) <= 64 * 1024)
+        if (wgs(2) >= 256) return conv_launch<2, NCH, MODE>(c, st);
+    conv_launch<1, NCH, MODE>(c, st);
+}
+template <int NJ, int MODE>
+void conv_direct(const ConvArgs &c, hipStream_t st)
+{
+    hipLaunchKernelGGL((k_conv3x3_direct<NJ, MODE>), dim3(nblk((long)c.N * c.H * c.W), c.Cout / (16 * NJ)), dim3(256), 0,
+                       st, c.xa, c.CA, c.xb, c.CB, c.N, c.H, c.W, c.Wt, c.Cout, c.bias, c.relu, c.out, c.ga, c.SA,
+                       c.acc_a, c.gb, c.acc_b);
+}
+// The channel counts of the network's layers have a staged instance.  It reads
+// the bias and stores in 16-byte pieces, which the direct kernel does not: a
+// tensor off that alignment takes the direct kernel.
+template <int MODE>
+void conv(const ConvArgs &c, hipStream_t st)
+{
+    const uintptr_t al = (uintptr_t)c.bias | (uintptr_t)c.out | (uintptr_t)c.ga | (uintptr_t)c.gb;
+    const int nch = (al & 15) ? 0 : (c.CA + c.CB) / 32;
+    if (nch == 1) return conv_staged<1, MODE>(c, st);
+    if (nch == 2) return conv_staged<2, MODE>(c, st);
+    if (nch == 3) return conv_staged<3, MODE>(c, st);
+    if (nch == 4) return conv_staged<4, MODE>(c, st);
+    if (nch == 6) return conv_staged<6, MODE>(c, st);
+    switch (conv_nj((long)c.N * c.H * c.W, c.Cout)) {
+    case 4: conv_direct<4, MODE>(c, st); break;
+    case 2: conv_direct<2, MODE>(c, st); break;
+    default: conv_direct<1, MODE>(c, st);
+    }
+}
 }  // namespace
 
 extern "C" {
@@ -810,17 +1034,7 @@ int glide_unet_conv3x3(const uint16_t *xa, int CA, const uint16_t *xb, int CB, i
     if (!xa || !weights || !bias || !out || (CB > 0 && !xb)) return ufail(GLIDE_E_NULL, "conv3x3: NULL argument");
     if (bad_ch(CA) || CA == 0 || bad_ch(CB) || bad_ch(Cout) || Cout == 0 || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3: channels must be positive multiples of 32, sizes positive");
-    const long P = (long)N * H * W;
-    const int nj = conv_nj(P, Cout);
-    if (nj == 4)
-        hipLaunchKernelGGL((k_conv3x3<4, 0>), dim3(nblk(P), Cout / 64), dim3(256), 0, SS(stream), xa, CA, xb, CB, N, H,
-                           W, weights, Cout, bias, relu, out, nullptr, 0, 0, nullptr, 0);
-    else if (nj == 2)
-        hipLaunchKernelGGL((k_conv3x3<2, 0>), dim3(nblk(P), Cout / 32), dim3(256), 0, SS(stream), xa, CA, xb, CB, N, H,
-                           W, weights, Cout, bias, relu, out, nullptr, 0, 0, nullptr, 0);
-    else
-        hipLaunchKernelGGL((k_conv3x3<1, 0>), dim3(nblk(P), Cout / 16), dim3(256), 0, SS(stream), xa, CA, xb, CB, N, H,
-                           W, weights, Cout, bias, relu, out, nullptr, 0, 0, nullptr, 0);
+    conv<0>(ConvArgs{xa, CA, xb, CB, N, H, W, weights, Cout, bias, relu, out, nullptr, 0, 0, nullptr, 0}, SS(stream));
     return ucheck("conv3x3");
 }
 
@@ -830,18 +1044,9 @@ int glide_unet_conv3x3_dgrad(const uint16_t *dz, int Cout, int N, int H, int W, 
     if (!dz || !wflip || !ga || (CB > 0 && !gb)) return ufail(GLIDE_E_NULL, "conv3x3_dgrad: NULL argument");
     if (bad_ch(Cout) || Cout == 0 || bad_ch(CA) || CA == 0 || bad_ch(CB) || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3_dgrad: channels must be positive multiples of 32, sizes positive");
-    const long P = (long)N * H * W;
-    const int Cin = CA + CB;   // output channels of the transposed convolution
-    const int nj = conv_nj(P, Cin);
-    if (nj == 4)
-        hipLaunchKernelGGL((k_conv3x3<4, 1>), dim3(nblk(P), Cin / 64), dim3(256), 0, SS(stream), dz, Cout, nullptr, 0,
-                           N, H, W, wflip, Cin, nullptr, 0, nullptr, ga, CA, acc_a, gb, acc_b);
-    else if (nj == 2)
-        hipLaunchKernelGGL((k_conv3x3<2, 1>), dim3(nblk(P), Cin / 32), dim3(256), 0, SS(stream), dz, Cout, nullptr, 0,
-                           N, H, W, wflip, Cin, nullptr, 0, nullptr, ga, CA, acc_a, gb, acc_b);
-    else
-        hipLaunchKernelGGL((k_conv3x3<1, 1>), dim3(nblk(P), Cin / 16), dim3(256), 0, SS(stream), dz, Cout, nullptr, 0,
-                           N, H, W, wflip, Cin, nullptr, 0, nullptr, ga, CA, acc_a, gb, acc_b);
+    // the transposed convolution: CA + CB output channels
+    conv<1>(ConvArgs{dz, Cout, nullptr, 0, N, H, W, wflip, CA + CB, nullptr, 0, nullptr, ga, CA, acc_a, gb, acc_b},
+            SS(stream));
     return ucheck("conv3x3_dgrad");
 }
 

@@ -20,6 +20,7 @@
 #include <cstdint>
 #include <cstring>
 #include <string>
+#include <type_traits>
 
 #include "glide_unet.h"
 
@@ -336,24 +337,31 @@ __global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict
 // in LDS as they lie (16-byte stores), and ds_read_b64_tr_b16 hands each lane
 // the four consecutive pixels of its channel that a fragment needs.  A tap's
 // column shift is a row offset into the staged pixels, so x is read from
-// memory once for its nine taps.  Wave w takes the three taps of image row
-// w - 1: per 32 pixels it reads 2 dz and 6 x fragments for 12 MFMAs.  The
-// pitch of 96 bytes puts the four pixels that 16 lanes read in different
-// banks.  Every (tap, co, ci) sums its chunk in steps of 32 pixels in pixel
-// order, so the bits depend on neither the tile nor the grid.
+// memory once for its nine taps.  Waves 0 to 2 take the three taps of image
+// row w - 1: per 32 pixels they read 2 dz and 6 x fragments for 12 MFMAs.
+// Wave 3 stages dz and, in the blocks of the first 32 input channels, adds up
+// the bias gradient from the same staged pixels, which costs no time beside
+// the MFMA waves.  The pitch of 96 bytes puts the four pixels that 16 lanes read in
+// different banks.  Every (tap, co, ci) sums its chunk in steps of 32 pixels in
+// pixel order, and every channel's bias gradient pixel by pixel, so the bits
+// depend on neither the tile nor the grid.
 //
-// Bound by LDS reads (16 of 512 bytes per wave and step against 12 MFMAs of
-// 16 cycles).  One tap per block and 2-byte transposing stores took 5.0 ms of
-// a 16 x 256^2 training step for its 13 layers; this takes 1.1 ms.
+// A block is a serial chain of chunk / WG_PX tiles (often one block per CU), so
+// what counts is the time of one tile: loads run two tiles ahead, and a tile
+// whose pixels all lie inside the image (most of them) loads without tests.
+// For a 16 x 256^2 training step's 13 layers: 5.0 ms with one tap per block and
+// 2-byte transposing stores (and 0.64 ms for the bias gradients by themselves),
+// 1.1 ms with loads one tile ahead and tested addresses, 0.72 ms now.
 // ---------------------------------------------------------------------------
 constexpr int WG_PX = 128;   // pixels per staged tile
 constexpr int WG_LD = 48;    // LDS pitch of a pixel's 32 channels (bf16)
+constexpr int WG_NR = WG_PX / 16 + 1;   // 16-byte pieces of a staged row per lane
 
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
-// the 8 pixels [0, 8) from row t (pitch WG_LD) of channel `16-lane group's
-// first channel + r16`, in pixel order; t: the lane's row + 4-channel group
+// rows 0-3 and 4-7 (pitch WG_LD) from t of one channel per lane, in row order;
+// t: the lane's row (lane % 16 / 4) and 4-channel group (lane % 4) of its 16 channels
 __device__ __forceinline__ Frag tr_frag(const bf16_t *t)
 {
     union {
@@ -365,10 +373,11 @@ __device__ __forceinline__ Frag tr_frag(const bf16_t *t)
     return u.f;
 }
 
-__global__ __launch_bounds__(192) void k_conv3x3_wgrad(const bf16_t *__restrict__ dz, int Cout,
-                                                       const bf16_t *__restrict__ xa, int CA,
-                                                       const bf16_t *__restrict__ xb, int CB, int N, int H, int W,
-                                                       long chunk, float *__restrict__ partial)
+__global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const bf16_t *__restrict__ dz, int Cout,
+                                                          const bf16_t *__restrict__ xa, int CA,
+                                                          const bf16_t *__restrict__ xb, int CB, int N, int H, int W,
+                                                          long chunk, float *__restrict__ partial,
+                                                          float *__restrict__ part_b)
 {
     __shared__ bf16_t sD[WG_PX][WG_LD];          // dz of pixel p0 + k
     __shared__ bf16_t sX[3][WG_PX + 2][WG_LD];   // x of pixel p0 - 1 + k, image row dy = -1, 0, 1
@@ -376,36 +385,48 @@ __global__ __launch_bounds__(192) void k_conv3x3_wgrad(const bf16_t *__restrict_
     const int ci0 = blockIdx.x * 32, co0 = blockIdx.y * 32;
     const long P = (long)N * H * W, HW = (long)H * W;
     const long p_lo = (long)blockIdx.z * chunk, p_hi = p_lo + chunk < P ? p_lo + chunk : P;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, dy = w - 1;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), dy = w - 1;
     const int r16 = lane & 15, kq = lane >> 4;
-    const bf16_t *xs = ci0 < CA ? xa + ci0 : xb + (ci0 - CA);
-    const int cs = ci0 < CA ? CA : CB;
-    constexpr int NX = ((WG_PX + 2) * 4 + 63) / 64;   // 16-byte pieces of the wave's x row per lane
-    constexpr int ND = (WG_PX * 4 + 191) / 192;       // ... and of dz per thread
-    uint4 rx[NX], rd[ND];
-    // position in its image of the staged x row's first pixel; its rows above
-    // (dy = -1) and below (dy = 1) the image are zero
-    long r0 = ((p_lo - 1 + (long)dy * W) % HW + HW) % HW;
-    const long bad_lo = dy < 0 ? HW - W : 0, bad_n = dy == 0 ? 0 : W;
-    auto load = [&](long p0) {
+    const bool is_x = w < 3;
+    // the row that this wave stages: element k is pixel p0 + shift + k of src
+    const bf16_t *src = is_x ? (ci0 < CA ? xa + ci0 : xb + (ci0 - CA)) : dz + co0;
+    const int cs = is_x ? (ci0 < CA ? CA : CB) : Cout;
+    const long shift = is_x ? (long)dy * W - 1 : 0;
+    const int len = is_x ? WG_PX + 2 : WG_PX;
+    bf16_t(*row)[WG_LD] = is_x ? sX[w] : sD;
+    const int s0 = lane >> 2;
+    const bf16_t *lsrc = src + (long)s0 * cs + 8 * (lane & 3);
+    // position in its image of the x row's first pixel; the rows above (dy = -1)
+    // and below (dy = 1) the image are zero
+    long r0 = is_x ? ((p_lo + shift) % HW + HW) % HW : 0;
+    const long bad_lo = dy < 0 ? HW - W : 0, bad_hi = dy == 0 ? 0 : bad_lo + W;
+    auto load = [&](long p0, uint4(&r)[WG_NR]) {
+        const long q0 = p0 + shift;
+        const bool inside = is_x ? q0 >= 0 && q0 + len <= P && r0 + len <= HW && (r0 + len <= bad_lo || r0 >= bad_hi)
+                                 : q0 + len <= p_hi;
+        const bf16_t *b = lsrc + q0 * cs;
+        if (inside) {
 #pragma unroll
-        for (int m = 0; m < NX; m++) {
-            const int s = (lane >> 2) + 16 * m;
-            const long q = p0 - 1 + (long)dy * W + s;
-            long r = r0 + s;
-            while (r >= HW) r -= HW;
-            const bool ok = s < WG_PX + 2 && q >= 0 && q < P && !(r >= bad_lo && r < bad_lo + bad_n);
-            rx[m] = ok ? *(const uint4 *)(xs + q * cs + 8 * (lane & 3)) : uint4{0u, 0u, 0u, 0u};
-        }
+            for (int m = 0; m < WG_NR; m++)
+                if (16 * m + s0 < len) r[m] = *(const uint4 *)(b + 16 * m * cs);
+        } else {
 #pragma unroll
-        for (int m = 0; m < ND; m++) {
-            const int e = tid + 192 * m;
-            const long p = p0 + (e >> 2);
-            const bool ok = e < WG_PX * 4 && p < p_hi;
-            rd[m] = ok ? *(const uint4 *)(dz + p * Cout + co0 + 8 * (e & 3)) : uint4{0u, 0u, 0u, 0u};
+            for (int m = 0; m < WG_NR; m++) {
+                const int s = s0 + 16 * m;
+                const long q = q0 + s;
+                bool ok = s < len && q >= 0 && q < (is_x ? P : p_hi);
+                if (is_x) {
+                    long k = r0 + s;
+                    while (k >= HW) k -= HW;
+                    ok = ok && !(k >= bad_lo && k < bad_hi);
+                }
+                r[m] = ok ? *(const uint4 *)(b + 16 * m * cs) : uint4{0u, 0u, 0u, 0u};
+            }
         }
-        r0 += WG_PX;
-        while (r0 >= HW) r0 -= HW;
+        if (is_x) {
+            r0 += WG_PX;
+            while (r0 >= HW) r0 -= HW;
+        }
     };
     f32x4 acc[3][2][2];
 #pragma unroll
@@ -414,101 +435,133 @@ __global__ __launch_bounds__(192) void k_conv3x3_wgrad(const bf16_t *__restrict_
         for (int a = 0; a < 2; a++)
 #pragma unroll
             for (int b = 0; b < 2; b++) acc[d][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float bsum = 0.0f;
     // column of the lane's first pixel (8 kq past the step's first)
     int col = (int)((p_lo + 8 * kq) % W);
     const int cstep = 32 % W;
     // the lane's corner of a fragment at step 0: pixel 8 kq + r16 / 4, channels 4 (r16 % 4)
     const int fo = (8 * kq + (r16 >> 2)) * WG_LD + 4 * (r16 & 3);
-    load(p_lo);
-    for (long p0 = p_lo; p0 < p_hi; p0 += WG_PX) {
-        __syncthreads();   // the previous tile has been read
+    const bf16_t *xrow = &sX[is_x ? w : 0][0][0];
+    auto step = [&](long p0, int st, auto plain) {
+        const int o = fo + 32 * st * WG_LD;
+        Frag A[2], B[3][2];
 #pragma unroll
-        for (int m = 0; m < NX; m++) {
-            const int s = (lane >> 2) + 16 * m;
-            if (s < WG_PX + 2) *(uint4 *)&sX[w][s][8 * (lane & 3)] = rx[m];
-        }
+        for (int a = 0; a < 2; a++) A[a] = tr_frag(&sD[0][0] + o + 16 * a);
 #pragma unroll
-        for (int m = 0; m < ND; m++) {
-            const int e = tid + 192 * m;
-            if (e < WG_PX * 4) *(uint4 *)&sD[e >> 2][8 * (e & 3)] = rd[m];
-        }
-        __syncthreads();
-        if (p0 + WG_PX < p_hi) load(p0 + WG_PX);
-        // 8 consecutive pixels lie in one image row where W % 8 == 0 (chunks start at multiples of 8)
-        const bool plain = (W & 7) == 0 && p0 + WG_PX <= p_hi;
-#pragma unroll 1
-        for (int st = 0; st < WG_PX / 32; st++) {
-            if (p0 + 32 * st >= p_hi) break;
-            const int o = fo + 32 * st * WG_LD;
-            Frag A[2], B[3][2];
+        for (int d = 0; d < 3; d++)
 #pragma unroll
-            for (int a = 0; a < 2; a++) A[a] = tr_frag(&sD[0][0] + o + 16 * a);
+            for (int b = 0; b < 2; b++) B[d][b] = tr_frag(xrow + o + d * WG_LD + 16 * b);
+        // x is 0 left of column 0 (tap dx = -1) and right of column W - 1 (dx = 1)
+        if (plain) {
+            const uint32_t ml = col == 0 ? 0xffff0000u : 0xffffffffu, mr = col == W - 8 ? 0x0000ffffu : 0xffffffffu;
+#pragma unroll
+            for (int b = 0; b < 2; b++) {
+                B[0][b].raw.x &= ml;
+                B[2][b].raw.w &= mr;
+            }
+        } else {
+            uint32_t m[3][4] = {};
+            int c = col;
+#pragma unroll
+            for (int e = 0; e < 8; e++) {
+                const uint32_t h = p0 + 32 * st + 8 * kq + e < p_hi ? 0xffffu << (16 * (e & 1)) : 0u;
+                m[0][e >> 1] |= c > 0 ? h : 0u;
+                m[1][e >> 1] |= h;
+                m[2][e >> 1] |= c < W - 1 ? h : 0u;
+                c = c + 1 == W ? 0 : c + 1;
+            }
 #pragma unroll
             for (int d = 0; d < 3; d++)
-#pragma unroll
-                for (int b = 0; b < 2; b++) B[d][b] = tr_frag(&sX[w][0][0] + o + d * WG_LD + 16 * b);
-            // x is 0 left of column 0 (tap dx = -1) and right of column W - 1 (dx = 1)
-            if (plain) {
-                const uint32_t ml = col == 0 ? 0xffff0000u : 0xffffffffu, mr = col == W - 8 ? 0x0000ffffu : 0xffffffffu;
 #pragma unroll
                 for (int b = 0; b < 2; b++) {
-                    B[0][b].raw.x &= ml;
-                    B[2][b].raw.w &= mr;
+                    B[d][b].raw.x &= m[d][0];
+                    B[d][b].raw.y &= m[d][1];
+                    B[d][b].raw.z &= m[d][2];
+                    B[d][b].raw.w &= m[d][3];
+                }
+        }
+        col += cstep;
+        col = col >= W ? col - W : col;
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int a = 0; a < 2; a++)
+#pragma unroll
+                for (int b = 0; b < 2; b++)
+                    acc[d][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a].v, B[d][b].v, acc[d][a][b], 0, 0, 0);
+    };
+    // lanes 0-31: bias gradient of channel co0 + lane, four pixels per read
+    const bool do_b = part_b && blockIdx.x == 0 && lane < 32;
+    const bf16_t *bcol = &sD[r16 >> 2][16 * (kq & 1) + 4 * (r16 & 3)];
+    auto tile = [&](long p0, uint4(&r)[WG_NR]) {
+        __syncthreads();   // the previous tile has been read
+#pragma unroll
+        for (int m = 0; m < WG_NR; m++)
+            if (16 * m + s0 < len) *(uint4 *)&row[16 * m + s0][8 * (lane & 3)] = r[m];
+        __syncthreads();
+        if (p0 + 2 * WG_PX < p_hi) load(p0 + 2 * WG_PX, r);
+        if (is_x) {
+            // 8 consecutive pixels lie in one image row where W % 8 == 0 (chunks start at multiples of 8)
+            if ((W & 7) == 0 && p0 + WG_PX <= p_hi) {
+#pragma unroll
+                for (int st = 0; st < WG_PX / 32; st++) step(p0, st, std::true_type{});
+            } else {
+#pragma unroll 1
+                for (int st = 0; st < WG_PX / 32 && p0 + 32 * st < p_hi; st++) step(p0, st, std::false_type{});
+            }
+        } else if (do_b) {
+            const int n = p_hi - p0 < WG_PX ? (int)(p_hi - p0) : WG_PX;
+            if (n == WG_PX) {
+#pragma unroll 8
+                for (int k = 0; k < WG_PX; k += 4) {
+                    const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(bcol + k * WG_LD));
+#pragma unroll
+                    for (int e = 0; e < 4; e++) bsum += bf2f((bf16_t)v[e]);
                 }
             } else {
-                uint32_t m[3][4] = {};
-                int c = col;
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const uint32_t h = p0 + 32 * st + 8 * kq + e < p_hi ? 0xffffu << (16 * (e & 1)) : 0u;
-                    m[0][e >> 1] |= c > 0 ? h : 0u;
-                    m[1][e >> 1] |= h;
-                    m[2][e >> 1] |= c < W - 1 ? h : 0u;
-                    c = c + 1 == W ? 0 : c + 1;
-                }
-#pragma unroll
-                for (int d = 0; d < 3; d++)
-#pragma unroll
-                    for (int b = 0; b < 2; b++) {
-                        B[d][b].raw.x &= m[d][0];
-                        B[d][b].raw.y &= m[d][1];
-                        B[d][b].raw.z &= m[d][2];
-                        B[d][b].raw.w &= m[d][3];
-                    }
+                for (int k = 0; k < n; k++) bsum += bf2f(sD[k][lane]);
             }
-            col += cstep;
-            col = col >= W ? col - W : col;
-#pragma unroll
-            for (int d = 0; d < 3; d++)
-#pragma unroll
-                for (int a = 0; a < 2; a++)
-#pragma unroll
-                    for (int b = 0; b < 2; b++)
-                        acc[d][a][b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A[a].v, B[d][b].v, acc[d][a][b], 0, 0, 0);
         }
+    };
+    uint4 ra[WG_NR], rb[WG_NR];
+#pragma unroll
+    for (int m = 0; m < WG_NR; m++) ra[m] = rb[m] = uint4{0u, 0u, 0u, 0u};
+    load(p_lo, ra);
+    if (p_lo + WG_PX < p_hi) load(p_lo + WG_PX, rb);
+    for (long p0 = p_lo; p0 < p_hi; p0 += 2 * WG_PX) {
+        tile(p0, ra);
+        if (p0 + WG_PX < p_hi) tile(p0 + WG_PX, rb);
     }
+    if (is_x) {
 #pragma unroll
-    for (int d = 0; d < 3; d++) {
-        float *dst = partial + ((long)blockIdx.z * 9 + 3 * w + d) * Cout * Cin;
+        for (int d = 0; d < 3; d++) {
+            float *dst = partial + ((long)blockIdx.z * 9 + 3 * w + d) * Cout * Cin;
 #pragma unroll
-        for (int a = 0; a < 2; a++)
+            for (int a = 0; a < 2; a++)
 #pragma unroll
-            for (int b = 0; b < 2; b++)
+                for (int b = 0; b < 2; b++)
 #pragma unroll
-                for (int i = 0; i < 4; i++)
-                    dst[(long)(co0 + 16 * a + 4 * kq + i) * Cin + ci0 + 16 * b + r16] = acc[d][a][b][i];
+                    for (int i = 0; i < 4; i++)
+                        dst[(long)(co0 + 16 * a + 4 * kq + i) * Cin + ci0 + 16 * b + r16] = acc[d][a][b][i];
+        }
+    } else if (do_b) {
+        part_b[(long)blockIdx.z * Cout + co0 + lane] = bsum;
     }
 }
 
-// out[k] = sum_z partial[z][k] in z order
-__global__ void k_reduce_chunks(const float *__restrict__ partial, long n, int nz, float *__restrict__ out)
+// out[k] = sum_z partial[z][k] in z order; out2 likewise from partial2 (n2 entries)
+__global__ void k_reduce_chunks(const float *__restrict__ partial, long n, int nz, float *__restrict__ out,
+                                const float *__restrict__ partial2, long n2, float *__restrict__ out2)
 {
     long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
+    if (k >= n + n2) return;
+    const bool first = k < n;
+    const float *p = first ? partial + k : partial2 + (k - n);
+    const long stride = first ? n : n2;
     float s = 0.0f;
 #pragma unroll 16   // loads of 16 chunks in flight, the additions in z order
-    for (int z = 0; z < nz; z++) s += partial[(long)z * n + k];
-    out[k] = s;
+    for (int z = 0; z < nz; z++) s += p[(long)z * stride];
+    (first ? out[k] : out2[k - n]) = s;
 }
 
 // Plain GEMM C[m][n] = sum_k A[m][k] B[n][k] (both K-contiguous, BF16; M, N
@@ -1052,22 +1105,28 @@ int glide_unet_conv3x3_dgrad(const uint16_t *dz, int Cout, int N, int H, int W, 
 
 long glide_unet_wgrad_chunks(int N, int H, int W) { return ((long)N * H * W + 4095) / 4096; }
 
-int glide_unet_conv3x3_wgrad(const uint16_t *dz, int Cout, const uint16_t *xa, int CA, const uint16_t *xb, int CB,
-                             int N, int H, int W, float *partial, float *dw, void *stream)
+int glide_unet_conv3x3_wgrad_bias(const uint16_t *dz, int Cout, const uint16_t *xa, int CA, const uint16_t *xb, int CB,
+                                  int N, int H, int W, float *partial, float *dw, float *db, void *stream)
 {
     if (!dz || !xa || !partial || !dw || (CB > 0 && !xb)) return ufail(GLIDE_E_NULL, "conv3x3_wgrad: NULL argument");
     if (bad_ch(Cout) || Cout == 0 || bad_ch(CA) || CA == 0 || bad_ch(CB) || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3_wgrad: channels must be positive multiples of 32, sizes positive");
-    const long P = (long)N * H * W, chunk = 4096;
+    const long chunk = 4096;
     const long nz = glide_unet_wgrad_chunks(N, H, W);
     const int Cin = CA + CB;
-    dim3 grid(Cin / 32, Cout / 32, (unsigned)nz);
-    hipLaunchKernelGGL(k_conv3x3_wgrad, grid, dim3(192), 0, SS(stream), dz, Cout, xa, CA, xb, CB, N, H, W, chunk,
-                       partial);
-    const long n = 9L * Cout * Cin;
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(n)), dim3(256), 0, SS(stream), partial, n, (int)nz, dw);
-    (void)P;
+    const long n = 9L * Cout * Cin, n2 = db ? Cout : 0;
+    float *part_b = db ? partial + nz * n : nullptr;
+    hipLaunchKernelGGL(k_conv3x3_wgrad, dim3(Cin / 32, Cout / 32, (unsigned)nz), dim3(256), 0, SS(stream), dz, Cout, xa,
+                       CA, xb, CB, N, H, W, chunk, partial, part_b);
+    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(n + n2)), dim3(256), 0, SS(stream), partial, n, (int)nz, dw, part_b, n2,
+                       db);
     return ucheck("conv3x3_wgrad");
+}
+
+int glide_unet_conv3x3_wgrad(const uint16_t *dz, int Cout, const uint16_t *xa, int CA, const uint16_t *xb, int CB,
+                             int N, int H, int W, float *partial, float *dw, void *stream)
+{
+    return glide_unet_conv3x3_wgrad_bias(dz, Cout, xa, CA, xb, CB, N, H, W, partial, dw, nullptr, stream);
 }
 
 int glide_unet_gemm_bf16(const uint16_t *A, const uint16_t *B, float *C, int M, int N, int K, void *stream)
@@ -1151,7 +1210,8 @@ int glide_unet_bias_grad(const uint16_t *dz, long P, int C, float *partial, floa
     else
         hipLaunchKernelGGL(k_bias_grad, dim3((C + 63) / 64, (unsigned)nz), dim3(64), 0, SS(stream), dz, P, C, 4096L,
                            partial);
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(C)), dim3(256), 0, SS(stream), partial, (long)C, (int)nz, db);
+    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(C)), dim3(256), 0, SS(stream), partial, (long)C, (int)nz, db,
+                       (const float *)nullptr, 0L, (float *)nullptr);
     return ucheck("bias_grad");
 }
 
@@ -1181,7 +1241,8 @@ int glide_unet_head_bwd(const float *dout, const uint16_t *x, long P, int C, int
     else
         hipLaunchKernelGGL(k_head_bwd_w, dim3((unsigned)nz), dim3(((nk + 63) / 64) * 64), 0, SS(stream), dout, x, P,
                            C, NO, 4096L, partial);
-    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(nk)), dim3(256), 0, SS(stream), partial, (long)nk, (int)nz, dwh_dbh);
+    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(nk)), dim3(256), 0, SS(stream), partial, (long)nk, (int)nz, dwh_dbh,
+                       (const float *)nullptr, 0L, (float *)nullptr);
     return ucheck("head_bwd");
 }
 

@@ -134,7 +134,7 @@ class UNet:
             for name, ins, co in LAYERS:
                 h, w = dims[LEVEL[name]]
                 nz = _lib.fn("glide_unet_wgrad_chunks")(N, h, w)
-                part = max(part, nz * 9 * co * SHAPES[name][1], _lib.fn("glide_unet_bias_chunks")(N * h * w) * co)
+                part = max(part, nz * (9 * co * SHAPES[name][1] + co))
             nk = N_OUT * CH[HEAD_IN] + N_OUT
             part = max(part, _lib.fn("glide_unet_bias_chunks")(N * H * W) * nk,
                        _lib.fn("glide_unet_mse_blocks")(N * H * W * N_OUT))
@@ -199,9 +199,8 @@ class UNet:
             _lib.call("glide_unet_relu_bwd", _p(g[name]), _p(acts[name]), n, _p(dz), st)
             xa, xb = acts[ins[0]], (acts[ins[1]] if len(ins) > 1 else None)
             ca, cb = CH[ins[0]], (CH[ins[1]] if xb is not None else 0)
-            _lib.call("glide_unet_conv3x3_wgrad", _p(dz), co, _p(xa), ca, _p(xb), cb, N, h, w, _p(b["partial"]),
-                      _p(self.grads[name + ".W"]), st)
-            _lib.call("glide_unet_bias_grad", _p(dz), N * h * w, co, _p(b["partial"]), _p(self.grads[name + ".b"]), st)
+            _lib.call("glide_unet_conv3x3_wgrad_bias", _p(dz), co, _p(xa), ca, _p(xb), cb, N, h, w, _p(b["partial"]),
+                      _p(self.grads[name + ".W"]), _p(self.grads[name + ".b"]), st)
             if ins == ["x0"]:
                 continue
             gb = g[ins[1]] if xb is not None else None

@@ -44,6 +44,12 @@ long glide_unet_wgrad_chunks(int N, int H, int W);
 int glide_unet_conv3x3_wgrad(const uint16_t *dz, int Cout, const uint16_t *xa, int CA, const uint16_t *xb,
                              int CB, int N, int H, int W, float *partial, float *dw, void *stream);
 
+/* glide_unet_conv3x3_wgrad and, from the same reading of dz, the bias gradient
+ * db[c] = sum_p dz[p][c] of glide_unet_bias_grad (the same sums): partial
+ * holds glide_unet_wgrad_chunks(N, H, W) x Cout more floats.  db may be NULL. */
+int glide_unet_conv3x3_wgrad_bias(const uint16_t *dz, int Cout, const uint16_t *xa, int CA, const uint16_t *xb,
+                                  int CB, int N, int H, int W, float *partial, float *dw, float *db, void *stream);
+
 /* C[m][n] = sum_k A[m][k] B[n][k] (BF16 in, FP32 out; M, N multiples of 16,
  * K of 32): the MFMA fragment layout the convolutions use, exposed for tests. */
 int glide_unet_gemm_bf16(const uint16_t *A, const uint16_t *B, float *C, int M, int N, int K, void *stream);

@@ -4,7 +4,8 @@ are not multiples of 8, several images, chunk remainders, and every 32-channel
 group of both inputs.
 
 Tolerance per entry: an FP32 sum of P products in any order is off by at most
-(P + 2) 2^-24 times the sum of the products' magnitudes."""
+(P + 2) 2^-24 times the sum of the products' magnitudes.  The bias gradient of
+the same launch equals glide_unet_bias_grad's bit for bit."""
 import ctypes
 
 import numpy as np
@@ -39,6 +40,13 @@ def test_wgrad_matches_oracle(N, H, W, CA, CB, Co):
     a, b, d = _dev(xa), (_dev(xb) if CB else None), _dev(dz)
     _lib.call("glide_unet_conv3x3_wgrad", d.data_ptr(), Co, a.data_ptr(), CA, b.data_ptr() if CB else None, CB, N, H,
               W, part.data_ptr(), dw.data_ptr(), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    part2 = torch.empty(part.numel() + _lib.fn("glide_unet_wgrad_chunks")(N, H, W) * Co, device=DEV)
+    dw2, db, db2 = torch.empty_like(dw), torch.empty(Co, device=DEV), torch.empty(Co, device=DEV)
+    st = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    _lib.call("glide_unet_conv3x3_wgrad_bias", d.data_ptr(), Co, a.data_ptr(), CA, b.data_ptr() if CB else None, CB, N,
+              H, W, part2.data_ptr(), dw2.data_ptr(), db.data_ptr(), st)
+    _lib.call("glide_unet_bias_grad", d.data_ptr(), P, Co, part2.data_ptr(), db2.data_ptr(), st)
+    assert torch.equal(dw, dw2) and torch.equal(db, db2)
     x = np.concatenate([xa, xb], -1)
     ref = U.conv3x3_wgrad(dz, x)
     mag = U.conv3x3_wgrad(np.abs(dz), np.abs(x))

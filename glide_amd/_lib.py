@@ -116,6 +116,13 @@ SIGNATURES = {
                                          c_void_p, c_void_p, c_void_p]),
     "glide_unet_conv3x3_wgrad_bias": (c_int, [c_void_p, c_int, c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int,
                                               c_void_p, c_void_p, c_void_p, c_void_p]),
+    "glide_unet_conv3x3_dgrad_relu": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
+                                              c_void_p, c_void_p]),
+    "glide_unet_head_bwd_relu": (c_int, [c_void_p, c_void_p, ctypes.c_long, c_int, c_int, c_void_p, c_void_p, c_void_p,
+                                         c_void_p, c_void_p]),
+    "glide_unet_pool2_bwd_relu": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p,
+                                          c_void_p]),
+    "glide_unet_up2_bwd_relu": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "glide_unet_gemm_bf16": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
     "glide_unet_prep_weights": (c_int, [c_void_p, c_int, c_int, c_void_p, c_void_p, c_void_p]),
     "glide_unet_relu_bwd": (c_int, [c_void_p, c_void_p, ctypes.c_long, c_void_p, c_void_p]),

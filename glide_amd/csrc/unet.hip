@@ -65,6 +65,11 @@ union Frag {
     uint4 raw;
     bf16x8 v;
 };
+// 8 channels in one 16-byte access
+union Bf8 {
+    uint4 raw;
+    bf16_t h[8];
+};
 
 // ---------------------------------------------------------------------------
 // 3x3 convolution, implicit GEMM on MFMA.
@@ -72,6 +77,9 @@ union Frag {
 //        x = concat(xa (CA ch), xb (CB ch)); act = ReLU when relu != 0.
 // MODE 1 (data gradient): the same sum without bias/act into FP32 outputs split
 //        by channel: co < SA -> ga[p][co] (+)= ..., else gb[p][co - SA] (+)= ...
+// MODE 2 (data gradient through the input's ReLU): out_bf16[p][co] =
+//        bf16(ya[p][co] > 0 ? sum : 0), what MODE 1 followed by the ReLU's
+//        backward gives without the FP32 gradient's round trip through memory.
 //
 // A workgroup of NW waves owns 2 NW rows x 32 columns of one image x 32 output
 // channels: it stages the (2 NW + 2) x 34 input pixels of every channel (NCH
@@ -107,8 +115,9 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
                                                      const bf16_t *__restrict__ xb, int H, int W, int tiles_x,
                                                      int tiles, const bf16_t *__restrict__ Wt, int Cout,
                                                      const float *__restrict__ bias, int relu,
-                                                     bf16_t *__restrict__ out, float *__restrict__ ga, int SA,
-                                                     int acc_a, float *__restrict__ gb, int acc_b)
+                                                     const bf16_t *__restrict__ ya, bf16_t *__restrict__ out,
+                                                     float *__restrict__ ga, int SA, int acc_a,
+                                                     float *__restrict__ gb, int acc_b)
 {
     constexpr int PW = CV_W + 2, NPX = (2 * NW + 2) * PW, Cin = 32 * NCH;
     __shared__ bf16_t sm[NCH * NPX * CV_LD];   // [chunk][pixel][CV_LD]
@@ -199,12 +208,17 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
         const int y = y0 + 2 * wave + (a >> 1), x = x0 + 16 * (a & 1) + r16;
         if (y >= H || x >= W) continue;
         const long p = img + (long)y * W + x;
-        if (MODE == 0) {
+        if (MODE != 1) {
             uint32_t h[8];
+            Bf8 y8;
+            if (MODE == 2) y8.raw = *(const uint4 *)(ya + p * Cout + co);
 #pragma unroll
             for (int i = 0; i < 8; i++) {
                 const float val = acc[a][i >> 2][i & 3] + bs[i];
-                h[i] = relu ? f2bf_num(fmaxf(val, 0.0f)) : (uint32_t)f2bf(val);   // fmaxf leaves no NaN
+                if (MODE == 0)
+                    h[i] = relu ? f2bf_num(fmaxf(val, 0.0f)) : (uint32_t)f2bf(val);   // fmaxf leaves no NaN
+                else
+                    h[i] = f2bf(bf2f(y8.h[i]) > 0.0f ? acc[a][i >> 2][i & 3] : 0.0f);
             }
             *(uint4 *)(out + p * Cout + co) =
                 uint4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
@@ -232,7 +246,8 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
 template <int NJ, int MODE>
 __global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict__ xa, int CA, const bf16_t *__restrict__ xb,
                                                         int CB, int N, int H, int W, const bf16_t *__restrict__ Wt, int Cout,
-                                                        const float *__restrict__ bias, int relu, bf16_t *__restrict__ out,
+                                                        const float *__restrict__ bias, int relu, const bf16_t *__restrict__ ya,
+                                                        bf16_t *__restrict__ out,
                                                         float *__restrict__ ga, int SA, int acc_a, float *__restrict__ gb,
                                                         int acc_b)
 {
@@ -314,6 +329,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict
                     val += bias[co];
                     if (relu) val = fmaxf(val, 0.0f);
                     out[p * Cout + co] = f2bf(val);
+                } else if (MODE == 2) {
+                    out[p * Cout + co] = f2bf(bf2f(ya[p * Cout + co]) > 0.0f ? val : 0.0f);
                 } else {
                     if (co < SA) {
                         float *d = ga + p * SA + co;
@@ -636,12 +653,6 @@ __global__ void k_pool2_bwd(const float *__restrict__ dy, int N, int H, int W, i
     const float g = 0.25f * dy[(((long)n * (H / 2) + y / 2) * (W / 2) + x / 2) * C + c];
     dx[k] = acc ? dx[k] + g : g;
 }
-// 8 channels in one 16-byte access
-union Bf8 {
-    uint4 raw;
-    bf16_t h[8];
-};
-
 // 2x2 average pooling over 8-channel groups (C % 8 == 0, 16-byte aligned
 // tensors): per channel the same sums as k_pool2
 __global__ void k_pool2_v8(const bf16_t *__restrict__ x, int N, int H, int W, int C, bf16_t *__restrict__ y)
@@ -692,6 +703,86 @@ __global__ void k_up2(const bf16_t *__restrict__ x, int N, int H, int W, int C, 
     const int yo = (int)(r % (2 * H)), n = (int)(r / (2 * H));
     y[k] = x[(((long)n * H + yo / 2) * W + xo / 2) * C + c];
 }
+// The backward passes that end at a ReLU's output: the gradient of 8 channels
+// formed as the FP32 kernels form it, masked and rounded to BF16 at once
+// (dz = bf16(y > 0 ? g : 0)); C % 8 == 0, tensors 16-byte aligned.  Bound by
+// memory: the FP32 gradient is neither written nor read again.  Level 0 of a
+// 16 x 256^2 training step: pooling 216 -> 52 us with its ReLU, the head's 157
+// -> 23 us, upsampling onto level 1 62 -> 41 us.
+__device__ __forceinline__ void relu_store(const float g[8], const bf16_t *y, bf16_t *dz)
+{
+    Bf8 a, o;
+    a.raw = *(const uint4 *)y;
+#pragma unroll
+    for (int i = 0; i < 8; i++) o.h[i] = f2bf(bf2f(a.h[i]) > 0.0f ? g[i] : 0.0f);
+    *(uint4 *)dz = o.raw;
+}
+__device__ __forceinline__ void load8(const float *p, float v[8])
+{
+    const float4 a = *(const float4 *)p, b = *(const float4 *)(p + 4);
+    v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w, v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+}
+// g + 0.25 dy (k_pool2_bwd accumulating into g)
+__global__ void k_pool2_bwd_relu(const float *__restrict__ dy, const float *__restrict__ g, int N, int H, int W, int C,
+                                 const bf16_t *__restrict__ y, bf16_t *__restrict__ dz)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int C8 = C / 8;
+    if (k >= (long)N * H * W * C8) return;
+    const int c8 = (int)(k % C8);
+    long r = k / C8;
+    const int px = (int)(r % W);
+    r /= W;
+    const int py = (int)(r % H), n = (int)(r / H);
+    float d[8], a[8];
+    load8(dy + (((long)n * (H / 2) + py / 2) * (W / 2) + px / 2) * C + 8 * c8, d);
+    load8(g + 8 * k, a);
+#pragma unroll
+    for (int i = 0; i < 8; i++) a[i] = a[i] + 0.25f * d[i];
+    relu_store(a, y + 8 * k, dz + 8 * k);
+}
+// k_up2_bwd
+__global__ void k_up2_bwd_relu(const float *__restrict__ dy, int N, int H, int W, int C, const bf16_t *__restrict__ y,
+                               bf16_t *__restrict__ dz)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int C8 = C / 8;
+    if (k >= (long)N * H * W * C8) return;
+    const int c8 = (int)(k % C8);
+    long r = k / C8;
+    const int px = (int)(r % W);
+    r /= W;
+    const int py = (int)(r % H), n = (int)(r / H);
+    const long W2 = 2L * W, b = (((long)n * 2 * H + 2 * py) * W2 + 2 * px) * C + 8 * c8;
+    float q0[8], q1[8], q2[8], q3[8];
+    load8(dy + b, q0);
+    load8(dy + b + C, q1);
+    load8(dy + b + W2 * C, q2);
+    load8(dy + b + W2 * C + C, q3);
+#pragma unroll
+    for (int i = 0; i < 8; i++) q0[i] = ((q0[i] + q1[i]) + q2[i]) + q3[i];
+    relu_store(q0, y + 8 * k, dz + 8 * k);
+}
+// k_head_bwd_x; x is the head's input, the ReLU's output
+template <int NO>
+__global__ void k_head_bwd_relu(const float *__restrict__ dout, const bf16_t *__restrict__ x, long P, int C,
+                                const float *__restrict__ Wh, bf16_t *__restrict__ dz)
+{
+    const long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int C8 = C / 8;
+    if (k >= P * C8) return;
+    const long p = k / C8;
+    const int c = 8 * (int)(k - p * C8);
+    float g[8];
+#pragma unroll
+    for (int o = 0; o < NO; o++) {
+        const float d = dout[NO * p + o];
+#pragma unroll
+        for (int i = 0; i < 8; i++) g[i] = o ? g[i] + d * Wh[o * C + c + i] : d * Wh[c + i];
+    }
+    relu_store(g, x + 8 * k, dz + 8 * k);
+}
+
 __global__ void k_up2_bwd(const float *__restrict__ dy, int N, int H, int W, int C, float *__restrict__ dx)
 {
     long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -826,60 +917,73 @@ __global__ void k_head_bwd_w(const float *__restrict__ dout, const bf16_t *__res
     part[(long)blockIdx.x * nk + k] = s;
 }
 
-// k_head_bwd_w with both tensors staged in LDS like k_bias_grad_v8 (C % 8 ==
-// 0, C <= 64, x 16-byte aligned): the same sums in the same pixel order.
-__global__ __launch_bounds__(256) void k_head_bwd_w_v8(const float *__restrict__ dout, const bf16_t *__restrict__ x,
-                                                       long P, int C, int NO, long chunk, float *__restrict__ part)
+// k_head_bwd_w with both tensors staged in LDS (C % 16 == 0, C <= 64, x 16-byte
+// aligned): the same sums in the same pixel order.  A lane's chain reads four
+// pixels of its channel at once (ds_read_b64_tr_b16) and four of its output's
+// gradient; the bias sums' lanes read a column of ones instead of x, so every
+// lane runs the same chain.  16 x 256^2 pixels, 32 channels, 3 outputs: 1226
+// us by k_head_bwd_w, 66 us by this.
+constexpr int HB_NT = 320;   // threads: NO C + NO <= 260 chains
+constexpr int HB_LD = 80;    // LDS pitch (bf16): up to 64 channels, 16 ones
+template <int NO>
+__global__ __launch_bounds__(HB_NT) void k_head_bwd_w_v8(const float *__restrict__ dout, const bf16_t *__restrict__ x,
+                                                         long P, int C, long chunk, float *__restrict__ part)
 {
-    __shared__ bf16_t t[SUM_PX][64];
-    __shared__ float d[SUM_PX * 4];
-    const int nk = NO * C + NO, n8 = C / 8, k = threadIdx.x;   // nk <= 260: lanes k and k + 256
+    __shared__ bf16_t t[SUM_PX][HB_LD];
+    __shared__ float d[4][SUM_PX];
+    const int nk = NO * C + NO, n8 = C / 8, k = threadIdx.x, r16 = k & 15;
     const long lo = (long)blockIdx.x * chunk, hi = lo + chunk < P ? lo + chunk : P;
-    const int g = threadIdx.x & 7, row = threadIdx.x >> 3;
-    uint4 r[SUM_PX / 32];
-    float rd[4];
+    constexpr int NX = (SUM_PX * 8 + HB_NT - 1) / HB_NT, ND = (SUM_PX * NO + HB_NT - 1) / HB_NT;
+    uint4 r[NX];
+    float rd[ND];
     auto load = [&](long p0) {
 #pragma unroll
-        for (int q = 0; q < SUM_PX / 32; q++) {
-            const long p = p0 + row + 32 * q;
-            r[q] = g < n8 && p < hi ? *(const uint4 *)(x + p * C + 8 * g) : uint4{0u, 0u, 0u, 0u};
+        for (int q = 0; q < NX; q++) {
+            const int e = k + HB_NT * q, px = e / n8;
+            r[q] = px < SUM_PX && p0 + px < hi ? *(const uint4 *)(x + (p0 + px) * C + 8 * (e - px * n8)) : uint4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const long e = (long)threadIdx.x + 256 * q;   // element of the tile's NO x SUM_PX values
-            rd[q] = q < NO && NO * p0 + e < NO * hi ? dout[NO * p0 + e] : 0.0f;
+        for (int q = 0; q < ND; q++) {
+            const int e = k + HB_NT * q;
+            rd[q] = e < SUM_PX * NO && NO * p0 + e < NO * hi ? dout[NO * p0 + e] : 0.0f;
         }
     };
+    for (int e = k; e < SUM_PX * 16; e += HB_NT) t[e >> 4][64 + (e & 15)] = 0x3f80;   // 1.0
     const bool prod = k < NO * C;
-    const int o = prod ? k / C : k - NO * C, c = prod ? k % C : 0;
-    const int o2 = k + 256 - NO * C;   // lane k's second sum (only where nk > 256): dbh[o2]
-    const bool two = k + 256 < nk;
-    float s = 0.0f, s2 = 0.0f;
+    const int o = prod ? k / C : (k < nk ? k - NO * C : 0), c16 = prod ? k % C - r16 : 64;
+    const bf16_t *tc = &t[r16 >> 2][c16 + 4 * (r16 & 3)];
+    float s = 0.0f;
     load(lo);
     for (long p0 = lo; p0 < hi; p0 += SUM_PX) {
         __syncthreads();   // the previous tile has been added
 #pragma unroll
-        for (int q = 0; q < SUM_PX / 32; q++)
-            if (g < n8) *(uint4 *)&t[row + 32 * q][8 * g] = r[q];
+        for (int q = 0; q < NX; q++) {
+            const int e = k + HB_NT * q, px = e / n8;
+            if (px < SUM_PX) *(uint4 *)&t[px][8 * (e - px * n8)] = r[q];
+        }
 #pragma unroll
-        for (int q = 0; q < 4; q++)
-            if (q < NO) d[threadIdx.x + 256 * q] = rd[q];
+        for (int q = 0; q < ND; q++) {
+            const int e = k + HB_NT * q;
+            if (e < SUM_PX * NO) d[e % NO][e / NO] = rd[q];
+        }
         __syncthreads();
         if (p0 + SUM_PX < hi) load(p0 + SUM_PX);
-        const int n = hi - p0 < SUM_PX ? (int)(hi - p0) : SUM_PX;
-        if (prod) {
-#pragma unroll 16
-            for (int q = 0; q < n; q++) s += d[NO * q + o] * bf2f(t[q][c]);
-        } else if (k < nk) {
-#pragma unroll 16
-            for (int q = 0; q < n; q++) s += d[NO * q + o];
-        }
-        if (two) {
-            for (int q = 0; q < n; q++) s2 += d[NO * q + o2];
+        if (k >= ((nk + 63) & ~63)) continue;   // a wave without a chain
+        if (p0 + SUM_PX <= hi) {
+#pragma unroll 8
+            for (int q = 0; q < SUM_PX; q += 4) {
+                const s16x4 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4 *)(tc + q * HB_LD));
+                const float4 g = *(const float4 *)&d[o][q];
+                s += g.x * bf2f((bf16_t)v[0]);
+                s += g.y * bf2f((bf16_t)v[1]);
+                s += g.z * bf2f((bf16_t)v[2]);
+                s += g.w * bf2f((bf16_t)v[3]);
+            }
+        } else {
+            for (int q = 0; q < (int)(hi - p0); q++) s += d[o][q] * bf2f(t[q][c16 + r16]);
         }
     }
     if (k < nk) part[(long)blockIdx.x * nk + k] = s;
-    if (two) part[(long)blockIdx.x * nk + k + 256] = s2;
 }
 
 // masked mean-squared error: loss partials and d(loss)/d(pred) = 2 m (pred - target) / count
@@ -996,6 +1100,23 @@ inline hipStream_t SS(void *s) { return (hipStream_t)s; }
 bool bad_ch(int c) { return c < 0 || c % 32 != 0 || c > 4096; }
 // 8-channel (16-byte) accesses apply: C % 8 == 0 and both tensors 16-byte aligned
 bool vec8(int C, const void *a, const void *b) { return C % 8 == 0 && (((uintptr_t)a | (uintptr_t)b) & 15) == 0; }
+// head weight-gradient partials, glide_unet_bias_chunks(P) x (NO C + NO)
+void head_bwd_w(const float *dout, const bf16_t *x, long P, int C, int NO, float *partial, hipStream_t st)
+{
+    const int nk = NO * C + NO;
+    const unsigned nz = (unsigned)((P + 4095) / 4096);
+    if (vec8(C, x, x) && C % 16 == 0 && C <= 64) {
+        auto go = [&](auto no) {
+            hipLaunchKernelGGL(k_head_bwd_w_v8<decltype(no)::value>, dim3(nz), dim3(HB_NT), 0, st, dout, x, P, C, 4096L,
+                               partial);
+        };
+        if (NO == 1) return go(std::integral_constant<int, 1>{});
+        if (NO == 2) return go(std::integral_constant<int, 2>{});
+        if (NO == 3) return go(std::integral_constant<int, 3>{});
+        return go(std::integral_constant<int, 4>{});
+    }
+    hipLaunchKernelGGL(k_head_bwd_w, dim3(nz), dim3(((nk + 63) / 64) * 64), 0, st, dout, x, P, C, NO, 4096L, partial);
+}
 // Output channels per wave (16 * NJ) of the direct 3x3 convolution over P
 // pixels: the
 // widest of 64, 32 and 16 that still gives at least 2048 waves (two per
@@ -1021,6 +1142,7 @@ struct ConvArgs {
     int Cout;
     const float *bias;
     int relu;
+    const bf16_t *ya;
     bf16_t *out;
     float *ga;
     int SA, acc_a;
@@ -1033,7 +1155,7 @@ void conv_launch(const ConvArgs &c, hipStream_t st)
 {
     const int tx = (c.W + CV_W - 1) / CV_W, tiles = tx * ((c.H + 2 * NW - 1) / (2 * NW));
     hipLaunchKernelGGL((k_conv3x3<NW, NCH, MODE>), dim3((unsigned)((long)tiles * c.N), c.Cout / 32), dim3(64 * NW), 0,
-                       st, c.xa, c.CA, c.xb, c.H, c.W, tx, tiles, c.Wt, c.Cout, c.bias, c.relu, c.out, c.ga, c.SA,
+                       st, c.xa, c.CA, c.xb, c.H, c.W, tx, tiles, c.Wt, c.Cout, c.bias, c.relu, c.ya, c.out, c.ga, c.SA,
                        c.acc_a, c.gb, c.acc_b);
 }
 // Waves per workgroup (tile rows / 2): the tallest tile reads the fewest halo
@@ -1055,7 +1177,7 @@ template <int NJ, int MODE>
 void conv_direct(const ConvArgs &c, hipStream_t st)
 {
     hipLaunchKernelGGL((k_conv3x3_direct<NJ, MODE>), dim3(nblk((long)c.N * c.H * c.W), c.Cout / (16 * NJ)), dim3(256), 0,
-                       st, c.xa, c.CA, c.xb, c.CB, c.N, c.H, c.W, c.Wt, c.Cout, c.bias, c.relu, c.out, c.ga, c.SA,
+                       st, c.xa, c.CA, c.xb, c.CB, c.N, c.H, c.W, c.Wt, c.Cout, c.bias, c.relu, c.ya, c.out, c.ga, c.SA,
                        c.acc_a, c.gb, c.acc_b);
 }
 // The channel counts of the network's layers have a staged instance.  It reads
@@ -1064,7 +1186,7 @@ void conv_direct(const ConvArgs &c, hipStream_t st)
 template <int MODE>
 void conv(const ConvArgs &c, hipStream_t st)
 {
-    const uintptr_t al = (uintptr_t)c.bias | (uintptr_t)c.out | (uintptr_t)c.ga | (uintptr_t)c.gb;
+    const uintptr_t al = (uintptr_t)c.bias | (uintptr_t)c.ya | (uintptr_t)c.out | (uintptr_t)c.ga | (uintptr_t)c.gb;
     const int nch = (al & 15) ? 0 : (c.CA + c.CB) / 32;
     if (nch == 1) return conv_staged<1, MODE>(c, st);
     if (nch == 2) return conv_staged<2, MODE>(c, st);
@@ -1087,7 +1209,8 @@ int glide_unet_conv3x3(const uint16_t *xa, int CA, const uint16_t *xb, int CB, i
     if (!xa || !weights || !bias || !out || (CB > 0 && !xb)) return ufail(GLIDE_E_NULL, "conv3x3: NULL argument");
     if (bad_ch(CA) || CA == 0 || bad_ch(CB) || bad_ch(Cout) || Cout == 0 || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3: channels must be positive multiples of 32, sizes positive");
-    conv<0>(ConvArgs{xa, CA, xb, CB, N, H, W, weights, Cout, bias, relu, out, nullptr, 0, 0, nullptr, 0}, SS(stream));
+    conv<0>(ConvArgs{xa, CA, xb, CB, N, H, W, weights, Cout, bias, relu, nullptr, out, nullptr, 0, 0, nullptr,
+                     0}, SS(stream));
     return ucheck("conv3x3");
 }
 
@@ -1098,9 +1221,22 @@ int glide_unet_conv3x3_dgrad(const uint16_t *dz, int Cout, int N, int H, int W, 
     if (bad_ch(Cout) || Cout == 0 || bad_ch(CA) || CA == 0 || bad_ch(CB) || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3_dgrad: channels must be positive multiples of 32, sizes positive");
     // the transposed convolution: CA + CB output channels
-    conv<1>(ConvArgs{dz, Cout, nullptr, 0, N, H, W, wflip, CA + CB, nullptr, 0, nullptr, ga, CA, acc_a, gb, acc_b},
+    conv<1>(ConvArgs{dz, Cout, nullptr, 0, N, H, W, wflip, CA + CB, nullptr, 0, nullptr, nullptr, ga, CA, acc_a,
+                     gb, acc_b},
             SS(stream));
     return ucheck("conv3x3_dgrad");
+}
+
+int glide_unet_conv3x3_dgrad_relu(const uint16_t *dz, int Cout, int N, int H, int W, const uint16_t *wflip, int Cin,
+                                  const uint16_t *y, uint16_t *dzin, void *stream)
+{
+    if (!dz || !wflip || !y || !dzin) return ufail(GLIDE_E_NULL, "conv3x3_dgrad_relu: NULL argument");
+    if (dz == dzin) return ufail(GLIDE_E_ARG, "conv3x3_dgrad_relu: dz and dzin must be distinct");
+    if (bad_ch(Cout) || Cout == 0 || bad_ch(Cin) || Cin == 0 || N < 1 || H < 1 || W < 1)
+        return ufail(GLIDE_E_SIZE, "conv3x3_dgrad_relu: channels must be positive multiples of 32, sizes positive");
+    conv<2>(ConvArgs{dz, Cout, nullptr, 0, N, H, W, wflip, Cin, nullptr, 0, y, dzin, nullptr, 0, 0, nullptr, 0},
+            SS(stream));
+    return ucheck("conv3x3_dgrad_relu");
 }
 
 long glide_unet_wgrad_chunks(int N, int H, int W) { return ((long)N * H * W + 4095) / 4096; }
@@ -1235,15 +1371,52 @@ int glide_unet_head_bwd(const float *dout, const uint16_t *x, long P, int C, int
     if (P < 1 || C < 1 || NO < 1 || NO > 4 || nk > 1024) return ufail(GLIDE_E_SIZE, "head_bwd: bad size");
     hipLaunchKernelGGL(k_head_bwd_x, dim3(nblk(P * C)), dim3(256), 0, SS(stream), dout, P, C, NO, wh, dx);
     const long nz = glide_unet_bias_chunks(P);
-    if (vec8(C, x, x) && C <= 64)
-        hipLaunchKernelGGL(k_head_bwd_w_v8, dim3((unsigned)nz), dim3(256), 0, SS(stream), dout, x, P, C, NO, 4096L,
-                           partial);
-    else
-        hipLaunchKernelGGL(k_head_bwd_w, dim3((unsigned)nz), dim3(((nk + 63) / 64) * 64), 0, SS(stream), dout, x, P,
-                           C, NO, 4096L, partial);
+    head_bwd_w(dout, x, P, C, NO, partial, SS(stream));
     hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(nk)), dim3(256), 0, SS(stream), partial, (long)nk, (int)nz, dwh_dbh,
                        (const float *)nullptr, 0L, (float *)nullptr);
     return ucheck("head_bwd");
+}
+
+int glide_unet_head_bwd_relu(const float *dout, const uint16_t *x, long P, int C, int NO, const float *wh, uint16_t *dz,
+                             float *partial, float *dwh_dbh, void *stream)
+{
+    if (!dout || !x || !wh || !dz || !partial || !dwh_dbh) return ufail(GLIDE_E_NULL, "head_bwd_relu: NULL argument");
+    const int nk = NO * C + NO;
+    if (P < 1 || C < 1 || C % 8 || NO < 1 || NO > 4 || nk > 1024) return ufail(GLIDE_E_SIZE, "head_bwd_relu: bad size");
+    if (!vec8(C, x, dz)) return ufail(GLIDE_E_ARG, "head_bwd_relu: x and dz must be 16-byte aligned");
+    const dim3 grid(nblk(P * (C / 8)));
+    hipStream_t st = SS(stream);
+    if (NO == 1) hipLaunchKernelGGL(k_head_bwd_relu<1>, grid, dim3(256), 0, st, dout, x, P, C, wh, dz);
+    if (NO == 2) hipLaunchKernelGGL(k_head_bwd_relu<2>, grid, dim3(256), 0, st, dout, x, P, C, wh, dz);
+    if (NO == 3) hipLaunchKernelGGL(k_head_bwd_relu<3>, grid, dim3(256), 0, st, dout, x, P, C, wh, dz);
+    if (NO == 4) hipLaunchKernelGGL(k_head_bwd_relu<4>, grid, dim3(256), 0, st, dout, x, P, C, wh, dz);
+    head_bwd_w(dout, x, P, C, NO, partial, st);
+    hipLaunchKernelGGL(k_reduce_chunks, dim3(nblk(nk)), dim3(256), 0, st, partial, (long)nk,
+                       (int)glide_unet_bias_chunks(P), dwh_dbh, (const float *)nullptr, 0L, (float *)nullptr);
+    return ucheck("head_bwd_relu");
+}
+
+int glide_unet_pool2_bwd_relu(const float *dy, const float *g, int N, int H, int W, int C, const uint16_t *y,
+                              uint16_t *dz, void *stream)
+{
+    if (!dy || !g || !y || !dz) return ufail(GLIDE_E_NULL, "pool2_bwd_relu: NULL argument");
+    if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C < 8 || C % 8)
+        return ufail(GLIDE_E_SIZE, "pool2_bwd_relu: even sizes and channels in multiples of 8 required");
+    if (!vec8(C, dy, g) || !vec8(C, y, dz)) return ufail(GLIDE_E_ARG, "pool2_bwd_relu: tensors must be 16-byte aligned");
+    hipLaunchKernelGGL(k_pool2_bwd_relu, dim3(nblk((long)N * H * W * (C / 8))), dim3(256), 0, SS(stream), dy, g, N, H, W,
+                       C, y, dz);
+    return ucheck("pool2_bwd_relu");
+}
+
+int glide_unet_up2_bwd_relu(const float *dy, int N, int H, int W, int C, const uint16_t *y, uint16_t *dz, void *stream)
+{
+    if (!dy || !y || !dz) return ufail(GLIDE_E_NULL, "up2_bwd_relu: NULL argument");
+    if (N < 1 || H < 1 || W < 1 || C < 8 || C % 8)
+        return ufail(GLIDE_E_SIZE, "up2_bwd_relu: positive sizes and channels in multiples of 8 required");
+    if (!vec8(C, dy, y) || !vec8(C, dz, dz)) return ufail(GLIDE_E_ARG, "up2_bwd_relu: tensors must be 16-byte aligned");
+    hipLaunchKernelGGL(k_up2_bwd_relu, dim3(nblk((long)N * H * W * (C / 8))), dim3(256), 0, SS(stream), dy, N, H, W, C, y,
+                       dz);
+    return ucheck("up2_bwd_relu");
 }
 
 long glide_unet_mse_blocks(long n) { return (n + 255) / 256; }

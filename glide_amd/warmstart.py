@@ -122,14 +122,15 @@ class UNet:
         b = {"acts": acts, "dims": dims,
              "pred": torch.empty(N * H * W * N_OUT, dtype=torch.float32, device=self.device)}
         if train:
+            # FP32 gradients of the pooled, upsampled and skip tensors; every other layer's gradient goes
+            # through its ReLU into dz as it is formed
             g = {}
-            for name in CH:
-                if name == "x0":
-                    continue
+            for name in list(POOLS) + list(UPS) + list(POOLS.values()):
                 h, w = dims[LEVEL[name]]
                 g[name] = torch.empty(N * h * w * CH[name], dtype=torch.float32, device=self.device)
             b["g"] = g
-            b["dz"] = torch.empty(max(a.numel() for a in acts.values()), dtype=torch.int16, device=self.device)
+            n_dz = max(a.numel() for a in acts.values())
+            b["dz"] = [torch.empty(n_dz, dtype=torch.int16, device=self.device) for _ in range(2)]
             part = 0
             for name, ins, co in LAYERS:
                 h, w = dims[LEVEL[name]]
@@ -188,33 +189,36 @@ class UNet:
         dpred = b["dpred"] if dpred is None else dpred
         P0 = N * H * W
         C = CH[HEAD_IN]
-        _lib.call("glide_unet_head_bwd", _p(dpred), _p(acts[HEAD_IN]), P0, C, N_OUT, _p(self.params["head.W"]),
-                  _p(g[HEAD_IN]), _p(b["partial"]), _p(b["head"]), st)
+        # dz of the layer at hand and of the one below it (a layer's data gradient reads one and writes the other)
+        dz, dz_next = b["dz"]
+        _lib.call("glide_unet_head_bwd_relu", _p(dpred), _p(acts[HEAD_IN]), P0, C, N_OUT, _p(self.params["head.W"]),
+                  _p(dz), _p(b["partial"]), _p(b["head"]), st)
         self.grads["head.W"].copy_(b["head"][:N_OUT * C].view(N_OUT, C))
         self.grads["head.b"].copy_(b["head"][N_OUT * C:])
-        dz = b["dz"]
         for name, ins, co in reversed(LAYERS):
             h, w = dims[LEVEL[name]]
-            n = N * h * w * co
-            _lib.call("glide_unet_relu_bwd", _p(g[name]), _p(acts[name]), n, _p(dz), st)
             xa, xb = acts[ins[0]], (acts[ins[1]] if len(ins) > 1 else None)
             ca, cb = CH[ins[0]], (CH[ins[1]] if xb is not None else 0)
             _lib.call("glide_unet_conv3x3_wgrad_bias", _p(dz), co, _p(xa), ca, _p(xb), cb, N, h, w, _p(b["partial"]),
                       _p(self.grads[name + ".W"]), _p(self.grads[name + ".b"]), st)
             if ins == ["x0"]:
                 continue
-            gb = g[ins[1]] if xb is not None else None
-            _lib.call("glide_unet_conv3x3_dgrad", _p(dz), co, N, h, w, _p(self.wf[name]), ca, _p(g[ins[0]]), 0, cb,
-                      _p(gb), 0, st)
-            for i in ins:
-                if i in UPS:
-                    src = UPS[i]
-                    hs, ws = dims[LEVEL[src]]
-                    _lib.call("glide_unet_up2_bwd", _p(g[i]), N, hs, ws, CH[src], _p(g[src]), st)
-                if i in POOLS:
-                    src = POOLS[i]
-                    hs, ws = dims[LEVEL[src]]
-                    _lib.call("glide_unet_pool2_bwd", _p(g[i]), N, hs, ws, CH[src], _p(g[src]), 1, st)
+            src = ins[0]
+            if src in POOLS or src in UPS:
+                _lib.call("glide_unet_conv3x3_dgrad", _p(dz), co, N, h, w, _p(self.wf[name]), ca, _p(g[src]), 0, cb,
+                          _p(g[ins[1]]) if xb is not None else None, 0, st)
+                below = POOLS.get(src) or UPS[src]
+                hs, ws = dims[LEVEL[below]]
+                if src in POOLS:
+                    _lib.call("glide_unet_pool2_bwd_relu", _p(g[src]), _p(g[below]), N, hs, ws, CH[below],
+                              _p(acts[below]), _p(dz_next), st)
+                else:
+                    _lib.call("glide_unet_up2_bwd_relu", _p(g[src]), N, hs, ws, CH[below], _p(acts[below]),
+                              _p(dz_next), st)
+            else:
+                _lib.call("glide_unet_conv3x3_dgrad_relu", _p(dz), co, N, h, w, _p(self.wf[name]), ca, _p(xa),
+                          _p(dz_next), st)
+            dz, dz_next = dz_next, dz
 
     def adam_step(self, lr: float, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8, weight_decay: float = 0.0):
         self.step_count += 1

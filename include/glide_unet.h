@@ -37,6 +37,12 @@ int glide_unet_conv3x3(const uint16_t *xa, int CA, const uint16_t *xb, int CB, i
 int glide_unet_conv3x3_dgrad(const uint16_t *dz, int Cout, int N, int H, int W, const uint16_t *wflip,
                              int CA, float *ga, int acc_a, int CB, float *gb, int acc_b, void *stream);
 
+/* The data gradient of a convolution whose one input is itself a ReLU's output
+ * y, through that ReLU: dzin = bf16(dx * (y > 0)) (Cin channels), the bits of
+ * glide_unet_conv3x3_dgrad followed by glide_unet_relu_bwd. */
+int glide_unet_conv3x3_dgrad_relu(const uint16_t *dz, int Cout, int N, int H, int W, const uint16_t *wflip,
+                                  int Cin, const uint16_t *y, uint16_t *dzin, void *stream);
+
 /* Weight gradient dw[t][co][ci] = sum_p dz[p][co] x[p+off_t][ci] (FP32),
  * split over pixel chunks into partial (glide_unet_wgrad_chunks(N, H, W) x 9
  * x Cout x (CA+CB) floats) and reduced in chunk order (deterministic). */
@@ -83,6 +89,19 @@ int glide_unet_head(const uint16_t *x, long P, int C, int NO, const float *wh, c
                     void *stream);
 int glide_unet_head_bwd(const float *dout, const uint16_t *x, long P, int C, int NO, const float *wh,
                         float *dx, float *partial, float *dwh_dbh, void *stream);
+
+/* Backward passes that end at a ReLU's output y, through it, with the bits of
+ * the FP32 pass followed by glide_unet_relu_bwd: of the head whose input x is
+ * that output (glide_unet_head_bwd with dz in dx's place), of 2x2 pooling
+ * added to the gradient g of y's other uses (glide_unet_pool2_bwd with
+ * accumulate), and of upsampling (N x H x W is y's size).  Channels in
+ * multiples of 8, tensors 16-byte aligned. */
+int glide_unet_head_bwd_relu(const float *dout, const uint16_t *x, long P, int C, int NO, const float *wh,
+                             uint16_t *dz, float *partial, float *dwh_dbh, void *stream);
+int glide_unet_pool2_bwd_relu(const float *dy, const float *g, int N, int H, int W, int C, const uint16_t *y,
+                              uint16_t *dz, void *stream);
+int glide_unet_up2_bwd_relu(const float *dy, int N, int H, int W, int C, const uint16_t *y, uint16_t *dz,
+                            void *stream);
 
 /* Masked MSE: grad = 2 m (pred - target) inv_count (mask per pixel of 2
  * values, may be NULL); per-block loss partials (glide_unet_mse_blocks(n)). */

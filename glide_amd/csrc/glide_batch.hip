@@ -102,10 +102,10 @@ __global__ __launch_bounds__(BTX *TY) void kb_residual(const BEntry *__restrict_
         const int lt = t - pre[e], tx = cdiv(A.g.nx, BTX);   // cell tiles; edge faces by the last tiles
         __syncthreads();   // the previous tile's readers of S are done
         if (CHILD)
-            residual_tile_lds<BTX, TY, true>(A.g, to_params(A.p), A.f, A.U, nullptr, A.r, A.bed, A.B, A.beta, A.mask,
+            residual_tile_lds<BTX, TY>(A.g, to_params(A.p), A.f, A.U, nullptr, A.r, A.bed, A.B, A.beta, A.mask,
                                              A.gamma, lt % tx, lt / tx, S);
         else
-            residual_tile_lds<BTX, TY, true>(A.g, to_params(A.p), A.r, A.U, A.f, nullptr, A.bed, A.B, A.beta, A.mask,
+            residual_tile_lds<BTX, TY>(A.g, to_params(A.p), A.r, A.U, A.f, nullptr, A.bed, A.B, A.beta, A.mask,
                                              A.gamma, lt % tx, lt / tx, S);
     });
 }

@@ -17,6 +17,7 @@
 #include <cstring>
 #include <mutex>
 #include <string>
+#include <type_traits>
 
 #include "glide_hip.h"
 #include "tiles_device.h"
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(TX *RTY) void k_residual(GlideGeom g, Params p, dou
     const int tx = cdiv(g.nx, TX), total = tx * cdiv(g.ny, RTY);   // cell tiles; edge faces by the last tiles
     tile_loop(total, [&](int t) {
         __syncthreads();   // the previous tile's readers of S are done
-        residual_tile_lds<TX, RTY, true>(g, p, r, U, f, sub, bed, B, beta, mask, gamma, t % tx, t / tx, S);
+        residual_tile_lds<TX, RTY>(g, p, r, U, f, sub, bed, B, beta, mask, gamma, t % tx, t / tx, S);
     });
 }
 
@@ -149,20 +150,25 @@ __global__ __launch_bounds__(TX *RTY) void k_residual(GlideGeom g, Params p, dou
 // (interior and general) must share.  Large levels take 2 (occupancy hides
 // the Newton chain's latency); small levels, whose few waves each run alone
 // on a SIMD, take 1 (the whole register file: no spills, longer schedules).
-template <bool LOCAL, int WPE>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_vanka(GlideGeom g, Params p,
-                                                                                   const double *__restrict__ U,
-                                              const double *__restrict__ f, const double *__restrict__ bed,
-                                              const double *__restrict__ B, const double *__restrict__ beta,
-                                              const double *__restrict__ gamma, const unsigned char *__restrict__ blk,
-                                              int nbx, int n_newton, double *__restrict__ cd)
+// LOOP: fewer workgroups than tiles, each looping over tiles (tile_loop); kept
+// apart because the loop's hoisted values cost the straight kernel 300 bytes
+// of spill per lane.
+template <bool LOCAL, int WPE, bool LOOP>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_vanka(
+    GlideGeom g, Params p, const double *__restrict__ U, const double *__restrict__ f, const double *__restrict__ bed,
+    const double *__restrict__ B, const double *__restrict__ beta, const double *__restrict__ gamma,
+    const unsigned char *__restrict__ blk, int nbx, int n_newton, double *__restrict__ cd)
 {
     __shared__ VankaLDS<TX, TY> L;
     const int tx = cdiv(g.nx, TX), total = tx * cdiv(g.ny, TY);
-    tile_loop(total, [&](int t) {
-        __syncthreads();   // the previous tile's readers of L are done
-        vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, t % tx, t / tx, L);
-    });
+    if (LOOP)
+        tile_loop(total, [&](int t) {
+            __syncthreads();   // the previous tile's readers of L are done
+            vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, t % tx, t / tx, L);
+        });
+    else if ((int)blockIdx.x < total)
+        vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, blockIdx.x % tx,
+                                  blockIdx.x / tx, L);
 }
 
 // Small-level sweep with the apply pass folded in (vanka_halo_tile): U -> Uo,
@@ -1151,75 +1157,44 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
 {
     const int nbx = nbx_of(g.nx);
     const bool small = (long)g.ny * g.nx <= g_small_max_cells;
-    const bool rows = small && g_small_variant == 1;
-    const dim3 rgrid(cdiv(g.nx, 64), g.ny), rblock(64, ROW_WAVES);
-    if (small && g_small_variant == 2) {
-        // The sweeps alternate the state between U and the scratch (5 nc >=
-        // nu + nv + nc doubles); an odd count runs its first sweep in place
-        // with the apply pass, so that the last sweep writes U.
+    const int variant = g_small_variant;
+    const bool rows = small && variant == 1;
+    const dim3 block(TX, TY), rblock(64, ROW_WAVES), rgrid(cdiv(g.nx, 64), g.ny);
+    const dim3 vgrid = vanka_grid(g.ny, g.nx), pgrid = point_grid(g.ny, g.nx), hgrid = halo_grid(g.ny, g.nx);
+    const bool loop = (long)vgrid.x < (long)cdiv(g.nx, TX) * cdiv(g.ny, TY);
+    auto sweep = [&](auto local) {   // one sweep in place: the smoother, then the apply pass
+        constexpr bool LOCAL = decltype(local)::value;
+        if (rows)
+            hipLaunchKernelGGL(k_vanka_rows<LOCAL>, rgrid, rblock, 0, st, g, p, U, f, bed, B, beta, gamma, blk, nbx,
+                               n_newton, scratch);
+        else if (small)
+            hipLaunchKernelGGL((loop ? k_vanka<LOCAL, 1, true> : k_vanka<LOCAL, 1, false>), vgrid, block, 0, st, g, p, U, f,
+                               bed, B, beta, gamma, blk, nbx, n_newton, scratch);
+        else
+            hipLaunchKernelGGL((loop ? k_vanka<LOCAL, 2, true> : k_vanka<LOCAL, 2, false>), vgrid, block, 0, st, g, p, U, f,
+                               bed, B, beta, gamma, blk, nbx, n_newton, scratch);
+        hipLaunchKernelGGL(k_vanka_apply<LOCAL>, pgrid, block, 0, st, g.ny, g.nx, U, scratch, blk, nbx);
+    };
+    auto run = [&](auto local) {
+        constexpr bool LOCAL = decltype(local)::value;
         int s = 0;
-        if (n_sweeps & 1) {
-            if (blk) {
-                hipLaunchKernelGGL((k_vanka<true, 1>), vanka_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, U, f, bed,
-                                   B, beta, gamma, blk, nbx, n_newton, scratch);
-                hipLaunchKernelGGL(k_vanka_apply<true>, point_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g.ny, g.nx, U,
-                                   scratch, blk, nbx);
-            } else {
-                hipLaunchKernelGGL((k_vanka<false, 1>), vanka_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, U, f, bed,
-                                   B, beta, gamma, blk, nbx, n_newton, scratch);
-                hipLaunchKernelGGL(k_vanka_apply<false>, point_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g.ny, g.nx, U,
-                                   scratch, blk, nbx);
-            }
-            s = 1;
-        }
-        for (; s < n_sweeps; s++) {
-            const bool to_u = ((n_sweeps - 1 - s) & 1) == 0;
-            const double *src = to_u ? scratch : U;
-            double *dst = to_u ? U : scratch;
-            if (blk)
-                hipLaunchKernelGGL(k_vanka_halo<true>, halo_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, src, dst, f,
-                                   bed, B, beta, gamma, blk, nbx, n_newton);
-            else
-                hipLaunchKernelGGL(k_vanka_halo<false>, halo_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, src, dst,
+        if (small && variant == 2) {
+            // The sweeps alternate the state between U and the scratch (5 nc >=
+            // nu + nv + nc doubles); an odd count runs its first sweep in place
+            // with the apply pass, so that the last sweep writes U.
+            if (n_sweeps & 1) sweep(local), s = 1;
+            for (; s < n_sweeps; s++) {
+                const bool to_u = ((n_sweeps - 1 - s) & 1) == 0;
+                hipLaunchKernelGGL(k_vanka_halo<LOCAL>, hgrid, block, 0, st, g, p, to_u ? scratch : U, to_u ? U : scratch,
                                    f, bed, B, beta, gamma, blk, nbx, n_newton);
-        }
-        return check_launch("vanka sweep");
-    }
-    for (int s = 0; s < n_sweeps; s++) {
-        if (rows) {
-            if (blk) {
-                hipLaunchKernelGGL(k_vanka_rows<true>, rgrid, rblock, 0, st, g, p, U, f, bed, B, beta, gamma, blk, nbx,
-                                   n_newton, scratch);
-                hipLaunchKernelGGL(k_vanka_apply<true>, point_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g.ny, g.nx, U,
-                                   scratch, blk, nbx);
-            } else {
-                hipLaunchKernelGGL(k_vanka_rows<false>, rgrid, rblock, 0, st, g, p, U, f, bed, B, beta, gamma, blk,
-                                   nbx, n_newton, scratch);
-                hipLaunchKernelGGL(k_vanka_apply<false>, point_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g.ny, g.nx, U,
-                                   scratch, blk, nbx);
             }
-            continue;
         }
-        if (blk) {
-            if (small)
-                hipLaunchKernelGGL((k_vanka<true, 1>), vanka_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, U, f, bed, B,
-                                   beta, gamma, blk, nbx, n_newton, scratch);
-            else
-                hipLaunchKernelGGL((k_vanka<true, 2>), vanka_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, U, f, bed, B,
-                                   beta, gamma, blk, nbx, n_newton, scratch);
-            hipLaunchKernelGGL(k_vanka_apply<true>, point_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g.ny, g.nx, U,
-                               scratch, blk, nbx);
-        } else {
-            if (small)
-                hipLaunchKernelGGL((k_vanka<false, 1>), vanka_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, U, f, bed,
-                                   B, beta, gamma, blk, nbx, n_newton, scratch);
-            else
-                hipLaunchKernelGGL((k_vanka<false, 2>), vanka_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g, p, U, f, bed,
-                                   B, beta, gamma, blk, nbx, n_newton, scratch);
-            hipLaunchKernelGGL(k_vanka_apply<false>, point_grid(g.ny, g.nx), dim3(TX, TY), 0, st, g.ny, g.nx, U,
-                               scratch, blk, nbx);
-        }
-    }
+        for (; s < n_sweeps; s++) sweep(local);
+    };
+    if (blk)
+        run(std::true_type{});
+    else
+        run(std::false_type{});
     return check_launch("vanka sweep");
 }
 

@@ -19,10 +19,10 @@
 //  - u - 0.25 d as one fma (0.25 d is exact);
 //  - the range handling of divisions, exp and log, whose arguments are in
 //    range here (recip, exp_mid, log_normal below).
-// 223 FP64 instructions an iteration instead of about 590 (781 VALU in all,
-// interior form).  Measured per sweep, 10 iterations, with its apply pass:
-// 32^2 20.2 -> 12.7 us, 512^2 65.1 -> 44.4 us; a 512^2 step to 1e-8 82.8 ->
-// 59.4 ms.
+// 348 FP64 instructions an iteration instead of about 590 (781 VALU in all,
+// interior form), 308 where the sigmoid is clamped (newton_iterate).  Measured
+// per sweep, 10 iterations, with its apply pass: 32^2 20.2 -> 12.1 us, 512^2
+// 65.1 -> 41.6 us; a 512^2 step to 1e-8 82.8 -> 56.8 ms.
 // Terms that vanish at the domain edge are multiplied by a factor held per
 // cell (1/(2 dx) or 0 per face, 1/dx or 0 per vertex), constants where the
 // whole tile is interior.  The only differences from the assembly are signs of
@@ -140,12 +140,10 @@ __host__ __device__ __forceinline__ double log_normal(double x)
 // dm_pow(x, p) for x >= 0: the short forms where x is normal and |p log x| <= 700
 __host__ __device__ __forceinline__ double pow_pos(double x, double p)
 {
-    if (x >= 2.2250738585072014e-308 && x <= 1.7976931348623157e308) {
-        const double y = p * log_normal(x);
-        if (fabs(y) <= 700.0) return exp_mid(y);
-        return dm_exp(y);
-    }
-    return dm_pow(x, p);
+    const double y = p * log_normal(x);
+    double r = exp_mid(y);
+    if (!(x >= 2.2250738585072014e-308 && x <= 1.7976931348623157e308 && fabs(y) <= 700.0)) r = dm_pow(x, p);
+    return r;
 }
 
 // sigm (ssa_device.h): the clamped argument keeps exp in range and 1 + exp in [1, 4.9e8]
@@ -153,6 +151,13 @@ __host__ __device__ __forceinline__ double sigm_mid(double z, double c)
 {
     const double s = fmin(fmax(c * z, -20.0), 20.0);
     return recip(1.0 + exp_mid(-s));
+}
+// sigm where the argument reaches the clamp (a NaN counts as -20, as in sigm):
+// 1 / (1 + e^-20) and 1 / (1 + e^20)
+__host__ __device__ __forceinline__ bool sigm_clamped(double z, double c) { return !(fabs(c * z) < 20.0); }
+__host__ __device__ __forceinline__ double sigm_end(double z, double c)
+{
+    return c * z > 0.0 ? 0x1.ffffffee4b79ap-1 : 0x1.1b4865556b5d5p-29;
 }
 __host__ __device__ __forceinline__ Ground ground_mid(double bed, double H, const Params &p)
 {
@@ -229,12 +234,15 @@ struct NewtonX {
     double u_l, u_r, v_t, v_b, H;
 };
 
-// One damped iteration x -= 0.25 A^-1 r, H = max(H, th).
+// One damped iteration x -= 0.25 A^-1 r, H = max(H, th).  CLAMPED: the cell's
+// sigmoid argument reaches its clamp; GL: p.gl_derivatives.
+template <bool CLAMPED, bool GL>
 __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const NewtonK &K, const Params &p, NewtonX &x)
 {
     const double u_l = x.u_l, u_r = x.u_r, v_t = x.v_t, v_b = x.v_b, H = x.H;
     // the cell's own sigmoid, drag and surface
-    const double g = sigm_mid(fma(0.917, H, C.bed), p.gl_c);
+    const double z = fma(0.917, H, C.bed);
+    const double g = CLAMPED ? sigm_end(z, p.gl_c) : sigm_mid(z, p.gl_c);
     const double g1 = 1.0 - g;
     const double be = fma(g, C.beta, g1 * p.water_drag);
     const double Hf = -0.917 * H;
@@ -246,30 +254,30 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
     const double cal = p.calving_rate * g1;
     double qH = K.idt + cal;
     r4 = r4 + cal * H;
-    if (p.gl_derivatives) qH = K.idt - fma(p.calving_rate * H, 0.917 * (p.gl_c * g * g1), -cal);
+    if (GL) qH = K.idt - fma(p.calving_rate * H, 0.917 * (p.gl_c * g * g1), -cal);
     const double s_l = C.H_l + H, s_r = H + C.H_r, s_t = C.H_t + H, s_b = H + C.H_b;
     double q0, q1, q2, q3;
     {   // twice the flux and its derivatives; the factors F carry 1/(2 dx)
         const double d = H - C.H_l, f = fma(s_l, u_l, -(fabs(u_l) * d));
-        q0 = -fma(-copysign(1.0, u_l), d, s_l) * C.F_l;
+        q0 = fma(copysign(1.0, u_l), d, -s_l) * C.F_l;
         qH = fma(-(u_l - fabs(u_l)), C.F_l, qH);
         r4 = fma(-f, C.F_l, r4);
     }
     {
         const double d = C.H_r - H, f = fma(s_r, u_r, -(fabs(u_r) * d));
-        q1 = fma(-copysign(1.0, u_r), d, s_r) * C.F_r;
+        q1 = -fma(copysign(1.0, u_r), d, -s_r) * C.F_r;
         qH = fma(u_r + fabs(u_r), C.F_r, qH);
         r4 = fma(f, C.F_r, r4);
     }
     {
         const double d = C.H_t - H, f = fma(s_t, v_t, -(fabs(v_t) * d));
-        q2 = fma(-copysign(1.0, v_t), d, s_t) * C.F_t;
+        q2 = -fma(copysign(1.0, v_t), d, -s_t) * C.F_t;
         qH = fma(v_t + fabs(v_t), C.F_t, qH);
         r4 = fma(f, C.F_t, r4);
     }
     {
         const double d = H - C.H_b, f = fma(s_b, v_b, -(fabs(v_b) * d));
-        q3 = -fma(-copysign(1.0, v_b), d, s_b) * C.F_b;
+        q3 = fma(copysign(1.0, v_b), d, -s_b) * C.F_b;
         qH = fma(-(v_b - fabs(v_b)), C.F_b, qH);
         r4 = fma(-f, C.F_b, r4);
     }
@@ -370,7 +378,7 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
         a2 = fma(-0.5, b_t, a2);
         r3 = fma(-0.5, b_b * v_b, r3);
         a3 = fma(-0.5, b_b, a3);
-        if (p.gl_derivatives) {
+        if (GL) {
             const double db = (0.917 * (p.gl_c * g * g1)) * (C.beta - p.water_drag);
             c0 = c0 + -0.5 * db * u_l;
             c1 = c1 + -0.5 * db * u_r;
@@ -445,6 +453,32 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
     x.v_t = fma(-0.25, x2, v_t);
     x.v_b = fma(-0.25, x3, v_b);
     x.H = fmax(fma(-0.25, x4, H), C.th);
+}
+
+// n_newton iterations.  Ice 200 m above or below flotation (at the default
+// sharpness) has its sigmoid clamped; where every lane of the wave has, which
+// is most of a sheet, an iteration takes the clamped form's 5 instructions for
+// the 40 of exp and division.  The branch selects whole iterations, so that each form is
+// scheduled as one block: the sigmoid's chain hides among the rest of the
+// assembly (as a branch of its own it cost waves at a grounding line 1.4%).
+// Ten sweeps of 1024^2: 1632 -> 1480 us.
+__host__ __device__ __forceinline__ void newton_iterate(const NewtonCell &C, const NewtonK &K, const Params &p, int n_newton,
+                                               NewtonX &x)
+{
+    if (p.gl_derivatives) {
+        for (int k = 0; k < n_newton; k++) newton_step<false, true>(C, K, p, x);
+        return;
+    }
+    for (int k = 0; k < n_newton; k++) {
+        bool clamped = sigm_clamped(fma(0.917, x.H, C.bed), p.gl_c);
+#if defined(__HIP_DEVICE_COMPILE__)
+        clamped = __builtin_amdgcn_ballot_w64(!clamped) == 0;
+#endif
+        if (clamped)
+            newton_step<true, false>(C, K, p, x);
+        else
+            newton_step<false, false>(C, K, p, x);
+    }
 }
 
 }  // namespace glide

@@ -37,21 +37,32 @@ __host__ __device__ inline size_t n_v(int ny, int nx) { return (size_t)(ny + 1) 
 __host__ __device__ inline size_t n_c(int ny, int nx) { return (size_t)ny * nx; }
 __host__ __device__ inline size_t n_t(int ny, int nx) { return n_u(ny, nx) + n_v(ny, nx) + n_c(ny, nx); }
 
+// Byte offsets of a tile's neighbourhood in a row-major field of `cols` columns:
+// a base that is the same for the whole tile (row rb, column cb) and 32-bit
+// offsets from it, so an access is one instruction (scalar base plus vector
+// offset) where 64-bit element arithmetic took four to six.  (r, c) must not
+// lie before (rb, cb) and at most 2^16 columns times some 20 rows after it.
+struct TileField {
+    uint32_t pitch;
+    size_t org;
+    __device__ __forceinline__ TileField(int cols, int rb, int cb) : pitch(8u * (uint32_t)cols), org((size_t)rb * cols + cb) {}
+    __device__ __forceinline__ const char *base(const double *a) const { return (const char *)(a + org); }
+};
+__device__ __forceinline__ double ld_off(const char *base, uint32_t off) { return *(const double *)(base + off); }
+
 template <class Body>
 __device__ __forceinline__ void tile_loop(int total, const Body &body)
 {
     const int G = gridDim.x, b = blockIdx.x;
-    if (G >= total) {
-        if (b < total) body(b);
-        return;
-    }
+    const bool one = G >= total;   // tile b only; one loop for both cases, so that the body is compiled once
     const int tch = max(1, min(TCH, total / (2 * NXCD)));
     const int x = b % NXCD, lane = b / NXCD;
     const int nwg = (G - x + NXCD - 1) / NXCD;
     const int nchunks = (total + tch - 1) / tch;
     const int my_chunks = nchunks > x ? (nchunks - x + NXCD - 1) / NXCD : 0;
-    for (int k = lane; k < my_chunks * tch; k += nwg) {
-        const int t = (x + NXCD * (k / tch)) * tch + k % tch;
+    const int first = one ? 0 : lane, end = one ? 1 : my_chunks * tch, step = one ? 1 : nwg;
+    for (int k = first; k < end; k += step) {
+        const int t = one ? b : (x + NXCD * (k / tch)) * tch + k % tch;
         if (t < total) body(t);
     }
 }
@@ -90,36 +101,65 @@ __device__ __forceinline__ void fill_eta_tile(double (*eta_s)[TX + 2], int i0, i
     }
 }
 
+// 2 eta of cell (i, j) (eta_cell, ssa_device.h) from its face velocities and
+// the next ones along each face's line (u_tl = u[i-1, j], v_lt = v[i, j-1], ...):
+// the factors of 1/2 of the corner shear rates, their mean square and eta
+// itself are exact and ride on one constant; corners on the domain edge get
+// the factor 0.
+__device__ __forceinline__ double eta2_from(int i, int j, int ny, int nx, double u_l, double u_r, double v_t, double v_b,
+                                            double u_tl, double u_tr, double u_bl, double u_br, double v_lt,
+                                            double v_rt, double v_lb, double v_rb, double Bc, const Params &p,
+                                            double glen_exp, double dxi)
+{
+    const double dudx = (u_r - u_l) * dxi, dvdy = (v_t - v_b) * dxi;
+    const bool t = i > 0, b = i < ny - 1, l = j > 0, r = j < nx - 1;
+    const double V_tl = t && l ? dxi : 0.0, V_tr = t && r ? dxi : 0.0, V_bl = b && l ? dxi : 0.0, V_br = b && r ? dxi : 0.0;
+    const double e_tl = fma(u_tl - u_l, V_tl, (v_t - v_lt) * V_tl);
+    const double e_tr = fma(u_tr - u_r, V_tr, (v_rt - v_t) * V_tr);
+    const double e_bl = fma(u_l - u_bl, V_bl, (v_b - v_lb) * V_bl);
+    const double e_br = fma(u_r - u_br, V_br, (v_rb - v_b) * V_br);
+    const double e2 = fma(e_br, e_br, fma(e_bl, e_bl, fma(e_tr, e_tr, e_tl * e_tl)));
+    const double eII = fma(0.0625, e2, fma(dudx, dvdy, fma(dvdy, dvdy, dudx * dudx))) + p.eps_reg;
+    return Bc * pow_pos(eII, glen_exp);
+}
 // ---------------------------------------------------------------------------
 // Residual r = F(U) - f (- sub)  (glide/cuda/residuals.cu:6-292), LDS-staged:
-// the tile's u, v (two-ring halo), H, bed, beta (one-ring halo) are staged
-// once; every cell's viscosity, grounding sigmoid, sigma_xx and sigma_yy and
-// every vertex's sigma_xy are evaluated once into LDS; each point then sums
-// its rows from LDS.  Every quantity is the same expression of the same
-// (clamped) values as in the per-point form of the reference and the oracle,
-// and each row sums its terms in the same order, so the bits are the same.
+// the tile's u and v (two-ring halo) are staged once; every cell of the tile
+// and the ring around it then yields 2 eta H, its normal stresses, surface and
+// drag, and every vertex its shear stress, each evaluated once into LDS; each
+// point sums its rows from LDS.
+//
+// Every row sums its terms in the order of the reference and the oracle, and
+// every term has their rounding: what differs is powers of two, which are
+// exact (2 eta H in eta H's place, the factors of the stresses, drags, fluxes
+// and averages on the constants 1/(2 dx) and 1/(8 dx)), the range handling of
+// the divisions, exp and log (newton_device.h), and terms that vanish at the
+// domain edge, which get a factor of 0.  So the bits are the same up to the
+// sign of zeros.
+//
+// Bound by FP64 issue: about half of it is the power law and the sigmoid per
+// haloed cell.  512^2: 11.5 -> 9.2 us; 1024^2 on new data each pass: 47.9 ->
+// 39.7 us (3.0 TB/s of compulsory traffic; 24 us at the rate of a large copy).
 // ---------------------------------------------------------------------------
 template <int TX, int TY>
 struct ResidLDS {
     double u[TY + 4][TX + 4];   // u[i0-2+a][j0-2+b] (clamped)
     double v[TY + 4][TX + 4];   // v[i0-2+a][j0-2+b] (clamped)
-    double H[TY + 2][TX + 2];   // cells [i0-1+a][j0-1+b] (clamped)
-    double bed[TY + 2][TX + 2];
-    double beta[TY + 2][TX + 2];
-    double E[TY + 2][TX + 2];   // viscosity (0 outside the domain)
-    double g[TY + 2][TX + 2];   // grounding sigmoid and its derivative
-    double gd[TY + 2][TX + 2];
-    double sxx[TY + 2][TX + 2]; // sigma_xx / sigma_yy residual parts
-    double syy[TY + 2][TX + 2];
-    double sxy[TY + 1][TX + 1]; // vertices [i0+a][j0+b]
+    double H[TY + 2][TX + 2];   // cells [i0-1+a][j0-1+b] (clamped); likewise:
+    double S[TY + 2][TX + 2];   // surface max(bed, -0.917 H) + H
+    double be[TY + 2][TX + 2];  // drag g beta + (1 - g) water_drag
+    double n[TY + 2][TX + 2];   // 2 eta H (0 outside the domain)
+    double sx[TY + 2][TX + 2];  // sigma_xx, sigma_yy (0 outside the domain)
+    double sy[TY + 2][TX + 2];
+    double cal[TY][TX];         // calving sink of cell [i0+a][j0+b]
+    double sxy[TY + 1][TX + 1]; // 8 sigma_xy at vertex [i0+a][j0+b]
 };
 
-// EDGE_FACES: the tiles cover the cells only (cdiv(nx, TX) x cdiv(ny, TY));
-// where a tile ends exactly at the last column (row), its last lane (row of
-// threads) also computes the u faces at j = nx (v faces at i = ny), so the
-// extra face column and row need no tiles of their own.  Without it the
-// tiles cover the points [0, ny] x [0, nx].  Same arithmetic per point.
-template <int TX, int TY, bool EDGE_FACES = false>
+// The tiles cover the cells only (cdiv(nx, TX) x cdiv(ny, TY)); where a tile
+// ends exactly at the last column (row), its last lane (row of threads) also
+// computes the u faces at j = nx (v faces at i = ny), so the extra face column
+// and row need no tiles of their own.
+template <int TX, int TY>
 __device__ __forceinline__ void residual_tile_lds(const GlideGeom &g, const Params &p, double *__restrict__ r,
                                                   const double *__restrict__ U, const double *__restrict__ f,
                                                   const double *__restrict__ sub, const double *__restrict__ bed,
@@ -127,140 +167,117 @@ __device__ __forceinline__ void residual_tile_lds(const GlideGeom &g, const Para
                                                   const double *__restrict__ mask, const double *__restrict__ gamma,
                                                   int bx, int by, ResidLDS<TX, TY> &S)
 {
-    constexpr int NT = TX * TY;
+    constexpr int NT = TX * TY, NC = ((TY + 2) * (TX + 2) + NT - 1) / NT;
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
     const double *u = U, *v = U + nu, *H = U + nu + nv;
     const int i0 = by * TY, j0 = bx * TX;
     const int tid = threadIdx.y * TX + threadIdx.x;
-    const double dx_inv = 1.0 / g.dx, dt = g.dt;
-    // 1. stage the inputs
+    const NewtonK K = newton_constants(g.dx, g.dt);
+    const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+    // 1. stage u and v; the cells' other inputs go to registers meanwhile
+    double h[NC], bd[NC], bt[NC], Bc[NC];
+#pragma unroll
+    for (int q = 0; q < NC; q++) {
+        const int k = tid + q * NT, a = k / (TX + 2), b = k - a * (TX + 2);
+        if (k < (TY + 2) * (TX + 2)) {
+            const size_t kc = (size_t)clampi(i0 - 1 + a, 0, ny - 1) * nx + clampi(j0 - 1 + b, 0, nx - 1);
+            h[q] = H[kc];
+            bd[q] = bed[kc];
+            bt[q] = beta[kc];
+            Bc[q] = B[kc];
+        }
+    }
     for (int k = tid; k < (TY + 4) * (TX + 4); k += NT) {
         const int a = k / (TX + 4), b = k - a * (TX + 4);
         S.u[a][b] = ld_u(u, i0 - 2 + a, j0 - 2 + b, ny, nx);
         S.v[a][b] = ld_v(v, i0 - 2 + a, j0 - 2 + b, ny, nx);
     }
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        S.H[a][b] = ld_c(H, i0 - 1 + a, j0 - 1 + b, ny, nx);
-        S.bed[a][b] = ld_c(bed, i0 - 1 + a, j0 - 1 + b, ny, nx);
-        S.beta[a][b] = ld_c(beta, i0 - 1 + a, j0 - 1 + b, ny, nx);
+    __syncthreads();
+    // 2. per cell (a, b): global (i0-1+a, j0-1+b), its u and v at [a+1][b+1]
+#pragma unroll
+    for (int q = 0; q < NC; q++) {
+        const int k = tid + q * NT, a = k / (TX + 2), b = k - a * (TX + 2);
+        if (k >= (TY + 2) * (TX + 2)) break;
+        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
+        const double u_l = S.u[a + 1][b + 1], u_r = S.u[a + 1][b + 2], v_t = S.v[a + 1][b + 1], v_b = S.v[a + 2][b + 1];
+        double n = 0.0;
+        if (ci >= 0 && ci < ny && cj >= 0 && cj < nx)
+            n = eta2_from(ci, cj, ny, nx, u_l, u_r, v_t, v_b, S.u[a][b + 1], S.u[a][b + 2], S.u[a + 2][b + 1],
+                          S.u[a + 2][b + 2], S.v[a + 1][b], S.v[a + 1][b + 2], S.v[a + 2][b], S.v[a + 2][b + 2], Bc[q], p,
+                          glen_exp, K.dxi) *
+                h[q];
+        const double du = u_r - u_l, dv = v_t - v_b;
+        S.n[a][b] = n;
+        S.sx[a][b] = n * fma(du, K.dxi2, dv * K.dxi);
+        S.sy[a][b] = n * fma(du, K.dxi, dv * K.dxi2);
+        const double gr = sigm_mid(fma(0.917, h[q], bd[q]), p.gl_c), g1 = 1.0 - gr;
+        S.H[a][b] = h[q];
+        S.S[a][b] = fmax(bd[q], -0.917 * h[q]) + h[q];
+        S.be[a][b] = fma(gr, bt[q], g1 * p.water_drag);
+        if (a >= 1 && a <= TY && b >= 1 && b <= TX) S.cal[a - 1][b - 1] = p.calving_rate * g1 * h[q];
     }
     __syncthreads();
-    auto UL = [&](int a, int b) { return S.u[a - i0 + 2][b - j0 + 2]; };   // global (a, b)
-    auto VL = [&](int a, int b) { return S.v[a - i0 + 2][b - j0 + 2]; };
-    auto HC = [&](int a, int b) { return S.H[a - i0 + 1][b - j0 + 1]; };
-    auto EC = [&](int a, int b) { return S.E[a - i0 + 1][b - j0 + 1]; };
-    // 2. per cell: viscosity and grounding sigmoid
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        S.E[a][b] = (ci >= 0 && ci < ny && cj >= 0 && cj < nx)
-                        ? eta_cell_acc(ci, cj, UL, VL, B[(size_t)ci * nx + cj], p, g.dx, ny, nx)
-                        : 0.0;
-        const Ground gr = ground(S.bed[a][b], S.H[a][b], p);
-        S.g[a][b] = gr.g;
-        S.gd[a][b] = gr.gd;
-    }
-    __syncthreads();
-    // 3. per cell normal stresses, per vertex shear stress
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        double sx = 0.0, sy = 0.0;
-        // cells [i0, i0+TY) x [j0-1, j0+TX), and j0+TX for the faces at j = nx
-        if (a >= 1 && a <= TY && b <= TX + (EDGE_FACES ? 1 : 0))
-            sx = sigma_xx(UL(ci, cj), UL(ci, cj + 1), VL(ci, cj), VL(ci + 1, cj), S.E[a][b] * S.H[a][b], dx_inv, cj,
-                          nx).res;
-        // cells [i0-1, i0+TY) x [j0, j0+TX), and i0+TY for the faces at i = ny
-        if (a <= TY + (EDGE_FACES ? 1 : 0) && b >= 1 && b <= TX)
-            sy = sigma_yy(UL(ci, cj), UL(ci, cj + 1), VL(ci, cj), VL(ci + 1, cj), S.E[a][b] * S.H[a][b], dx_inv, ci,
-                          ny).res;
-        S.sxx[a][b] = sx;
-        S.syy[a][b] = sy;
-    }
+    // 3. per vertex shear stress, 0 on the domain edge
     for (int k = tid; k < (TY + 1) * (TX + 1); k += NT) {
-        const int a = k / (TX + 1), b = k - a * (TX + 1);
+        const int a = k / (TX + 1), b = k - a * (TX + 1);   // vertex (i0 + a, j0 + b): cells [a..a+1][b..b+1]
         const int vi = i0 + a, vj = j0 + b;
-        const double eH = etaH_vertex(EC(vi - 1, vj - 1), EC(vi - 1, vj), EC(vi, vj - 1), EC(vi, vj),
-                                      HC(vi - 1, vj - 1), HC(vi - 1, vj), HC(vi, vj - 1), HC(vi, vj));
-        S.sxy[a][b] = sigma_xy(UL(vi - 1, vj), UL(vi, vj), VL(vi, vj - 1), VL(vi, vj), eH, dx_inv, vi, vj, ny, nx).res;
+        const double V = vi > 0 && vi < ny && vj > 0 && vj < nx ? K.dxi : 0.0;
+        const double m = ((S.n[a][b] + S.n[a][b + 1]) + S.n[a + 1][b]) + S.n[a + 1][b + 1];
+        S.sxy[a][b] = m * fma(S.u[a + 1][b + 2] - S.u[a + 2][b + 2], V, (S.v[a + 2][b + 2] - S.v[a + 2][b + 1]) * V);
     }
     __syncthreads();
     // 4. rows of point (i, j): cell (i < ny, j < nx), u face (i < ny), v face (j < nx)
-    auto SXX = [&](int ci, int cj) { return S.sxx[ci - i0 + 1][cj - j0 + 1]; };
-    auto SYY = [&](int ci, int cj) { return S.syy[ci - i0 + 1][cj - j0 + 1]; };
-    auto SXY = [&](int vi, int vj) { return S.sxy[vi - i0][vj - j0]; };
     auto rows = [&](int i, int j) {
-    const int a = i - i0 + 1, b = j - j0 + 1;   // cell (i, j) in the one-ring arrays
-    if (i < ny && j < nx) {
-        double H_c = S.H[a][b];
-        const size_t kc = (size_t)i * nx + j;
-        double rH = H_c / dt - (f ? f[nu + nv + kc] : 0.0);
-        Calv jc = calving_g(H_c, Ground{S.g[a][b], S.gd[a][b]}, p);
-        rH -= jc.res;
-        double H_l = S.H[a][b - 1];
-        Flux q = flux_x(UL(i, j), H_l, H_c, j, nx);
-        rH -= q.res * dx_inv;
-        double H_r = S.H[a][b + 1];
-        q = flux_x(UL(i, j + 1), H_c, H_r, j + 1, nx);
-        rH += q.res * dx_inv;
-        double H_t = S.H[a - 1][b];
-        q = flux_y(VL(i, j), H_t, H_c, i, ny);
-        rH += q.res * dx_inv;
-        double H_b = S.H[a + 1][b];
-        q = flux_y(VL(i + 1, j), H_c, H_b, i + 1, ny);
-        rH -= q.res * dx_inv;
-        double m = mask[kc];
-        double th = gamma[kc];
-        double val = (1.0 - m) * rH + m * (H_c - th);
-        size_t k = nu + nv + kc;
-        r[k] = sub ? val - sub[k] : val;
-    }
-    if (i < ny) {
-        const size_t k = (size_t)i * (nx + 1) + j;
-        double ru = f ? -f[k] : -0.0;
-        ru += SXX(i, j) * dx_inv;
-        ru -= SXX(i, j - 1) * dx_inv;
-        ru += SXY(i, j) * dx_inv;
-        ru -= SXY(i + 1, j) * dx_inv;
-        {
-            TauB t = tau_b_g(UL(i, j), S.g[a][b - 1], S.g[a][b], S.gd[a][b - 1], S.gd[a][b], S.beta[a][b - 1],
-                             S.beta[a][b], p);
-            ru += t.res;
+        const int a = i - i0 + 1, b = j - j0 + 1;   // cell (i, j) in the one-ring arrays
+        const bool il = j > 0, ir = j + 1 < nx, it = i > 0, ib = i + 1 < ny;
+        const double H_c = S.H[a][b], H_l = S.H[a][b - 1], H_t = S.H[a - 1][b];
+        const double u_l = S.u[a + 1][b + 1], v_t = S.v[a + 1][b + 1];
+        const double s_l = H_l + H_c, s_t = H_t + H_c;
+        const double F_l = il && j < nx ? K.hdx : 0.0, F_t = it && i < ny ? K.hdx : 0.0;
+        if (i < ny && j < nx) {
+            const size_t kc = (size_t)i * nx + j;
+            const double H_r = S.H[a][b + 1], H_b = S.H[a + 1][b], u_r = S.u[a + 1][b + 2], v_b = S.v[a + 2][b + 1];
+            const double F_r = ir ? K.hdx : 0.0, F_b = ib ? K.hdx : 0.0;
+            double rH = div_refined(H_c, K.dt, K.rdt) - (f ? f[nu + nv + kc] : 0.0);
+            rH += S.cal[a - 1][b - 1];
+            rH -= fma(s_l, u_l, -(fabs(u_l) * (H_c - H_l))) * F_l;
+            rH += fma(H_c + H_r, u_r, -(fabs(u_r) * (H_r - H_c))) * F_r;
+            rH += fma(s_t, v_t, -(fabs(v_t) * (H_t - H_c))) * F_t;
+            rH -= fma(H_c + H_b, v_b, -(fabs(v_b) * (H_c - H_b))) * F_b;
+            const double m = mask[kc], th = gamma[kc];
+            const double val = (1.0 - m) * rH + m * (H_c - th);
+            const size_t k = nu + nv + kc;
+            r[k] = sub ? val - sub[k] : val;
         }
-        {
-            TauD t = tau_dx(S.H[a][b - 1], S.H[a][b], S.bed[a][b - 1], S.bed[a][b], dx_inv, j, nx);
-            ru -= t.res;
+        if (i < ny) {
+            const size_t k = (size_t)i * (nx + 1) + j;
+            double ru = f ? -f[k] : -0.0;
+            ru += S.sx[a][b] * K.dxi;
+            ru -= S.sx[a][b - 1] * K.dxi;
+            ru += S.sxy[a - 1][b - 1] * K.edx;
+            ru -= S.sxy[a][b - 1] * K.edx;
+            ru = fma(-0.5, (S.be[a][b - 1] + S.be[a][b]) * u_l, ru);
+            ru -= (s_l * (S.S[a][b] - S.S[a][b - 1])) * F_l;
+            r[k] = sub ? ru - sub[k] : ru;
         }
-        r[k] = sub ? ru - sub[k] : ru;
-    }
-    if (j < nx) {
-        const size_t k = nu + (size_t)i * nx + j;
-        double rv = f ? -f[k] : -0.0;
-        rv += SYY(i - 1, j) * dx_inv;
-        rv -= SYY(i, j) * dx_inv;
-        rv -= SXY(i, j) * dx_inv;
-        rv += SXY(i, j + 1) * dx_inv;
-        {
-            TauB t = tau_b_g(VL(i, j), S.g[a - 1][b], S.g[a][b], S.gd[a - 1][b], S.gd[a][b], S.beta[a - 1][b],
-                             S.beta[a][b], p);
-            rv += t.res;
+        if (j < nx) {
+            const size_t k = nu + (size_t)i * nx + j;
+            double rv = f ? -f[k] : -0.0;
+            rv += S.sy[a - 1][b] * K.dxi;
+            rv -= S.sy[a][b] * K.dxi;
+            rv -= S.sxy[a - 1][b - 1] * K.edx;
+            rv += S.sxy[a - 1][b] * K.edx;
+            rv = fma(-0.5, (S.be[a - 1][b] + S.be[a][b]) * v_t, rv);
+            rv -= (s_t * (S.S[a - 1][b] - S.S[a][b])) * F_t;
+            r[k] = sub ? rv - sub[k] : rv;
         }
-        {
-            TauD t = tau_dy(S.H[a - 1][b], S.H[a][b], S.bed[a - 1][b], S.bed[a][b], dx_inv, i, ny);
-            rv -= t.res;
-        }
-        r[k] = sub ? rv - sub[k] : rv;
-    }
     };
     const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
     if (i > ny || j > nx) return;
     rows(i, j);
-    if (EDGE_FACES) {
-        if (j == nx - 1 && j0 + TX == nx && i < ny) rows(i, nx);   // u face at j = nx
-        if (i == ny - 1 && i0 + TY == ny && j < nx) rows(ny, j);   // v face at i = ny
-    }
+    if (j == nx - 1 && j0 + TX == nx && i < ny) rows(i, nx);   // u face at j = nx
+    if (i == ny - 1 && i0 + TY == ny && j < nx) rows(ny, j);   // v face at i = ny
 }
 
 template <class EtaFn>
@@ -315,103 +332,145 @@ struct VankaLDS {
     double be[TY + 2][TX + 2];
 };
 
-// 2 eta of cell (i, j) (eta_cell, ssa_device.h): the factors of 1/2 of the
-// corner shear rates, their mean square and eta itself are exact and ride on
-// one constant; corners on the domain edge get the factor 0.
-__device__ __forceinline__ double eta2_cell(int i, int j, const double *__restrict__ u, const double *__restrict__ v,
-                                            double Bc, const Params &p, double glen_exp, double dxi, int ny, int nx)
-{
-    const double u_l = ld_u(u, i, j, ny, nx), u_r = ld_u(u, i, j + 1, ny, nx);
-    const double v_t = ld_v(v, i, j, ny, nx), v_b = ld_v(v, i + 1, j, ny, nx);
-    const double dudx = (u_r - u_l) * dxi, dvdy = (v_t - v_b) * dxi;
-    const bool t = i > 0, b = i < ny - 1, l = j > 0, r = j < nx - 1;
-    const double V_tl = t && l ? dxi : 0.0, V_tr = t && r ? dxi : 0.0, V_bl = b && l ? dxi : 0.0, V_br = b && r ? dxi : 0.0;
-    const double e_tl = fma(ld_u(u, i - 1, j, ny, nx) - u_l, V_tl, (v_t - ld_v(v, i, j - 1, ny, nx)) * V_tl);
-    const double e_tr = fma(ld_u(u, i - 1, j + 1, ny, nx) - u_r, V_tr, (ld_v(v, i, j + 1, ny, nx) - v_t) * V_tr);
-    const double e_bl = fma(u_l - ld_u(u, i + 1, j, ny, nx), V_bl, (v_b - ld_v(v, i + 1, j - 1, ny, nx)) * V_bl);
-    const double e_br = fma(u_r - ld_u(u, i + 1, j + 1, ny, nx), V_br, (ld_v(v, i + 1, j + 1, ny, nx) - v_b) * V_br);
-    const double e2 = fma(e_br, e_br, fma(e_bl, e_bl, fma(e_tr, e_tr, e_tl * e_tl)));
-    const double eII = fma(0.0625, e2, fma(dudx, dvdy, fma(dvdy, dvdy, dudx * dudx))) + p.eps_reg;
-    return Bc * pow_pos(eII, glen_exp);
-}
+// A thread's share of the staged cells [i0-1, i0+TY] x [j0-1, j0+TX], cell q =
+// tid + q TX TY: load() issues all its reads, compute() evaluates and stores
+// to LDS.  Between the two the thread issues its own cell's reads as well, so a
+// tile waits out one memory latency instead of three (two workgroups per CU
+// leave little else to run meanwhile); together with 32-bit offsets a sweep's
+// staging at 1024^2 went from 53.3 to 50.8 us.  INTERIOR: the cells lie in [1, ny-2] x
+// [1, nx-2], so nothing is clamped.
+template <bool INTERIOR, int TX, int TY>
+struct VankaStage {
+    static constexpr int NT = TX * TY, NALL = (TY + 2) * (TX + 2), NC = (NALL + NT - 1) / NT;
+    double u[NC][6], v[NC][6];   // rows i-1, i, i+1 of u x columns j, j+1; rows i, i+1 of v x columns j-1, j, j+1
+    double h[NC], bd[NC], bt[NC], Bc[NC];
 
-// cells [i0-1, i0+TY] x [j0-1, j0+TX]
-template <int TX, int TY>
-__device__ __forceinline__ void vanka_stage(VankaLDS<TX, TY> &L, int i0, int j0, const double *__restrict__ u,
-                                            const double *__restrict__ v, const double *__restrict__ H,
-                                            const double *__restrict__ bed, const double *__restrict__ B,
-                                            const double *__restrict__ beta, const Params &p, double dxi, int ny, int nx)
-{
-    const int tid = threadIdx.y * TX + threadIdx.x;
-    const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += TX * TY) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        const int ic = clampi(ci, 0, ny - 1), jc = clampi(cj, 0, nx - 1);
-        const size_t kc = (size_t)ic * nx + jc;
-        const double h = H[kc], bd = bed[kc];
-        const double e2 = ic == ci && jc == cj ? eta2_cell(ci, cj, u, v, B[kc], p, glen_exp, dxi, ny, nx) : 0.0;
-        const double g = sigm_mid(fma(0.917, h, bd), p.gl_c);
-        L.e2[a][b] = e2;
-        L.n[a][b] = e2 * h;
-        L.H[a][b] = h;
-        L.S[a][b] = fmax(bd, -0.917 * h) + h;
-        L.be[a][b] = fma(g, beta[kc], (1.0 - g) * p.water_drag);
+    __device__ __forceinline__ void load(int i0, int j0, int rb, int cb, const double *__restrict__ U,
+                                         const double *__restrict__ bed, const double *__restrict__ B,
+                                         const double *__restrict__ beta, int ny, int nx)
+    {
+        const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+        const TileField tu(nx + 1, rb, cb), tc(nx, rb, cb);
+        const char *bu = tu.base(U), *bv = tc.base(U + nu), *bH = tc.base(U + nu + nv), *bbed = tc.base(bed),
+                   *bB = tc.base(B), *bbeta = tc.base(beta);
+        const int tid = threadIdx.y * TX + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            const int k = tid + q * NT, a = k / (TX + 2), b = k - a * (TX + 2);
+            if (k >= NALL) break;
+            const int ci = i0 - 1 + a, cj = j0 - 1 + b;
+            const int ic = INTERIOR ? ci : clampi(ci, 0, ny - 1), jc = INTERIOR ? cj : clampi(cj, 0, nx - 1);
+            const uint32_t r0 = ic - rb, c0 = 8u * (jc - cb), u0 = r0 * tu.pitch, v0 = r0 * tc.pitch, kc = v0 + c0;
+            // row i+1 of v and column j+1 of u exist for every cell
+            const uint32_t v1 = v0 + tc.pitch;
+            const uint32_t ut = INTERIOR || ic > 0 ? u0 - tu.pitch : u0, ub = INTERIOR || ic < ny - 1 ? u0 + tu.pitch : u0;
+            const uint32_t cl = INTERIOR || jc > 0 ? c0 - 8 : c0, cr = INTERIOR || jc < nx - 1 ? c0 + 8 : c0;
+            h[q] = ld_off(bH, kc);
+            bd[q] = ld_off(bbed, kc);
+            bt[q] = ld_off(bbeta, kc);
+            Bc[q] = ld_off(bB, kc);
+            u[q][0] = ld_off(bu, ut + c0);
+            u[q][1] = ld_off(bu, ut + c0 + 8);
+            u[q][2] = ld_off(bu, u0 + c0);
+            u[q][3] = ld_off(bu, u0 + c0 + 8);
+            u[q][4] = ld_off(bu, ub + c0);
+            u[q][5] = ld_off(bu, ub + c0 + 8);
+            v[q][0] = ld_off(bv, v0 + cl);
+            v[q][1] = ld_off(bv, v0 + c0);
+            v[q][2] = ld_off(bv, v0 + cr);
+            v[q][3] = ld_off(bv, v1 + cl);
+            v[q][4] = ld_off(bv, v1 + c0);
+            v[q][5] = ld_off(bv, v1 + cr);
+        }
     }
-}
+    __device__ __forceinline__ void compute(VankaLDS<TX, TY> &L, int i0, int j0, const Params &p, double dxi, int ny,
+                                            int nx) const
+    {
+        const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+        const int tid = threadIdx.y * TX + threadIdx.x;
+#pragma unroll
+        for (int q = 0; q < NC; q++) {
+            const int k = tid + q * NT, a = k / (TX + 2), b = k - a * (TX + 2);
+            if (k >= NALL) break;
+            const int ci = i0 - 1 + a, cj = j0 - 1 + b;
+            double e2 = 0.0;
+            if (INTERIOR || (ci >= 0 && ci < ny && cj >= 0 && cj < nx))
+                e2 = eta2_from(INTERIOR ? 1 : ci, INTERIOR ? 1 : cj, INTERIOR ? 3 : ny, INTERIOR ? 3 : nx, u[q][2], u[q][3],
+                               v[q][1], v[q][4], u[q][0], u[q][1], u[q][4], u[q][5], v[q][0], v[q][2], v[q][3], v[q][5],
+                               Bc[q], p, glen_exp, dxi);
+            const double g = sigm_mid(fma(0.917, h[q], bd[q]), p.gl_c);
+            L.e2[a][b] = e2;
+            L.n[a][b] = e2 * h[q];
+            L.H[a][b] = h[q];
+            L.S[a][b] = fmax(bd[q], -0.917 * h[q]) + h[q];
+            L.be[a][b] = fma(g, bt[q], (1.0 - g) * p.water_drag);
+        }
+    }
+};
 
 // ---------------------------------------------------------------------------
-// One cell's Vanka update (glide/cuda/vanka.cu:56-439): its neighbourhood
-// (a, b index the staged arrays), n_newton damped Newton iterations
-// (newton_step) and the per-cell deltas.  INTERIOR: the cell lies in
-// [1, ny-2] x [1, nx-2], so no read is clamped and no term vanishes.
+// One cell's Vanka update (glide/cuda/vanka.cu:56-439): the tile's cells are
+// staged (VankaStage), then each thread takes its cell's neighbourhood, runs
+// n_newton damped Newton iterations (newton_iterate) and returns the per-cell
+// deltas.  (i, j) is the cell, (i0, j0) the tile's first cell, so that the cell
+// is [i - i0 + 1][j - j0 + 1] of the staged arrays.  INTERIOR: the tile's ring
+// lies in [1, ny-2] x [1, nx-2], so no read is clamped and no term vanishes.
 // ---------------------------------------------------------------------------
 template <bool INTERIOR, int TX, int TY>
 __device__ __forceinline__ void vanka_cell_deltas(const GlideGeom &g, const Params &p, const NewtonK &K,
-                                                  const VankaLDS<TX, TY> &L, int a, int b,
-                                                  const double *__restrict__ u, const double *__restrict__ v,
+                                                  VankaLDS<TX, TY> &L, const double *__restrict__ U,
                                                   const double *__restrict__ f, const double *__restrict__ bed,
-                                                  const double *__restrict__ beta, const double *__restrict__ gamma,
-                                                  int n_newton, int i, int j, double d5[5])
+                                                  const double *__restrict__ B, const double *__restrict__ beta,
+                                                  const double *__restrict__ gamma, int n_newton, int i0, int j0, int i,
+                                                  int j, double d5[5])
 {
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
-    // offsets of the rows above, at and below, and of the columns around (clamped at the edge)
-    auto row = [&](int q, int hi) { return INTERIOR ? q : clampi(q, 0, hi); };
-    const double *u0 = u + (size_t)i * (nx + 1), *ut = u + (size_t)row(i - 1, ny - 1) * (nx + 1),
-                 *ub = u + (size_t)row(i + 1, ny - 1) * (nx + 1);
-    const double *v0 = v + (size_t)i * nx, *v1 = v + (size_t)(i + 1) * nx, *vt = v + (size_t)row(i - 1, ny) * nx,
-                 *vb = v + (size_t)row(i + 2, ny) * nx;
-    const int jl = row(j - 1, nx - 1), jr = row(j + 1, nx - 1), jrr = row(j + 2, nx);
+    // a row and column not after the first that the tile's cells read
+    const int rb = INTERIOR ? i0 - 2 : max(i0 - 2, 0), cb = INTERIOR ? j0 - 2 : max(j0 - 2, 0);
+    VankaStage<INTERIOR, TX, TY> stage;
+    stage.load(i0, j0, rb, cb, U, bed, B, beta, ny, nx);
+    const TileField tu(nx + 1, rb, cb), tc(nx, rb, cb);
+    const char *bu = tu.base(U), *bv = tc.base(U + nu), *fu = tu.base(f), *fv = tc.base(f + nu),
+               *fH = tc.base(f + nu + nv);
+    // rows i-1, i, i+1 of u and i-1, i, i+1, i+2 of v; columns j-1, j, j+1 and, of u, j+2 (clamped at the edge)
+    const uint32_t r0 = i - rb, c0 = 8u * (j - cb);
+    const uint32_t u0 = r0 * tu.pitch, v0 = r0 * tc.pitch, v1 = v0 + tc.pitch;
+    const uint32_t ut = INTERIOR || i > 0 ? u0 - tu.pitch : u0, ub = INTERIOR || i < ny - 1 ? u0 + tu.pitch : u0;
+    const uint32_t vt = INTERIOR || i > 0 ? v0 - tc.pitch : v0, vb = INTERIOR || i < ny - 1 ? v1 + tc.pitch : v1;
+    const uint32_t cl = INTERIOR || j > 0 ? c0 - 8 : c0, cr = INTERIOR || j < nx - 1 ? c0 + 8 : c0;
+    const uint32_t crr = INTERIOR || j < nx - 1 ? c0 + 16 : c0 + 8;
     NewtonX x;
-    x.u_l = u0[j];
-    x.u_r = u0[j + 1];
-    x.v_t = v0[j];
-    x.v_b = v1[j];
+    NewtonCell C;
+    x.u_l = ld_off(bu, u0 + c0);
+    x.u_r = ld_off(bu, u0 + c0 + 8);
+    x.v_t = ld_off(bv, v0 + c0);
+    x.v_b = ld_off(bv, v1 + c0);
+    C.u_ll = ld_off(bu, u0 + cl);
+    C.u_rr = ld_off(bu, u0 + crr);
+    C.u_tl = ld_off(bu, ut + c0);
+    C.u_tr = ld_off(bu, ut + c0 + 8);
+    C.u_bl = ld_off(bu, ub + c0);
+    C.u_br = ld_off(bu, ub + c0 + 8);
+    C.v_lt = ld_off(bv, v0 + cl);
+    C.v_lb = ld_off(bv, v1 + cl);
+    C.v_rt = ld_off(bv, v0 + cr);
+    C.v_rb = ld_off(bv, v1 + cr);
+    C.v_tt = ld_off(bv, vt + c0);
+    C.v_bb = ld_off(bv, vb + c0);
+    C.f0 = ld_off(fu, u0 + c0);
+    C.f1 = ld_off(fu, u0 + c0 + 8);
+    C.f2 = ld_off(fv, v0 + c0);
+    C.f3 = ld_off(fv, v1 + c0);
+    C.f4 = ld_off(fH, v0 + c0);
+    C.bed = ld_off(tc.base(bed), v0 + c0);
+    C.beta = ld_off(tc.base(beta), v0 + c0);
+    C.th = ld_off(tc.base(gamma), v0 + c0);
+    stage.compute(L, i0, j0, p, K.dxi, ny, nx);
+    __syncthreads();
+    const int a = i - i0 + 1, b = j - j0 + 1;
     x.H = L.H[a][b];
     const NewtonX x0 = x;
-    NewtonCell C;
-    C.u_ll = u0[row(j - 1, nx)];
-    C.u_rr = u0[jrr];
-    C.u_tl = ut[j];
-    C.u_tr = ut[j + 1];
-    C.u_bl = ub[j];
-    C.u_br = ub[j + 1];
-    C.v_lt = v0[jl];
-    C.v_lb = v1[jl];
-    C.v_rt = v0[jr];
-    C.v_rb = v1[jr];
-    C.v_tt = vt[j];
-    C.v_bb = vb[j];
-    const size_t ku = (size_t)i * (nx + 1) + j, kv = nu + (size_t)i * nx + j, kc = (size_t)i * nx + j;
-    C.f0 = f[ku];
-    C.f1 = f[ku + 1];
-    C.f2 = f[kv];
-    C.f3 = f[kv + nx];
-    C.f4 = f[kv + nv];
-    C.bed = bed[kc];
-    C.beta = beta[kc];
-    C.th = gamma[kc];
     C.e2 = L.e2[a][b];
     C.n_l = L.n[a][b - 1];
     C.n_r = L.n[a][b + 1];
@@ -438,7 +497,7 @@ __device__ __forceinline__ void vanka_cell_deltas(const GlideGeom &g, const Para
     C.d_t = C.u_tr - C.u_tl;
     C.d_b = C.u_br - C.u_bl;
     newton_edges<INTERIOR>(C, K, i, j, ny, nx);
-    for (int k = 0; k < n_newton; k++) newton_step(C, K, p, x);
+    newton_iterate(C, K, p, n_newton, x);
     d5[0] = 0.5 * (x.u_l - x0.u_l);
     d5[1] = 0.5 * (x.u_r - x0.u_r);
     d5[2] = 0.5 * (x.v_t - x0.v_t);
@@ -461,10 +520,8 @@ __device__ __forceinline__ void vanka_tile(const GlideGeom &g, const Params &p, 
 {
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx), nc = n_c(ny, nx);
-    const double *u = U, *v = U + nu, *H = U + nu + nv;
     const int i0 = by * TY, j0 = bx * TX;
-    const int a = threadIdx.y + 1, b = threadIdx.x + 1;
-    const int i = i0 - 1 + a, j = j0 - 1 + b;
+    const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
     const bool mine = (i < ny && j < nx);
     // A local sweep smooths every cell of a tile that holds an active cell:
     // the apply pass reads only the active cells' updates, so the idle
@@ -475,17 +532,15 @@ __device__ __forceinline__ void vanka_tile(const GlideGeom &g, const Params &p, 
         if (!__syncthreads_or(mine && blk[(i / RB) * nbx + j / RB])) return;   // uniform: the whole tile is idle
     }
     const NewtonK K = newton_constants(g.dx, g.dt);
-    vanka_stage<TX, TY>(L, i0, j0, u, v, H, bed, B, beta, p, K.dxi, ny, nx);
-    __syncthreads();
-    if (!mine) return;
-    // A tile whose cells all lie in [1, ny-2] x [1, nx-2] runs the interior
-    // form (same bits).  The whole per-cell body is instantiated twice so
-    // that no value is live across the branch.
     double d5[5];
-    if (i0 >= 1 && i0 + TY <= ny - 1 && j0 >= 1 && j0 + TX <= nx - 1)
-        vanka_cell_deltas<true>(g, p, K, L, a, b, u, v, f, bed, beta, gamma, n_newton, i, j, d5);
+    // the whole per-cell body is instantiated twice so that no value is live
+    // across the branch; threads past the level's edge take its nearest cell
+    if (i0 >= 2 && i0 + TY <= ny - 2 && j0 >= 2 && j0 + TX <= nx - 2)
+        vanka_cell_deltas<true>(g, p, K, L, U, f, bed, B, beta, gamma, n_newton, i0, j0, i, j, d5);
     else
-        vanka_cell_deltas<false>(g, p, K, L, a, b, u, v, f, bed, beta, gamma, n_newton, i, j, d5);
+        vanka_cell_deltas<false>(g, p, K, L, U, f, bed, B, beta, gamma, n_newton, i0, j0, min(i, ny - 1), min(j, nx - 1),
+                                 d5);
+    if (!mine) return;
     const size_t ci = (size_t)i * nx + j;
 #pragma unroll
     for (int q = 0; q < 5; q++) cd[q * nc + ci] = d5[q];
@@ -554,16 +609,13 @@ __device__ __forceinline__ void vanka_halo_tile(const GlideGeom &g, const Params
     if (LOCAL) run = __syncthreads_or(in && act(i, j));   // uniform
     if (run) {
         const NewtonK K = newton_constants(g.dx, g.dt);
-        vanka_stage<TX, TY>(L, i0 - 1, j0 - 1, u, v, H, bed, B, beta, p, K.dxi, ny, nx);
-        __syncthreads();
-        const int ic = min(max(i, 0), ny - 1), jc = min(max(j, 0), nx - 1);
-        const int la = ic - i0 + 2, lb = jc - j0 + 2;   // the cell in the staged arrays
         double d5[5];
-        // every run cell in [1, ny-2] x [1, nx-2]: the interior form
-        if (i0 >= 2 && i0 + TY <= ny && j0 >= 2 && j0 + TX <= nx)
-            vanka_cell_deltas<true>(g, p, K, L, la, lb, u, v, f, bed, beta, gamma, n_newton, ic, jc, d5);
+        // the run cells are a tile at (i0 - 1, j0 - 1)
+        if (i0 >= 3 && i0 + TY <= ny - 1 && j0 >= 3 && j0 + TX <= nx - 1)
+            vanka_cell_deltas<true>(g, p, K, L, U, f, bed, B, beta, gamma, n_newton, i0 - 1, j0 - 1, i, j, d5);
         else
-            vanka_cell_deltas<false>(g, p, K, L, la, lb, u, v, f, bed, beta, gamma, n_newton, ic, jc, d5);
+            vanka_cell_deltas<false>(g, p, K, L, U, f, bed, B, beta, gamma, n_newton, i0 - 1, j0 - 1,
+                                     clampi(i, 0, ny - 1), clampi(j, 0, nx - 1), d5);
 #pragma unroll
         for (int q = 0; q < 5; q++) cd_s[q][a][b] = d5[q];
         __syncthreads();

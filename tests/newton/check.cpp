@@ -42,6 +42,9 @@ static int functions()
             if (!same(pow_pos(x, q), dm_pow(x, q))) return std::printf("pow_pos(%g, %g)\n", x, q), 1;
     for (double z : {0.0, 1e9, -1e9, (double)NAN, (double)INFINITY})
         if (!same(sigm_mid(z, 0.1), sigm(z, 0.1))) return std::printf("sigm_mid(%g)\n", z), 1;
+    for (double z : {200.0, -200.0, 1e9, -1e9, (double)NAN, (double)INFINITY, -(double)INFINITY})
+        if (!sigm_clamped(z, 0.1) || !same(sigm_end(z, 0.1), sigm(z, 0.1))) return std::printf("sigm_end(%g)\n", z), 1;
+    if (sigm_clamped(199.99, 0.1) || sigm_clamped(-199.99, 0.1)) return std::printf("sigm_clamped\n"), 1;
     return 0;
 }
 
@@ -51,7 +54,7 @@ int main()
     std::mt19937_64 rng(99);
     std::uniform_real_distribution<double> U(0.5, 2.0), S(-1.0, 1.0), P(0.0, 1.0);
     const int sizes[][2] = {{2, 2}, {2, 9}, {3, 3}, {4, 7}, {16, 16}, {33, 20}};
-    long cells = 0, limited = 0, floating = 0;
+    long cells = 0, limited = 0, floating = 0, clamped = 0;
     for (int gl = 0; gl < 2; gl++)
         for (double dt : {1.0, 10.0, 0.3})
             for (auto &sz : sizes) {
@@ -115,6 +118,7 @@ int main()
                                 vanka_assemble<0>(N, p, i, j, ny, nx, dxi, dt, y.u_l, y.u_r, y.v_t, y.v_b, y.H, th, false, J, r);
                                 limited += J[20] == 0.0 && J[21] == 0.0 && J[24] == 2.0;
                                 floating += N.bed_c < -0.917 * y.H;
+                                clamped += sigm_clamped(fma(0.917, y.H, N.bed_c), p.gl_c);
                                 lu5_solve(J, r, e);
                                 y.u_l -= 0.25 * e[0];
                                 y.u_r -= 0.25 * e[1];
@@ -122,7 +126,7 @@ int main()
                                 y.v_b -= 0.25 * e[3];
                                 y.H -= 0.25 * e[4];
                                 y.H = fmax(y.H, th);
-                                newton_step(C, K, p, x);
+                                newton_iterate(C, K, p, 1, x);
                                 if (!same(x.u_l, y.u_l) || !same(x.u_r, y.u_r) || !same(x.v_t, y.v_t) ||
                                     !same(x.v_b, y.v_b) || !same(x.H, y.H)) {
                                     std::printf("cell (%d, %d) of %d x %d, gl %d, iteration %d: %.17g %.17g %.17g %.17g %.17g, "
@@ -134,8 +138,8 @@ int main()
                             cells++;
                         }
             }
-    if (limited < 100 || floating < 100) {
-        std::printf("only %ld limited and %ld floating iterations\n", limited, floating);
+    if (limited < 100 || floating < 100 || clamped < 100 || clamped > 6 * cells - 100) {
+        std::printf("%ld limited, %ld floating, %ld clamped of %ld iterations\n", limited, floating, clamped, 6 * cells);
         return 1;
     }
     std::printf("ok %ld\n", cells);

@@ -76,20 +76,18 @@ std::atomic<int> g_wg_per_cu[2] = {{64}, {8}};
 // for variant 0 in an earlier build.
 std::atomic<long> g_small_max_cells{128 * 128};
 std::atomic<int> g_small_variant{2};
-// Tile heights (64 x TY points) of the single-level residual (4, 8, 16; 0 =
-// by level size) and of the JVP / VJP (0 = the per-point form, 4, 6, 8); set
-// by glide_set_tile_height.  Launch shapes only: results are the same bits.
-// Measured at 512^2: residual 64 x 16 tiles 11.3 us, 64 x 8 12.0, 64 x 4 13.4;
-// at 1024^2: 64 x 8 39.7 us, 64 x 16 42.0, 64 x 4 46.4 (8 workgroups per CU).
-// VJP at 512^2: 64 x 4 22.5 us, 64 x 8 26.1, 64 x 6 31.8, per point 39.6.
+// Tile heights (64 x TY cells) of the single-level residual (4, 8, 16; 0 = 8)
+// and of the JVP / VJP (0 = the per-point form, 4, 6, 8; initially by level
+// size, lin_ty); set by glide_set_tile_height.  Launch shapes only: results are
+// the same bits.  Residual, 64 x 4 / 8 / 16 tiles: 256^2 7.8 / 7.9 / 9.4 us,
+// 512^2 11.5 / 10.4 / 11.2, 768^2 24.6 / 25.4 / 32.4, 1024^2 39.1 / 35.3 /
+// 43.8, 2048^2 153 / 139 / 173.
 std::atomic<int> g_res_ty{0};
-std::atomic<int> g_lin_ty{4};
-int residual_ty(int ny, int nx)
+std::atomic<int> g_lin_ty{-1};
+int residual_ty()
 {
     const int ty = g_res_ty;
-    if (ty) return ty;
-    const long nc = (long)ny * nx;
-    return nc > (1L << 18) ? 8 : (nc >= (1L << 16) ? 16 : 4);
+    return ty ? ty : 8;
 }
 
 int n_cu()
@@ -930,37 +928,52 @@ __global__ __launch_bounds__(NT) void k_vjp_point(GlideGeom g, Params p, double 
     }
 }
 
-// LDS-staged JVP and VJP on 64 x LTY point tiles (lin_tile_lds).  Tiles are
+// LDS-staged JVP and VJP on 64 x LTY cell tiles (lin_tile_lds).  Tiles are
 // numbered down the columns of tiles and dealt to the XCDs in chunks of
 // consecutive tiles (chunked_tile), so a chunk's vertical neighbours, which
 // share the larger halos, meet in one L2.
 template <int LTY>
-__global__ __launch_bounds__(TX *LTY) void k_jvp(GlideGeom g, Params p, double *__restrict__ jo,
+__global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_jvp(GlideGeom g, Params p, double *__restrict__ jo,
                                                  const double *__restrict__ U, const double *__restrict__ dU,
                                                  const double *__restrict__ bed, const double *__restrict__ B,
                                                  const double *__restrict__ beta, const double *__restrict__ mask)
 {
     __shared__ LinLDS<TX, LTY> S;
-    const int tiles_y = cdiv(g.ny + 1, LTY), total = cdiv(g.nx + 1, TX) * tiles_y;
+    const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
     lin_tile_lds<TX, LTY, false>(g, p, jo, nullptr, U, dU, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
 }
 template <int LTY>
-__global__ __launch_bounds__(TX *LTY) void k_vjp(GlideGeom g, Params p, double *__restrict__ out,
+__global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, Params p, double *__restrict__ out,
                                                  const double *__restrict__ base, const double *__restrict__ U,
                                                  const double *__restrict__ lam, const double *__restrict__ bed,
                                                  const double *__restrict__ B, const double *__restrict__ beta,
                                                  const double *__restrict__ mask)
 {
     __shared__ LinLDS<TX, LTY> S;
-    const int tiles_y = cdiv(g.ny + 1, LTY), total = cdiv(g.nx + 1, TX) * tiles_y;
+    const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
     lin_tile_lds<TX, LTY, true>(g, p, out, base, U, lam, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
 }
+// Height of the staged JVP / VJP tiles.  While all tiles are resident at once
+// (two 64 x 6 tiles of the JVP or three 64 x 4 tiles of the VJP a CU, which is
+// what their registers allow without spills) the short tiles have the shorter
+// chain; beyond that the 64 x 8 tiles' smaller halo and four waves a SIMD pay.
+// JVP, 64 x 6 / 64 x 8: 256^2 7.9 / 8.8 us, 384^2 11.4 / 13.3, 512^2 18.0 /
+// 13.4, 1024^2 56.7 / 47.5.  VJP, 64 x 4 / 64 x 8: 256^2 8.5 / 10.0, 384^2 13.1
+// / 15.1, 512^2 18.5 / 15.5, 1024^2 59.9 / 56.9.
+inline int lin_ty(const GlideGeom &g, bool vjp)
+{
+    const int ty = g_lin_ty;
+    if (ty >= 0) return ty;
+    const long tx = cdiv(g.nx, TX);
+    if (vjp) return tx * cdiv(g.ny, 4) <= 3L * n_cu() ? 4 : 8;
+    return tx * cdiv(g.ny, 6) <= 2L * n_cu() ? 6 : 8;
+}
 // grid of the staged JVP / VJP
-inline dim3 lin_grid(const GlideGeom &g, int ty) { return dim3(chunked_grid(cdiv(g.nx + 1, TX) * cdiv(g.ny + 1, ty))); }
+inline dim3 lin_grid(const GlideGeom &g, int ty) { return dim3(chunked_grid(cdiv(g.nx, TX) * cdiv(g.ny, ty))); }
 
 // Adjoint red-black Vanka pass, in place: cells of one colour own disjoint
 // dofs, so lam is read and written by one lane per dof
@@ -1135,7 +1148,7 @@ int launch_residual(const GlideGeom &g, const Params &p, double *r, const double
                     const double *bed, const double *B, const double *beta, const double *mask, const double *gamma,
                     hipStream_t st, int *zero = nullptr)
 {
-    const int ty = residual_ty(g.ny, g.nx);
+    const int ty = residual_ty();
     if (ty == 16)
         hipLaunchKernelGGL(k_residual<16>, residual_grid(g.ny, g.nx, 16), dim3(TX, 16), 0, st, g, p, r, U, f, sub, bed,
                            B, beta, mask, gamma, zero);
@@ -1403,7 +1416,7 @@ int fascd(const GlideLevel *L, int n, int k, bool finest, double thklim, const G
 int launch_vjp(const GlideGeom &g, const Params &p, double *out, const double *base, const double *U, const double *lam,
                const double *bed, const double *B, const double *beta, const double *mask, hipStream_t st)
 {
-    const int ty = g_lin_ty;
+    const int ty = lin_ty(g, true);
     const dim3 grid4 = lin_grid(g, 4), grid8 = lin_grid(g, 8), grid6 = lin_grid(g, 6);
     if (ty == 8)
         hipLaunchKernelGGL(k_vjp<8>, grid8, dim3(TX, 8), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
@@ -1669,7 +1682,7 @@ int glide_jvp(const GlideGeom *g, const GlideParams *p, double *j, const double 
     TRY(check_geom(g));
     if (!p || !j || !U || !dU || !bed || !B || !beta || !mask) return fail(GLIDE_E_NULL, "jvp: NULL argument");
     (void)gamma;
-    const int ty = g_lin_ty;
+    const int ty = lin_ty(*g, false);
     const dim3 grid4 = lin_grid(*g, 4), grid8 = lin_grid(*g, 8), grid6 = lin_grid(*g, 6);
     if (ty == 8)
         hipLaunchKernelGGL(k_jvp<8>, grid8, dim3(TX, 8), 0, S(stream), *g, to_params(*p), j, U, dU, bed, B, beta, mask);

@@ -724,35 +724,57 @@ __device__ __forceinline__ double prol_H_at(const double *hc, const double *wc, 
 // Linearisation, LDS-staged like the residual: JVP j = J(U) d
 // (glide/cuda/residuals.cu:299-579) and the gather-form VJP l = J(U)^T lambda
 // (residuals.cu:586-1023; the (u, v) block through its symmetry, as a JVP
-// along lambda with a zero thickness direction).  The tile's u, v and the
-// direction (two-ring halo) and H, bed, beta and the thickness direction (or
-// lambda_H (1 - mask)) (one-ring halo) are staged once; each cell's dual
-// viscosity, grounding sigmoid and the directional derivatives of sigma_xx
-// and sigma_yy, and each vertex's of sigma_xy, are evaluated once; each point
-// then sums its terms from LDS.  Every quantity is the expression of the
-// per-point form on the same clamped values and every output sums its terms
-// in the same order, so the bits are those of the per-point form.
-// Tiles cover the points [0, ny] x [0, nx].
+// along lambda with a zero thickness direction).  Every cell of the tile and
+// the ring around it yields 2 eta H and its derivative, the directional
+// derivatives of its normal stresses, its surface, drag and the direction (or
+// lambda_H (1 - mask)) once into LDS, every vertex the derivative of its shear
+// stress; each point then sums its terms from LDS.  The velocities are read
+// from the caches, where a tile's rows stay, which leaves the LDS to four
+// workgroups per CU instead of three.
+//
+// Rounding as in the residual: every output sums its terms in the per-point
+// form's order, with powers of two on the constants, the short exp and log,
+// and a factor of 0 where a term vanishes at the domain edge, so the bits are
+// those of the per-point form up to the sign of zeros.  JVP of 512^2: 21.2 ->
+// 13.4 us, 1024^2: 71 -> 47.5; VJP of 333 x 517: 16.5 -> 14.2 (the staged form
+// before, which kept the velocities in LDS and evaluated each face's terms).
+//
+// The tiles cover the cells (cdiv(nx, TX) x cdiv(ny, TY)); the faces at j = nx
+// and i = ny go with the last tiles as in the residual.
 // ---------------------------------------------------------------------------
 template <int TX, int TY>
 struct LinLDS {
-    double u[TY + 4][TX + 4], v[TY + 4][TX + 4];     // state, clamped, global (i0-2+a, j0-2+b)
-    double du[TY + 4][TX + 4], dv[TY + 4][TX + 4];   // direction (JVP) or lambda (VJP), clamped
-    double H[TY + 2][TX + 2], dH[TY + 2][TX + 2];    // cells (i0-1+a, j0-1+b), clamped; dH: direction or lambda_H (1 - mask)
-    double bed[TY + 2][TX + 2], beta[TY + 2][TX + 2];
-    double ev[TY + 2][TX + 2], ed[TY + 2][TX + 2];   // dual viscosity (0 outside the domain)
-    double g[TY + 2][TX + 2], gd[TY + 2][TX + 2];    // grounding sigmoid and its derivative
-    double txx[TY + 2][TX + 2], tyy[TY + 2][TX + 2]; // directional derivatives of sigma_xx, sigma_yy
-    double txy[TY + 1][TX + 1];                      // ... of sigma_xy, vertices (i0+a, j0+b)
+    // cells [i0-1+a][j0-1+b], clamped
+    double n[TY + 2][TX + 2];    // 2 eta H (0 outside the domain)
+    double hd[TY + 2][TX + 2];   // H (2 eta)' (0 outside)
+    double eh[TY + 2][TX + 2];   // JVP: 2 eta H' (0 outside); VJP: 2 eta
+    double tx[TY + 2][TX + 2], ty[TY + 2][TX + 2];   // derivatives of sigma_xx, sigma_yy (0 outside)
+    double H[TY + 2][TX + 2];
+    double dH[TY + 2][TX + 2];   // direction, or lambda_H (1 - mask)
+    double S[TY + 2][TX + 2];    // surface
+    double sl[TY + 2][TX + 2];   // d surface / d H
+    double be[TY + 2][TX + 2];   // drag
+    double db[TY + 2][TX + 2];   // d drag / d H (gl_derivatives)
+    double cd[TY][TX];           // -d calving / d H of cell [i0+a][j0+b]
+    double txy[TY + 1][TX + 1];  // 8 x derivative of sigma_xy, vertices [i0+a][j0+b]
 };
 
-// eta*H as a Dual: cell and vertex average (viscosity.cu:150-217)
-__device__ __forceinline__ Dual eH_cell_dual(Dual eta, Dual Hh) { return Dual{Hh.v * eta.v, Hh.v * eta.d + eta.v * Hh.d}; }
-__device__ __forceinline__ Dual eH_vertex_dual(Dual a, Dual b, Dual c, Dual d, Dual Ha, Dual Hb, Dual Hc, Dual Hdd)
+// the general form's eII^q and its derivative factor, for arguments out of the short forms' range
+__device__ __forceinline__ void glen_pow_dual(double x, double q, double &v, double &c)
 {
-    return Dual{etaH_vertex(a.v, b.v, c.v, d.v, Ha.v, Hb.v, Hc.v, Hdd.v),
-                0.25 * Ha.v * a.d + 0.25 * a.v * Ha.d + 0.25 * Hb.v * b.d + 0.25 * b.v * Hb.d + 0.25 * Hc.v * c.d +
-                    0.25 * c.v * Hc.d + 0.25 * Hdd.v * d.d + 0.25 * d.v * Hdd.d};
+    const double lg = log_normal(x), y0 = q * lg, y1 = (q - 1.0) * lg;
+    v = exp_mid(y0);
+    c = q * exp_mid(y1);
+    if (!(x >= 2.2250738585072014e-308 && x <= 1.7976931348623157e308 && fabs(y0) <= 700.0 && fabs(y1) <= 700.0)) {
+        if (x == 0.0) {   // dm_pow's own value at 0 (only reachable with eps_reg = 0)
+            v = dm_pow(x, q);
+            c = q * dm_pow(x, q - 1.0);
+        } else {
+            const double l = dm_log(x);
+            v = dm_exp(q * l);
+            c = q * dm_exp((q - 1.0) * l);
+        }
+    }
 }
 
 // VJP: out = base - l when base != NULL (the adjoint residual f_adj - J^T lambda)
@@ -763,242 +785,243 @@ __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p
                                              const double *__restrict__ B, const double *__restrict__ beta,
                                              const double *__restrict__ mask, int bx, int by, LinLDS<TX, TY> &S)
 {
-    constexpr int NT = TX * TY;
+    constexpr int NT = TX * TY, NALL = (TY + 2) * (TX + 2);
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
-    const double *u = U, *v = U + nu, *H = U + nu + nv;
-    const double *du = D, *dv = D + nu, *dH = D + nu + nv;
     const int i0 = by * TY, j0 = bx * TX;
+    const int rb = max(i0 - 2, 0), cb = max(j0 - 2, 0);
+    const TileField tu(nx + 1, rb, cb), tc(nx, rb, cb);
+    const char *bu = tu.base(U), *bv = tc.base(U + nu), *bH = tc.base(U + nu + nv);
+    const char *du = tu.base(D), *dv = tc.base(D + nu), *dH = tc.base(D + nu + nv);
+    const char *bbed = tc.base(bed), *bB = tc.base(B), *bbeta = tc.base(beta), *bmask = tc.base(mask);
     const int tid = threadIdx.y * TX + threadIdx.x;
-    const double dx_inv = 1.0 / g.dx, dt = g.dt;
-    // 1. stage the inputs
-    for (int k = tid; k < (TY + 4) * (TX + 4); k += NT) {
-        const int a = k / (TX + 4), b = k - a * (TX + 4);
-        const int gi = i0 - 2 + a, gj = j0 - 2 + b;
-        S.u[a][b] = ld_u(u, gi, gj, ny, nx);
-        S.v[a][b] = ld_v(v, gi, gj, ny, nx);
-        S.du[a][b] = ld_u(du, gi, gj, ny, nx);
-        S.dv[a][b] = ld_v(dv, gi, gj, ny, nx);
-    }
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
+    const NewtonK K = newton_constants(g.dx, g.dt);
+    const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+    // byte offsets of (row, column), clamped to the field
+    auto ou = [&](int i, int j) { return (uint32_t)(clampi(i, 0, ny - 1) - rb) * tu.pitch + 8u * (clampi(j, 0, nx) - cb); };
+    auto ov = [&](int i, int j) { return (uint32_t)(clampi(i, 0, ny) - rb) * tc.pitch + 8u * (clampi(j, 0, nx - 1) - cb); };
+    // 1. per cell
+#pragma unroll 1
+    for (int k = tid; k < NALL; k += NT) {
         const int a = k / (TX + 2), b = k - a * (TX + 2);
         const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        S.H[a][b] = ld_c(H, ci, cj, ny, nx);
-        S.bed[a][b] = ld_c(bed, ci, cj, ny, nx);
-        S.beta[a][b] = ld_c(beta, ci, cj, ny, nx);
-        S.dH[a][b] = VJP ? ld_c(dH, ci, cj, ny, nx) * (1.0 - ld_c(mask, ci, cj, ny, nx)) : ld_c(dH, ci, cj, ny, nx);
-    }
-    __syncthreads();
-    auto UL = [&](int a, int b) { return S.u[a - i0 + 2][b - j0 + 2]; };   // global (a, b)
-    auto VL = [&](int a, int b) { return S.v[a - i0 + 2][b - j0 + 2]; };
-    auto DU = [&](int a, int b) { return S.du[a - i0 + 2][b - j0 + 2]; };
-    auto DV = [&](int a, int b) { return S.dv[a - i0 + 2][b - j0 + 2]; };
-    auto Ud = [&](int a, int b) { return Dual{UL(a, b), DU(a, b)}; };
-    auto Vd = [&](int a, int b) { return Dual{VL(a, b), DV(a, b)}; };
-    auto HC = [&](int a, int b) { return S.H[a - i0 + 1][b - j0 + 1]; };
-    auto LM = [&](int a, int b) { return S.dH[a - i0 + 1][b - j0 + 1]; };   // VJP: lambda_H (1 - mask)
-    auto Hd = [&](int a, int b) { return Dual{HC(a, b), VJP ? 0.0 : S.dH[a - i0 + 1][b - j0 + 1]}; };
-    auto E = [&](int a, int b) { return Dual{S.ev[a - i0 + 1][b - j0 + 1], S.ed[a - i0 + 1][b - j0 + 1]}; };
-    auto G = [&](int a, int b) { return Ground{S.g[a - i0 + 1][b - j0 + 1], S.gd[a - i0 + 1][b - j0 + 1]}; };
-    auto BED = [&](int a, int b) { return S.bed[a - i0 + 1][b - j0 + 1]; };
-    auto BETA = [&](int a, int b) { return S.beta[a - i0 + 1][b - j0 + 1]; };
-    // 2. per cell: dual viscosity and grounding sigmoid
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        const Dual e = (ci >= 0 && ci < ny && cj >= 0 && cj < nx)
-                           ? eta_cell_dual_acc(ci, cj, Ud, Vd, B[(size_t)ci * nx + cj], p, g.dx, ny, nx)
-                           : Dual{0.0, 0.0};
-        S.ev[a][b] = e.v;
-        S.ed[a][b] = e.d;
-        const Ground gr = ground(S.bed[a][b], S.H[a][b], p);
-        S.g[a][b] = gr.g;
-        S.gd[a][b] = gr.gd;
-    }
-    __syncthreads();
-    // 3. directional derivatives of the stresses: sigma_xx on cells [i0, i0+TY) x
-    //    [j0-1, j0+TX), sigma_yy on [i0-1, i0+TY) x [j0, j0+TX), sigma_xy on the vertices
-    for (int k = tid; k < (TY + 2) * (TX + 2); k += NT) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        double tx = 0.0, ty = 0.0;
-        if ((a >= 1 && a <= TY && b <= TX) || (a <= TY && b >= 1 && b <= TX)) {
-            const Dual eH = eH_cell_dual(E(ci, cj), Hd(ci, cj));
-            const Dual ul = Ud(ci, cj), ur = Ud(ci, cj + 1), vt = Vd(ci, cj), vb = Vd(ci + 1, cj);
-            if (a >= 1 && a <= TY && b <= TX) {
-                const SigN s = sigma_xx(ul.v, ur.v, vt.v, vb.v, eH.v, dx_inv, cj, nx);
-                tx = sigN_jvp(s, ul.d, ur.d, vt.d, vb.d, eH.d);
-            }
-            if (a <= TY && b >= 1 && b <= TX) {
-                const SigN s = sigma_yy(ul.v, ur.v, vt.v, vb.v, eH.v, dx_inv, ci, ny);
-                ty = sigN_jvp(s, ul.d, ur.d, vt.d, vb.d, eH.d);
-            }
+        const int ic = clampi(ci, 0, ny - 1), jc = clampi(cj, 0, nx - 1);
+        const uint32_t r0 = ic - rb, c0 = 8u * (jc - cb), u0 = r0 * tu.pitch + c0, v0 = r0 * tc.pitch + c0;
+        const double h = ld_off(bH, v0), bd = ld_off(bbed, v0), bt = ld_off(bbeta, v0);
+        double hd = ld_off(dH, v0);
+        if (VJP) hd = hd * (1.0 - ld_off(bmask, v0));
+        double n = 0.0, nh = 0.0, ne = 0.0, tx = 0.0, ty = 0.0;
+        if (ic == ci && jc == cj) {
+            const uint32_t v1 = v0 + tc.pitch;   // row i+1 of v and column j+1 of u exist for every cell
+            const bool t = ci > 0, bo = ci < ny - 1, l = cj > 0, r = cj < nx - 1;
+            const uint32_t ut = t ? u0 - tu.pitch : u0, ub = bo ? u0 + tu.pitch : u0, cl = l ? 8u : 0u, cr = r ? 8u : 0u;
+            const double u_l = ld_off(bu, u0), u_r = ld_off(bu, u0 + 8), v_t = ld_off(bv, v0), v_b = ld_off(bv, v1);
+            const double x_l = ld_off(du, u0), x_r = ld_off(du, u0 + 8), y_t = ld_off(dv, v0), y_b = ld_off(dv, v1);
+            const double V_tl = t && l ? K.dxi : 0.0, V_tr = t && r ? K.dxi : 0.0, V_bl = bo && l ? K.dxi : 0.0,
+                         V_br = bo && r ? K.dxi : 0.0;
+            // corner shear rates (doubled) and their derivatives
+            const double e_tl = (ld_off(bu, ut) - u_l) * V_tl + (v_t - ld_off(bv, v0 - cl)) * V_tl;
+            const double e_tr = (ld_off(bu, ut + 8) - u_r) * V_tr + (ld_off(bv, v0 + cr) - v_t) * V_tr;
+            const double e_bl = (u_l - ld_off(bu, ub)) * V_bl + (v_b - ld_off(bv, v1 - cl)) * V_bl;
+            const double e_br = (u_r - ld_off(bu, ub + 8)) * V_br + (ld_off(bv, v1 + cr) - v_b) * V_br;
+            const double d_tl = (ld_off(du, ut) - x_l) * V_tl + (y_t - ld_off(dv, v0 - cl)) * V_tl;
+            const double d_tr = (ld_off(du, ut + 8) - x_r) * V_tr + (ld_off(dv, v0 + cr) - y_t) * V_tr;
+            const double d_bl = (x_l - ld_off(du, ub)) * V_bl + (y_b - ld_off(dv, v1 - cl)) * V_bl;
+            const double d_br = (x_r - ld_off(du, ub + 8)) * V_br + (ld_off(dv, v1 + cr) - y_b) * V_br;
+            const double a_ = u_r - u_l, b_ = v_t - v_b;
+            const double ux = a_ * K.dxi, vy = b_ * K.dxi, uxd = (x_r - x_l) * K.dxi, vyd = (y_t - y_b) * K.dxi;
+            const double e2 = ((e_tl * e_tl + e_tr * e_tr) + e_bl * e_bl) + e_br * e_br;
+            const double e2d = ((fma(e_tl, d_tl, d_tl * e_tl) + fma(e_tr, d_tr, d_tr * e_tr)) + fma(e_bl, d_bl, d_bl * e_bl)) +
+                               fma(e_br, d_br, d_br * e_br);
+            const double eII = fma(0.0625, e2, (ux * ux + vy * vy) + ux * vy) + p.eps_reg;
+            const double eIId = fma(0.0625, e2d, (fma(ux, uxd, uxd * ux) + fma(vy, vyd, vyd * vy)) + fma(ux, vyd, uxd * vy));
+            double pv, pc;
+            glen_pow_dual(eII, glen_exp, pv, pc);
+            const double Bc = ld_off(bB, v0);
+            const double ev = pv * Bc, ed = (pc * eIId) * Bc;   // 2 eta and its derivative
+            n = ev * h;
+            nh = h * ed;
+            ne = VJP ? ev : ev * hd;
+            const double nd = VJP ? nh : nh + ne;
+            const double ex = fma(a_, K.dxi2, b_ * K.dxi), ey = fma(a_, K.dxi, b_ * K.dxi2);
+            const double p1 = n * K.dxi, p2 = p1 + p1;
+            tx = (((p2 * x_r - p2 * x_l) + p1 * y_t) - p1 * y_b) + ex * nd;
+            ty = (((p1 * x_r - p1 * x_l) + p2 * y_t) - p2 * y_b) + ey * nd;
         }
-        S.txx[a][b] = tx;
-        S.tyy[a][b] = ty;
-    }
-    for (int k = tid; k < (TY + 1) * (TX + 1); k += NT) {
-        const int a = k / (TX + 1), b = k - a * (TX + 1);
-        const int vi = i0 + a, vj = j0 + b;
-        const Dual eH = eH_vertex_dual(E(vi - 1, vj - 1), E(vi - 1, vj), E(vi, vj - 1), E(vi, vj), Hd(vi - 1, vj - 1),
-                                       Hd(vi - 1, vj), Hd(vi, vj - 1), Hd(vi, vj));
-        const Dual ut = Ud(vi - 1, vj), ub = Ud(vi, vj), vl = Vd(vi, vj - 1), vr = Vd(vi, vj);
-        const SigS s = sigma_xy(ut.v, ub.v, vl.v, vr.v, eH.v, dx_inv, vi, vj, ny, nx);
-        S.txy[a][b] = sigS_jvp(s, ut.d, ub.d, vl.d, vr.d, eH.d);
+        const double z = fma(0.917, h, bd), gr = sigm_mid(z, p.gl_c), g1 = 1.0 - gr, Hf = -0.917 * h;
+        double njd = p.calving_rate * g1, db = 0.0;
+        if (p.gl_derivatives) {
+            const double dg = 0.917 * (p.gl_c * gr * g1);
+            njd = -fma(p.calving_rate * h, dg, -njd);
+            db = dg * (bt - p.water_drag);
+        }
+        S.n[a][b] = n;
+        S.hd[a][b] = nh;
+        S.eh[a][b] = ne;
+        S.tx[a][b] = tx;
+        S.ty[a][b] = ty;
+        S.H[a][b] = h;
+        S.dH[a][b] = hd;
+        S.S[a][b] = fmax(bd, Hf) + h;
+        S.sl[a][b] = bd > Hf ? 1.0 : 1.0 + -0.917;
+        S.be[a][b] = fma(gr, bt, g1 * p.water_drag);
+        S.db[a][b] = db;
+        if (a >= 1 && a <= TY && b >= 1 && b <= TX) S.cd[a - 1][b - 1] = njd;
     }
     __syncthreads();
-    auto TXX = [&](int ci, int cj) { return S.txx[ci - i0 + 1][cj - j0 + 1]; };
-    auto TYY = [&](int ci, int cj) { return S.tyy[ci - i0 + 1][cj - j0 + 1]; };
-    auto TXY = [&](int vi, int vj) { return S.txy[vi - i0][vj - j0]; };
-    // 2 eps_xy at vertex (vi, vj), 0 on boundary vertices
-    auto EXY = [&](int vi, int vj) {
-        return sigma_xy(UL(vi - 1, vj), UL(vi, vj), VL(vi, vj - 1), VL(vi, vj), 0.0, dx_inv, vi, vj, ny, nx).d_eta_H;
-    };
+    // 2. per vertex, 0 on the domain edge
+#pragma unroll 1
+    for (int k = tid; k < (TY + 1) * (TX + 1); k += NT) {
+        const int a = k / (TX + 1), b = k - a * (TX + 1);   // vertex (i0 + a, j0 + b): cells [a..a+1][b..b+1]
+        const int vi = i0 + a, vj = j0 + b;
+        double t8 = 0.0;
+        if (vi > 0 && vi < ny && vj > 0 && vj < nx) {
+            const uint32_t ub = (uint32_t)(vi - rb) * tu.pitch + 8u * (vj - cb), ut = ub - tu.pitch;
+            const uint32_t vr = (uint32_t)(vi - rb) * tc.pitch + 8u * (vj - cb), vl = vr - 8;
+            const double m = ((S.n[a][b] + S.n[a][b + 1]) + S.n[a + 1][b]) + S.n[a + 1][b + 1];
+            const double md =
+                VJP ? ((S.hd[a][b] + S.hd[a][b + 1]) + S.hd[a + 1][b]) + S.hd[a + 1][b + 1]
+                    : ((((((S.hd[a][b] + S.eh[a][b]) + S.hd[a][b + 1]) + S.eh[a][b + 1]) + S.hd[a + 1][b]) + S.eh[a + 1][b]) +
+                       S.hd[a + 1][b + 1]) +
+                          S.eh[a + 1][b + 1];
+            const double q = m * K.dxi;
+            const double x = fma(ld_off(bu, ut) - ld_off(bu, ub), K.dxi, (ld_off(bv, vr) - ld_off(bv, vl)) * K.dxi);
+            t8 = (((q * ld_off(du, ut) - q * ld_off(du, ub)) - q * ld_off(dv, vl)) + q * ld_off(dv, vr)) + x * md;
+        }
+        S.txy[a][b] = t8;
+    }
+    __syncthreads();
     const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
     if (i > ny || j > nx) return;
     auto emit = [&](size_t k, double val) { out[k] = (VJP && base) ? base[k] - val : val; };
-    // 4a. u row (i, j): J_u d (glide/cuda/residuals.cu:378-499)
-    if (i < ny) {
-        double d = 0.0;
-        d += TXX(i, j) * dx_inv;
-        d -= TXX(i, j - 1) * dx_inv;
-        d += TXY(i, j) * dx_inv;
-        d -= TXY(i + 1, j) * dx_inv;
-        const Dual ul = Ud(i, j), Hl = Hd(i, j - 1), Hc = Hd(i, j);
-        {
-            const Ground gl = G(i, j - 1), gc = G(i, j);
-            TauB t = tau_b_g(ul.v, gl.g, gc.g, gl.gd, gc.gd, BETA(i, j - 1), BETA(i, j), p);
-            d += t.d_u * ul.d + t.d_H_l * Hl.d + t.d_H_r * Hc.d;
-        }
-        {
-            TauD t = tau_dx(Hl.v, Hc.v, BED(i, j - 1), BED(i, j), dx_inv, j, nx);
-            d -= t.d_H_l * Hl.d + t.d_H_r * Hc.d;
-        }
-        if (VJP) {   // plus the mass rows through the fluxes of this face
-            Flux q = flux_x(ul.v, HC(i, j - 1), HC(i, j), j, nx);
-            double acc = 0.0;
-            if (j > 0) acc += LM(i, j - 1) * q.d_u * dx_inv;
-            if (j < nx) acc += -LM(i, j) * q.d_u * dx_inv;
-            acc += d;
-            d = acc;
+    // 3a. u face (i, j): J_u d (glide/cuda/residuals.cu:378-499)
+    auto urow = [&](int i, int j) {
+        const int a = i - i0 + 1, b = j - j0 + 1;
+        const uint32_t o = ou(i, j);
+        const double u_l = ld_off(bu, o), x_l = ld_off(du, o);
+        const double H_l = S.H[a][b - 1], H_c = S.H[a][b], s = H_l + H_c, F = j > 0 && j < nx ? K.hdx : 0.0;
+        double d = S.tx[a][b] * K.dxi;
+        d -= S.tx[a][b - 1] * K.dxi;
+        d += S.txy[a - 1][b - 1] * K.edx;
+        d -= S.txy[a][b - 1] * K.edx;
+        double q = (S.be[a][b - 1] + S.be[a][b]) * x_l;
+        if (!VJP) {
+            if (p.gl_derivatives)
+                q = (q + (S.db[a][b - 1] * u_l) * S.dH[a][b - 1]) + (S.db[a][b] * u_l) * S.dH[a][b];
+            d = fma(-0.5, q, d);
+            const double dS = (S.S[a][b] - S.S[a][b - 1]) * F;
+            d -= fma(-(s * S.sl[a][b - 1]), F, dS) * S.dH[a][b - 1] + fma(s * S.sl[a][b], F, dS) * S.dH[a][b];
+        } else {   // plus the mass rows through the fluxes of this face
+            d = fma(-0.5, q, d);
+            const double D2 = fma(-copysign(1.0, u_l), H_c - H_l, s);
+            d = ((S.dH[a][b - 1] * D2) * F - (S.dH[a][b] * D2) * F) + d;
         }
         emit((size_t)i * (nx + 1) + j, d);
-    }
-    // 4b. v row (i, j) (residuals.cu:501-576)
-    if (j < nx) {
-        double d = 0.0;
-        d += TYY(i - 1, j) * dx_inv;
-        d -= TYY(i, j) * dx_inv;
-        d -= TXY(i, j) * dx_inv;
-        d += TXY(i, j + 1) * dx_inv;
-        const Dual vt = Vd(i, j), Ht = Hd(i - 1, j), Hc = Hd(i, j);
-        {
-            const Ground gt = G(i - 1, j), gc = G(i, j);
-            TauB t = tau_b_g(vt.v, gt.g, gc.g, gt.gd, gc.gd, BETA(i - 1, j), BETA(i, j), p);
-            d += t.d_u * vt.d + t.d_H_l * Ht.d + t.d_H_r * Hc.d;
-        }
-        {
-            TauD t = tau_dy(Ht.v, Hc.v, BED(i - 1, j), BED(i, j), dx_inv, i, ny);
-            d -= t.d_H_l * Ht.d + t.d_H_r * Hc.d;
-        }
-        if (VJP) {
-            Flux q = flux_y(vt.v, HC(i - 1, j), HC(i, j), i, ny);
-            double acc = 0.0;
-            if (i > 0) acc += -LM(i - 1, j) * q.d_u * dx_inv;
-            if (i < ny) acc += LM(i, j) * q.d_u * dx_inv;
-            acc += d;
-            d = acc;
+    };
+    // 3b. v face (i, j) (residuals.cu:501-576)
+    auto vrow = [&](int i, int j) {
+        const int a = i - i0 + 1, b = j - j0 + 1;
+        const uint32_t o = ov(i, j);
+        const double v_t = ld_off(bv, o), y_t = ld_off(dv, o);
+        const double H_t = S.H[a - 1][b], H_c = S.H[a][b], s = H_t + H_c, F = i > 0 && i < ny ? K.hdx : 0.0;
+        double d = S.ty[a - 1][b] * K.dxi;
+        d -= S.ty[a][b] * K.dxi;
+        d -= S.txy[a - 1][b - 1] * K.edx;
+        d += S.txy[a - 1][b] * K.edx;
+        double q = (S.be[a - 1][b] + S.be[a][b]) * y_t;
+        if (!VJP) {
+            if (p.gl_derivatives)
+                q = (q + (S.db[a - 1][b] * v_t) * S.dH[a - 1][b]) + (S.db[a][b] * v_t) * S.dH[a][b];
+            d = fma(-0.5, q, d);
+            const double dS = (S.S[a - 1][b] - S.S[a][b]) * F;
+            d -= fma(s * S.sl[a - 1][b], F, dS) * S.dH[a - 1][b] + fma(-(s * S.sl[a][b]), F, dS) * S.dH[a][b];
+        } else {
+            d = fma(-0.5, q, d);
+            const double D2 = fma(-copysign(1.0, v_t), H_t - H_c, s);
+            d = ((S.dH[a][b] * D2) * F - (S.dH[a - 1][b] * D2) * F) + d;
         }
         emit(nu + (size_t)i * nx + j, d);
-    }
+    };
+    if (i < ny) urow(i, j);
+    if (j < nx) vrow(i, j);
+    if (j == nx - 1 && j0 + TX == nx && i < ny) urow(i, nx);   // u face at j = nx
+    if (i == ny - 1 && i0 + TY == ny && j < nx) vrow(ny, j);   // v face at i = ny
     if (i >= ny || j >= nx) return;
+    // 3c. cell (i, j)
+    const int a = i - i0 + 1, b = j - j0 + 1;
     const size_t kc = (size_t)i * nx + j;
-    if (!VJP) {   // 4c. mass row of cell (i, j) (residuals.cu:343-375)
-        const Dual H_c = Hd(i, j);
-        double d = H_c.d / dt;
-        Calv jc = calving_g(H_c.v, G(i, j), p);
-        d -= jc.d_H * H_c.d;
-        Flux q = flux_x(UL(i, j), HC(i, j - 1), H_c.v, j, nx);
-        d -= (q.d_u * DU(i, j) + q.d_H_l * Hd(i, j - 1).d + q.d_H_r * H_c.d) * dx_inv;
-        q = flux_x(UL(i, j + 1), H_c.v, HC(i, j + 1), j + 1, nx);
-        d += (q.d_u * DU(i, j + 1) + q.d_H_l * H_c.d + q.d_H_r * Hd(i, j + 1).d) * dx_inv;
-        q = flux_y(VL(i, j), HC(i - 1, j), H_c.v, i, ny);
-        d += (q.d_u * DV(i, j) + q.d_H_l * Hd(i - 1, j).d + q.d_H_r * H_c.d) * dx_inv;
-        q = flux_y(VL(i + 1, j), H_c.v, HC(i + 1, j), i + 1, ny);
-        d -= (q.d_u * DV(i + 1, j) + q.d_H_l * H_c.d + q.d_H_r * Hd(i + 1, j).d) * dx_inv;
+    const uint32_t u0 = ou(i, j), v0 = ov(i, j), v1 = v0 + tc.pitch;
+    const double u_l = ld_off(bu, u0), u_r = ld_off(bu, u0 + 8), v_t = ld_off(bv, v0), v_b = ld_off(bv, v1);
+    const double x_l = ld_off(du, u0), x_r = ld_off(du, u0 + 8), y_t = ld_off(dv, v0), y_b = ld_off(dv, v1);
+    const double F_l = j > 0 ? K.hdx : 0.0, F_r = j + 1 < nx ? K.hdx : 0.0, F_t = i > 0 ? K.hdx : 0.0,
+                 F_b = i + 1 < ny ? K.hdx : 0.0;
+    const double H = S.H[a][b], H_l = S.H[a][b - 1], H_r = S.H[a][b + 1], H_t = S.H[a - 1][b], H_b = S.H[a + 1][b];
+    const double s_l = H_l + H, s_r = H + H_r, s_t = H_t + H, s_b = H + H_b;
+    const double m_l = u_l - fabs(u_l), q_r = u_r + fabs(u_r), q_t = v_t + fabs(v_t), m_b = v_b - fabs(v_b);
+    const double h = S.dH[a][b], h_l = S.dH[a][b - 1], h_r = S.dH[a][b + 1], h_t = S.dH[a - 1][b], h_b = S.dH[a + 1][b];
+    if (!VJP) {   // mass row (residuals.cu:343-375)
+        double d = div_refined(h, K.dt, K.rdt);
+        d += S.cd[a - 1][b - 1] * h;
+        d -= ((fma(-copysign(1.0, u_l), H - H_l, s_l) * x_l + (u_l + fabs(u_l)) * h_l) + m_l * h) * F_l;
+        d += ((fma(-copysign(1.0, u_r), H_r - H, s_r) * x_r + q_r * h) + (u_r - fabs(u_r)) * h_r) * F_r;
+        d += ((fma(-copysign(1.0, v_t), H_t - H, s_t) * y_t + (v_t - fabs(v_t)) * h_t) + q_t * h) * F_t;
+        d -= ((fma(-copysign(1.0, v_b), H - H_b, s_b) * y_b + m_b * h) + (v_b + fabs(v_b)) * h_b) * F_b;
         const double m = mask[kc];
-        out[nu + nv + kc] = (1.0 - m) * d + m * H_c.d;
+        out[nu + nv + kc] = (1.0 - m) * d + m * h;
         return;
     }
-    // 4c. VJP, cell (i, j): every row's derivative with respect to H(i, j)
-    const double Hc = HC(i, j), eta = E(i, j).v;
-    const double Hl = HC(i, j - 1), Hr = HC(i, j + 1), Ht = HC(i - 1, j), Hb = HC(i + 1, j);
-    const double lc = LM(i, j);
-    Flux qxl = flux_x(UL(i, j), Hl, Hc, j, nx);
-    Flux qxr = flux_x(UL(i, j + 1), Hc, Hr, j + 1, nx);
-    Flux qyt = flux_y(VL(i, j), Ht, Hc, i, ny);
-    Flux qyb = flux_y(VL(i + 1, j), Hc, Hb, i + 1, ny);
-    Calv jc = calving_g(Hc, G(i, j), p);
-    // own mass row (residuals.cu:648-690)
-    double acc = lc / dt;
-    acc += -lc * jc.d_H;
-    acc += -lc * qxl.d_H_r * dx_inv;
-    acc += lc * qxr.d_H_l * dx_inv;
-    acc += lc * qyt.d_H_r * dx_inv;
-    acc += -lc * qyb.d_H_l * dx_inv;
-    acc += dH[kc] * mask[kc];
+    // VJP: every row's derivative with respect to H(i, j).  Own mass row (residuals.cu:648-690)
+    double acc = div_refined(h, K.dt, K.rdt);
+    acc += h * S.cd[a - 1][b - 1];
+    acc -= (h * m_l) * F_l;
+    acc += (h * q_r) * F_r;
+    acc += (h * q_t) * F_t;
+    acc -= (h * m_b) * F_b;
+    acc += ld_off(dH, v0) * ld_off(bmask, v0);
     // neighbours' mass rows through the shared faces
-    if (j > 0) acc += LM(i, j - 1) * qxl.d_H_r * dx_inv;
-    if (j < nx - 1) acc += -LM(i, j + 1) * qxr.d_H_l * dx_inv;
-    if (i > 0) acc += -LM(i - 1, j) * qyt.d_H_r * dx_inv;
-    if (i < ny - 1) acc += LM(i + 1, j) * qyb.d_H_l * dx_inv;
+    acc += (h_l * m_l) * F_l;
+    acc -= (h_r * q_r) * F_r;
+    acc -= (h_t * q_t) * F_t;
+    acc += (h_b * m_b) * F_b;
     // momentum rows through eta*H of this cell: normal stresses
-    const double ul = UL(i, j), ur = UL(i, j + 1), vt = VL(i, j), vb = VL(i + 1, j);
-    SigN sx = sigma_xx(ul, ur, vt, vb, 0.0, dx_inv, j, nx);
-    SigN sy = sigma_yy(ul, ur, vt, vb, 0.0, dx_inv, i, ny);
-    const double lu_l = DU(i, j), lu_r = DU(i, j + 1), lv_t = DV(i, j), lv_b = DV(i + 1, j);
-    acc += lu_l * sx.d_eta_H * eta * dx_inv;
-    acc += -lu_r * sx.d_eta_H * eta * dx_inv;
-    acc += -lv_t * sy.d_eta_H * eta * dx_inv;
-    acc += lv_b * sy.d_eta_H * eta * dx_inv;
+    const double e2 = S.eh[a][b];
+    {
+        const double du_ = u_r - u_l, dv_ = v_t - v_b;
+        const double ex = fma(du_, K.dxi2, dv_ * K.dxi), ey = fma(du_, K.dxi, dv_ * K.dxi2);
+        acc += ((x_l * ex) * e2) * K.dxi;
+        acc -= ((x_r * ex) * e2) * K.dxi;
+        acc -= ((y_t * ey) * e2) * K.dxi;
+        acc += ((y_b * ey) * e2) * K.dxi;
+    }
     // shear stresses of the four corner vertices
-    const double q4 = 0.25 * eta;
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-        const int a = i + (c >> 1), b = j + (c & 1);
-        const double dv_ = EXY(a, b);
-        const double w = DU(a, b) - DU(a - 1, b) - DV(a, b) + DV(a, b - 1);
-        acc += w * dv_ * q4 * dx_inv;
+    {
+        const uint32_t ut = i > 0 ? u0 - tu.pitch : u0, ub = i < ny - 1 ? u0 + tu.pitch : u0, cl = j > 0 ? 8u : 0u,
+                       cr = j < nx - 1 ? 8u : 0u;
+        const double V_tl = i > 0 && j > 0 ? K.dxi : 0.0, V_tr = i > 0 && j < nx - 1 ? K.dxi : 0.0,
+                     V_bl = i < ny - 1 && j > 0 ? K.dxi : 0.0, V_br = i < ny - 1 && j < nx - 1 ? K.dxi : 0.0;
+        double e = fma(ld_off(bu, ut) - u_l, V_tl, (v_t - ld_off(bv, v0 - cl)) * V_tl);
+        double w = ((x_l - ld_off(du, ut)) - y_t) + ld_off(dv, v0 - cl);
+        acc += ((w * e) * e2) * K.edx;
+        e = fma(ld_off(bu, ut + 8) - u_r, V_tr, (ld_off(bv, v0 + cr) - v_t) * V_tr);
+        w = ((x_r - ld_off(du, ut + 8)) - ld_off(dv, v0 + cr)) + y_t;
+        acc += ((w * e) * e2) * K.edx;
+        e = fma(u_l - ld_off(bu, ub), V_bl, (v_b - ld_off(bv, v1 - cl)) * V_bl);
+        w = ((ld_off(du, ub) - x_l) - y_b) + ld_off(dv, v1 - cl);
+        acc += ((w * e) * e2) * K.edx;
+        e = fma(u_r - ld_off(bu, ub + 8), V_br, (ld_off(bv, v1 + cr) - v_b) * V_br);
+        w = ((ld_off(du, ub + 8) - x_r) - ld_off(dv, v1 + cr)) + y_b;
+        acc += ((w * e) * e2) * K.edx;
     }
     // basal drag (grounding-line derivatives) and driving stress on the four faces
-    {
-        const Ground ga = G(i, j - 1), gb = G(i, j);
-        TauB t = tau_b_g(ul, ga.g, gb.g, ga.gd, gb.gd, BETA(i, j - 1), BETA(i, j), p);
-        TauD d = tau_dx(Hl, Hc, BED(i, j - 1), BED(i, j), dx_inv, j, nx);
-        acc += lu_l * t.d_H_r;
-        acc += -lu_l * d.d_H_r;
-    }
-    {
-        const Ground ga = G(i, j), gb = G(i, j + 1);
-        TauB t = tau_b_g(ur, ga.g, gb.g, ga.gd, gb.gd, BETA(i, j), BETA(i, j + 1), p);
-        TauD d = tau_dx(Hc, Hr, BED(i, j), BED(i, j + 1), dx_inv, j + 1, nx);
-        acc += lu_r * t.d_H_l;
-        acc += -lu_r * d.d_H_l;
-    }
-    {
-        const Ground ga = G(i - 1, j), gb = G(i, j);
-        TauB t = tau_b_g(vt, ga.g, gb.g, ga.gd, gb.gd, BETA(i - 1, j), BETA(i, j), p);
-        TauD d = tau_dy(Ht, Hc, BED(i - 1, j), BED(i, j), dx_inv, i, ny);
-        acc += lv_t * t.d_H_r;
-        acc += -lv_t * d.d_H_r;
-    }
-    {
-        const Ground ga = G(i, j), gb = G(i + 1, j);
-        TauB t = tau_b_g(vb, ga.g, gb.g, ga.gd, gb.gd, BETA(i, j), BETA(i + 1, j), p);
-        TauD d = tau_dy(Hc, Hb, BED(i, j), BED(i + 1, j), dx_inv, i + 1, ny);
-        acc += lv_b * t.d_H_l;
-        acc += -lv_b * d.d_H_l;
-    }
+    const double Sc = S.S[a][b], sl = S.sl[a][b], db = -0.5 * S.db[a][b];
+    if (p.gl_derivatives) acc += x_l * (db * u_l);
+    acc -= x_l * fma(s_l * sl, F_l, (Sc - S.S[a][b - 1]) * F_l);
+    if (p.gl_derivatives) acc += x_r * (db * u_r);
+    acc -= x_r * fma(-(s_r * sl), F_r, (S.S[a][b + 1] - Sc) * F_r);
+    if (p.gl_derivatives) acc += y_t * (db * v_t);
+    acc -= y_t * fma(-(s_t * sl), F_t, (S.S[a - 1][b] - Sc) * F_t);
+    if (p.gl_derivatives) acc += y_b * (db * v_b);
+    acc -= y_b * fma(s_b * sl, F_b, (Sc - S.S[a + 1][b]) * F_b);
     emit(nu + nv + kc, acc);
 }
 

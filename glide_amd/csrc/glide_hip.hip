@@ -938,7 +938,7 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_jvp(GlideGeom g, 
                                                  const double *__restrict__ bed, const double *__restrict__ B,
                                                  const double *__restrict__ beta, const double *__restrict__ mask)
 {
-    __shared__ LinLDS<TX, LTY> S;
+    __shared__ LinLDS0<TX, LTY> S;
     const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
@@ -951,7 +951,7 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, 
                                                  const double *__restrict__ B, const double *__restrict__ beta,
                                                  const double *__restrict__ mask)
 {
-    __shared__ LinLDS<TX, LTY> S;
+    __shared__ LinLDS0<TX, LTY> S;
     const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
@@ -963,14 +963,16 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, 
 // chain; beyond that the 64 x 8 tiles' smaller halo and four waves a SIMD pay.
 // JVP, 64 x 6 / 64 x 8: 256^2 7.9 / 8.8 us, 384^2 11.4 / 13.3, 512^2 18.0 /
 // 13.4, 1024^2 56.7 / 47.5.  VJP, 64 x 4 / 64 x 8: 256^2 8.5 / 10.0, 384^2 13.1
-// / 15.1, 512^2 18.5 / 15.5, 1024^2 59.9 / 56.9.
+// / 15.1, 512^2 18.5 / 15.5, 1024^2 59.9 / 56.9.  The adjoint colours (k_adjoint)
+// change over at the VJP's line: 256^2 9.6 / 10.4, 384^2 18.0 / 19.3, 512^2 22.4
+// / 20.3, 1024^2 82.4 / 74.7.
+inline bool lin_tall(const GlideGeom &g) { return (long)cdiv(g.nx, TX) * cdiv(g.ny, 4) > 3L * n_cu(); }
 inline int lin_ty(const GlideGeom &g, bool vjp)
 {
     const int ty = g_lin_ty;
     if (ty >= 0) return ty;
-    const long tx = cdiv(g.nx, TX);
-    if (vjp) return tx * cdiv(g.ny, 4) <= 3L * n_cu() ? 4 : 8;
-    return tx * cdiv(g.ny, 6) <= 2L * n_cu() ? 6 : 8;
+    if (vjp) return lin_tall(g) ? 8 : 4;
+    return (long)cdiv(g.nx, TX) * cdiv(g.ny, 6) <= 2L * n_cu() ? 6 : 8;
 }
 // grid of the staged JVP / VJP
 inline dim3 lin_grid(const GlideGeom &g, int ty) { return dim3(chunked_grid(cdiv(g.nx, TX) * cdiv(g.ny, ty))); }
@@ -1021,6 +1023,24 @@ __global__ __launch_bounds__(NT) void k_vanka_adj(GlideGeom g, Params p, double 
     lam_out[kv0] = l2 + 0.5 * omega * d[2];
     lam_out[kv1] = l3 + 0.5 * omega * d[3];
     lam_out[kh] = l4 + omega * d[4];
+}
+
+// r = f_adj - J^T lam and one colour's update of lam into lam_out (adjoint_tile);
+// per colour, against k_vjp and k_vanka_adj: 64^2 17 -> 9.2 us, 256^2 17 -> 9.6
+// (an adjoint cycle of 256^2 3.08 -> 1.84 ms), 512^2 27 -> 20.3
+template <int LTY>
+__global__ __launch_bounds__(TX *LTY) void k_adjoint(GlideGeom g, Params p, double *__restrict__ lam_out,
+                                                     double *__restrict__ r, const double *__restrict__ f_adj,
+                                                     const double *__restrict__ U, const double *__restrict__ lam,
+                                                     const double *__restrict__ bed, const double *__restrict__ B,
+                                                     const double *__restrict__ beta, const double *__restrict__ mask,
+                                                     int color, double omega)
+{
+    __shared__ AdjLDS<TX, LTY> S;
+    const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
+    const int t = chunked_tile(blockIdx.x, total);
+    if (t >= total) return;
+    adjoint_tile<TX, LTY>(g, p, lam_out, r, f_adj, U, lam, bed, B, beta, mask, color, omega, t / tiles_y, t % tiles_y, S);
 }
 
 // grad_beta = lambda . dR/dbeta, gather form in the oracle's summation order
@@ -1441,13 +1461,20 @@ int compute_mask(const GlideLevel &A, hipStream_t st)
 int adjoint_sweeps(const GlideLevel &A, int n, double omega, hipStream_t st)
 {
     const Params p = to_params(A.p);
+    const bool tall = lin_tall(A.g);
+    const dim3 grid = lin_grid(A.g, tall ? 8 : 4), block(TX, tall ? 8 : 4);
     for (int s = 0; s < n; s++) {
-        for (int color = 0; color < 2; color++) {
-            TRY(launch_vjp(A.g, p, A.r_adj, A.f_adj, A.U, A.Lambda, A.bed, A.B, A.beta, A.mask, st));
-            hipLaunchKernelGGL(k_vanka_adj, cell_grid(A.g.ny, A.g.nx), dim3(TX, TY), 0, st, A.g, p, A.Lambda, A.Lambda,
-                               A.mask, A.r_adj, A.U, A.bed, A.B, A.beta, A.gamma, color, omega);
-            TRY(check_launch("vanka adjoint"));
+        for (int color = 0; color < 2; color++) {   // red into the Vanka scratch (5 values a cell), black back
+            double *out = color ? A.Lambda : A.scratch;
+            const double *lam = color ? A.scratch : A.Lambda;
+            if (tall)
+                hipLaunchKernelGGL(k_adjoint<8>, grid, block, 0, st, A.g, p, out, A.r_adj, A.f_adj, A.U, lam, A.bed, A.B,
+                                   A.beta, A.mask, color, omega);
+            else
+                hipLaunchKernelGGL(k_adjoint<4>, grid, block, 0, st, A.g, p, out, A.r_adj, A.f_adj, A.U, lam, A.bed, A.B,
+                                   A.beta, A.mask, color, omega);
         }
+        TRY(check_launch("adjoint sweep"));
     }
     return GLIDE_OK;
 }
@@ -1598,7 +1625,7 @@ int glide_set_tile_height(int kernel, int ty)
 {
     if (kernel == 0) {
         if (ty != 0 && ty != 4 && ty != 8 && ty != 16)
-            return fail(GLIDE_E_ARG, "residual tile height must be 0 (by level size), 4, 8 or 16");
+            return fail(GLIDE_E_ARG, "residual tile height must be 0 (the default), 4, 8 or 16");
         g_res_ty = ty;
     } else if (kernel == 1) {
         if (ty != 0 && ty != 4 && ty != 6 && ty != 8) return fail(GLIDE_E_ARG, "JVP/VJP tile height must be 0, 4, 6 or 8");

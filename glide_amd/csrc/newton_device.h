@@ -234,27 +234,51 @@ struct NewtonX {
     double u_l, u_r, v_t, v_b, H;
 };
 
-// One damped iteration x -= 0.25 A^-1 r, H = max(H, th).  CLAMPED: the cell's
-// sigmoid argument reaches its clamp; GL: p.gl_derivatives.
+// What the cell's own thickness gives: drag, surface and its slope, calving rate
+// times (1 - g), d mass row / d H without the fluxes, d drag / d H.
+struct NewtonCentre {
+    double be, S, sl, cal, qH, db;
+};
+// CLAMPED: the cell's sigmoid argument reaches its clamp; GL: p.gl_derivatives
 template <bool CLAMPED, bool GL>
-__host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const NewtonK &K, const Params &p, NewtonX &x)
+__host__ __device__ __forceinline__ NewtonCentre newton_centre(const NewtonCell &C, const NewtonK &K, const Params &p, double H)
 {
-    const double u_l = x.u_l, u_r = x.u_r, v_t = x.v_t, v_b = x.v_b, H = x.H;
-    // the cell's own sigmoid, drag and surface
+    NewtonCentre M;
     const double z = fma(0.917, H, C.bed);
     const double g = CLAMPED ? sigm_end(z, p.gl_c) : sigm_mid(z, p.gl_c);
     const double g1 = 1.0 - g;
-    const double be = fma(g, C.beta, g1 * p.water_drag);
+    M.be = fma(g, C.beta, g1 * p.water_drag);
     const double Hf = -0.917 * H;
-    const double S = fmax(C.bed, Hf) + H;
-    const double sl = C.bed > Hf ? 1.0 : 1.0 + -0.917;   // 1 + d base / d H
+    M.S = fmax(C.bed, Hf) + H;
+    M.sl = C.bed > Hf ? 1.0 : 1.0 + -0.917;   // 1 + d base / d H
+    M.cal = p.calving_rate * g1;
+    M.qH = K.idt + M.cal;
+    M.db = 0.0;
+    if (GL) {
+        const double dg = 0.917 * (p.gl_c * g * g1);
+        M.qH = K.idt - fma(p.calving_rate * H, dg, -M.cal);
+        M.db = dg * (C.beta - p.water_drag);
+    }
+    return M;
+}
 
+// The block [[a0, t2, t, -t, c0], [t2, a1, -t, t, c1], [t, -t, a2, t2, c2],
+// [-t, t, t2, a3, c3], [q0, q1, q2, q3, qH]] and its right-hand side
+struct NewtonSystem {
+    double a0, a1, a2, a3, t, c0, c1, c2, c3, q0, q1, q2, q3, qH;
+    double r0, r1, r2, r3, r4;
+};
+// ADJ: the block alone, its mass row the identity where `masked`
+template <bool GL, bool ADJ>
+__host__ __device__ __forceinline__ NewtonSystem newton_system(const NewtonCell &C, const NewtonK &K, const NewtonCentre &M,
+                                                              const NewtonX &x, bool masked)
+{
+    const double u_l = x.u_l, u_r = x.u_r, v_t = x.v_t, v_b = x.v_b, H = x.H;
+    const double be = M.be, S = M.S, sl = M.sl;
     // mass row (J20..J23 = q0..q3, J24 = qH): H/dt, calving, the four upwind fluxes
     double r4 = div_refined(H, K.dt, K.rdt) - C.f4;
-    const double cal = p.calving_rate * g1;
-    double qH = K.idt + cal;
-    r4 = r4 + cal * H;
-    if (GL) qH = K.idt - fma(p.calving_rate * H, 0.917 * (p.gl_c * g * g1), -cal);
+    double qH = M.qH;
+    r4 = r4 + M.cal * H;
     const double s_l = C.H_l + H, s_r = H + C.H_r, s_t = C.H_t + H, s_b = H + C.H_b;
     double q0, q1, q2, q3;
     {   // twice the flux and its derivatives; the factors F carry 1/(2 dx)
@@ -281,7 +305,7 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
         qH = fma(-(v_b - fabs(v_b)), C.F_b, qH);
         r4 = fma(-f, C.F_b, r4);
     }
-    if ((H - K.dt * r4) <= C.th) {
+    if (ADJ ? masked : (H - K.dt * r4) <= C.th) {
         q0 = q1 = q2 = q3 = 0.0;
         qH = 1.0;
         r4 = H - C.th;
@@ -379,11 +403,10 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
         r3 = fma(-0.5, b_b * v_b, r3);
         a3 = fma(-0.5, b_b, a3);
         if (GL) {
-            const double db = (0.917 * (p.gl_c * g * g1)) * (C.beta - p.water_drag);
-            c0 = c0 + -0.5 * db * u_l;
-            c1 = c1 + -0.5 * db * u_r;
-            c2 = c2 + -0.5 * db * v_t;
-            c3 = c3 + -0.5 * db * v_b;
+            c0 = c0 + -0.5 * M.db * u_l;
+            c1 = c1 + -0.5 * M.db * u_r;
+            c2 = c2 + -0.5 * M.db * v_t;
+            c3 = c3 + -0.5 * M.db * v_b;
         }
     }
     {   // driving stress
@@ -397,16 +420,17 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
         r3 = r3 - (s_b * d_b) * C.F_b;
         c3 = c3 - fma(s_b * sl, C.F_b, d_b * C.F_b);
     }
-    a0 = a0 - 1.0;
-    a1 = a1 - 1.0;
-    a2 = a2 - 1.0;
-    a3 = a3 - 1.0;
-    qH = qH + 1.0;
+    return {a0, a1, a2, a3, t, c0, c1, c2, c3, q0, q1, q2, q3, qH, r0, r1, r2, r3, r4};
+}
 
-    // LU of [[a0, t2, t, -t, c0], [t2, a1, -t, t, c1], [t, -t, a2, t2, c2],
-    // [-t, t, t2, a3, c3], [q0, q1, q2, q3, qH]] as lu5_solve takes it
+// x = A^-1 r as lu5_solve takes it
+__host__ __device__ __forceinline__ void newton_solve(const NewtonSystem &A, double &x0, double &x1, double &x2, double &x3,
+                                                      double &x4)
+{
+    const double t = A.t, t2 = t + t, a0 = A.a0, c0 = A.c0, r0 = A.r0;
+    double a1 = A.a1, a2 = A.a2, a3 = A.a3, c1 = A.c1, c2 = A.c2, c3 = A.c3, q1 = A.q1, q2 = A.q2, q3 = A.q3, qH = A.qH;
     const double i0 = recip(a0);
-    const double m = t * i0, m2 = m + m, l0 = q0 * i0;   // column 0 below a0: m2, m, -m, l0
+    const double m = t * i0, m2 = m + m, l0 = A.q0 * i0;   // column 0 below a0: m2, m, -m, l0
     a1 = fma(-m2, t2, a1);
     const double B = fma(-m2, t, -t);
     c1 = fma(-m2, c0, c1);
@@ -439,20 +463,45 @@ __host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const 
     const double l3 = q3 * i3;
     qH = fma(-l3, c3, qH);
     const double i4 = recip(qH);
-    const double y1 = fma(-m2, r0, r1);
-    const double y2 = fma(-k, y1, fma(-m, r0, r2));
-    const double y3 = fma(-w, y2, fma(k, y1, fma(m, r0, r3)));
-    const double y4 = fma(-l3, y3, fma(-l2, y2, fma(-l1, y1, fma(-l0, r0, r4))));
-    const double x4 = y4 * i4;
-    const double x3 = fma(-c3, x4, y3) * i3;
-    const double x2 = fma(-D, x3, fma(-c2, x4, y2)) * i2;
-    const double x1 = fma(-B, x2, fma(B, x3, fma(-c1, x4, y1))) * i1;
-    const double x0 = fma(-t2, x1, fma(-t, x2, fma(t, x3, fma(-c0, x4, r0)))) * i0;
-    x.u_l = fma(-0.25, x0, u_l);
-    x.u_r = fma(-0.25, x1, u_r);
-    x.v_t = fma(-0.25, x2, v_t);
-    x.v_b = fma(-0.25, x3, v_b);
-    x.H = fmax(fma(-0.25, x4, H), C.th);
+    const double y1 = fma(-m2, r0, A.r1);
+    const double y2 = fma(-k, y1, fma(-m, r0, A.r2));
+    const double y3 = fma(-w, y2, fma(k, y1, fma(m, r0, A.r3)));
+    const double y4 = fma(-l3, y3, fma(-l2, y2, fma(-l1, y1, fma(-l0, r0, A.r4))));
+    x4 = y4 * i4;
+    x3 = fma(-c3, x4, y3) * i3;
+    x2 = fma(-D, x3, fma(-c2, x4, y2)) * i2;
+    x1 = fma(-B, x2, fma(B, x3, fma(-c1, x4, y1))) * i1;
+    x0 = fma(-t2, x1, fma(-t, x2, fma(t, x3, fma(-c0, x4, r0)))) * i0;
+}
+
+// One damped iteration x -= 0.25 A^-1 r, H = max(H, th)
+template <bool CLAMPED, bool GL>
+__host__ __device__ __forceinline__ void newton_step(const NewtonCell &C, const NewtonK &K, const Params &p, NewtonX &x)
+{
+    NewtonSystem A = newton_system<GL, false>(C, K, newton_centre<CLAMPED, GL>(C, K, p, x.H), x, false);
+    A.a0 = A.a0 - 1.0;
+    A.a1 = A.a1 - 1.0;
+    A.a2 = A.a2 - 1.0;
+    A.a3 = A.a3 - 1.0;
+    A.qH = A.qH + 1.0;
+    double x0, x1, x2, x3, x4;
+    newton_solve(A, x0, x1, x2, x3, x4);
+    x.u_l = fma(-0.25, x0, x.u_l);
+    x.u_r = fma(-0.25, x1, x.u_r);
+    x.v_t = fma(-0.25, x2, x.v_t);
+    x.v_b = fma(-0.25, x3, x.v_b);
+    x.H = fmax(fma(-0.25, x4, x.H), C.th);
+}
+
+// d = A^-T r of the adjoint block (vanka_assemble<1>): the velocity block is
+// symmetric, so the transpose swaps the H column and the mass row.
+template <bool GL>
+__host__ __device__ __forceinline__ void newton_adjoint(const NewtonCell &C, const NewtonK &K, const NewtonCentre &M,
+                                                        const NewtonX &x, bool masked, const double r[5], double d[5])
+{
+    const NewtonSystem A = newton_system<GL, true>(C, K, M, x, masked);
+    newton_solve({A.a0, A.a1, A.a2, A.a3, A.t, A.q0, A.q1, A.q2, A.q3, A.c0, A.c1, A.c2, A.c3, A.qH, r[0], r[1], r[2], r[3], r[4]},
+                 d[0], d[1], d[2], d[3], d[4]);
 }
 
 // n_newton iterations.  Ice 200 m above or below flotation (at the default

@@ -777,125 +777,161 @@ __device__ __forceinline__ void glen_pow_dual(double x, double q, double &v, dou
     }
 }
 
-// VJP: out = base - l when base != NULL (the adjoint residual f_adj - J^T lambda)
-template <int TX, int TY, bool VJP>
-__device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p, double *__restrict__ out,
-                                             const double *__restrict__ base, const double *__restrict__ U,
-                                             const double *__restrict__ D, const double *__restrict__ bed,
-                                             const double *__restrict__ B, const double *__restrict__ beta,
-                                             const double *__restrict__ mask, int bx, int by, LinLDS<TX, TY> &S)
-{
-    constexpr int NT = TX * TY, NALL = (TY + 2) * (TX + 2);
-    const int ny = g.ny, nx = g.nx;
-    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
-    const int i0 = by * TY, j0 = bx * TX;
-    const int rb = max(i0 - 2, 0), cb = max(j0 - 2, 0);
-    const TileField tu(nx + 1, rb, cb), tc(nx, rb, cb);
-    const char *bu = tu.base(U), *bv = tc.base(U + nu), *bH = tc.base(U + nu + nv);
-    const char *du = tu.base(D), *dv = tc.base(D + nu), *dH = tc.base(D + nu + nv);
-    const char *bbed = tc.base(bed), *bB = tc.base(B), *bbeta = tc.base(beta), *bmask = tc.base(mask);
-    const int tid = threadIdx.y * TX + threadIdx.x;
-    const NewtonK K = newton_constants(g.dx, g.dt);
-    const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+template <int TX, int TY>
+struct LinLDS0 : LinLDS<TX, TY> {
+    __device__ __forceinline__ void keep(int, int, double, double) {}
+};
+// ... with the smoother's 2 eta and 2 eta H, whose viscosity rounds differently (fma, eta2_from)
+template <int TX, int TY>
+struct AdjLDS : LinLDS<TX, TY> {
+    double s_e2[TY + 2][TX + 2], s_n[TY + 2][TX + 2];
+    __device__ __forceinline__ void keep(int a, int b, double e2, double n)
+    {
+        s_e2[a][b] = e2;
+        s_n[a][b] = n;
+    }
+};
+
+// One tile: stage() fills the LDS (all threads), then the rows may be asked
+// for: u faces (i0.., j0..j0+TX), v faces (i0..i0+TY, j0..), cells.  ADJ: LDS is an AdjLDS.
+template <int TX, int TY, bool VJP, bool ADJ>
+struct LinTile {
+    using LDS = typename std::conditional<ADJ, AdjLDS<TX, TY>, LinLDS0<TX, TY>>::type;
+    static constexpr int NT = TX * TY, NALL = (TY + 2) * (TX + 2);
+    LDS &S;
+    const Params &p;
+    const int ny, nx, i0, j0, rb, cb;
+    const TileField tu, tc;
+    const char *bu, *bv, *bH, *du, *dv, *dH, *bbed, *bB, *bbeta, *bmask;
+    const NewtonK K;
+
+    __device__ __forceinline__ LinTile(LDS &S_, const GlideGeom &g, const Params &p_, const double *__restrict__ U,
+                                       const double *__restrict__ D, const double *__restrict__ bed,
+                                       const double *__restrict__ B, const double *__restrict__ beta,
+                                       const double *__restrict__ mask, int bx, int by)
+        : S(S_), p(p_), ny(g.ny), nx(g.nx), i0(by * TY), j0(bx * TX), rb(max(i0 - 2, 0)), cb(max(j0 - 2, 0)),
+          tu(nx + 1, rb, cb), tc(nx, rb, cb), K(newton_constants(g.dx, g.dt))
+    {
+        const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+        bu = tu.base(U), bv = tc.base(U + nu), bH = tc.base(U + nu + nv);
+        du = tu.base(D), dv = tc.base(D + nu), dH = tc.base(D + nu + nv);
+        bbed = tc.base(bed), bB = tc.base(B), bbeta = tc.base(beta), bmask = tc.base(mask);
+    }
     // byte offsets of (row, column), clamped to the field
-    auto ou = [&](int i, int j) { return (uint32_t)(clampi(i, 0, ny - 1) - rb) * tu.pitch + 8u * (clampi(j, 0, nx) - cb); };
-    auto ov = [&](int i, int j) { return (uint32_t)(clampi(i, 0, ny) - rb) * tc.pitch + 8u * (clampi(j, 0, nx - 1) - cb); };
-    // 1. per cell
-#pragma unroll 1
-    for (int k = tid; k < NALL; k += NT) {
-        const int a = k / (TX + 2), b = k - a * (TX + 2);
-        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
-        const int ic = clampi(ci, 0, ny - 1), jc = clampi(cj, 0, nx - 1);
-        const uint32_t r0 = ic - rb, c0 = 8u * (jc - cb), u0 = r0 * tu.pitch + c0, v0 = r0 * tc.pitch + c0;
-        const double h = ld_off(bH, v0), bd = ld_off(bbed, v0), bt = ld_off(bbeta, v0);
-        double hd = ld_off(dH, v0);
-        if (VJP) hd = hd * (1.0 - ld_off(bmask, v0));
-        double n = 0.0, nh = 0.0, ne = 0.0, tx = 0.0, ty = 0.0;
-        if (ic == ci && jc == cj) {
-            const uint32_t v1 = v0 + tc.pitch;   // row i+1 of v and column j+1 of u exist for every cell
-            const bool t = ci > 0, bo = ci < ny - 1, l = cj > 0, r = cj < nx - 1;
-            const uint32_t ut = t ? u0 - tu.pitch : u0, ub = bo ? u0 + tu.pitch : u0, cl = l ? 8u : 0u, cr = r ? 8u : 0u;
-            const double u_l = ld_off(bu, u0), u_r = ld_off(bu, u0 + 8), v_t = ld_off(bv, v0), v_b = ld_off(bv, v1);
-            const double x_l = ld_off(du, u0), x_r = ld_off(du, u0 + 8), y_t = ld_off(dv, v0), y_b = ld_off(dv, v1);
-            const double V_tl = t && l ? K.dxi : 0.0, V_tr = t && r ? K.dxi : 0.0, V_bl = bo && l ? K.dxi : 0.0,
-                         V_br = bo && r ? K.dxi : 0.0;
-            // corner shear rates (doubled) and their derivatives
-            const double e_tl = (ld_off(bu, ut) - u_l) * V_tl + (v_t - ld_off(bv, v0 - cl)) * V_tl;
-            const double e_tr = (ld_off(bu, ut + 8) - u_r) * V_tr + (ld_off(bv, v0 + cr) - v_t) * V_tr;
-            const double e_bl = (u_l - ld_off(bu, ub)) * V_bl + (v_b - ld_off(bv, v1 - cl)) * V_bl;
-            const double e_br = (u_r - ld_off(bu, ub + 8)) * V_br + (ld_off(bv, v1 + cr) - v_b) * V_br;
-            const double d_tl = (ld_off(du, ut) - x_l) * V_tl + (y_t - ld_off(dv, v0 - cl)) * V_tl;
-            const double d_tr = (ld_off(du, ut + 8) - x_r) * V_tr + (ld_off(dv, v0 + cr) - y_t) * V_tr;
-            const double d_bl = (x_l - ld_off(du, ub)) * V_bl + (y_b - ld_off(dv, v1 - cl)) * V_bl;
-            const double d_br = (x_r - ld_off(du, ub + 8)) * V_br + (ld_off(dv, v1 + cr) - y_b) * V_br;
-            const double a_ = u_r - u_l, b_ = v_t - v_b;
-            const double ux = a_ * K.dxi, vy = b_ * K.dxi, uxd = (x_r - x_l) * K.dxi, vyd = (y_t - y_b) * K.dxi;
-            const double e2 = ((e_tl * e_tl + e_tr * e_tr) + e_bl * e_bl) + e_br * e_br;
-            const double e2d = ((fma(e_tl, d_tl, d_tl * e_tl) + fma(e_tr, d_tr, d_tr * e_tr)) + fma(e_bl, d_bl, d_bl * e_bl)) +
-                               fma(e_br, d_br, d_br * e_br);
-            const double eII = fma(0.0625, e2, (ux * ux + vy * vy) + ux * vy) + p.eps_reg;
-            const double eIId = fma(0.0625, e2d, (fma(ux, uxd, uxd * ux) + fma(vy, vyd, vyd * vy)) + fma(ux, vyd, uxd * vy));
-            double pv, pc;
-            glen_pow_dual(eII, glen_exp, pv, pc);
-            const double Bc = ld_off(bB, v0);
-            const double ev = pv * Bc, ed = (pc * eIId) * Bc;   // 2 eta and its derivative
-            n = ev * h;
-            nh = h * ed;
-            ne = VJP ? ev : ev * hd;
-            const double nd = VJP ? nh : nh + ne;
-            const double ex = fma(a_, K.dxi2, b_ * K.dxi), ey = fma(a_, K.dxi, b_ * K.dxi2);
-            const double p1 = n * K.dxi, p2 = p1 + p1;
-            tx = (((p2 * x_r - p2 * x_l) + p1 * y_t) - p1 * y_b) + ex * nd;
-            ty = (((p1 * x_r - p1 * x_l) + p2 * y_t) - p2 * y_b) + ey * nd;
-        }
-        const double z = fma(0.917, h, bd), gr = sigm_mid(z, p.gl_c), g1 = 1.0 - gr, Hf = -0.917 * h;
-        double njd = p.calving_rate * g1, db = 0.0;
-        if (p.gl_derivatives) {
-            const double dg = 0.917 * (p.gl_c * gr * g1);
-            njd = -fma(p.calving_rate * h, dg, -njd);
-            db = dg * (bt - p.water_drag);
-        }
-        S.n[a][b] = n;
-        S.hd[a][b] = nh;
-        S.eh[a][b] = ne;
-        S.tx[a][b] = tx;
-        S.ty[a][b] = ty;
-        S.H[a][b] = h;
-        S.dH[a][b] = hd;
-        S.S[a][b] = fmax(bd, Hf) + h;
-        S.sl[a][b] = bd > Hf ? 1.0 : 1.0 + -0.917;
-        S.be[a][b] = fma(gr, bt, g1 * p.water_drag);
-        S.db[a][b] = db;
-        if (a >= 1 && a <= TY && b >= 1 && b <= TX) S.cd[a - 1][b - 1] = njd;
+    __device__ __forceinline__ uint32_t ou(int i, int j) const
+    {
+        return (uint32_t)(clampi(i, 0, ny - 1) - rb) * tu.pitch + 8u * (clampi(j, 0, nx) - cb);
     }
-    __syncthreads();
-    // 2. per vertex, 0 on the domain edge
-#pragma unroll 1
-    for (int k = tid; k < (TY + 1) * (TX + 1); k += NT) {
-        const int a = k / (TX + 1), b = k - a * (TX + 1);   // vertex (i0 + a, j0 + b): cells [a..a+1][b..b+1]
-        const int vi = i0 + a, vj = j0 + b;
-        double t8 = 0.0;
-        if (vi > 0 && vi < ny && vj > 0 && vj < nx) {
-            const uint32_t ub = (uint32_t)(vi - rb) * tu.pitch + 8u * (vj - cb), ut = ub - tu.pitch;
-            const uint32_t vr = (uint32_t)(vi - rb) * tc.pitch + 8u * (vj - cb), vl = vr - 8;
-            const double m = ((S.n[a][b] + S.n[a][b + 1]) + S.n[a + 1][b]) + S.n[a + 1][b + 1];
-            const double md =
-                VJP ? ((S.hd[a][b] + S.hd[a][b + 1]) + S.hd[a + 1][b]) + S.hd[a + 1][b + 1]
-                    : ((((((S.hd[a][b] + S.eh[a][b]) + S.hd[a][b + 1]) + S.eh[a][b + 1]) + S.hd[a + 1][b]) + S.eh[a + 1][b]) +
-                       S.hd[a + 1][b + 1]) +
-                          S.eh[a + 1][b + 1];
-            const double q = m * K.dxi;
-            const double x = fma(ld_off(bu, ut) - ld_off(bu, ub), K.dxi, (ld_off(bv, vr) - ld_off(bv, vl)) * K.dxi);
-            t8 = (((q * ld_off(du, ut) - q * ld_off(du, ub)) - q * ld_off(dv, vl)) + q * ld_off(dv, vr)) + x * md;
-        }
-        S.txy[a][b] = t8;
+    __device__ __forceinline__ uint32_t ov(int i, int j) const
+    {
+        return (uint32_t)(clampi(i, 0, ny) - rb) * tc.pitch + 8u * (clampi(j, 0, nx - 1) - cb);
     }
-    __syncthreads();
-    const int i = i0 + threadIdx.y, j = j0 + threadIdx.x;
-    if (i > ny || j > nx) return;
-    auto emit = [&](size_t k, double val) { out[k] = (VJP && base) ? base[k] - val : val; };
-    // 3a. u face (i, j): J_u d (glide/cuda/residuals.cu:378-499)
-    auto urow = [&](int i, int j) {
+
+    __device__ __forceinline__ void stage() const
+    {
+        const int tid = threadIdx.y * TX + threadIdx.x;
+        const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+        // 1. per cell
+    #pragma unroll 1
+        for (int k = tid; k < NALL; k += NT) {
+            const int a = k / (TX + 2), b = k - a * (TX + 2);
+            const int ci = i0 - 1 + a, cj = j0 - 1 + b;
+            const int ic = clampi(ci, 0, ny - 1), jc = clampi(cj, 0, nx - 1);
+            const uint32_t r0 = ic - rb, c0 = 8u * (jc - cb), u0 = r0 * tu.pitch + c0, v0 = r0 * tc.pitch + c0;
+            const double h = ld_off(bH, v0), bd = ld_off(bbed, v0), bt = ld_off(bbeta, v0);
+            double hd = ld_off(dH, v0);
+            if (VJP) hd = hd * (1.0 - ld_off(bmask, v0));
+            double n = 0.0, nh = 0.0, ne = 0.0, tx = 0.0, ty = 0.0, se = 0.0;
+            if (ic == ci && jc == cj) {
+                const uint32_t v1 = v0 + tc.pitch;   // row i+1 of v and column j+1 of u exist for every cell
+                const bool t = ci > 0, bo = ci < ny - 1, l = cj > 0, r = cj < nx - 1;
+                const uint32_t ut = t ? u0 - tu.pitch : u0, ub = bo ? u0 + tu.pitch : u0, cl = l ? 8u : 0u, cr = r ? 8u : 0u;
+                const double u_l = ld_off(bu, u0), u_r = ld_off(bu, u0 + 8), v_t = ld_off(bv, v0), v_b = ld_off(bv, v1);
+                const double x_l = ld_off(du, u0), x_r = ld_off(du, u0 + 8), y_t = ld_off(dv, v0), y_b = ld_off(dv, v1);
+                const double V_tl = t && l ? K.dxi : 0.0, V_tr = t && r ? K.dxi : 0.0, V_bl = bo && l ? K.dxi : 0.0,
+                             V_br = bo && r ? K.dxi : 0.0;
+                // corner shear rates (doubled) and their derivatives
+                const double e_tl = (ld_off(bu, ut) - u_l) * V_tl + (v_t - ld_off(bv, v0 - cl)) * V_tl;
+                const double e_tr = (ld_off(bu, ut + 8) - u_r) * V_tr + (ld_off(bv, v0 + cr) - v_t) * V_tr;
+                const double e_bl = (u_l - ld_off(bu, ub)) * V_bl + (v_b - ld_off(bv, v1 - cl)) * V_bl;
+                const double e_br = (u_r - ld_off(bu, ub + 8)) * V_br + (ld_off(bv, v1 + cr) - v_b) * V_br;
+                const double d_tl = (ld_off(du, ut) - x_l) * V_tl + (y_t - ld_off(dv, v0 - cl)) * V_tl;
+                const double d_tr = (ld_off(du, ut + 8) - x_r) * V_tr + (ld_off(dv, v0 + cr) - y_t) * V_tr;
+                const double d_bl = (x_l - ld_off(du, ub)) * V_bl + (y_b - ld_off(dv, v1 - cl)) * V_bl;
+                const double d_br = (x_r - ld_off(du, ub + 8)) * V_br + (ld_off(dv, v1 + cr) - y_b) * V_br;
+                const double a_ = u_r - u_l, b_ = v_t - v_b;
+                const double ux = a_ * K.dxi, vy = b_ * K.dxi, uxd = (x_r - x_l) * K.dxi, vyd = (y_t - y_b) * K.dxi;
+                const double e2 = ((e_tl * e_tl + e_tr * e_tr) + e_bl * e_bl) + e_br * e_br;
+                const double e2d = ((fma(e_tl, d_tl, d_tl * e_tl) + fma(e_tr, d_tr, d_tr * e_tr)) + fma(e_bl, d_bl, d_bl * e_bl)) +
+                                   fma(e_br, d_br, d_br * e_br);
+                if (ADJ) {
+                    se = eta2_from(ci, cj, ny, nx, u_l, u_r, v_t, v_b, ld_off(bu, ut), ld_off(bu, ut + 8), ld_off(bu, ub),
+                                             ld_off(bu, ub + 8), ld_off(bv, v0 - cl), ld_off(bv, v0 + cr), ld_off(bv, v1 - cl),
+                                             ld_off(bv, v1 + cr), ld_off(bB, v0), p, glen_exp, K.dxi);
+                }
+                const double eII = fma(0.0625, e2, (ux * ux + vy * vy) + ux * vy) + p.eps_reg;
+                const double eIId = fma(0.0625, e2d, (fma(ux, uxd, uxd * ux) + fma(vy, vyd, vyd * vy)) + fma(ux, vyd, uxd * vy));
+                double pv, pc;
+                glen_pow_dual(eII, glen_exp, pv, pc);
+                const double Bc = ld_off(bB, v0);
+                const double ev = pv * Bc, ed = (pc * eIId) * Bc;   // 2 eta and its derivative
+                n = ev * h;
+                nh = h * ed;
+                ne = VJP ? ev : ev * hd;
+                const double nd = VJP ? nh : nh + ne;
+                const double ex = fma(a_, K.dxi2, b_ * K.dxi), ey = fma(a_, K.dxi, b_ * K.dxi2);
+                const double p1 = n * K.dxi, p2 = p1 + p1;
+                tx = (((p2 * x_r - p2 * x_l) + p1 * y_t) - p1 * y_b) + ex * nd;
+                ty = (((p1 * x_r - p1 * x_l) + p2 * y_t) - p2 * y_b) + ey * nd;
+            }
+            const double z = fma(0.917, h, bd), gr = sigm_mid(z, p.gl_c), g1 = 1.0 - gr, Hf = -0.917 * h;
+            double njd = p.calving_rate * g1, db = 0.0;
+            if (p.gl_derivatives) {
+                const double dg = 0.917 * (p.gl_c * gr * g1);
+                njd = -fma(p.calving_rate * h, dg, -njd);
+                db = dg * (bt - p.water_drag);
+            }
+            S.n[a][b] = n;
+            S.keep(a, b, se, se * h);
+            S.hd[a][b] = nh;
+            S.eh[a][b] = ne;
+            S.tx[a][b] = tx;
+            S.ty[a][b] = ty;
+            S.H[a][b] = h;
+            S.dH[a][b] = hd;
+            S.S[a][b] = fmax(bd, Hf) + h;
+            S.sl[a][b] = bd > Hf ? 1.0 : 1.0 + -0.917;
+            S.be[a][b] = fma(gr, bt, g1 * p.water_drag);
+            S.db[a][b] = db;
+            if (a >= 1 && a <= TY && b >= 1 && b <= TX) S.cd[a - 1][b - 1] = njd;
+        }
+        __syncthreads();
+        // 2. per vertex, 0 on the domain edge
+    #pragma unroll 1
+        for (int k = tid; k < (TY + 1) * (TX + 1); k += NT) {
+            const int a = k / (TX + 1), b = k - a * (TX + 1);   // vertex (i0 + a, j0 + b): cells [a..a+1][b..b+1]
+            const int vi = i0 + a, vj = j0 + b;
+            double t8 = 0.0;
+            if (vi > 0 && vi < ny && vj > 0 && vj < nx) {
+                const uint32_t ub = (uint32_t)(vi - rb) * tu.pitch + 8u * (vj - cb), ut = ub - tu.pitch;
+                const uint32_t vr = (uint32_t)(vi - rb) * tc.pitch + 8u * (vj - cb), vl = vr - 8;
+                const double m = ((S.n[a][b] + S.n[a][b + 1]) + S.n[a + 1][b]) + S.n[a + 1][b + 1];
+                const double md =
+                    VJP ? ((S.hd[a][b] + S.hd[a][b + 1]) + S.hd[a + 1][b]) + S.hd[a + 1][b + 1]
+                        : ((((((S.hd[a][b] + S.eh[a][b]) + S.hd[a][b + 1]) + S.eh[a][b + 1]) + S.hd[a + 1][b]) + S.eh[a + 1][b]) +
+                           S.hd[a + 1][b + 1]) +
+                              S.eh[a + 1][b + 1];
+                const double q = m * K.dxi;
+                const double x = fma(ld_off(bu, ut) - ld_off(bu, ub), K.dxi, (ld_off(bv, vr) - ld_off(bv, vl)) * K.dxi);
+                t8 = (((q * ld_off(du, ut) - q * ld_off(du, ub)) - q * ld_off(dv, vl)) + q * ld_off(dv, vr)) + x * md;
+            }
+            S.txy[a][b] = t8;
+        }
+        __syncthreads();
+    }
+    // u face (i, j): J_u d (glide/cuda/residuals.cu:378-499)
+    __device__ __forceinline__ double u_row(int i, int j) const
+    {
         const int a = i - i0 + 1, b = j - j0 + 1;
         const uint32_t o = ou(i, j);
         const double u_l = ld_off(bu, o), x_l = ld_off(du, o);
@@ -916,10 +952,11 @@ __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p
             const double D2 = fma(-copysign(1.0, u_l), H_c - H_l, s);
             d = ((S.dH[a][b - 1] * D2) * F - (S.dH[a][b] * D2) * F) + d;
         }
-        emit((size_t)i * (nx + 1) + j, d);
-    };
-    // 3b. v face (i, j) (residuals.cu:501-576)
-    auto vrow = [&](int i, int j) {
+        return d;
+    }
+    // v face (i, j) (residuals.cu:501-576)
+    __device__ __forceinline__ double v_row(int i, int j) const
+    {
         const int a = i - i0 + 1, b = j - j0 + 1;
         const uint32_t o = ov(i, j);
         const double v_t = ld_off(bv, o), y_t = ld_off(dv, o);
@@ -940,89 +977,216 @@ __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p
             const double D2 = fma(-copysign(1.0, v_t), H_t - H_c, s);
             d = ((S.dH[a][b] * D2) * F - (S.dH[a - 1][b] * D2) * F) + d;
         }
-        emit(nu + (size_t)i * nx + j, d);
-    };
+        return d;
+    }
+    // cell (i, j)
+    __device__ __forceinline__ double h_row(int i, int j) const
+    {
+        const int a = i - i0 + 1, b = j - j0 + 1;
+        const uint32_t u0 = ou(i, j), v0 = ov(i, j), v1 = v0 + tc.pitch;
+        const double u_l = ld_off(bu, u0), u_r = ld_off(bu, u0 + 8), v_t = ld_off(bv, v0), v_b = ld_off(bv, v1);
+        const double x_l = ld_off(du, u0), x_r = ld_off(du, u0 + 8), y_t = ld_off(dv, v0), y_b = ld_off(dv, v1);
+        const double F_l = j > 0 ? K.hdx : 0.0, F_r = j + 1 < nx ? K.hdx : 0.0, F_t = i > 0 ? K.hdx : 0.0,
+                     F_b = i + 1 < ny ? K.hdx : 0.0;
+        const double H = S.H[a][b], H_l = S.H[a][b - 1], H_r = S.H[a][b + 1], H_t = S.H[a - 1][b], H_b = S.H[a + 1][b];
+        const double s_l = H_l + H, s_r = H + H_r, s_t = H_t + H, s_b = H + H_b;
+        const double m_l = u_l - fabs(u_l), q_r = u_r + fabs(u_r), q_t = v_t + fabs(v_t), m_b = v_b - fabs(v_b);
+        const double h = S.dH[a][b], h_l = S.dH[a][b - 1], h_r = S.dH[a][b + 1], h_t = S.dH[a - 1][b], h_b = S.dH[a + 1][b];
+        if (!VJP) {   // mass row (residuals.cu:343-375)
+            double d = div_refined(h, K.dt, K.rdt);
+            d += S.cd[a - 1][b - 1] * h;
+            d -= ((fma(-copysign(1.0, u_l), H - H_l, s_l) * x_l + (u_l + fabs(u_l)) * h_l) + m_l * h) * F_l;
+            d += ((fma(-copysign(1.0, u_r), H_r - H, s_r) * x_r + q_r * h) + (u_r - fabs(u_r)) * h_r) * F_r;
+            d += ((fma(-copysign(1.0, v_t), H_t - H, s_t) * y_t + (v_t - fabs(v_t)) * h_t) + q_t * h) * F_t;
+            d -= ((fma(-copysign(1.0, v_b), H - H_b, s_b) * y_b + m_b * h) + (v_b + fabs(v_b)) * h_b) * F_b;
+            const double m = ld_off(bmask, v0);
+            return (1.0 - m) * d + m * h;
+        }
+        // VJP: every row's derivative with respect to H(i, j).  Own mass row (residuals.cu:648-690)
+        double acc = div_refined(h, K.dt, K.rdt);
+        acc += h * S.cd[a - 1][b - 1];
+        acc -= (h * m_l) * F_l;
+        acc += (h * q_r) * F_r;
+        acc += (h * q_t) * F_t;
+        acc -= (h * m_b) * F_b;
+        acc += ld_off(dH, v0) * ld_off(bmask, v0);
+        // neighbours' mass rows through the shared faces
+        acc += (h_l * m_l) * F_l;
+        acc -= (h_r * q_r) * F_r;
+        acc -= (h_t * q_t) * F_t;
+        acc += (h_b * m_b) * F_b;
+        // momentum rows through eta*H of this cell: normal stresses
+        const double e2 = S.eh[a][b];
+        {
+            const double du_ = u_r - u_l, dv_ = v_t - v_b;
+            const double ex = fma(du_, K.dxi2, dv_ * K.dxi), ey = fma(du_, K.dxi, dv_ * K.dxi2);
+            acc += ((x_l * ex) * e2) * K.dxi;
+            acc -= ((x_r * ex) * e2) * K.dxi;
+            acc -= ((y_t * ey) * e2) * K.dxi;
+            acc += ((y_b * ey) * e2) * K.dxi;
+        }
+        // shear stresses of the four corner vertices
+        {
+            const uint32_t ut = i > 0 ? u0 - tu.pitch : u0, ub = i < ny - 1 ? u0 + tu.pitch : u0, cl = j > 0 ? 8u : 0u,
+                           cr = j < nx - 1 ? 8u : 0u;
+            const double V_tl = i > 0 && j > 0 ? K.dxi : 0.0, V_tr = i > 0 && j < nx - 1 ? K.dxi : 0.0,
+                         V_bl = i < ny - 1 && j > 0 ? K.dxi : 0.0, V_br = i < ny - 1 && j < nx - 1 ? K.dxi : 0.0;
+            double e = fma(ld_off(bu, ut) - u_l, V_tl, (v_t - ld_off(bv, v0 - cl)) * V_tl);
+            double w = ((x_l - ld_off(du, ut)) - y_t) + ld_off(dv, v0 - cl);
+            acc += ((w * e) * e2) * K.edx;
+            e = fma(ld_off(bu, ut + 8) - u_r, V_tr, (ld_off(bv, v0 + cr) - v_t) * V_tr);
+            w = ((x_r - ld_off(du, ut + 8)) - ld_off(dv, v0 + cr)) + y_t;
+            acc += ((w * e) * e2) * K.edx;
+            e = fma(u_l - ld_off(bu, ub), V_bl, (v_b - ld_off(bv, v1 - cl)) * V_bl);
+            w = ((ld_off(du, ub) - x_l) - y_b) + ld_off(dv, v1 - cl);
+            acc += ((w * e) * e2) * K.edx;
+            e = fma(u_r - ld_off(bu, ub + 8), V_br, (ld_off(bv, v1 + cr) - v_b) * V_br);
+            w = ((ld_off(du, ub + 8) - x_r) - ld_off(dv, v1 + cr)) + y_b;
+            acc += ((w * e) * e2) * K.edx;
+        }
+        // basal drag (grounding-line derivatives) and driving stress on the four faces
+        const double Sc = S.S[a][b], sl = S.sl[a][b], db = -0.5 * S.db[a][b];
+        if (p.gl_derivatives) acc += x_l * (db * u_l);
+        acc -= x_l * fma(s_l * sl, F_l, (Sc - S.S[a][b - 1]) * F_l);
+        if (p.gl_derivatives) acc += x_r * (db * u_r);
+        acc -= x_r * fma(-(s_r * sl), F_r, (S.S[a][b + 1] - Sc) * F_r);
+        if (p.gl_derivatives) acc += y_t * (db * v_t);
+        acc -= y_t * fma(-(s_t * sl), F_t, (S.S[a - 1][b] - Sc) * F_t);
+        if (p.gl_derivatives) acc += y_b * (db * v_b);
+        acc -= y_b * fma(s_b * sl, F_b, (Sc - S.S[a + 1][b]) * F_b);
+        return acc;
+    }
+};
+
+// VJP: out = base - l when base != NULL (the adjoint residual f_adj - J^T lambda)
+template <int TX, int TY, bool VJP>
+__device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p, double *__restrict__ out,
+                                             const double *__restrict__ base, const double *__restrict__ U,
+                                             const double *__restrict__ D, const double *__restrict__ bed,
+                                             const double *__restrict__ B, const double *__restrict__ beta,
+                                             const double *__restrict__ mask, int bx, int by, LinLDS0<TX, TY> &S)
+{
+    const LinTile<TX, TY, VJP, false> T(S, g, p, U, D, bed, B, beta, mask, bx, by);
+    T.stage();
+    const int ny = g.ny, nx = g.nx, i = T.i0 + threadIdx.y, j = T.j0 + threadIdx.x;
+    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+    if (i > ny || j > nx) return;
+    auto emit = [&](size_t k, double val) { out[k] = (VJP && base) ? base[k] - val : val; };
+    auto urow = [&](int i, int j) { emit((size_t)i * (nx + 1) + j, T.u_row(i, j)); };
+    auto vrow = [&](int i, int j) { emit(nu + (size_t)i * nx + j, T.v_row(i, j)); };
     if (i < ny) urow(i, j);
     if (j < nx) vrow(i, j);
-    if (j == nx - 1 && j0 + TX == nx && i < ny) urow(i, nx);   // u face at j = nx
-    if (i == ny - 1 && i0 + TY == ny && j < nx) vrow(ny, j);   // v face at i = ny
+    if (j == nx - 1 && T.j0 + TX == nx && i < ny) urow(i, nx);   // u face at j = nx
+    if (i == ny - 1 && T.i0 + TY == ny && j < nx) vrow(ny, j);   // v face at i = ny
+    if (i < ny && j < nx) emit(nu + nv + (size_t)i * nx + j, T.h_row(i, j));
+}
+
+// ---------------------------------------------------------------------------
+// One colour of the adjoint smoother in one pass (glide/grid.py:319-330,
+// glide/cuda/vanka.cu:441-840): r = f_adj - J^T lam, then every cell of the
+// colour solves its transposed block against r and updates its five dofs.  A
+// pass of its own for r and another for the solve cost two launches, two
+// stagings and the trip of r through memory, each of them more than the
+// arithmetic on the levels that fit the chip at once.
+//
+// The tiles read their neighbours' lam, so the updated lam goes to another
+// array, every dof written once: by its cell of the colour (the cells of one
+// colour own disjoint dofs), the thickness of the other cells and the domain
+// edge faces of cells of the other colour by those.  The cells of the colour
+// take the first half of the threads, so that whole waves solve.
+// ---------------------------------------------------------------------------
+template <int TX, int TY>
+__device__ __forceinline__ void adjoint_tile(const GlideGeom &g, const Params &p, double *__restrict__ lam_out,
+                                             double *__restrict__ r, const double *__restrict__ f_adj,
+                                             const double *__restrict__ U, const double *__restrict__ lam,
+                                             const double *__restrict__ bed, const double *__restrict__ B,
+                                             const double *__restrict__ beta, const double *__restrict__ mask, int color,
+                                             double omega, int bx, int by, AdjLDS<TX, TY> &S)
+{
+    const LinTile<TX, TY, true, true> T(S, g, p, U, lam, bed, B, beta, mask, bx, by);
+    T.stage();
+    const int ny = g.ny, nx = g.nx;
+    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+    const int tid = threadIdx.y * TX + threadIdx.x, half = tid >= TX * TY / 2, q = tid - half * (TX * TY / 2);
+    const int a = q / (TX / 2) + 1, i = T.i0 + a - 1, b = 2 * (q % (TX / 2)) + 1 + ((color + i + half) & 1), j = T.j0 + b - 1;
     if (i >= ny || j >= nx) return;
-    // 3c. cell (i, j)
-    const int a = i - i0 + 1, b = j - j0 + 1;
-    const size_t kc = (size_t)i * nx + j;
-    const uint32_t u0 = ou(i, j), v0 = ov(i, j), v1 = v0 + tc.pitch;
-    const double u_l = ld_off(bu, u0), u_r = ld_off(bu, u0 + 8), v_t = ld_off(bv, v0), v_b = ld_off(bv, v1);
-    const double x_l = ld_off(du, u0), x_r = ld_off(du, u0 + 8), y_t = ld_off(dv, v0), y_b = ld_off(dv, v1);
-    const double F_l = j > 0 ? K.hdx : 0.0, F_r = j + 1 < nx ? K.hdx : 0.0, F_t = i > 0 ? K.hdx : 0.0,
-                 F_b = i + 1 < ny ? K.hdx : 0.0;
-    const double H = S.H[a][b], H_l = S.H[a][b - 1], H_r = S.H[a][b + 1], H_t = S.H[a - 1][b], H_b = S.H[a + 1][b];
-    const double s_l = H_l + H, s_r = H + H_r, s_t = H_t + H, s_b = H + H_b;
-    const double m_l = u_l - fabs(u_l), q_r = u_r + fabs(u_r), q_t = v_t + fabs(v_t), m_b = v_b - fabs(v_b);
-    const double h = S.dH[a][b], h_l = S.dH[a][b - 1], h_r = S.dH[a][b + 1], h_t = S.dH[a - 1][b], h_b = S.dH[a + 1][b];
-    if (!VJP) {   // mass row (residuals.cu:343-375)
-        double d = div_refined(h, K.dt, K.rdt);
-        d += S.cd[a - 1][b - 1] * h;
-        d -= ((fma(-copysign(1.0, u_l), H - H_l, s_l) * x_l + (u_l + fabs(u_l)) * h_l) + m_l * h) * F_l;
-        d += ((fma(-copysign(1.0, u_r), H_r - H, s_r) * x_r + q_r * h) + (u_r - fabs(u_r)) * h_r) * F_r;
-        d += ((fma(-copysign(1.0, v_t), H_t - H, s_t) * y_t + (v_t - fabs(v_t)) * h_t) + q_t * h) * F_t;
-        d -= ((fma(-copysign(1.0, v_b), H - H_b, s_b) * y_b + m_b * h) + (v_b + fabs(v_b)) * h_b) * F_b;
-        const double m = mask[kc];
-        out[nu + nv + kc] = (1.0 - m) * d + m * h;
+    const size_t ku = (size_t)i * (nx + 1) + j, kv0 = nu + (size_t)i * nx + j, kv1 = kv0 + nx, kh = kv0 + nv;
+    if (half) {
+        r[kh] = f_adj[kh] - T.h_row(i, j);
+        lam_out[kh] = lam[kh];
+        auto edge = [&](size_t k, double row) {
+            r[k] = f_adj[k] - row;
+            lam_out[k] = lam[k];
+        };
+        if (j == 0) edge(ku, T.u_row(i, 0));
+        if (j == nx - 1) edge(ku + 1, T.u_row(i, nx));
+        if (i == 0) edge(kv0, T.v_row(0, j));
+        if (i == ny - 1) edge(kv1, T.v_row(ny, j));
         return;
     }
-    // VJP: every row's derivative with respect to H(i, j).  Own mass row (residuals.cu:648-690)
-    double acc = div_refined(h, K.dt, K.rdt);
-    acc += h * S.cd[a - 1][b - 1];
-    acc -= (h * m_l) * F_l;
-    acc += (h * q_r) * F_r;
-    acc += (h * q_t) * F_t;
-    acc -= (h * m_b) * F_b;
-    acc += ld_off(dH, v0) * ld_off(bmask, v0);
-    // neighbours' mass rows through the shared faces
-    acc += (h_l * m_l) * F_l;
-    acc -= (h_r * q_r) * F_r;
-    acc -= (h_t * q_t) * F_t;
-    acc += (h_b * m_b) * F_b;
-    // momentum rows through eta*H of this cell: normal stresses
-    const double e2 = S.eh[a][b];
-    {
-        const double du_ = u_r - u_l, dv_ = v_t - v_b;
-        const double ex = fma(du_, K.dxi2, dv_ * K.dxi), ey = fma(du_, K.dxi, dv_ * K.dxi2);
-        acc += ((x_l * ex) * e2) * K.dxi;
-        acc -= ((x_r * ex) * e2) * K.dxi;
-        acc -= ((y_t * ey) * e2) * K.dxi;
-        acc += ((y_b * ey) * e2) * K.dxi;
-    }
-    // shear stresses of the four corner vertices
-    {
-        const uint32_t ut = i > 0 ? u0 - tu.pitch : u0, ub = i < ny - 1 ? u0 + tu.pitch : u0, cl = j > 0 ? 8u : 0u,
-                       cr = j < nx - 1 ? 8u : 0u;
-        const double V_tl = i > 0 && j > 0 ? K.dxi : 0.0, V_tr = i > 0 && j < nx - 1 ? K.dxi : 0.0,
-                     V_bl = i < ny - 1 && j > 0 ? K.dxi : 0.0, V_br = i < ny - 1 && j < nx - 1 ? K.dxi : 0.0;
-        double e = fma(ld_off(bu, ut) - u_l, V_tl, (v_t - ld_off(bv, v0 - cl)) * V_tl);
-        double w = ((x_l - ld_off(du, ut)) - y_t) + ld_off(dv, v0 - cl);
-        acc += ((w * e) * e2) * K.edx;
-        e = fma(ld_off(bu, ut + 8) - u_r, V_tr, (ld_off(bv, v0 + cr) - v_t) * V_tr);
-        w = ((x_r - ld_off(du, ut + 8)) - ld_off(dv, v0 + cr)) + y_t;
-        acc += ((w * e) * e2) * K.edx;
-        e = fma(u_l - ld_off(bu, ub), V_bl, (v_b - ld_off(bv, v1 - cl)) * V_bl);
-        w = ((ld_off(du, ub) - x_l) - y_b) + ld_off(dv, v1 - cl);
-        acc += ((w * e) * e2) * K.edx;
-        e = fma(u_r - ld_off(bu, ub + 8), V_br, (ld_off(bv, v1 + cr) - v_b) * V_br);
-        w = ((ld_off(du, ub + 8) - x_r) - ld_off(dv, v1 + cr)) + y_b;
-        acc += ((w * e) * e2) * K.edx;
-    }
-    // basal drag (grounding-line derivatives) and driving stress on the four faces
-    const double Sc = S.S[a][b], sl = S.sl[a][b], db = -0.5 * S.db[a][b];
-    if (p.gl_derivatives) acc += x_l * (db * u_l);
-    acc -= x_l * fma(s_l * sl, F_l, (Sc - S.S[a][b - 1]) * F_l);
-    if (p.gl_derivatives) acc += x_r * (db * u_r);
-    acc -= x_r * fma(-(s_r * sl), F_r, (S.S[a][b + 1] - Sc) * F_r);
-    if (p.gl_derivatives) acc += y_t * (db * v_t);
-    acc -= y_t * fma(-(s_t * sl), F_t, (S.S[a - 1][b] - Sc) * F_t);
-    if (p.gl_derivatives) acc += y_b * (db * v_b);
-    acc -= y_b * fma(s_b * sl, F_b, (Sc - S.S[a + 1][b]) * F_b);
-    emit(nu + nv + kc, acc);
+    double rhs[5], d[5];
+    rhs[0] = f_adj[ku] - T.u_row(i, j);
+    rhs[1] = f_adj[ku + 1] - T.u_row(i, j + 1);
+    rhs[2] = f_adj[kv0] - T.v_row(i, j);
+    rhs[3] = f_adj[kv1] - T.v_row(i + 1, j);
+    rhs[4] = f_adj[kh] - T.h_row(i, j);
+    r[ku] = rhs[0];
+    r[ku + 1] = rhs[1];
+    r[kv0] = rhs[2];
+    r[kv1] = rhs[3];
+    r[kh] = rhs[4];
+    const char *bu = T.bu, *bv = T.bv;
+    const uint32_t u0 = T.ou(i, j), v0 = T.ov(i, j), v1 = v0 + T.tc.pitch;
+    const uint32_t ut = T.ou(i - 1, j), ub = T.ou(i + 1, j);
+    NewtonX x;
+    NewtonCell C{};
+    x.u_l = ld_off(bu, u0);
+    x.u_r = ld_off(bu, u0 + 8);
+    x.v_t = ld_off(bv, v0);
+    x.v_b = ld_off(bv, v1);
+    x.H = S.H[a][b];
+    C.u_tl = ld_off(bu, ut);
+    C.u_tr = ld_off(bu, ut + 8);
+    C.u_bl = ld_off(bu, ub);
+    C.u_br = ld_off(bu, ub + 8);
+    C.v_lt = ld_off(bv, T.ov(i, j - 1));
+    C.v_lb = ld_off(bv, T.ov(i + 1, j - 1));
+    C.v_rt = ld_off(bv, T.ov(i, j + 1));
+    C.v_rb = ld_off(bv, T.ov(i + 1, j + 1));
+    C.e2 = S.s_e2[a][b];
+    C.n_l = S.s_n[a][b - 1];
+    C.n_r = S.s_n[a][b + 1];
+    C.n_t = S.s_n[a - 1][b];
+    C.n_b = S.s_n[a + 1][b];
+    C.p_tl = (S.s_n[a - 1][b - 1] + C.n_t) + C.n_l;
+    C.p_tr = C.n_t + S.s_n[a - 1][b + 1];
+    C.n_bl = S.s_n[a + 1][b - 1];
+    C.n_br = S.s_n[a + 1][b + 1];
+    C.H_l = S.H[a][b - 1];
+    C.H_r = S.H[a][b + 1];
+    C.H_t = S.H[a - 1][b];
+    C.H_b = S.H[a + 1][b];
+    C.S_l = S.S[a][b - 1];
+    C.S_r = S.S[a][b + 1];
+    C.S_t = S.S[a - 1][b];
+    C.S_b = S.S[a + 1][b];
+    C.be_l = S.be[a][b - 1];
+    C.be_r = S.be[a][b + 1];
+    C.be_t = S.be[a - 1][b];
+    C.be_b = S.be[a + 1][b];
+    newton_edges<false>(C, T.K, i, j, ny, nx);
+    const double cd = S.cd[a - 1][b - 1];
+    const NewtonCentre M{S.be[a][b], S.S[a][b], S.sl[a][b], 0.0, T.K.idt + cd, S.db[a][b]};
+    const bool masked = mask[(size_t)i * nx + j] > 0.5;
+    if (p.gl_derivatives)
+        newton_adjoint<true>(C, T.K, M, x, masked, rhs, d);
+    else
+        newton_adjoint<false>(C, T.K, M, x, masked, rhs, d);
+    lam_out[ku] = lam[ku] + 0.5 * omega * d[0];
+    lam_out[ku + 1] = lam[ku + 1] + 0.5 * omega * d[1];
+    lam_out[kv0] = lam[kv0] + 0.5 * omega * d[2];
+    lam_out[kv1] = lam[kv1] + 0.5 * omega * d[3];
+    lam_out[kh] = lam[kh] + omega * d[4];
 }
 
 }  // namespace glide

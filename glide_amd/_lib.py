@@ -109,6 +109,8 @@ SIGNATURES = {
     "glide_batch_time_restriction": (c_int, [c_void_p, c_int, c_int, POINTER(c_double), POINTER(c_double), c_void_p]),
     "glide_unet_conv3x3": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p,
                                    c_int, c_void_p, c_void_p]),
+    "glide_unet_conv3x3_up_pool": (c_int, [c_void_p, c_int, c_int, c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int,
+                                           c_void_p, c_int, c_void_p, c_void_p, c_void_p]),
     "glide_unet_conv3x3_dgrad": (c_int, [c_void_p, c_int, c_int, c_int, c_int, c_void_p, c_int, c_void_p, c_int,
                                          c_int, c_void_p, c_int, c_void_p]),
     "glide_unet_wgrad_chunks": (ctypes.c_long, [c_int, c_int, c_int]),

@@ -110,22 +110,31 @@ __device__ __forceinline__ uint32_t f2bf_num(float f)
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
-template <int NW, int NCH, int MODE>
-__global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ xa, int CA,
+// 16-byte pieces a thread stages per round: all of them where that is at most 12 (18 for 6 chunks) loads in flight
+constexpr int conv_round(int ne, int nch)
+{
+    const int most = (nch > 4 ? 18 : 12) / nch, rounds = (ne + most - 1) / most;
+    return (ne + rounds - 1) / rounds;
+}
+
+template <int NW, int NG, int NCH, int MODE>
+__global__ __launch_bounds__(64 * NW * NG) void k_conv3x3(const bf16_t *__restrict__ xa, int CA, int up,
                                                      const bf16_t *__restrict__ xb, int H, int W, int tiles_x,
                                                      int tiles, const bf16_t *__restrict__ Wt, int Cout,
                                                      const float *__restrict__ bias, int relu,
                                                      const bf16_t *__restrict__ ya, bf16_t *__restrict__ out,
+                                                     bf16_t *__restrict__ pool,
                                                      float *__restrict__ ga, int SA, int acc_a,
                                                      float *__restrict__ gb, int acc_b)
 {
     constexpr int PW = CV_W + 2, NPX = (2 * NW + 2) * PW, Cin = 32 * NCH;
     __shared__ bf16_t sm[NCH * NPX * CV_LD];   // [chunk][pixel][CV_LD]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int NT = 64 * NW * NG;
+    const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % NW;
     const int r16 = lane & 15, kq = lane >> 4;   // fragment row / k-quarter
     const int n = blockIdx.x / tiles, tl = blockIdx.x - n * tiles;
     const int y0 = (tl / tiles_x) * 2 * NW, x0 = (tl % tiles_x) * CV_W;
-    const int co0 = blockIdx.y * 32;
+    const int co0 = (blockIdx.y * NG + (tid >> 6) / NW) * 32;
     const long img = (long)n * H * W;
 
     // weight fragments of step (t, c): row m of fragment j is channel co0 + 8 (m / 4) + 4 j + m % 4
@@ -136,31 +145,34 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
         B[0].raw = *(const uint4 *)(b + wlane);
         B[1].raw = *(const uint4 *)(b + 8 * Cin + wlane);
     };
-    Frag B[3][2];
+    constexpr int D = NCH == 1 ? 3 : NCH == 3 ? 9 : 6;   // steps ahead, a divisor of the 3 NCH steps of a row of taps
+    Frag B[D][2];
 #pragma unroll
-    for (int s = 0; s < 3; s++) wload(s / NCH, s % NCH, B[s]);
+    for (int s = 0; s < D; s++) wload(s / NCH, s % NCH, B[s]);
 
     // stage the input: 16-byte pieces, 4 per pixel and chunk
-    constexpr int NE = (NPX * 4 + 64 * NW - 1) / (64 * NW), NB = NCH > 2 ? 2 : 4;   // pieces per thread, in flight x NCH
+    constexpr int NE = (NPX * 4 + NT - 1) / NT, NB = conv_round(NE, NCH);   // pieces per thread, in flight x NCH
     const int CB = Cin - CA, ncha = CA / 32;
 #pragma unroll
     for (int e0 = 0; e0 < NE; e0 += NB) {
         uint4 v[NB][NCH];
 #pragma unroll
         for (int k = 0; k < NB; k++) {
-            const int e = tid + 64 * NW * (e0 + k), px = e >> 2, q = e & 3;
+            const int e = tid + NT * (e0 + k), px = e >> 2, q = e & 3;
             const int ry = px / PW, rx = px - ry * PW;
             const int y = y0 - 1 + ry, x = x0 - 1 + rx;
             const bool ok = e < NPX * 4 && y >= 0 && y < H && x >= 0 && x < W;
             const long p = img + (long)y * W + x;
-            const bf16_t *a = xa + p * CA + 8 * q, *b = xb + p * CB + 8 * q;
+            // xa at half the resolution: its pixel under this one
+            const long pa = MODE == 0 && up ? ((long)n * (H / 2) + (y >> 1)) * (W / 2) + (x >> 1) : p;
+            const bf16_t *a = xa + pa * CA + 8 * q, *b = xb + p * CB + 8 * q;
 #pragma unroll
             for (int c = 0; c < NCH; c++)
                 v[k][c] = ok ? *(const uint4 *)(c < ncha ? a + 32 * c : b + 32 * (c - ncha)) : uint4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
         for (int k = 0; k < NB; k++) {
-            const int e = tid + 64 * NW * (e0 + k);
+            const int e = tid + NT * (e0 + k);
             if (e < NPX * 4) {
 #pragma unroll
                 for (int c = 0; c < NCH; c++) *(uint4 *)(sm + (c * NPX + (e >> 2)) * CV_LD + 8 * (e & 3)) = v[k][c];
@@ -188,10 +200,10 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
             for (int j = 0; j < 2; j++)
 #pragma unroll
                 for (int a = 0; a < 4; a++)
-                    acc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[s % 3][j].v, A[a].v, acc[a][j], 0, 0, 0);
-            const int q = s + 3;   // past the last step: the last tap again
+                    acc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[s % D][j].v, A[a].v, acc[a][j], 0, 0, 0);
+            const int q = s + D;   // past the last step: the last tap again
             const int t = 3 * dy + q / NCH;
-            wload(t < 9 ? t : 8, q % NCH, B[s % 3]);
+            wload(t < 9 ? t : 8, q % NCH, B[s % D]);
         }
         base += PW * CV_LD;
     }
@@ -203,9 +215,11 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
         const float4 b0 = *(const float4 *)(bias + co), b1 = *(const float4 *)(bias + co + 4);
         bs[0] = b0.x, bs[1] = b0.y, bs[2] = b0.z, bs[3] = b0.w, bs[4] = b1.x, bs[5] = b1.y, bs[6] = b1.z, bs[7] = b1.w;
     }
+    uint4 o4[4];
 #pragma unroll
     for (int a = 0; a < 4; a++) {
         const int y = y0 + 2 * wave + (a >> 1), x = x0 + 16 * (a & 1) + r16;
+        o4[a] = uint4{0u, 0u, 0u, 0u};
         if (y >= H || x >= W) continue;
         const long p = img + (long)y * W + x;
         if (MODE != 1) {
@@ -220,8 +234,8 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
                 else
                     h[i] = f2bf(bf2f(y8.h[i]) > 0.0f ? acc[a][i >> 2][i & 3] : 0.0f);
             }
-            *(uint4 *)(out + p * Cout + co) =
-                uint4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+            o4[a] = uint4{h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6] | h[7] << 16};
+            *(uint4 *)(out + p * Cout + co) = o4[a];
         } else {
             const bool first = co0 < SA;   // 32-channel groups lie in one of the outputs
             float4 *d = (float4 *)(first ? ga + p * SA + co : gb + p * (Cout - SA) + (co - SA));
@@ -236,6 +250,29 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
             d[1] = v1;
         }
     }
+    // 2x2 mean of the output as k_pool2 forms it: the lane's two rows and the next lane's (H and W even)
+    if (MODE == 0 && pool) {
+#pragma unroll
+        for (int a = 0; a < 2; a++) {
+            Bf8 q0, q1, q2, q3, o;
+            q0.raw = o4[a];
+            q2.raw = o4[a + 2];
+            auto next = [](uint4 v) {
+                return uint4{(uint32_t)__shfl_xor((int)v.x, 1), (uint32_t)__shfl_xor((int)v.y, 1),
+                             (uint32_t)__shfl_xor((int)v.z, 1), (uint32_t)__shfl_xor((int)v.w, 1)};
+            };
+            q1.raw = next(q0.raw);
+            q3.raw = next(q2.raw);
+            const int y = y0 + 2 * wave, x = x0 + 16 * a + r16;
+            if (y >= H || x >= W || (r16 & 1)) continue;
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                const float s = ((bf2f(q0.h[i]) + bf2f(q1.h[i])) + bf2f(q2.h[i])) + bf2f(q3.h[i]);
+                o.h[i] = f2bf(0.25f * s);
+            }
+            *(uint4 *)(pool + (((long)n * (H / 2) + y / 2) * (W / 2) + x / 2) * Cout + co) = o.raw;
+        }
+    }
 }
 
 // The same convolution reading every tap's pixels from the caches, for input
@@ -244,7 +281,8 @@ __global__ __launch_bounds__(64 * NW) void k_conv3x3(const bf16_t *__restrict__ 
 // channels.  Grid: x = pixel blocks of 256 (4
 // waves x 64), y = output-channel groups of 16 NJ.  The same sums, bit for bit.
 template <int NJ, int MODE>
-__global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict__ xa, int CA, const bf16_t *__restrict__ xb,
+__global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict__ xa, int CA, int up,
+                                                        const bf16_t *__restrict__ xb,
                                                         int CB, int N, int H, int W, const bf16_t *__restrict__ Wt, int Cout,
                                                         const float *__restrict__ bias, int relu, const bf16_t *__restrict__ ya,
                                                         bf16_t *__restrict__ out,
@@ -289,7 +327,8 @@ __global__ __launch_bounds__(256) void k_conv3x3_direct(const bf16_t *__restrict
         for (int a = 0; a < 4; a++) {
             const int y = py[a] + dy, x = px[a] + dx;
             const bool ok = pv[a] && y >= 0 && y < H && x >= 0 && x < W;
-            const long src = ok ? (((long)pn[a] * H + y) * W + x) : 0;
+            const int h = MODE == 0 && up && c0 < CA;   // xa at half the resolution
+            const long src = ok ? (((long)pn[a] * (H >> h) + (y >> h)) * (W >> h) + (x >> h)) : 0;
             A[a].raw = ok ? *(const uint4 *)(xs + src * cs + cc) : uint4{0u, 0u, 0u, 0u};
         }
 #pragma unroll
@@ -868,22 +907,27 @@ __global__ void k_head(const bf16_t *__restrict__ x, long P, int C, int NO, cons
 }
 // k_head reading 8 channels per 16-byte access (C % 8 == 0, aligned): the
 // same sums in the same order
-__global__ void k_head_v8(const bf16_t *__restrict__ x, long P, int C, int NO, const float *__restrict__ Wh,
+template <int NO>
+__global__ void k_head_v8(const bf16_t *__restrict__ x, long P, int C, const float *__restrict__ Wh,
                           const float *__restrict__ bh, float *__restrict__ out)
 {
     long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= P) return;
-    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    float s[NO];
+#pragma unroll
     for (int o = 0; o < NO; o++) s[o] = bh[o];
+#pragma unroll 4
     for (int c = 0; c < C; c += 8) {
         Bf8 q;
         q.raw = *(const uint4 *)(x + p * C + c);
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             const float v = bf2f(q.h[i]);
+#pragma unroll
             for (int o = 0; o < NO; o++) s[o] += Wh[o * C + c + i] * v;
         }
     }
+#pragma unroll
     for (int o = 0; o < NO; o++) out[NO * p + o] = s[o];
 }
 // dx[p][c] = sum_o dout[p][o] Wh[o][c]
@@ -1042,7 +1086,8 @@ __global__ void k_features(const double *__restrict__ H, const double *__restric
                            const double *__restrict__ B, int ny, int nx, double dx, bf16_t *__restrict__ x)
 {
     long k = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= (long)ny * nx) return;
+    const long n = (long)ny * nx, k0 = k;
+    k = k < n ? k : n - 1;
     const int i = (int)(k / nx), j = (int)(k % nx);
     const int jl = j > 0 ? j - 1 : j, jr = j < nx - 1 ? j + 1 : j;
     const int it = i > 0 ? i - 1 : i, ib = i < ny - 1 ? i + 1 : i;
@@ -1051,8 +1096,26 @@ __global__ void k_features(const double *__restrict__ H, const double *__restric
     float f[7] = {(float)(H[k] / 1000.0), (float)tanh((bed[k] + 0.917 * H[k]) / 200.0),
                   (float)(100.0 * sqrt(sx * sx + sy * sy)), (float)(log(beta[k]) + 2.0), (float)(B[k] / 24.0 - 1.0),
                   (float)(100.0 * sx), (float)(100.0 * sy)};
-    bf16_t *o = x + k * 32;
-    for (int c = 0; c < 32; c++) o[c] = c < 7 ? f2bf(f[c]) : (bf16_t)0;
+    uint32_t h[8] = {};
+#pragma unroll
+    for (int c = 0; c < 7; c++) h[c] = f2bf(f[c]);
+    const uint4 q = {h[0] | h[1] << 16, h[2] | h[3] << 16, h[4] | h[5] << 16, h[6]};
+    if ((uintptr_t)x & 15) {
+        if (k0 < n)
+            for (int c = 0; c < 32; c++) x[k * 32 + c] = (bf16_t)(c < 8 ? h[c & 7] : 0u);
+        return;
+    }
+    // four consecutive lanes store one cell's 64 bytes
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int s = 0; s < 4; s++) {
+        const int src = 16 * s + (lane >> 2);
+        uint4 v = {(uint32_t)__shfl((int)q.x, src), (uint32_t)__shfl((int)q.y, src), (uint32_t)__shfl((int)q.z, src),
+                   (uint32_t)__shfl((int)q.w, src)};
+        if (lane & 3) v = uint4{0u, 0u, 0u, 0u};
+        const long c = k0 - lane + src;
+        if (c < n) *(uint4 *)(x + c * 32 + 8 * (lane & 3)) = v;
+    }
 }
 // targets (FP32, 3 per cell): cell-centred (u_l + u_r)/2 and (v_t + v_b)/2
 // times scale, and the thickness change (H - H_prev) times hscale
@@ -1133,9 +1196,17 @@ int conv_nj(long P, int C)
 // LDS bytes of a workgroup of nw waves
 constexpr size_t conv_lds(int nw, int nch) { return (size_t)nch * (2 * nw + 2) * (CV_W + 2) * CV_LD * sizeof(bf16_t); }
 
+void pool2(const bf16_t *x, int N, int H, int W, int C, bf16_t *y, hipStream_t st)
+{
+    const long n = (long)N * (H / 2) * (W / 2) * C;
+    if (vec8(C, x, y))
+        hipLaunchKernelGGL(k_pool2_v8, dim3(nblk(n / 8)), dim3(256), 0, st, x, N, H, W, C, y);
+    else
+        hipLaunchKernelGGL(k_pool2, dim3(nblk(n)), dim3(256), 0, st, x, N, H, W, C, y);
+}
 struct ConvArgs {
     const bf16_t *xa;
-    int CA;
+    int CA, up;   // up: xa is at half the resolution
     const bf16_t *xb;
     int CB, N, H, W;
     const bf16_t *Wt;
@@ -1143,61 +1214,73 @@ struct ConvArgs {
     const float *bias;
     int relu;
     const bf16_t *ya;
-    bf16_t *out;
+    bf16_t *out, *pool;
     float *ga;
     int SA, acc_a;
     float *gb;
     int acc_b;
 };
 
-template <int NW, int NCH, int MODE>
+template <int NW, int NG, int NCH, int MODE>
 void conv_launch(const ConvArgs &c, hipStream_t st)
 {
     const int tx = (c.W + CV_W - 1) / CV_W, tiles = tx * ((c.H + 2 * NW - 1) / (2 * NW));
-    hipLaunchKernelGGL((k_conv3x3<NW, NCH, MODE>), dim3((unsigned)((long)tiles * c.N), c.Cout / 32), dim3(64 * NW), 0,
-                       st, c.xa, c.CA, c.xb, c.H, c.W, tx, tiles, c.Wt, c.Cout, c.bias, c.relu, c.ya, c.out, c.ga, c.SA,
-                       c.acc_a, c.gb, c.acc_b);
+    hipLaunchKernelGGL((k_conv3x3<NW, NG, NCH, MODE>), dim3((unsigned)((long)tiles * c.N), c.Cout / (32 * NG)),
+                       dim3(64 * NW * NG), 0, st, c.xa, c.CA, c.up, c.xb, c.H, c.W, tx, tiles, c.Wt, c.Cout, c.bias,
+                       c.relu, c.ya, c.out, c.pool, c.ga, c.SA, c.acc_a, c.gb, c.acc_b);
 }
-// Waves per workgroup (tile rows / 2): the tallest tile reads the fewest halo
-// rows, so 4 where that still gives a workgroup per CU and the input fits 64
-// KB of LDS, else 2, else 1.
-template <int NCH, int MODE>
+// Row pairs per workgroup (tile rows / 2): the tallest tile reads the fewest
+// halo rows, so 4 where that still gives a workgroup per CU and the input fits
+// 64 KB of LDS, else 2, else 1.
+template <int NG, int NCH, int MODE>
 void conv_staged(const ConvArgs &c, hipStream_t st)
 {
     auto wgs = [&](int nw) {
-        return (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * nw - 1) / (2 * nw)) * c.N * (c.Cout / 32);
+        return (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * nw - 1) / (2 * nw)) * c.N * (c.Cout / (32 * NG));
     };
     if constexpr (conv_lds(4, NCH) <= 64 * 1024)
-        if (wgs(4) >= 256) return conv_launch<4, NCH, MODE>(c, st);
+        if (wgs(4) >= 256) return conv_launch<4, NG, NCH, MODE>(c, st);
     if constexpr (conv_lds(2, NCH) <= 64 * 1024)
-        if (wgs(2) >= 256) return conv_launch<2, NCH, MODE>(c, st);
-    conv_launch<1, NCH, MODE>(c, st);
+        if (wgs(2) >= 256) return conv_launch<2, NG, NCH, MODE>(c, st);
+    conv_launch<1, NG, NCH, MODE>(c, st);
+}
+// The workgroup's waves share the staged input among up to 3 groups of 32 output channels.
+template <int NCH, int MODE>
+void conv_groups(const ConvArgs &c, hipStream_t st)
+{
+    const int ng = c.Cout / 32;
+    if (ng % 3 == 0) return conv_staged<3, NCH, MODE>(c, st);
+    if (ng % 2 == 0) return conv_staged<2, NCH, MODE>(c, st);
+    conv_staged<1, NCH, MODE>(c, st);
 }
 template <int NJ, int MODE>
 void conv_direct(const ConvArgs &c, hipStream_t st)
 {
     hipLaunchKernelGGL((k_conv3x3_direct<NJ, MODE>), dim3(nblk((long)c.N * c.H * c.W), c.Cout / (16 * NJ)), dim3(256), 0,
-                       st, c.xa, c.CA, c.xb, c.CB, c.N, c.H, c.W, c.Wt, c.Cout, c.bias, c.relu, c.ya, c.out, c.ga, c.SA,
+                       st, c.xa, c.CA, c.up, c.xb, c.CB, c.N, c.H, c.W, c.Wt, c.Cout, c.bias, c.relu, c.ya, c.out, c.ga, c.SA,
                        c.acc_a, c.gb, c.acc_b);
 }
 // The channel counts of the network's layers have a staged instance.  It reads
 // the bias and stores in 16-byte pieces, which the direct kernel does not: a
 // tensor off that alignment takes the direct kernel.
 template <int MODE>
-void conv(const ConvArgs &c, hipStream_t st)
+void conv(ConvArgs c, hipStream_t st)
 {
-    const uintptr_t al = (uintptr_t)c.bias | (uintptr_t)c.ya | (uintptr_t)c.out | (uintptr_t)c.ga | (uintptr_t)c.gb;
-    const int nch = (al & 15) ? 0 : (c.CA + c.CB) / 32;
-    if (nch == 1) return conv_staged<1, MODE>(c, st);
-    if (nch == 2) return conv_staged<2, MODE>(c, st);
-    if (nch == 3) return conv_staged<3, MODE>(c, st);
-    if (nch == 4) return conv_staged<4, MODE>(c, st);
-    if (nch == 6) return conv_staged<6, MODE>(c, st);
+    const uintptr_t al = (uintptr_t)c.bias | (uintptr_t)c.ya | (uintptr_t)c.out | (uintptr_t)c.pool | (uintptr_t)c.ga |
+                         (uintptr_t)c.gb;
+    switch ((al & 15) ? 0 : (c.CA + c.CB) / 32) {
+    case 1: return conv_groups<1, MODE>(c, st);
+    case 2: return conv_groups<2, MODE>(c, st);
+    case 3: return conv_groups<3, MODE>(c, st);
+    case 4: return conv_groups<4, MODE>(c, st);
+    case 6: return conv_groups<6, MODE>(c, st);
+    }
     switch (conv_nj((long)c.N * c.H * c.W, c.Cout)) {
     case 4: conv_direct<4, MODE>(c, st); break;
     case 2: conv_direct<2, MODE>(c, st); break;
     default: conv_direct<1, MODE>(c, st);
     }
+    if (c.pool) pool2(c.out, c.N, c.H, c.W, c.Cout, c.pool, st);
 }
 }  // namespace
 
@@ -1209,8 +1292,21 @@ int glide_unet_conv3x3(const uint16_t *xa, int CA, const uint16_t *xb, int CB, i
     if (!xa || !weights || !bias || !out || (CB > 0 && !xb)) return ufail(GLIDE_E_NULL, "conv3x3: NULL argument");
     if (bad_ch(CA) || CA == 0 || bad_ch(CB) || bad_ch(Cout) || Cout == 0 || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3: channels must be positive multiples of 32, sizes positive");
-    conv<0>(ConvArgs{xa, CA, xb, CB, N, H, W, weights, Cout, bias, relu, nullptr, out, nullptr, 0, 0, nullptr,
+    conv<0>(ConvArgs{xa, CA, 0, xb, CB, N, H, W, weights, Cout, bias, relu, nullptr, out, nullptr, nullptr, 0, 0, nullptr,
                      0}, SS(stream));
+    return ucheck("conv3x3");
+}
+
+int glide_unet_conv3x3_up_pool(const uint16_t *xa, int CA, int up_a, const uint16_t *xb, int CB, int N, int H, int W,
+                               const uint16_t *weights, int Cout, const float *bias, int relu, uint16_t *out,
+                               uint16_t *pooled, void *stream)
+{
+    if (!xa || !weights || !bias || !out || (CB > 0 && !xb)) return ufail(GLIDE_E_NULL, "conv3x3: NULL argument");
+    if (bad_ch(CA) || CA == 0 || bad_ch(CB) || bad_ch(Cout) || Cout == 0 || N < 1 || H < 1 || W < 1)
+        return ufail(GLIDE_E_SIZE, "conv3x3: channels must be positive multiples of 32, sizes positive");
+    if ((up_a || pooled) && (H % 2 || W % 2)) return ufail(GLIDE_E_SIZE, "conv3x3: even sizes required");
+    conv<0>(ConvArgs{xa, CA, up_a != 0, xb, CB, N, H, W, weights, Cout, bias, relu, nullptr, out, pooled, nullptr, 0, 0,
+                     nullptr, 0}, SS(stream));
     return ucheck("conv3x3");
 }
 
@@ -1221,7 +1317,7 @@ int glide_unet_conv3x3_dgrad(const uint16_t *dz, int Cout, int N, int H, int W, 
     if (bad_ch(Cout) || Cout == 0 || bad_ch(CA) || CA == 0 || bad_ch(CB) || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3_dgrad: channels must be positive multiples of 32, sizes positive");
     // the transposed convolution: CA + CB output channels
-    conv<1>(ConvArgs{dz, Cout, nullptr, 0, N, H, W, wflip, CA + CB, nullptr, 0, nullptr, nullptr, ga, CA, acc_a,
+    conv<1>(ConvArgs{dz, Cout, 0, nullptr, 0, N, H, W, wflip, CA + CB, nullptr, 0, nullptr, nullptr, nullptr, ga, CA, acc_a,
                      gb, acc_b},
             SS(stream));
     return ucheck("conv3x3_dgrad");
@@ -1234,7 +1330,7 @@ int glide_unet_conv3x3_dgrad_relu(const uint16_t *dz, int Cout, int N, int H, in
     if (dz == dzin) return ufail(GLIDE_E_ARG, "conv3x3_dgrad_relu: dz and dzin must be distinct");
     if (bad_ch(Cout) || Cout == 0 || bad_ch(Cin) || Cin == 0 || N < 1 || H < 1 || W < 1)
         return ufail(GLIDE_E_SIZE, "conv3x3_dgrad_relu: channels must be positive multiples of 32, sizes positive");
-    conv<2>(ConvArgs{dz, Cout, nullptr, 0, N, H, W, wflip, Cin, nullptr, 0, y, dzin, nullptr, 0, 0, nullptr, 0},
+    conv<2>(ConvArgs{dz, Cout, 0, nullptr, 0, N, H, W, wflip, Cin, nullptr, 0, y, dzin, nullptr, nullptr, 0, 0, nullptr, 0},
             SS(stream));
     return ucheck("conv3x3_dgrad_relu");
 }
@@ -1295,11 +1391,7 @@ int glide_unet_pool2(const uint16_t *x, int N, int H, int W, int C, uint16_t *y,
 {
     if (!x || !y) return ufail(GLIDE_E_NULL, "pool2: NULL argument");
     if (N < 1 || H < 2 || W < 2 || H % 2 || W % 2 || C < 1) return ufail(GLIDE_E_SIZE, "pool2: even sizes required");
-    const long n = (long)N * (H / 2) * (W / 2) * C;
-    if (vec8(C, x, y))
-        hipLaunchKernelGGL(k_pool2_v8, dim3(nblk(n / 8)), dim3(256), 0, SS(stream), x, N, H, W, C, y);
-    else
-        hipLaunchKernelGGL(k_pool2, dim3(nblk(n)), dim3(256), 0, SS(stream), x, N, H, W, C, y);
+    pool2(x, N, H, W, C, y, SS(stream));
     return ucheck("pool2");
 }
 
@@ -1356,10 +1448,18 @@ int glide_unet_head(const uint16_t *x, long P, int C, int NO, const float *wh, c
 {
     if (!x || !wh || !bh || !out) return ufail(GLIDE_E_NULL, "head: NULL argument");
     if (P < 1 || C < 1 || NO < 1 || NO > 4) return ufail(GLIDE_E_SIZE, "head: bad size (1 <= outputs <= 4)");
-    if (vec8(C, x, x))
-        hipLaunchKernelGGL(k_head_v8, dim3(nblk(P)), dim3(256), 0, SS(stream), x, P, C, NO, wh, bh, out);
+    const dim3 grid(nblk(P)), block(256);
+    hipStream_t st = SS(stream);
+    if (!vec8(C, x, x))
+        hipLaunchKernelGGL(k_head, grid, block, 0, st, x, P, C, NO, wh, bh, out);
+    else if (NO == 1)
+        hipLaunchKernelGGL(k_head_v8<1>, grid, block, 0, st, x, P, C, wh, bh, out);
+    else if (NO == 2)
+        hipLaunchKernelGGL(k_head_v8<2>, grid, block, 0, st, x, P, C, wh, bh, out);
+    else if (NO == 3)
+        hipLaunchKernelGGL(k_head_v8<3>, grid, block, 0, st, x, P, C, wh, bh, out);
     else
-        hipLaunchKernelGGL(k_head, dim3(nblk(P)), dim3(256), 0, SS(stream), x, P, C, NO, wh, bh, out);
+        hipLaunchKernelGGL(k_head_v8<4>, grid, block, 0, st, x, P, C, wh, bh, out);
     return ucheck("head");
 }
 

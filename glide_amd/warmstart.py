@@ -37,6 +37,7 @@ LAYERS = [
     ("d1a", ["u1", "e1"], 32), ("d1", ["d1a"], 32),
 ]
 POOLS = {"p1": "e1", "p2": "e2", "p3": "e3"}
+POOLED = {src: name for name, src in POOLS.items()}
 UPS = {"u3": "b", "u2": "d3", "u1": "d2"}
 IN_CH = 32
 HEAD_IN = "d1"
@@ -115,7 +116,7 @@ class UNet:
         dims = {lv: (H >> lv, W >> lv) for lv in range(4)}
         acts = {}
         for name in CH:
-            if name == "x0":
+            if name == "x0" or (name in UPS and not train):   # without training the upsampling is part of its convolution
                 continue
             h, w = dims[LEVEL[name]]
             acts[name] = torch.empty(N * h * w * CH[name], dtype=torch.int16, device=self.device)
@@ -155,19 +156,18 @@ class UNet:
         acts, dims, st = b["acts"], b["dims"], self._stream()
         acts["x0"] = x0
         for name, ins, co in LAYERS:
-            for i in ins:
-                if i in POOLS:
-                    src = POOLS[i]
-                    h, w = dims[LEVEL[src]]
-                    _lib.call("glide_unet_pool2", _p(acts[src]), N, h, w, CH[src], _p(acts[i]), st)
-                if i in UPS:
-                    src = UPS[i]
-                    h, w = dims[LEVEL[src]]
-                    _lib.call("glide_unet_up2", _p(acts[src]), N, h, w, CH[src], _p(acts[i]), st)
             h, w = dims[LEVEL[name]]
-            xa, xb = acts[ins[0]], (acts[ins[1]] if len(ins) > 1 else None)
-            _lib.call("glide_unet_conv3x3", _p(xa), CH[ins[0]], _p(xb), CH[ins[1]] if xb is not None else 0, N, h, w,
-                      _p(self.wb[name]), co, _p(self.params[name + ".b"]), 1, _p(acts[name]), st)
+            xa, xb = acts.get(ins[0]), (acts[ins[1]] if len(ins) > 1 else None)
+            up = 0
+            if ins[0] in UPS:
+                src = UPS[ins[0]]
+                if train:   # the weight gradient reads the upsampled tensor
+                    _lib.call("glide_unet_up2", _p(acts[src]), N, h // 2, w // 2, CH[src], _p(xa), st)
+                else:
+                    xa, up = acts[src], 1
+            _lib.call("glide_unet_conv3x3_up_pool", _p(xa), CH[ins[0]], up, _p(xb), CH[ins[1]] if xb is not None else 0, N,
+                      h, w, _p(self.wb[name]), co, _p(self.params[name + ".b"]), 1, _p(acts[name]),
+                      _p(acts[POOLED[name]]) if name in POOLED else None, st)
         _lib.call("glide_unet_head", _p(acts[HEAD_IN]), N * H * W, CH[HEAD_IN], N_OUT, _p(self.params["head.W"]),
                   _p(self.params["head.b"]), _p(b["pred"]), st)
         return b["pred"]

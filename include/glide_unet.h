@@ -31,6 +31,14 @@ int glide_unet_conv3x3(const uint16_t *xa, int CA, const uint16_t *xb, int CB, i
                        const uint16_t *weights, int Cout, const float *bias, int relu, uint16_t *out,
                        void *stream);
 
+/* glide_unet_conv3x3 with the network's resampling around it: up_a != 0 reads
+ * xa at half the resolution (N x H/2 x W/2, as if upsampled by glide_unet_up2
+ * first), pooled (if not NULL) receives the output's glide_unet_pool2.  H and W
+ * must be even where either is asked for. */
+int glide_unet_conv3x3_up_pool(const uint16_t *xa, int CA, int up_a, const uint16_t *xb, int CB, int N, int H, int W,
+                               const uint16_t *weights, int Cout, const float *bias, int relu, uint16_t *out,
+                               uint16_t *pooled, void *stream);
+
 /* Data gradient of glide_unet_conv3x3: from dz (BF16, Cout channels) and the
  * flipped weights of glide_unet_prep_weights, writes FP32 gradients of the
  * two inputs: ga (CA channels) and gb (CB channels); acc_* != 0 adds. */

@@ -85,8 +85,8 @@ union Bf8 {
 // channels: it stages the (2 NW + 2) x 34 input pixels of every channel (NCH
 // chunks of 32) in LDS once (zero outside the image), so the nine taps read
 // memory once, and a wave takes 2 rows (4 MFMA blocks of 16 pixels).  An LDS
-// pixel is 32 channels at a pitch of 80 bytes, which puts the 16-byte reads of
-// 8 consecutive pixels in different banks.  Weight fragments come from the
+// pixel is 32 channels in 64 bytes, its four 16-byte pieces swapped by its
+// column / 4, which puts the reads of 16 consecutive pixels in different banks.  Weight fragments come from the
 // caches, three steps ahead.  The weights are the MFMA's row operand, in an
 // order that leaves a lane with 8 consecutive output channels of its pixel:
 // one 16-byte store (two for FP32) instead of 8 of 2 bytes.  The K loop walks
@@ -100,7 +100,7 @@ union Bf8 {
 // (7 us at the rate of a large copy).
 // ---------------------------------------------------------------------------
 constexpr int CV_W = 32;      // tile columns
-constexpr int CV_LD = 40;     // LDS pitch of a pixel's 32 channels (bf16)
+constexpr int CV_LD = 32;     // LDS pitch of a pixel's 32 channels (bf16)
 
 // f2bf without the NaN case (a NaN becomes some other value)
 __device__ __forceinline__ uint32_t f2bf_num(float f)
@@ -117,8 +117,13 @@ constexpr int conv_round(int ne, int nch)
     return (ne + rounds - 1) / rounds;
 }
 
+constexpr size_t conv_lds(int nw, int nch) { return (size_t)nch * (2 * nw + 2) * (CV_W + 2) * CV_LD * sizeof(bf16_t); }
+constexpr size_t conv_wlds(int ng, int nch) { return (size_t)9 * nch * 32 * ng * CV_LD * sizeof(bf16_t); }
+// the weights go through LDS too where waves share them and a CU's 160 KB hold both
+constexpr bool conv_wl(int nw, int ng, int nch) { return nw == 4 && conv_lds(nw, nch) + conv_wlds(ng, nch) <= 160 * 1024; }
+
 template <int NW, int NG, int NCH, int MODE>
-__global__ __launch_bounds__(64 * NW * NG) void k_conv3x3(const bf16_t *__restrict__ xa, int CA, int up,
+__global__ __launch_bounds__(64 * NW * NG, NCH == 1 ? 5 : NCH == 6 ? 2 : NCH == 3 ? 3 : 4) void k_conv3x3(const bf16_t *__restrict__ xa, int CA, int up,
                                                      const bf16_t *__restrict__ xb, int H, int W, int tiles_x,
                                                      int tiles, const bf16_t *__restrict__ Wt, int Cout,
                                                      const float *__restrict__ bias, int relu,
@@ -128,7 +133,9 @@ __global__ __launch_bounds__(64 * NW * NG) void k_conv3x3(const bf16_t *__restri
                                                      float *__restrict__ gb, int acc_b)
 {
     constexpr int PW = CV_W + 2, NPX = (2 * NW + 2) * PW, Cin = 32 * NCH;
+    constexpr bool WL = conv_wl(NW, NG, NCH);
     __shared__ bf16_t sm[NCH * NPX * CV_LD];   // [chunk][pixel][CV_LD]
+    __shared__ bf16_t smw[WL ? 9 * NCH * 32 * NG * CV_LD : 1];   // [tap][chunk][output channel][CV_LD]
     constexpr int NT = 64 * NW * NG;
     const int tid = threadIdx.x, lane = tid & 63, wave = (tid >> 6) % NW;
     const int r16 = lane & 15, kq = lane >> 4;   // fragment row / k-quarter
@@ -147,8 +154,21 @@ __global__ __launch_bounds__(64 * NW * NG) void k_conv3x3(const bf16_t *__restri
     };
     constexpr int D = NCH == 1 ? 3 : NCH == 3 ? 9 : 6;   // steps ahead, a divisor of the 3 NCH steps of a row of taps
     Frag B[D][2];
+    if (!WL) {
 #pragma unroll
-    for (int s = 0; s < D; s++) wload(s / NCH, s % NCH, B[s]);
+        for (int s = 0; s < D; s++) wload(s / NCH, s % NCH, B[s]);
+    }
+    // staged weights: a tap's rows of this workgroup's channels are one block of memory
+    constexpr int NWP = 9 * NCH * 128 * NG, NWE = WL ? (NWP + NT - 1) / NT : 1;
+    uint4 wv[NWE];
+    if (WL) {
+#pragma unroll
+        for (int k = 0; k < NWE; k++) {
+            const int e = tid + NT * k, t = e / (NCH * 128 * NG), r = e - t * (NCH * 128 * NG);
+            wv[k] = e < NWP ? *(const uint4 *)((const char *)Wt + t * tap + (long)blockIdx.y * (NCH * 2048 * NG) + 16 * r)
+                            : uint4{0u, 0u, 0u, 0u};
+        }
+    }
 
     // stage the input: 16-byte pieces, 4 per pixel and chunk
     constexpr int NE = (NPX * 4 + NT - 1) / NT, NB = conv_round(NE, NCH);   // pieces per thread, in flight x NCH
@@ -174,9 +194,18 @@ __global__ __launch_bounds__(64 * NW * NG) void k_conv3x3(const bf16_t *__restri
         for (int k = 0; k < NB; k++) {
             const int e = tid + NT * (e0 + k);
             if (e < NPX * 4) {
+                const int px = e >> 2, lds = px * CV_LD + 8 * ((e & 3) ^ ((px % PW) >> 2 & 3));
 #pragma unroll
-                for (int c = 0; c < NCH; c++) *(uint4 *)(sm + (c * NPX + (e >> 2)) * CV_LD + 8 * (e & 3)) = v[k][c];
+                for (int c = 0; c < NCH; c++) *(uint4 *)(sm + c * NPX * CV_LD + lds) = v[k][c];
             }
+        }
+    }
+    if (WL) {
+#pragma unroll
+        for (int k = 0; k < NWE; k++) {
+            const int e = tid + NT * k, t = e / (NCH * 128 * NG), r = e - t * (NCH * 128 * NG);
+            const int row = r / (4 * NCH), c = r % (4 * NCH) >> 2, q = r & 3;
+            if (e < NWP) *(uint4 *)(smw + ((t * NCH + c) * 32 * NG + row) * CV_LD + 8 * (q ^ (row >> 3 & 3))) = wv[k];
         }
     }
     __syncthreads();
@@ -186,26 +215,66 @@ __global__ __launch_bounds__(64 * NW * NG) void k_conv3x3(const bf16_t *__restri
     for (int a = 0; a < 4; a++)
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[a][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // pixel block a: row 2 wave + a / 2, columns 16 (a % 2) + r16
-    const bf16_t *base = sm + (2 * wave * PW + r16) * CV_LD + 8 * kq;
+    // pixel block a: row 2 wave + a / 2, columns 16 (a % 2) + r16; per column offset of the taps its swizzled address
+    const bf16_t *base[3];
+#pragma unroll
+    for (int dx = 0; dx < 3; dx++)
+        base[dx] = sm + (2 * wave * PW + r16 + dx) * CV_LD + 8 * (kq ^ ((r16 + dx) >> 2 & 3));
+    auto aload = [&](int s, Frag(&A)[4]) {   // step s of a row of taps: tap s / NCH, chunk s % NCH
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+            A[a].raw = *(const uint4 *)(base[s / NCH] + (s % NCH * NPX + (a >> 1) * PW + 16 * (a & 1)) * CV_LD);
+    };
+    const bf16_t *wbase = smw + (32 * ((tid >> 6) / NW) + 8 * (r16 >> 2) + (r16 & 3)) * CV_LD + 8 * (kq ^ (r16 >> 2));
+    auto bload = [&](int s, Frag(&b)[2]) {
+        const bf16_t *w = wbase + s * 32 * NG * CV_LD;
+        b[0].raw = *(const uint4 *)w;
+        b[1].raw = *(const uint4 *)(w + 4 * CV_LD);
+    };
+    // with more channels fewer waves fit: the pixels of the next step load ahead (NA a divisor of a row's 3 NCH steps)
+    constexpr int NA = NCH == 1 ? 1 : NCH == 3 ? 3 : 2;
+    Frag A[NA][4];
+    Frag Bl[NA][2];
+    if (NA > 1) {
+        aload(0, A[0]);
+        if (WL) bload(0, Bl[0]);
+    }
 #pragma unroll 1
     for (int dy = 0; dy < 3; dy++) {
 #pragma unroll
         for (int s = 0; s < 3 * NCH; s++) {   // step 3 NCH dy + s: tap 3 dy + s / NCH, chunk s % NCH
-            const bf16_t *p = base + (s / NCH + s % NCH * NPX) * CV_LD;
-            Frag A[4];
+            constexpr int S = 3 * NCH;
+            if (NA == 1) {
+                aload(s, A[0]);
+                if (WL) bload(s, Bl[0]);
+            }
+            if (NA > 1 && s + 1 < S) {
+                aload(s + 1, A[(s + 1) % NA]);
+                if (WL) bload(s + 1, Bl[(s + 1) % NA]);
+            }
+            if (NA > 1 && s + 1 == S) {   // past the last row: the last row again
 #pragma unroll
-            for (int a = 0; a < 4; a++) A[a].raw = *(const uint4 *)(p + ((a >> 1) * PW + 16 * (a & 1)) * CV_LD);
+                for (int dx = 0; dx < 3; dx++) base[dx] += dy < 2 ? PW * CV_LD : 0;
+                wbase += dy < 2 ? S * 32 * NG * CV_LD : 0;
+                aload(0, A[0]);
+                if (WL) bload(0, Bl[0]);
+            }
 #pragma unroll
             for (int j = 0; j < 2; j++)
 #pragma unroll
                 for (int a = 0; a < 4; a++)
-                    acc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(B[s % D][j].v, A[a].v, acc[a][j], 0, 0, 0);
+                    acc[a][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(WL ? Bl[s % NA][j].v : B[s % D][j].v, A[s % NA][a].v,
+                                                                        acc[a][j], 0, 0, 0);
+            if (WL) continue;
             const int q = s + D;   // past the last step: the last tap again
             const int t = 3 * dy + q / NCH;
             wload(t < 9 ? t : 8, q % NCH, B[s % D]);
         }
-        base += PW * CV_LD;
+        if (NA == 1) {
+#pragma unroll
+            for (int dx = 0; dx < 3; dx++) base[dx] += PW * CV_LD;
+            wbase += 3 * NCH * 32 * NG * CV_LD;
+        }
     }
 
     // D fragment: row 4*kq + i of fragment j = channel co0 + 8*kq + 4*j + i, column r16 = pixel
@@ -1194,7 +1263,6 @@ int conv_nj(long P, int C)
     return 1;
 }
 // LDS bytes of a workgroup of nw waves
-constexpr size_t conv_lds(int nw, int nch) { return (size_t)nch * (2 * nw + 2) * (CV_W + 2) * CV_LD * sizeof(bf16_t); }
 
 void pool2(const bf16_t *x, int N, int H, int W, int C, bf16_t *y, hipStream_t st)
 {
@@ -1238,7 +1306,7 @@ void conv_staged(const ConvArgs &c, hipStream_t st)
     auto wgs = [&](int nw) {
         return (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * nw - 1) / (2 * nw)) * c.N * (c.Cout / (32 * NG));
     };
-    if constexpr (conv_lds(4, NCH) <= 64 * 1024)
+    if constexpr (conv_lds(4, NCH) <= 64 * 1024 || conv_wl(4, NG, NCH))
         if (wgs(4) >= 256) return conv_launch<4, NG, NCH, MODE>(c, st);
     if constexpr (conv_lds(2, NCH) <= 64 * 1024)
         if (wgs(2) >= 256) return conv_launch<2, NG, NCH, MODE>(c, st);

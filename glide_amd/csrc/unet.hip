@@ -170,6 +170,16 @@ __global__ __launch_bounds__(64 * NW * NG, NCH == 1 ? 5 : NCH == 6 ? 2 : NCH == 
         }
     }
 
+    // The weights are not in the L2s when a layer starts, and the workgroups of an XCD walk them in step, each prefetch
+    // a miss: so every XCD's workgroups first touch all of them, a line of 128 bytes a thread
+    uint32_t touched = 0;
+    if (!WL) {
+        const long lines = (9 * tap + 127) / 128;
+        const unsigned b = blockIdx.x + gridDim.x * blockIdx.y, nb = (gridDim.x * gridDim.y + 7) / 8;
+        const long l = (long)(b / 8) * NT + tid;
+        if (l < lines) touched = *(const uint32_t *)((const char *)Wt + 128 * l);
+        if (l + (long)nb * NT < lines) touched ^= *(const uint32_t *)((const char *)Wt + 128 * (l + (long)nb * NT));
+    }
     // stage the input: 16-byte pieces, 4 per pixel and chunk
     constexpr int NE = (NPX * 4 + NT - 1) / NT, NB = conv_round(NE, NCH);   // pieces per thread, in flight x NCH
     const int CB = Cin - CA, ncha = CA / 32;
@@ -208,6 +218,7 @@ __global__ __launch_bounds__(64 * NW * NG, NCH == 1 ? 5 : NCH == 6 ? 2 : NCH == 
             if (e < NWP) *(uint4 *)(smw + ((t * NCH + c) * 32 * NG + row) * CV_LD + 8 * (q ^ (row >> 3 & 3))) = wv[k];
         }
     }
+    if (!WL) asm volatile("" ::"v"(touched));
     __syncthreads();
 
     f32x4 acc[4][2];

@@ -493,10 +493,10 @@ def level_sweep_roofline(ph, level: int, n_sweeps: int, reps: int = 3):
     ms = e0.elapsed_time(e1) / (reps * n_sweeps)
     nc = g.ny * g.nx
     tf = sweep_flops(nc) / (ms * 1e-3) / 1e12
-    return {"kernel": f"k_vanka_halo<false> (full sweep of the {g.ny}x{g.nx} level, apply pass folded in)",
+    return {"kernel": f"k_vanka_multi<false> (full sweep of the {g.ny}x{g.nx} level, up to 3 sweeps a launch)",
             "bound": "valu", "note": "FP64 vector arithmetic (no MFMA); peak = MI355X FP64 78.6 TFLOP/s; one "
-            "lane per cell (each workgroup also runs the ring around its 62 x 2 cells), latency of the per-cell "
-            "Newton chain plus one launch per sweep",
+            "lane per cell (16 x 16 cells a workgroup, those at its sides redone by several), latency of the "
+            "per-cell Newton chain plus a launch per 2 or 3 sweeps",
             "achieved": round(tf, 4), "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s",
             "frac": round(tf / PEAK_FP64_TFLOPS, 5), "traffic": None, "ms_per_launch": round(ms, 5),
             "work": f"{nc} cells x (eta + 10 Newton x {FLOPS_NEWTON_ITER} flop) = {sweep_flops(nc)} flop per sweep"}

@@ -67,14 +67,14 @@ inline hipStream_t S(void *s) { return (hipStream_t)s; }
 std::atomic<int> g_wg_per_cu[2] = {{64}, {8}};
 // Levels with at most g_small_max_cells cells sweep with the small-level
 // kernel: variant 0 = k_vanka compiled for one wave per SIMD (the whole
-// register file), 1 = the row split (k_vanka_rows), 2 = k_vanka_halo (the
-// apply pass folded into the sweep, the state alternating between U and the
-// Vanka scratch); set by glide_set_small_levels.  Measured (one sweep with
-// its apply, 10 Newton iterations, HIP events over 10 sweeps): 32^2 22.2 /
-// 19.9 us, 64^2 23.4 / 20.5, 128^2 23.7-24.6 / 20.7-21.1 (variant 0 / 2);
-// the row split measured 23.2, 24.0 and 24.1 against 22.5, 23.6 and 23.4
-// for variant 0 in an earlier build.
-std::atomic<long> g_small_max_cells{128 * 128};
+// register file), 1 = the row split (k_vanka_rows), 2 = k_vanka_multi (up to
+// 3 sweeps a launch, the state alternating between U and the Vanka scratch)
+// where its workgroups have a CU each, else as 0; set by
+// glide_set_small_levels.  One sweep of ten, 10 Newton iterations, the larger
+// levels' kernels / variant 2: 32^2 14.2 / 9.0 us, 128^2 15.7 / 10.7, 192^2
+// 16.1 / 12.5, 208^2 (13 x 13 cells on each of 256 CUs, the most that fits)
+// 15.2 / 12.7.
+std::atomic<long> g_small_max_cells{208 * 208};
 std::atomic<int> g_small_variant{2};
 // Tile heights (64 x TY cells) of the single-level residual (4, 8, 16; 0 = 8)
 // and of the JVP / VJP (0 = the per-point form, 4, 6, 8; initially by level
@@ -169,21 +169,29 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                                   blockIdx.x / tx, L);
 }
 
-// Small-level sweep with the apply pass folded in (vanka_halo_tile): U -> Uo,
-// one workgroup per 62 x 2 owned cells, one wave per SIMD.
+// ns small-level sweeps in one launch (vanka_multi_tile): U -> Uo, another
+// buffer unless the level is one workgroup's
 template <bool LOCAL>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(1))) void k_vanka_halo(
-    GlideGeom g, Params p, const double *__restrict__ U, double *__restrict__ Uo, const double *__restrict__ f,
-    const double *__restrict__ bed, const double *__restrict__ B, const double *__restrict__ beta,
-    const double *__restrict__ gamma, const unsigned char *__restrict__ blk, int nbx, int n_newton)
+__global__ __launch_bounds__(MS *MS) __attribute__((amdgpu_waves_per_eu(1))) void k_vanka_multi(
+    GlideGeom g, Params p, const double *U, double *Uo, const double *__restrict__ f, const double *__restrict__ bed,
+    const double *__restrict__ B, const double *__restrict__ beta, const double *__restrict__ gamma,
+    const unsigned char *__restrict__ blk, int nbx, int n_newton, int ns)
 {
-    __shared__ VankaLDS<TX, TY> L;
-    __shared__ double cd_s[5][TY][TX];
-    vanka_halo_tile<TX, TY, LOCAL>(g, p, U, Uo, f, bed, B, beta, gamma, blk, nbx, n_newton, blockIdx.x, blockIdx.y,
-                                   L, cd_s);
+    __shared__ MultiLDS L;
+    vanka_multi_tile<LOCAL>(g, p, U, Uo, f, bed, B, beta, gamma, blk, nbx, n_newton, ns, blockIdx.x, blockIdx.y, L);
 }
-dim3 halo_grid(int ny, int nx) { return dim3(cdiv(nx, TX - 2), cdiv(ny, TY - 2)); }
-
+dim3 multi_grid(int ny, int nx, int ns) { return dim3(cdiv(nx, multi_own(nx, ns)), cdiv(ny, multi_own(ny, ns))); }
+// sweeps a launch: as many as leave every workgroup a CU of its own (a second
+// one on a CU takes its SIMDs' issue, which bounds the chain); 0: none do
+int multi_sweeps(int ny, int nx, int cus)
+{
+    if (ny <= MS && nx <= MS) return 256;
+    for (int ns = 3; ns >= 1; ns--) {
+        const dim3 w = multi_grid(ny, nx, ns);
+        if ((long)w.x * w.y <= cus) return ns;
+    }
+    return 0;
+}
 
 // ---------------------------------------------------------------------------
 // Row-split Vanka sweep for small levels, where a sweep takes as long as one
@@ -1193,7 +1201,7 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
     const int variant = g_small_variant;
     const bool rows = small && variant == 1;
     const dim3 block(TX, TY), rblock(64, ROW_WAVES), rgrid(cdiv(g.nx, 64), g.ny);
-    const dim3 vgrid = vanka_grid(g.ny, g.nx), pgrid = point_grid(g.ny, g.nx), hgrid = halo_grid(g.ny, g.nx);
+    const dim3 vgrid = vanka_grid(g.ny, g.nx), pgrid = point_grid(g.ny, g.nx);
     const bool loop = (long)vgrid.x < (long)cdiv(g.nx, TX) * cdiv(g.ny, TY);
     auto sweep = [&](auto local) {   // one sweep in place: the smoother, then the apply pass
         constexpr bool LOCAL = decltype(local)::value;
@@ -1211,15 +1219,27 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
     auto run = [&](auto local) {
         constexpr bool LOCAL = decltype(local)::value;
         int s = 0;
-        if (small && variant == 2) {
-            // The sweeps alternate the state between U and the scratch (5 nc >=
-            // nu + nv + nc doubles); an odd count runs its first sweep in place
-            // with the apply pass, so that the last sweep writes U.
-            if (n_sweeps & 1) sweep(local), s = 1;
-            for (; s < n_sweeps; s++) {
-                const bool to_u = ((n_sweeps - 1 - s) & 1) == 0;
-                hipLaunchKernelGGL(k_vanka_halo<LOCAL>, hgrid, block, 0, st, g, p, to_u ? scratch : U, to_u ? U : scratch,
-                                   f, bed, B, beta, gamma, blk, nbx, n_newton);
+        const int per = small && variant == 2 ? multi_sweeps(g.ny, g.nx, n_cu()) : 0;
+        if (per) {
+            // The launches alternate the state between U and the scratch (5 nc >=
+            // nu + nv + nc doubles) and the last one writes U: an odd count of
+            // them has one more, of fewer sweeps each, or runs its first sweep in
+            // place with the apply pass.  A level of one workgroup stays in U.
+            const bool one = g.ny <= MS && g.nx <= MS;
+            int launches = cdiv(n_sweeps, per);
+            if (!one && (launches & 1)) {
+                if (launches < n_sweeps)
+                    launches++;
+                else
+                    sweep(local), s = 1, launches--;
+            }
+            for (; launches > 0; launches--) {
+                const int ns = cdiv(n_sweeps - s, launches);
+                const bool to_u = one || (launches & 1);
+                hipLaunchKernelGGL(k_vanka_multi<LOCAL>, multi_grid(g.ny, g.nx, ns), dim3(MS, MS), 0, st, g, p,
+                                   one || !to_u ? U : scratch, to_u ? U : scratch, f, bed, B, beta, gamma, blk, nbx,
+                                   n_newton, ns);
+                s += ns;
             }
         }
         for (; s < n_sweeps; s++) sweep(local);

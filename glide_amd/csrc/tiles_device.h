@@ -574,72 +574,171 @@ __device__ __forceinline__ void apply_tile(int ny, int nx, double *__restrict__ 
     }
 }
 
-// One Vanka sweep with its apply pass folded in, from the state U into Uo
-// (another buffer).  The workgroup's TX x TY threads run the cells
-// [i0-1, i0+TY-2] x [j0-1, j0+TX-2]: the (TX-2) x (TY-2) cells it owns,
-// (i0, j0) = (by (TY-2), bx (TX-2)), and the ring around them, whose
-// updates the owned faces also receive.  The per-cell updates meet in LDS
-// and every point the workgroup owns gets U + 0.5 d with d summed as the
-// apply pass sums it: the u faces and H of its cells, their top v faces,
-// and the level's last face column and row where its cells reach them.
-// Each point of the level is owned once, so Uo is written whole.  Threads
-// whose cell lies outside the level run the nearest cell of the level and
-// drop the result (a wave with idle lanes ran its chain slower).  With
-// LOCAL, idle cells' updates are not read (as in the apply pass), and a
-// workgroup whose cells are all idle runs no chain.  Same bits as vanka_tile
-// followed by apply_tile.  The grid is cdiv(nx, TX-2) x cdiv(ny, TY-2).
-template <int TX, int TY, bool LOCAL>
-__device__ __forceinline__ void vanka_halo_tile(const GlideGeom &g, const Params &p, const double *__restrict__ U,
-                                                double *__restrict__ Uo, const double *__restrict__ f,
-                                                const double *__restrict__ bed, const double *__restrict__ B,
-                                                const double *__restrict__ beta, const double *__restrict__ gamma,
-                                                const unsigned char *__restrict__ blk, int nbx, int n_newton, int bx,
-                                                int by, VankaLDS<TX, TY> &L, double (*cd_s)[TY][TX])
+// Several Vanka sweeps in one launch, for levels whose sweeps leave most of the
+// chip idle: there a sweep by itself is one wave's Newton chain (0.61 us an
+// iteration) and as much again for the launch, the first loads and the stores
+// (5.9 us at 16^2 to 128^2).  A workgroup of MS x MS threads keeps MS x MS
+// cells' state in LDS, one cell a thread, and runs ns sweeps on it.  A cell's
+// update reads faces that cells up to 2 away update, so 2 rows and columns a
+// sweep go stale at each side of the tile that is not the level's edge; what
+// is left of the tile after ns sweeps is the (MS + 1 - 4 ns)^2 cells that the
+// workgroup owns (their left and top faces, the level's last face column and
+// row where its cells reach them).  Level dimensions up to MS have no such
+// sides and any number of sweeps.  Cells are computed by several workgroups,
+// from the same inputs with the same bits as by vanka_tile and apply_tile.
+// A sweep of ten, before (one to a launch, its apply pass in the kernel) and
+// after: 16^2 12.0 -> 7.7 us, 32^2 12.0 -> 9.1, 64^2 12.3 -> 9.1, 128^2 12.5 -> 10.0.
+// At 13 x 13 cells a workgroup and one sweep a launch it still beats the sweep
+// and apply kernels: 208^2 15.2 -> 12.7 us.  The 128^2 reference step took 24.4 ms,
+// 17.7 now.
+constexpr int MS = 16;
+struct MultiLDS {
+    double u[MS + 2][MS + 1];   // rows i0-1 .. i0+MS (clamped), face columns j0 .. j0+MS
+    double v[MS + 1][MS + 2];   // face rows i0 .. i0+MS, columns j0-1 .. j0+MS (clamped)
+    double H[MS + 2][MS + 2], n[MS + 2][MS + 2], S[MS + 2][MS + 2], be[MS + 2][MS + 2];   // the cells and a ring
+    double cdr[MS][MS], cdb[MS][MS];   // the cells' updates of their right and bottom faces
+};
+// cells of a dimension of n that a workgroup owns after ns sweeps
+__host__ __device__ inline int multi_own(int n, int ns) { return n <= MS ? n : MS + 1 - 4 * ns; }
+
+template <bool LOCAL>
+__device__ __forceinline__ void vanka_multi_tile(const GlideGeom &g, const Params &p, const double *U, double *Uo,
+                                                 const double *__restrict__ f, const double *__restrict__ bed,
+                                                 const double *__restrict__ B, const double *__restrict__ beta,
+                                                 const double *__restrict__ gamma, const unsigned char *__restrict__ blk,
+                                                 int nbx, int n_newton, int ns, int bx, int by, MultiLDS &L)
 {
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
-    const double *u = U, *v = U + nu, *H = U + nu + nv;
-    const int i0 = by * (TY - 2), j0 = bx * (TX - 2);   // owned cells [i0, ie) x [j0, je)
-    const int ie = min(i0 + TY - 2, ny), je = min(j0 + TX - 2, nx);
-    const int a = threadIdx.y, b = threadIdx.x;
-    const int i = i0 - 1 + a, j = j0 - 1 + b;
-    const bool in = i >= 0 && i < ny && j >= 0 && j < nx;
-    auto act = [&](int ci, int cj) { return !LOCAL || blk[(ci / RB) * nbx + cj / RB] != 0; };
-    bool run = true;
-    if (LOCAL) run = __syncthreads_or(in && act(i, j));   // uniform
-    if (run) {
+    const int oy = multi_own(ny, ns), ox = multi_own(nx, ns);
+    const int io = by * oy, jo = bx * ox;   // owned cells [io, io + oy) x [jo, jo + ox)
+    // the tile: 2 ns cells more at the top and left, and inside the level where that has room
+    const int i0 = max(min(io - 2 * ns, ny - MS), 0), j0 = max(min(jo - 2 * ns, nx - MS), 0);
+    const int tid = threadIdx.y * MS + threadIdx.x;
+    const bool in = i0 + (int)threadIdx.y < ny && j0 + (int)threadIdx.x < nx;
+    // threads past the level's edge run its nearest cell and drop the result (a
+    // wave with idle lanes ran its chain slower)
+    const int i = min(i0 + (int)threadIdx.y, ny - 1), j = min(j0 + (int)threadIdx.x, nx - 1), a = i - i0, b = j - j0;
+    for (int k = tid; k < (MS + 2) * (MS + 1); k += MS * MS) {
+        const int ru = k / (MS + 1), cu = k - ru * (MS + 1);
+        L.u[ru][cu] = U[(size_t)clampi(i0 - 1 + ru, 0, ny - 1) * (nx + 1) + min(j0 + cu, nx)];
+        const int rv = k / (MS + 2), cv = k - rv * (MS + 2);
+        L.v[rv][cv] = U[nu + (size_t)min(i0 + rv, ny) * nx + clampi(j0 - 1 + cv, 0, nx - 1)];
+    }
+    const size_t ku = (size_t)i * (nx + 1) + j, kv = nu + (size_t)i * nx + j, kc = (size_t)i * nx + j;
+    double H = U[nu + nv + kc];
+    const bool act = !LOCAL || blk[(i / RB) * nbx + j / RB] != 0;
+    if (!LOCAL || __syncthreads_or(in && act)) {   // uniform
+        NewtonCell C;
+        C.f0 = f[ku];
+        C.f1 = f[ku + 1];
+        C.f2 = f[kv];
+        C.f3 = f[kv + nx];
+        C.f4 = f[nu + nv + kc];
+        C.bed = bed[kc];
+        C.beta = beta[kc];
+        C.th = gamma[kc];
+        const double Bc = B[kc], glen_exp = (1.0 - p.n) / (2.0 * p.n);
         const NewtonK K = newton_constants(g.dx, g.dt);
-        double d5[5];
-        // the run cells are a tile at (i0 - 1, j0 - 1)
-        if (i0 >= 3 && i0 + TY <= ny - 1 && j0 >= 3 && j0 + TX <= nx - 1)
-            vanka_cell_deltas<true>(g, p, K, L, U, f, bed, B, beta, gamma, n_newton, i0 - 1, j0 - 1, i, j, d5);
-        else
-            vanka_cell_deltas<false>(g, p, K, L, U, f, bed, B, beta, gamma, n_newton, i0 - 1, j0 - 1,
-                                     clampi(i, 0, ny - 1), clampi(j, 0, nx - 1), d5);
-#pragma unroll
-        for (int q = 0; q < 5; q++) cd_s[q][a][b] = d5[q];
-        __syncthreads();
+        newton_edges<false>(C, K, i, j, ny, nx);
+        for (int k = tid; k < (MS + 2) * (MS + 2); k += MS * MS) {   // the ring: 0 beyond the level's edge and the tile
+            (&L.H[0][0])[k] = 0.0;
+            (&L.n[0][0])[k] = 0.0;
+            (&L.S[0][0])[k] = 0.0;
+            (&L.be[0][0])[k] = 0.0;
+        }
+        const int bl = max(b - 1, 0), br = min(b + 2, MS), at = max(a - 1, 0), ab = min(a + 2, MS);
+        for (int s = 0; s < ns; s++) {
+            __syncthreads();   // the state (and, first, the cleared ring) is there
+            NewtonX x;
+            x.u_l = L.u[a + 1][b];
+            x.u_r = L.u[a + 1][b + 1];
+            x.v_t = L.v[a][b + 1];
+            x.v_b = L.v[a + 1][b + 1];
+            x.H = H;
+            C.u_tl = L.u[a][b];
+            C.u_tr = L.u[a][b + 1];
+            C.u_bl = L.u[a + 2][b];
+            C.u_br = L.u[a + 2][b + 1];
+            C.v_lt = L.v[a][b];
+            C.v_rt = L.v[a][b + 2];
+            C.v_lb = L.v[a + 1][b];
+            C.v_rb = L.v[a + 1][b + 2];
+            C.u_ll = L.u[a + 1][bl];
+            C.u_rr = L.u[a + 1][br];
+            C.v_tt = L.v[at][b + 1];
+            C.v_bb = L.v[ab][b + 1];
+            C.e2 = eta2_from(i, j, ny, nx, x.u_l, x.u_r, x.v_t, x.v_b, C.u_tl, C.u_tr, C.u_bl, C.u_br, C.v_lt, C.v_rt,
+                             C.v_lb, C.v_rb, Bc, p, glen_exp, K.dxi);
+            const double sg = sigm_mid(fma(0.917, H, C.bed), p.gl_c), be = fma(sg, C.beta, (1.0 - sg) * p.water_drag);
+            if (in) {
+                L.H[a + 1][b + 1] = H;
+                L.n[a + 1][b + 1] = C.e2 * H;
+                L.S[a + 1][b + 1] = fmax(C.bed, -0.917 * H) + H;
+                L.be[a + 1][b + 1] = be;
+                // beyond the level's edge stands the edge cell's drag
+                if (i == 0) L.be[a][b + 1] = be;
+                if (i == ny - 1) L.be[a + 2][b + 1] = be;
+                if (j == 0) L.be[a + 1][b] = be;
+                if (j == nx - 1) L.be[a + 1][b + 2] = be;
+            }
+            __syncthreads();
+            C.n_l = L.n[a + 1][b];
+            C.n_r = L.n[a + 1][b + 2];
+            C.n_t = L.n[a][b + 1];
+            C.n_b = L.n[a + 2][b + 1];
+            C.p_tl = (L.n[a][b] + C.n_t) + C.n_l;
+            C.p_tr = C.n_t + L.n[a][b + 2];
+            C.n_bl = L.n[a + 2][b];
+            C.n_br = L.n[a + 2][b + 2];
+            C.H_l = L.H[a + 1][b];
+            C.H_r = L.H[a + 1][b + 2];
+            C.H_t = L.H[a][b + 1];
+            C.H_b = L.H[a + 2][b + 1];
+            C.S_l = L.S[a + 1][b];
+            C.S_r = L.S[a + 1][b + 2];
+            C.S_t = L.S[a][b + 1];
+            C.S_b = L.S[a + 2][b + 1];
+            C.be_l = L.be[a + 1][b];
+            C.be_r = L.be[a + 1][b + 2];
+            C.be_t = L.be[a][b + 1];
+            C.be_b = L.be[a + 2][b + 1];
+            C.c_l = (C.v_lt - C.v_lb) * K.dxi;
+            C.c_r = (C.v_rt - C.v_rb) * K.dxi;
+            C.d_t = C.u_tr - C.u_tl;
+            C.d_b = C.u_br - C.u_bl;
+            const NewtonX x0 = x;
+            newton_iterate(C, K, p, n_newton, x);
+            // an idle cell's updates count as 0
+            const double d0 = act ? 0.5 * (x.u_l - x0.u_l) : 0.0, d1 = act ? 0.5 * (x.u_r - x0.u_r) : 0.0;
+            const double d2 = act ? 0.5 * (x.v_t - x0.v_t) : 0.0, d3 = act ? 0.5 * (x.v_b - x0.v_b) : 0.0;
+            const double dH = act ? x.H - x0.H : 0.0;
+            if (in) {
+                L.cdr[a][b] = d1;
+                L.cdb[a][b] = d3;
+            }
+            __syncthreads();   // all have read the state, too
+            H = x0.H + 0.5 * dH;
+            if (in) {
+                double d = 0.0;
+                if (b > 0) d = d + L.cdr[a][b - 1];
+                L.u[a + 1][b] = x0.u_l + 0.5 * (d + d0);
+                d = 0.0;
+                if (a > 0) d = d + L.cdb[a - 1][b];
+                L.v[a][b + 1] = x0.v_t + 0.5 * (d + d2);
+                if (j == nx - 1) L.u[a + 1][b + 1] = x0.u_r + 0.5 * (0.0 + d1);
+                if (i == ny - 1) L.v[a + 1][b + 1] = x0.v_b + 0.5 * (0.0 + d3);
+            }
+        }
     }
-    auto cdv = [&](int q, int ci, int cj) { return cd_s[q][ci - i0 + 1][cj - j0 + 1]; };
-    double *uo = Uo, *vo = Uo + nu, *Ho = Uo + nu + nv;
-    if (i >= i0 && i < ie && j >= j0 && (j < je || j == nx)) {
-        double d = 0.0;
-        if (j > 0 && act(i, j - 1)) d = d + cdv(1, i, j - 1);
-        if (j < nx && act(i, j)) d = d + cdv(0, i, j);
-        const size_t k = (size_t)i * (nx + 1) + j;
-        uo[k] = u[k] + 0.5 * d;
-    }
-    if (j >= j0 && j < je && i >= i0 && (i < ie || i == ny)) {
-        double d = 0.0;
-        if (i > 0 && act(i - 1, j)) d = d + cdv(3, i - 1, j);
-        if (i < ny && act(i, j)) d = d + cdv(2, i, j);
-        const size_t k = (size_t)i * nx + j;
-        vo[k] = v[k] + 0.5 * d;
-    }
-    if (i >= i0 && i < ie && j >= j0 && j < je) {
-        const size_t k = (size_t)i * nx + j;
-        const double d = act(i, j) ? cdv(4, i, j) : 0.0;
-        Ho[k] = H[k] + 0.5 * d;
+    // each thread stores the points that it updated itself
+    if (LOCAL) __syncthreads();   // or, in an idle tile, that others loaded
+    if (in && i >= io && i < io + oy && j >= jo && j < jo + ox) {
+        Uo[ku] = L.u[a + 1][b];
+        Uo[kv] = L.v[a][b + 1];
+        Uo[nu + nv + kc] = H;
+        if (j == nx - 1) Uo[ku + 1] = L.u[a + 1][b + 1];
+        if (i == ny - 1) Uo[kv + nx] = L.v[a + 1][b + 1];
     }
 }
 

@@ -359,11 +359,11 @@ int glide_set_tile_height(int kernel, int ty);
 
 /* Vanka kernel of the small levels, whose sweeps are bound by the latency
  * of one wave's Newton chain: levels with at most max_cells cells (default
- * 128 x 128) sweep with `variant` 0 = one lane per cell with the whole
+ * 208 x 208) sweep with `variant` 0 = one lane per cell with the whole
  * register file, 1 = row split (five waves per 64 cells, each assembling one
- * row of the local block), or 2 (default) = variant 0 with the apply pass
- * folded into the sweep (each workgroup also runs the ring of cells around
- * the 62 x 2 cells it owns; the state alternates between U and the scratch);
+ * row of the local block), or 2 (default) = up to 3 sweeps a launch, each
+ * workgroup of 16 x 16 cells redoing those at its sides (the state alternates
+ * between U and the scratch), on levels whose workgroups have a CU each;
  * larger levels sweep one lane per cell at two waves per SIMD.  A launch
  * shape only: results are bitwise the same.
  * Process-wide (atomic); no reference counterpart. */

@@ -47,7 +47,11 @@ constexpr int SHAPE_PTY = 2;      // index of TY = 4
 enum TilingKind { TK_POINT = 0, TK_CELL = 1, TK_BLOCK = 2 };
 // table index inside a phase: ((child * 3) + kind) * NSHAPE + shape
 __host__ __device__ constexpr int table_id(int child, int kind, int shape) { return (child * 3 + kind) * NSHAPE + shape; }
-constexpr int NTABLE = 2 * 3 * NSHAPE;
+constexpr int NTILING = 2 * 3 * NSHAPE;
+// then the tilings of several sweeps a launch (vanka_multi_tile): 1 .. MULTI_MAX
+constexpr int MULTI_MAX = 3;
+constexpr int NTABLE = NTILING + MULTI_MAX;
+__host__ __device__ constexpr int multi_table(int ns) { return NTILING + ns - 1; }
 
 struct BEntry {
     GlideLevel L;   // this level
@@ -137,6 +141,22 @@ __global__ __launch_bounds__(BTX *PTY) void kb_apply(const BEntry *__restrict__ 
         const int lt = t - pre[e], tx = cdiv(A.g.nx + 1, BTX);
         apply_tile<BTX, PTY, LOCAL>(A.g.ny, A.g.nx, A.U, A.scratch, A.active, A.g.nx / RB + 1, lt % tx, lt / tx);
     });
+}
+
+// ns sweeps in one launch, the state from U to the scratch or back (to_u), a
+// tile a workgroup (vanka_multi_tile)
+template <bool LOCAL>
+__global__ __launch_bounds__(MS *MS) __attribute__((amdgpu_waves_per_eu(1))) void kb_vanka_multi(
+    const BEntry *__restrict__ E, const int *__restrict__ pre, int n, const unsigned char *__restrict__ on, int n_newton,
+    int ns, int to_u)
+{
+    __shared__ MultiLDS L;
+    const int t = blockIdx.x, e = find_entry(pre, n, t);
+    const GlideLevel &A = E[e].L;
+    if (!on[E[e].member]) return;
+    const int lt = t - pre[e], tx = cdiv(A.g.nx, multi_own(A.g.nx, ns));
+    vanka_multi_tile<LOCAL>(A.g, to_params(A.p), to_u ? A.scratch : A.U, to_u ? A.U : A.scratch, A.f, A.bed, A.B, A.beta,
+                            A.gamma, A.active, A.g.nx / RB + 1, n_newton, ns, lt % tx, lt / tx, L);
 }
 
 __global__ __launch_bounds__(256) void kb_activation(const BEntry *__restrict__ E, const int *__restrict__ pre, int n,
@@ -458,7 +478,19 @@ int b_sweeps(const GlideBatch *b, int p, bool local, int n_sweeps, int n_newton,
     const int kern = local ? BK_VANKA_LOCAL : BK_VANKA;
     const int apt = table_id(0, TK_POINT, SHAPE_PTY);
     const unsigned ga = grid_of(b, P.total[apt], 8);
-    for (int s = 0; s < n_sweeps; s++) {
+    // phases whose tiles have a CU each take several sweeps a launch, the state
+    // alternating between U and the scratch: an even count of launches, or the
+    // first sweep in place (as the single-level sweeps)
+    int per = 0, launches = 0, in_place = n_sweeps;
+    for (int ns = MULTI_MAX; ns >= 1 && !per; ns--)
+        if (P.total[multi_table(ns)] <= b->n_cu) per = ns;
+    if (per) {
+        launches = cdiv(n_sweeps, per);
+        if ((launches & 1) && launches < n_sweeps) launches++;
+        in_place = launches & 1;
+        launches -= in_place;
+    }
+    for (int s = 0; s < in_place; s++) {
         BTRY(b_vanka(b, p, local, P.shape[kern], P.occ[kern], n_newton, st));
         if (local)
             hipLaunchKernelGGL(kb_apply<true>, dim3(ga), dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, apt), P.n,
@@ -467,7 +499,14 @@ int b_sweeps(const GlideBatch *b, int p, bool local, int n_sweeps, int n_newton,
             hipLaunchKernelGGL(kb_apply<false>, dim3(ga), dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, apt), P.n,
                                b->d_on);
     }
-    return bcheck("batched apply");
+    for (int s = in_place; launches > 0; launches--) {
+        const int ns = cdiv(n_sweeps - s, launches);
+        hipLaunchKernelGGL((local ? kb_vanka_multi<true> : kb_vanka_multi<false>), dim3(P.total[multi_table(ns)]),
+                           dim3(MS, MS), 0, st, entries(b, p), table(b, p, multi_table(ns)), P.n, b->d_on, n_newton, ns,
+                           launches & 1);
+        s += ns;
+    }
+    return bcheck("batched sweeps");
 }
 
 template <int OP>
@@ -653,6 +692,16 @@ int glide_batch_create(const GlideLevel *const *members, const int *n_levels, in
                     P.total[table_id(child, kind, s)] = acc;
                     max_tiles = std::max(max_tiles, (size_t)acc);
                 }
+        for (int ns = 1; ns <= MULTI_MAX; ns++) {
+            int acc = 0;
+            b->h_tables.push_back(0);
+            for (int q = 0; q < P.n; q++) {
+                const GlideGeom &g = b->h_entries[P.off + q].L.g;
+                acc += cdiv(g.nx, multi_own(g.nx, ns)) * cdiv(g.ny, multi_own(g.ny, ns));
+                b->h_tables.push_back(acc);
+            }
+            P.total[multi_table(ns)] = acc;
+        }
     }
     hipError_t e = hipSuccess;
     const size_t eb = b->h_entries.size() * sizeof(BEntry), tb = b->h_tables.size() * sizeof(int);

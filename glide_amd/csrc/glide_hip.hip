@@ -169,6 +169,28 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
                                   blockIdx.x / tx, L);
 }
 
+// A large level's sweep with no apply pass (vanka_fold_tile), one of several:
+// U -> Uo, pending updates in sets `set ^ 1` -> `set` of the scratch
+template <bool LOCAL>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_vanka_fold(
+    GlideGeom g, Params p, const double *__restrict__ U, double *__restrict__ Uo, double *scratch, int set, int first,
+    const double *__restrict__ f, const double *__restrict__ bed, const double *__restrict__ B,
+    const double *__restrict__ beta, const double *__restrict__ gamma, const unsigned char *__restrict__ blk, int nbx,
+    int n_newton)
+{
+    __shared__ FoldLDS<TX, TY> F;
+    const int tx = cdiv(g.nx, TX);
+    vanka_fold_tile<TX, TY, LOCAL>(g, p, U, Uo, fold_pending<TX, TY>(scratch, g.ny, g.nx, set ^ 1),
+                                   fold_pending<TX, TY>(scratch, g.ny, g.nx, set), first != 0, f, bed, B, beta, gamma, blk,
+                                   nbx, n_newton, blockIdx.x % tx, blockIdx.x / tx, F);
+}
+__global__ __launch_bounds__(TX) void k_fold_finish(int ny, int nx, double *__restrict__ U, double *scratch, int set)
+{
+    const int tx = cdiv(nx, TX);
+    fold_finish_tile<TX, TY>(ny, nx, U, fold_pending<TX, TY>(scratch, ny, nx, set), blockIdx.x % tx, blockIdx.x / tx,
+                             threadIdx.x);
+}
+
 // ns small-level sweeps in one launch (vanka_multi_tile): U -> Uo, another
 // buffer unless the level is one workgroup's
 template <bool LOCAL>
@@ -1197,8 +1219,10 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
                   double *scratch, hipStream_t st)
 {
     const int nbx = nbx_of(g.nx);
-    const bool small = (long)g.ny * g.nx <= g_small_max_cells;
     const int variant = g_small_variant;
+    const bool few = (long)g.ny * g.nx <= g_small_max_cells;
+    const int per = few && variant == 2 ? multi_sweeps(g.ny, g.nx, n_cu()) : 0;
+    const bool small = few && (variant != 2 || per);
     const bool rows = small && variant == 1;
     const dim3 block(TX, TY), rblock(64, ROW_WAVES), rgrid(cdiv(g.nx, 64), g.ny);
     const dim3 vgrid = vanka_grid(g.ny, g.nx), pgrid = point_grid(g.ny, g.nx);
@@ -1219,7 +1243,6 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
     auto run = [&](auto local) {
         constexpr bool LOCAL = decltype(local)::value;
         int s = 0;
-        const int per = small && variant == 2 ? multi_sweeps(g.ny, g.nx, n_cu()) : 0;
         if (per) {
             // The launches alternate the state between U and the scratch (5 nc >=
             // nu + nv + nc doubles) and the last one writes U: an odd count of
@@ -1241,6 +1264,15 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
                                    n_newton, ns);
                 s += ns;
             }
+        } else if (!small && !loop && n_sweeps > 1 && fold_fits(g.ny, g.nx, TX, TY)) {
+            // an even count of sweeps that alternate the state between U and the
+            // scratch, an odd one's first in place
+            if (n_sweeps & 1) sweep(local), s = 1;
+            const dim3 tiles(cdiv(g.nx, TX) * cdiv(g.ny, TY));
+            for (int k = 0; s < n_sweeps; s++, k++)
+                hipLaunchKernelGGL(k_vanka_fold<LOCAL>, tiles, block, 0, st, g, p, k & 1 ? scratch : U, k & 1 ? U : scratch,
+                                   scratch, k & 1, k == 0, f, bed, B, beta, gamma, blk, nbx, n_newton);
+            hipLaunchKernelGGL(k_fold_finish, tiles, dim3(TX), 0, st, g.ny, g.nx, U, scratch, 1);
         }
         for (; s < n_sweeps; s++) sweep(local);
     };

@@ -332,6 +332,37 @@ struct VankaLDS {
     double be[TY + 2][TX + 2];
 };
 
+// cell [a][b]'s neighbours from the staged values; what follows from those and the faces
+template <int TX, int TY>
+__device__ __forceinline__ void cell_from_lds(NewtonCell &C, const VankaLDS<TX, TY> &L, const NewtonK &K, int a, int b)
+{
+    C.e2 = L.e2[a][b];
+    C.n_l = L.n[a][b - 1];
+    C.n_r = L.n[a][b + 1];
+    C.n_t = L.n[a - 1][b];
+    C.n_b = L.n[a + 1][b];
+    C.p_tl = (L.n[a - 1][b - 1] + C.n_t) + C.n_l;
+    C.p_tr = C.n_t + L.n[a - 1][b + 1];
+    C.n_bl = L.n[a + 1][b - 1];
+    C.n_br = L.n[a + 1][b + 1];
+    C.H_l = L.H[a][b - 1];
+    C.H_r = L.H[a][b + 1];
+    C.H_t = L.H[a - 1][b];
+    C.H_b = L.H[a + 1][b];
+    C.S_l = L.S[a][b - 1];
+    C.S_r = L.S[a][b + 1];
+    C.S_t = L.S[a - 1][b];
+    C.S_b = L.S[a + 1][b];
+    C.be_l = L.be[a][b - 1];
+    C.be_r = L.be[a][b + 1];
+    C.be_t = L.be[a - 1][b];
+    C.be_b = L.be[a + 1][b];
+    C.c_l = (C.v_lt - C.v_lb) * K.dxi;
+    C.c_r = (C.v_rt - C.v_rb) * K.dxi;
+    C.d_t = C.u_tr - C.u_tl;
+    C.d_b = C.u_br - C.u_bl;
+}
+
 // A thread's share of the staged cells [i0-1, i0+TY] x [j0-1, j0+TX], cell q =
 // tid + q TX TY: load() issues all its reads, compute() evaluates and stores
 // to LDS.  Between the two the thread issues its own cell's reads as well, so a
@@ -471,31 +502,7 @@ __device__ __forceinline__ void vanka_cell_deltas(const GlideGeom &g, const Para
     const int a = i - i0 + 1, b = j - j0 + 1;
     x.H = L.H[a][b];
     const NewtonX x0 = x;
-    C.e2 = L.e2[a][b];
-    C.n_l = L.n[a][b - 1];
-    C.n_r = L.n[a][b + 1];
-    C.n_t = L.n[a - 1][b];
-    C.n_b = L.n[a + 1][b];
-    C.p_tl = (L.n[a - 1][b - 1] + C.n_t) + C.n_l;
-    C.p_tr = C.n_t + L.n[a - 1][b + 1];
-    C.n_bl = L.n[a + 1][b - 1];
-    C.n_br = L.n[a + 1][b + 1];
-    C.H_l = L.H[a][b - 1];
-    C.H_r = L.H[a][b + 1];
-    C.H_t = L.H[a - 1][b];
-    C.H_b = L.H[a + 1][b];
-    C.S_l = L.S[a][b - 1];
-    C.S_r = L.S[a][b + 1];
-    C.S_t = L.S[a - 1][b];
-    C.S_b = L.S[a + 1][b];
-    C.be_l = L.be[a][b - 1];
-    C.be_r = L.be[a][b + 1];
-    C.be_t = L.be[a - 1][b];
-    C.be_b = L.be[a + 1][b];
-    C.c_l = (C.v_lt - C.v_lb) * K.dxi;
-    C.c_r = (C.v_rt - C.v_rb) * K.dxi;
-    C.d_t = C.u_tr - C.u_tl;
-    C.d_b = C.u_br - C.u_bl;
+    cell_from_lds(C, L, K, a, b);
     newton_edges<INTERIOR>(C, K, i, j, ny, nx);
     newton_iterate(C, K, p, n_newton, x);
     d5[0] = 0.5 * (x.u_l - x0.u_l);
@@ -571,6 +578,265 @@ __device__ __forceinline__ void apply_tile(int ny, int nx, double *__restrict__ 
         size_t ci = (size_t)i * nx + j;
         double d = act(i, j) ? cd[4 * nc + ci] : 0.0;
         U[nu + nv + ci] += 0.5 * d;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// A sweep of a large level without an apply pass: from the state U into Uo
+// (another buffer).  Inside a tile the faces' updates meet in LDS; a face
+// between two tiles keeps its value in Uo, and the two cells' updates of it
+// go to the pending arrays, which whoever reads the face in the next sweep
+// adds (k_fold_finish after the last one): v faces on the tiles' top rows,
+// u faces on their left columns.  So a sweep reads and writes the state once
+// where the two kernels wrote five values a cell, read them again and read and
+// wrote the state; and the tile's state is staged in LDS, 5.5 loads a thread
+// where each took its cells' 56 through the vector cache.  Same bits as
+// vanka_tile and apply_tile.  A sweep of ten, before and
+// after: 256^2 17.2 -> 14.0 us, 387 x 501 local 44.2 -> 40.2, 512^2 42.7 -> 38.0,
+// 1024^2 149 -> 138.
+// ---------------------------------------------------------------------------
+template <int TX, int TY>
+struct FoldLDS {
+    VankaLDS<TX, TY> L;
+    double u[TY + 4][TX + 3];   // rows i0-2 .. i0+TY+1, face columns j0-1 .. j0+TX+1 (clamped)
+    double v[TY + 3][TX + 4];   // face rows i0-1 .. i0+TY+1, columns j0-2 .. j0+TX+1 (clamped)
+    double cdr[TY][TX], cdb[TY][TX];   // the cells' updates of their right and bottom faces
+};
+// pending updates: v faces of row by * TY from the cells above and below, u
+// faces of column bx * TX from the cells at the left and right
+struct FoldPending {
+    double *top, *bot, *lft, *rgt;
+    __host__ __device__ FoldPending(double *a, int ny, int nx, int ntx, int nty)
+        : top(a), bot(a + (size_t)nty * nx), lft(a + 2 * (size_t)nty * nx), rgt(a + 2 * (size_t)nty * nx + (size_t)ny * ntx)
+    {
+    }
+    __host__ __device__ static size_t doubles(int ny, int nx, int ntx, int nty)
+    {
+        return 2 * (size_t)nty * nx + 2 * (size_t)ny * ntx;
+    }
+};
+// the scratch of 5 nc doubles holds the other state and two sets of pending updates
+__host__ __device__ inline bool fold_fits(int ny, int nx, int tx, int ty)
+{
+    return n_t(ny, nx) + 2 * FoldPending::doubles(ny, nx, cdiv(nx, tx), cdiv(ny, ty)) <= 5 * n_c(ny, nx);
+}
+template <int TX, int TY>
+__host__ __device__ inline FoldPending fold_pending(double *scratch, int ny, int nx, int set)
+{
+    const int ntx = cdiv(nx, TX), nty = cdiv(ny, TY);
+    return FoldPending(scratch + n_t(ny, nx) + set * FoldPending::doubles(ny, nx, ntx, nty), ny, nx, ntx, nty);
+}
+
+// stages the tile's faces, its own cell and what follows from them; then as vanka_cell_deltas
+template <bool INTERIOR, int TX, int TY>
+__device__ __forceinline__ void fold_cell(const GlideGeom &g, const Params &p, const NewtonK &K, FoldLDS<TX, TY> &F,
+                                          const double *__restrict__ U, const FoldPending &P, bool first,
+                                          const double *__restrict__ f, const double *__restrict__ bed,
+                                          const double *__restrict__ B, const double *__restrict__ beta,
+                                          const double *__restrict__ gamma, int n_newton, int bx, int by, int i, int j,
+                                          NewtonX &x, NewtonX &x0)
+{
+    constexpr int NT = TX * TY, UC = TX + 3, VC = TX + 4, NU = (TY + 4) * UC, NV = (TY + 3) * VC;
+    constexpr int QU = (NU + NT - 1) / NT, QV = (NV + NT - 1) / NT, NALL = (TY + 2) * (TX + 2), QC = (NALL + NT - 1) / NT;
+    static_assert(2 * VC <= NT && 2 * (TY + 4) <= NT, "one pending face a thread");
+    const int ny = g.ny, nx = g.nx, i0 = by * TY, j0 = bx * TX;
+    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+    const int rb = INTERIOR ? i0 - 2 : max(i0 - 2, 0), cb = INTERIOR ? j0 - 2 : max(j0 - 2, 0);
+    const TileField tu(nx + 1, rb, cb), tc(nx, rb, cb);
+    const char *bu = tu.base(U), *bv = tc.base(U + nu), *bH = tc.base(U + nu + nv), *bbed = tc.base(bed),
+               *bB = tc.base(B), *bbeta = tc.base(beta);
+    const int tid = threadIdx.y * TX + threadIdx.x;
+    auto clip = [](int k, int n) { return INTERIOR ? k : clampi(k, 0, n); };
+    double ur[QU], vr[QV], h[QC], bd[QC], bt[QC], Bc[QC];
+#pragma unroll
+    for (int q = 0; q < QU; q++) {
+        const int k = tid + q * NT, r = k / UC, c = k - r * UC;
+        if (k >= NU) break;
+        ur[q] = ld_off(bu, (clip(i0 - 2 + r, ny - 1) - rb) * tu.pitch + 8u * (clip(j0 - 1 + c, nx) - cb));
+    }
+#pragma unroll
+    for (int q = 0; q < QV; q++) {
+        const int k = tid + q * NT, r = k / VC, c = k - r * VC;
+        if (k >= NV) break;
+        vr[q] = ld_off(bv, (clip(i0 - 1 + r, ny) - rb) * tc.pitch + 8u * (clip(j0 - 2 + c, nx - 1) - cb));
+    }
+#pragma unroll
+    for (int q = 0; q < QC; q++) {
+        const int k = tid + q * NT, a = k / (TX + 2), b = k - a * (TX + 2);
+        if (k >= NALL) break;
+        const uint32_t kc = (clip(i0 - 1 + a, ny - 1) - rb) * tc.pitch + 8u * (clip(j0 - 1 + b, nx - 1) - cb);
+        h[q] = ld_off(bH, kc);
+        bd[q] = ld_off(bbed, kc);
+        bt[q] = ld_off(bbeta, kc);
+        Bc[q] = ld_off(bB, kc);
+    }
+    // the faces with pending updates: v on rows i0 and i0 + TY, u on columns j0 and j0 + TX
+    const bool top = !first && by > 0, bot = !first && i0 + TY < ny, lft = !first && bx > 0, rgt = !first && j0 + TX < nx;
+    double pv = 0.0, pu = 0.0;
+    const int vs = tid >= VC, vc = tid - vs * VC, us = tid & 1, ru = tid >> 1;   // thread's row and column of v, of u
+    const bool pend_v = tid < 2 * VC && (vs ? bot : top), pend_u = tid < 2 * (TY + 4) && (us ? rgt : lft);
+    if (pend_v) {
+        const size_t k = (size_t)(by + vs) * nx + clip(j0 - 2 + vc, nx - 1);
+        const double a = P.bot[k], b = P.top[k];
+        pv = ld_off(bv, (i0 + vs * TY - rb) * tc.pitch + 8u * (clip(j0 - 2 + vc, nx - 1) - cb)) + 0.5 * ((0.0 + a) + b);
+    }
+    if (pend_u) {
+        const int r = clip(i0 - 2 + ru, ny - 1);
+        const size_t k = (size_t)(bx + us) * ny + r;
+        const double a = P.rgt[k], b = P.lft[k];
+        pu = ld_off(bu, (r - rb) * tu.pitch + 8u * (j0 + us * TX - cb)) + 0.5 * ((0.0 + a) + b);
+    }
+    NewtonCell C;
+    {
+        const uint32_t r0 = i - rb, c0 = 8u * (j - cb), u0 = r0 * tu.pitch + c0, v0 = r0 * tc.pitch + c0;
+        const char *fu = tu.base(f), *fv = tc.base(f + nu);
+        C.f0 = ld_off(fu, u0);
+        C.f1 = ld_off(fu, u0 + 8);
+        C.f2 = ld_off(fv, v0);
+        C.f3 = ld_off(fv, v0 + tc.pitch);
+        C.f4 = ld_off(tc.base(f + nu + nv), v0);
+        C.bed = ld_off(bbed, v0);
+        C.beta = ld_off(bbeta, v0);
+        C.th = ld_off(tc.base(gamma), v0);
+    }
+#pragma unroll
+    for (int q = 0; q < QU; q++) {
+        const int k = tid + q * NT, r = k / UC, c = k - r * UC;
+        if (k < NU && !(c == 1 && lft) && !(c == TX + 1 && rgt)) F.u[r][c] = ur[q];
+    }
+#pragma unroll
+    for (int q = 0; q < QV; q++) {
+        const int k = tid + q * NT, r = k / VC, c = k - r * VC;
+        if (k < NV && !(r == 1 && top) && !(r == TY + 1 && bot)) F.v[r][c] = vr[q];
+    }
+    if (pend_v) F.v[1 + vs * TY][vc] = pv;
+    if (pend_u) F.u[ru][1 + us * TX] = pu;
+    __syncthreads();
+    const double glen_exp = (1.0 - p.n) / (2.0 * p.n);
+#pragma unroll
+    for (int q = 0; q < QC; q++) {
+        const int k = tid + q * NT, a = k / (TX + 2), b = k - a * (TX + 2);
+        if (k >= NALL) break;
+        const int ci = i0 - 1 + a, cj = j0 - 1 + b;
+        double e2 = 0.0;
+        if (INTERIOR || (ci >= 0 && ci < ny && cj >= 0 && cj < nx))
+            e2 = eta2_from(INTERIOR ? 1 : ci, INTERIOR ? 1 : cj, INTERIOR ? 3 : ny, INTERIOR ? 3 : nx, F.u[a + 1][b],
+                           F.u[a + 1][b + 1], F.v[a][b + 1], F.v[a + 1][b + 1], F.u[a][b], F.u[a][b + 1], F.u[a + 2][b],
+                           F.u[a + 2][b + 1], F.v[a][b], F.v[a][b + 2], F.v[a + 1][b], F.v[a + 1][b + 2], Bc[q], p,
+                           glen_exp, K.dxi);
+        const double sg = sigm_mid(fma(0.917, h[q], bd[q]), p.gl_c);
+        F.L.e2[a][b] = e2;
+        F.L.n[a][b] = e2 * h[q];
+        F.L.H[a][b] = h[q];
+        F.L.S[a][b] = fmax(bd[q], -0.917 * h[q]) + h[q];
+        F.L.be[a][b] = fma(sg, bt[q], (1.0 - sg) * p.water_drag);
+    }
+    __syncthreads();
+    const int a = i - i0, b = j - j0;
+    x.u_l = F.u[a + 2][b + 1];
+    x.u_r = F.u[a + 2][b + 2];
+    x.v_t = F.v[a + 1][b + 2];
+    x.v_b = F.v[a + 2][b + 2];
+    C.u_ll = F.u[a + 2][b];
+    C.u_rr = F.u[a + 2][b + 3];
+    C.u_tl = F.u[a + 1][b + 1];
+    C.u_tr = F.u[a + 1][b + 2];
+    C.u_bl = F.u[a + 3][b + 1];
+    C.u_br = F.u[a + 3][b + 2];
+    C.v_lt = F.v[a + 1][b + 1];
+    C.v_lb = F.v[a + 2][b + 1];
+    C.v_rt = F.v[a + 1][b + 3];
+    C.v_rb = F.v[a + 2][b + 3];
+    C.v_tt = F.v[a][b + 2];
+    C.v_bb = F.v[a + 3][b + 2];
+    cell_from_lds(C, F.L, K, a + 1, b + 1);
+    newton_edges<INTERIOR>(C, K, i, j, ny, nx);
+    x.H = F.L.H[a + 1][b + 1];
+    x0 = x;
+    newton_iterate(C, K, p, n_newton, x);
+}
+
+// P_in, P_out: pending updates of the last sweep and of this one; first: there are none yet
+template <int TX, int TY, bool LOCAL>
+__device__ __forceinline__ void vanka_fold_tile(const GlideGeom &g, const Params &p, const double *__restrict__ U,
+                                                double *__restrict__ Uo, const FoldPending &Pi, const FoldPending &Po,
+                                                bool first, const double *__restrict__ f, const double *__restrict__ bed,
+                                                const double *__restrict__ B, const double *__restrict__ beta,
+                                                const double *__restrict__ gamma, const unsigned char *__restrict__ blk,
+                                                int nbx, int n_newton, int bx, int by, FoldLDS<TX, TY> &F)
+{
+    const int ny = g.ny, nx = g.nx;
+    const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
+    const int i0 = by * TY, j0 = bx * TX, a = threadIdx.y, b = threadIdx.x;
+    const int i = i0 + a, j = j0 + b;
+    const bool in = i < ny && j < nx;
+    const bool act = !LOCAL || (in && blk[(i / RB) * nbx + j / RB] != 0);
+    const size_t ku = (size_t)i * (nx + 1) + j, kv = nu + (size_t)i * nx + j, kH = nu + nv + (size_t)i * nx + j;
+    // faces between tiles at this cell
+    const bool pt = a == 0 && by > 0, pb = a == TY - 1 && i + 1 < ny, pl = b == 0 && bx > 0, pr = b == TX - 1 && j + 1 < nx;
+    const size_t kt = (size_t)by * nx + j, kl = (size_t)bx * ny + i;
+    if (LOCAL) {
+        if (!__syncthreads_or(act)) {   // uniform: the whole tile is idle.  Both buffers hold its inner points from the first sweep on
+            if (!in) return;
+            if (pt || first) Uo[kv] = pt && !first ? U[kv] + 0.5 * ((0.0 + Pi.bot[kt]) + Pi.top[kt]) : U[kv];
+            if (pl || first) Uo[ku] = pl && !first ? U[ku] + 0.5 * ((0.0 + Pi.rgt[kl]) + Pi.lft[kl]) : U[ku];
+            if (first) {
+                Uo[kH] = U[kH];
+                if (j == nx - 1) Uo[ku + 1] = U[ku + 1];
+                if (i == ny - 1) Uo[kv + nx] = U[kv + nx];
+            }
+            if (pt) Po.top[kt] = 0.0;
+            if (pb) Po.bot[kt + nx] = 0.0;
+            if (pl) Po.lft[kl] = 0.0;
+            if (pr) Po.rgt[kl + ny] = 0.0;
+            return;
+        }
+    }
+    const NewtonK K = newton_constants(g.dx, g.dt);
+    NewtonX x, x0;
+    // as in vanka_tile
+    if (i0 >= 2 && i0 + TY <= ny - 2 && j0 >= 2 && j0 + TX <= nx - 2)
+        fold_cell<true>(g, p, K, F, U, Pi, first, f, bed, B, beta, gamma, n_newton, bx, by, i, j, x, x0);
+    else
+        fold_cell<false>(g, p, K, F, U, Pi, first, f, bed, B, beta, gamma, n_newton, bx, by, min(i, ny - 1), min(j, nx - 1),
+                         x, x0);
+    // an idle cell's updates count as 0
+    const double d0 = act ? 0.5 * (x.u_l - x0.u_l) : 0.0, d1 = act ? 0.5 * (x.u_r - x0.u_r) : 0.0;
+    const double d2 = act ? 0.5 * (x.v_t - x0.v_t) : 0.0, d3 = act ? 0.5 * (x.v_b - x0.v_b) : 0.0;
+    const double dH = act ? x.H - x0.H : 0.0;
+    F.cdr[a][b] = d1;
+    F.cdb[a][b] = d3;
+    __syncthreads();
+    if (!in) return;
+    double d = 0.0;
+    if (b > 0) d = d + F.cdr[a][b - 1];
+    Uo[ku] = pl ? x0.u_l : x0.u_l + 0.5 * (d + d0);
+    d = 0.0;
+    if (a > 0) d = d + F.cdb[a - 1][b];
+    Uo[kv] = pt ? x0.v_t : x0.v_t + 0.5 * (d + d2);
+    Uo[kH] = x0.H + 0.5 * dH;
+    if (j == nx - 1) Uo[ku + 1] = x0.u_r + 0.5 * (0.0 + d1);
+    if (i == ny - 1) Uo[kv + nx] = x0.v_b + 0.5 * (0.0 + d3);
+    if (pt) Po.top[kt] = d2;
+    if (pb) Po.bot[kt + nx] = d3;
+    if (pl) Po.lft[kl] = d0;
+    if (pr) Po.rgt[kl + ny] = d1;
+}
+
+// adds the last sweep's pending updates of tile (bx, by)'s top row and left column; a wave a tile
+template <int TX, int TY>
+__device__ __forceinline__ void fold_finish_tile(int ny, int nx, double *__restrict__ U, const FoldPending &P, int bx, int by,
+                                                 int lane)
+{
+    static_assert(TX == 64 && TY <= 64, "a wave covers the tile's top row and left column");
+    const int i0 = by * TY, j0 = bx * TX, j = j0 + lane, i = i0 + lane;
+    if (by > 0 && j < nx) {
+        const size_t k = (size_t)by * nx + j;
+        U[n_u(ny, nx) + (size_t)i0 * nx + j] += 0.5 * ((0.0 + P.bot[k]) + P.top[k]);
+    }
+    if (bx > 0 && lane < TY && i < ny) {
+        const size_t k = (size_t)bx * ny + i;
+        U[(size_t)i * (nx + 1) + j0] += 0.5 * ((0.0 + P.rgt[k]) + P.lft[k]);
     }
 }
 

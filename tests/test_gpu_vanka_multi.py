@@ -49,7 +49,7 @@ def test_sweeps_of_one_launch_bitwise(shape, n, local):
             torch.cuda.synchronize()
             out.append(U.cpu().numpy())
     finally:
-        _lib.call("glide_set_small_levels", 128 * 128, 2)
+        _lib.call("glide_set_small_levels", 208 * 208, 2)
     assert np.isfinite(out[0]).all()
     assert np.array_equal(out[0], out[1])
     if n <= 2 and ny * nx <= 5000:

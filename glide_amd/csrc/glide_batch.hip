@@ -159,6 +159,42 @@ __global__ __launch_bounds__(MS *MS) __attribute__((amdgpu_waves_per_eu(1))) voi
                             A.gamma, A.active, A.g.nx / RB + 1, n_newton, ns, lt % tx, lt / tx, L);
 }
 
+// a sweep with no apply pass, one of several (vanka_fold_tile): U -> the scratch
+// where set = 0, back where set = 1; pending updates in sets set ^ 1 -> set.  A
+// tile a workgroup: looping over tiles spilled 200 bytes a lane (an eight-member
+// V-cycle 34.0 ms; smoother and apply pass 32.0, this 26.1).
+template <bool LOCAL>
+__global__ __launch_bounds__(BTX *PTY) __attribute__((amdgpu_waves_per_eu(2))) void kb_vanka_fold(
+    const BEntry *__restrict__ E, const int *__restrict__ pre, int n, const unsigned char *__restrict__ on, int n_newton,
+    int set, int first)
+{
+    __shared__ FoldLDS<BTX, PTY> F;
+    const int t = chunked_tile(blockIdx.x, pre[n]);
+    if (t >= pre[n]) return;
+    const int e = find_entry(pre, n, t);
+    const GlideLevel &A = E[e].L;
+    if (!on[E[e].member]) return;
+    const int lt = t - pre[e], tx = cdiv(A.g.nx, BTX);
+    vanka_fold_tile<BTX, PTY, LOCAL>(A.g, to_params(A.p), set ? A.scratch : A.U, set ? A.U : A.scratch,
+                                     fold_pending<BTX, PTY>(A.scratch, A.g.ny, A.g.nx, set ^ 1),
+                                     fold_pending<BTX, PTY>(A.scratch, A.g.ny, A.g.nx, set), first != 0, A.f, A.bed, A.B,
+                                     A.beta, A.gamma, A.active, A.g.nx / RB + 1, n_newton, lt % tx, lt / tx, F);
+}
+
+// a wave a tile
+__global__ __launch_bounds__(BTX *PTY) void kb_fold_finish(const BEntry *__restrict__ E, const int *__restrict__ pre, int n,
+                                                           const unsigned char *__restrict__ on)
+{
+    const int t = blockIdx.x * PTY + threadIdx.y;
+    if (t >= pre[n]) return;
+    const int e = find_entry(pre, n, t);
+    const GlideLevel &A = E[e].L;
+    if (!on[E[e].member]) return;
+    const int lt = t - pre[e], tx = cdiv(A.g.nx, BTX);
+    fold_finish_tile<BTX, PTY>(A.g.ny, A.g.nx, A.U, fold_pending<BTX, PTY>(A.scratch, A.g.ny, A.g.nx, 1), lt % tx, lt / tx,
+                               threadIdx.x);
+}
+
 __global__ __launch_bounds__(256) void kb_activation(const BEntry *__restrict__ E, const int *__restrict__ pre, int n,
                                                      const unsigned char *__restrict__ on, int *__restrict__ any_active)
 {
@@ -350,6 +386,7 @@ struct BPhase {
     int n = 0, off = 0, toff = 0;     // entries, first entry, first table int
     int total[NTABLE] = {};           // tiles per table
     bool any_finest = false;
+    bool fold = true;                 // every entry's scratch holds what vanka_fold_tile keeps there
     int shape[BK_COUNT] = {SHAPE_PTY, SHAPE_PTY, SHAPE_PTY, SHAPE_PTY};
     int occ[BK_COUNT] = {0, 0, 0, 0};  // workgroups per CU (0: kernel default)
 };
@@ -478,17 +515,21 @@ int b_sweeps(const GlideBatch *b, int p, bool local, int n_sweeps, int n_newton,
     const int kern = local ? BK_VANKA_LOCAL : BK_VANKA;
     const int apt = table_id(0, TK_POINT, SHAPE_PTY);
     const unsigned ga = grid_of(b, P.total[apt], 8);
-    // phases whose tiles have a CU each take several sweeps a launch, the state
-    // alternating between U and the scratch: an even count of launches, or the
-    // first sweep in place (as the single-level sweeps)
+    // phases whose tiles have a CU each take several sweeps a launch, larger ones
+    // fold the apply pass into the next sweep; both alternate the state between U
+    // and the scratch: an even count of launches, or the first sweep in place (as
+    // the single-level sweeps)
     int per = 0, launches = 0, in_place = n_sweeps;
     for (int ns = MULTI_MAX; ns >= 1 && !per; ns--)
         if (P.total[multi_table(ns)] <= b->n_cu) per = ns;
+    const bool fold = !per && P.fold && n_sweeps > 1;
     if (per) {
         launches = cdiv(n_sweeps, per);
         if ((launches & 1) && launches < n_sweeps) launches++;
         in_place = launches & 1;
         launches -= in_place;
+    } else if (fold) {
+        in_place = n_sweeps & 1;
     }
     for (int s = 0; s < in_place; s++) {
         BTRY(b_vanka(b, p, local, P.shape[kern], P.occ[kern], n_newton, st));
@@ -505,6 +546,14 @@ int b_sweeps(const GlideBatch *b, int p, bool local, int n_sweeps, int n_newton,
                            dim3(MS, MS), 0, st, entries(b, p), table(b, p, multi_table(ns)), P.n, b->d_on, n_newton, ns,
                            launches & 1);
         s += ns;
+    }
+    if (fold) {
+        const int tid = table_id(0, TK_CELL, SHAPE_PTY), total = P.total[tid];
+        for (int s = in_place, k = 0; s < n_sweeps; s++, k++)
+            hipLaunchKernelGGL((local ? kb_vanka_fold<true> : kb_vanka_fold<false>), dim3(chunked_grid(total)),
+                               dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, tid), P.n, b->d_on, n_newton, k & 1, k == 0);
+        hipLaunchKernelGGL(kb_fold_finish, dim3(cdiv(total, PTY)), dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, tid), P.n,
+                           b->d_on);
     }
     return bcheck("batched sweeps");
 }
@@ -670,6 +719,7 @@ int glide_batch_create(const GlideLevel *const *members, const int *n_levels, in
             e.level = k;
             e.finest = k == 0;
             P.any_finest = P.any_finest || e.finest;
+            P.fold = P.fold && fold_fits(e.L.g.ny, e.L.g.nx, BTX, PTY);
             b->h_entries.push_back(e);
             P.n++;
         }

@@ -511,6 +511,8 @@ __host__ __device__ __forceinline__ void newton_adjoint(const NewtonCell &C, con
 // scheduled as one block: the sigmoid's chain hides among the rest of the
 // assembly (as a branch of its own it cost waves at a grounding line 1.4%).
 // Ten sweeps of 1024^2: 1632 -> 1480 us.
+// AHEAD: the wave's issue priority rises half way (vanka_fold_tile).
+template <bool AHEAD = false>
 __host__ __device__ __forceinline__ void newton_iterate(const NewtonCell &C, const NewtonK &K, const Params &p, int n_newton,
                                                NewtonX &x)
 {
@@ -519,6 +521,9 @@ __host__ __device__ __forceinline__ void newton_iterate(const NewtonCell &C, con
         return;
     }
     for (int k = 0; k < n_newton; k++) {
+#if defined(__HIP_DEVICE_COMPILE__)
+        if (AHEAD && 2 * k >= n_newton) __builtin_amdgcn_s_setprio(2);
+#endif
         bool clamped = sigm_clamped(fma(0.917, x.H, C.bed), p.gl_c);
 #if defined(__HIP_DEVICE_COMPILE__)
         clamped = __builtin_amdgcn_ballot_w64(!clamped) == 0;

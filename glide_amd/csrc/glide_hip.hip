@@ -972,10 +972,11 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_jvp(GlideGeom g, 
     const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
-    lin_tile_lds<TX, LTY, false>(g, p, jo, nullptr, U, dU, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
+    lin_tile_lds<TX, LTY, false, TX * LTY>(g, p, jo, nullptr, U, dU, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
 }
-template <int LTY>
-__global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, Params p, double *__restrict__ out,
+// WY: rows of threads; those past the tile's only stage (lin_helpers)
+template <int LTY, int WY = LTY>
+__global__ __launch_bounds__(TX *WY, WY > LTY ? 2 : LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, Params p, double *__restrict__ out,
                                                  const double *__restrict__ base, const double *__restrict__ U,
                                                  const double *__restrict__ lam, const double *__restrict__ bed,
                                                  const double *__restrict__ B, const double *__restrict__ beta,
@@ -985,7 +986,7 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, 
     const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
-    lin_tile_lds<TX, LTY, true>(g, p, out, base, U, lam, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
+    lin_tile_lds<TX, LTY, true, TX * WY>(g, p, out, base, U, lam, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
 }
 // Height of the staged JVP / VJP tiles.  While all tiles are resident at once
 // (two 64 x 6 tiles of the JVP or three 64 x 4 tiles of the VJP a CU, which is
@@ -994,8 +995,14 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, 
 // JVP, 64 x 6 / 64 x 8: 256^2 7.9 / 8.8 us, 384^2 11.4 / 13.3, 512^2 18.0 /
 // 13.4, 1024^2 56.7 / 47.5.  VJP, 64 x 4 / 64 x 8: 256^2 8.5 / 10.0, 384^2 13.1
 // / 15.1, 512^2 18.5 / 15.5, 1024^2 59.9 / 56.9.  The adjoint colours (k_adjoint)
-// change over at the VJP's line: 256^2 9.6 / 10.4, 384^2 18.0 / 19.3, 512^2 22.4
+// change over at the VJP's line: 256^2 (without helpers) 9.6 / 10.4, 384^2 18.0 / 19.3, 512^2 22.4
 // / 20.3, 1024^2 82.4 / 74.7.
+// Levels whose 64 x 4 tiles have a CU each: four more rows of threads take the
+// second round of the VJP's and the adjoint colours' staging (396 cells for 256
+// threads), whose loads and power laws are a serial chain.  An adjoint cycle of
+// 256^2 1.85 -> 1.64 ms, of 64^2 1.02 -> 0.91, a VJP of 200 x 220 8.2 -> 7.6 us.
+// With more tiles than CUs the extra waves only take the others' issue.
+inline bool lin_helpers(const GlideGeom &g) { return (long)cdiv(g.nx, TX) * cdiv(g.ny, 4) <= n_cu(); }
 inline bool lin_tall(const GlideGeom &g) { return (long)cdiv(g.nx, TX) * cdiv(g.ny, 4) > 3L * n_cu(); }
 inline int lin_ty(const GlideGeom &g, bool vjp)
 {
@@ -1057,9 +1064,9 @@ __global__ __launch_bounds__(NT) void k_vanka_adj(GlideGeom g, Params p, double 
 
 // r = f_adj - J^T lam and one colour's update of lam into lam_out (adjoint_tile);
 // per colour, against k_vjp and k_vanka_adj: 64^2 17 -> 9.2 us, 256^2 17 -> 9.6
-// (an adjoint cycle of 256^2 3.08 -> 1.84 ms), 512^2 27 -> 20.3
-template <int LTY>
-__global__ __launch_bounds__(TX *LTY) void k_adjoint(GlideGeom g, Params p, double *__restrict__ lam_out,
+// (an adjoint cycle of 256^2 3.08 -> 1.84 ms, 1.64 with lin_helpers), 512^2 27 -> 20.3
+template <int LTY, int WY = LTY>
+__global__ __launch_bounds__(TX *WY) void k_adjoint(GlideGeom g, Params p, double *__restrict__ lam_out,
                                                      double *__restrict__ r, const double *__restrict__ f_adj,
                                                      const double *__restrict__ U, const double *__restrict__ lam,
                                                      const double *__restrict__ bed, const double *__restrict__ B,
@@ -1070,7 +1077,7 @@ __global__ __launch_bounds__(TX *LTY) void k_adjoint(GlideGeom g, Params p, doub
     const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
-    adjoint_tile<TX, LTY>(g, p, lam_out, r, f_adj, U, lam, bed, B, beta, mask, color, omega, t / tiles_y, t % tiles_y, S);
+    adjoint_tile<TX, LTY, TX * WY>(g, p, lam_out, r, f_adj, U, lam, bed, B, beta, mask, color, omega, t / tiles_y, t % tiles_y, S);
 }
 
 // grad_beta = lambda . dR/dbeta, gather form in the oracle's summation order
@@ -1494,6 +1501,8 @@ int launch_vjp(const GlideGeom &g, const Params &p, double *out, const double *b
         hipLaunchKernelGGL(k_vjp<8>, grid8, dim3(TX, 8), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
     else if (ty == 6)
         hipLaunchKernelGGL(k_vjp<6>, grid6, dim3(TX, 6), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
+    else if (ty == 4 && lin_helpers(g))
+        hipLaunchKernelGGL((k_vjp<4, 8>), grid4, dim3(TX, 8), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
     else if (ty == 4)
         hipLaunchKernelGGL(k_vjp<4>, grid4, dim3(TX, 4), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
     else
@@ -1513,14 +1522,17 @@ int compute_mask(const GlideLevel &A, hipStream_t st)
 int adjoint_sweeps(const GlideLevel &A, int n, double omega, hipStream_t st)
 {
     const Params p = to_params(A.p);
-    const bool tall = lin_tall(A.g);
-    const dim3 grid = lin_grid(A.g, tall ? 8 : 4), block(TX, tall ? 8 : 4);
+    const bool tall = lin_tall(A.g), helpers = lin_helpers(A.g);
+    const dim3 grid = lin_grid(A.g, tall ? 8 : 4), block(TX, tall || helpers ? 8 : 4);
     for (int s = 0; s < n; s++) {
         for (int color = 0; color < 2; color++) {   // red into the Vanka scratch (5 values a cell), black back
             double *out = color ? A.Lambda : A.scratch;
             const double *lam = color ? A.scratch : A.Lambda;
             if (tall)
                 hipLaunchKernelGGL(k_adjoint<8>, grid, block, 0, st, A.g, p, out, A.r_adj, A.f_adj, A.U, lam, A.bed, A.B,
+                                   A.beta, A.mask, color, omega);
+            else if (helpers)
+                hipLaunchKernelGGL((k_adjoint<4, 8>), grid, block, 0, st, A.g, p, out, A.r_adj, A.f_adj, A.U, lam, A.bed, A.B,
                                    A.beta, A.mask, color, omega);
             else
                 hipLaunchKernelGGL(k_adjoint<4>, grid, block, 0, st, A.g, p, out, A.r_adj, A.f_adj, A.U, lam, A.bed, A.B,

@@ -1174,10 +1174,10 @@ struct AdjLDS : LinLDS<TX, TY> {
 
 // One tile: stage() fills the LDS (all threads), then the rows may be asked
 // for: u faces (i0.., j0..j0+TX), v faces (i0..i0+TY, j0..), cells.  ADJ: LDS is an AdjLDS.
-template <int TX, int TY, bool VJP, bool ADJ>
+template <int TX, int TY, bool VJP, bool ADJ, int NT = TX * TY>
 struct LinTile {
     using LDS = typename std::conditional<ADJ, AdjLDS<TX, TY>, LinLDS0<TX, TY>>::type;
-    static constexpr int NT = TX * TY, NALL = (TY + 2) * (TX + 2);
+    static constexpr int NALL = (TY + 2) * (TX + 2);
     LDS &S;
     const Params &p;
     const int ny, nx, i0, j0, rb, cb;
@@ -1439,15 +1439,16 @@ struct LinTile {
 };
 
 // VJP: out = base - l when base != NULL (the adjoint residual f_adj - J^T lambda)
-template <int TX, int TY, bool VJP>
+template <int TX, int TY, bool VJP, int NT>
 __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p, double *__restrict__ out,
                                              const double *__restrict__ base, const double *__restrict__ U,
                                              const double *__restrict__ D, const double *__restrict__ bed,
                                              const double *__restrict__ B, const double *__restrict__ beta,
                                              const double *__restrict__ mask, int bx, int by, LinLDS0<TX, TY> &S)
 {
-    const LinTile<TX, TY, VJP, false> T(S, g, p, U, D, bed, B, beta, mask, bx, by);
+    const LinTile<TX, TY, VJP, false, NT> T(S, g, p, U, D, bed, B, beta, mask, bx, by);
     T.stage();
+    if (threadIdx.y >= TY) return;   // threads that only staged
     const int ny = g.ny, nx = g.nx, i = T.i0 + threadIdx.y, j = T.j0 + threadIdx.x;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
     if (i > ny || j > nx) return;
@@ -1475,7 +1476,7 @@ __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p
 // edge faces of cells of the other colour by those.  The cells of the colour
 // take the first half of the threads, so that whole waves solve.
 // ---------------------------------------------------------------------------
-template <int TX, int TY>
+template <int TX, int TY, int NT>
 __device__ __forceinline__ void adjoint_tile(const GlideGeom &g, const Params &p, double *__restrict__ lam_out,
                                              double *__restrict__ r, const double *__restrict__ f_adj,
                                              const double *__restrict__ U, const double *__restrict__ lam,
@@ -1483,8 +1484,9 @@ __device__ __forceinline__ void adjoint_tile(const GlideGeom &g, const Params &p
                                              const double *__restrict__ beta, const double *__restrict__ mask, int color,
                                              double omega, int bx, int by, AdjLDS<TX, TY> &S)
 {
-    const LinTile<TX, TY, true, true> T(S, g, p, U, lam, bed, B, beta, mask, bx, by);
+    const LinTile<TX, TY, true, true, NT> T(S, g, p, U, lam, bed, B, beta, mask, bx, by);
     T.stage();
+    if (threadIdx.y >= TY) return;   // threads that only staged
     const int ny = g.ny, nx = g.nx;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
     const int tid = threadIdx.y * TX + threadIdx.x, half = tid >= TX * TY / 2, q = tid - half * (TX * TY / 2);

@@ -21,7 +21,7 @@ DEV = torch.device("cuda")
 
 
 @pytest.mark.parametrize("gl", [False, True])
-@pytest.mark.parametrize("shape", [(2, 2), (3, 63), (4, 64), (5, 65), (33, 130), (130, 66)])
+@pytest.mark.parametrize("shape", [(2, 2), (3, 63), (4, 64), (5, 65), (33, 130), (130, 66), (512, 70), (260, 258), (520, 380)])
 def test_colour_in_one_pass_same_bits(gl, shape):
     ny, nx = shape
     s = random_state(ny=ny, nx=nx, seed=ny + 7 * nx)

@@ -32,6 +32,11 @@ class GlideGeom(ctypes.Structure):
     _fields_ = [("ny", c_int), ("nx", c_int), ("dx", c_double), ("dt", c_double)]
 
 
+class GlideAdamItem(ctypes.Structure):
+    _fields_ = [("w", c_void_p), ("g", c_void_p), ("m", c_void_p), ("v", c_void_p), ("n", ctypes.c_long),
+                ("wb", c_void_p), ("wflip", c_void_p), ("cout", c_int), ("cin", c_int)]
+
+
 DP = c_void_p   # device pointers travel as plain addresses
 
 _LEVEL_PTRS = ["U", "f", "r", "w", "z", "Lambda", "Lambda_out", "f_adj", "r_adj",
@@ -142,6 +147,8 @@ SIGNATURES = {
                                c_void_p]),
     "glide_unet_adam": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, ctypes.c_long, ctypes.c_float,
                                 ctypes.c_float, ctypes.c_float, ctypes.c_float, c_int, ctypes.c_float, c_void_p]),
+    "glide_unet_adam_items": (c_int, [c_void_p, c_int, ctypes.c_float, ctypes.c_float, ctypes.c_float, ctypes.c_float,
+                                      c_int, ctypes.c_float, c_void_p]),
     "glide_unet_features": (c_int, [DP, DP, DP, DP, c_int, c_int, c_double, c_void_p, c_void_p]),
     "glide_unet_targets": (c_int, [DP, DP, DP, DP, c_int, c_int, c_double, c_double, c_void_p, c_void_p]),
     "glide_unet_apply_prediction": (c_int, [c_void_p, c_int, c_int, c_double, c_double, DP, DP, DP, DP, DP,

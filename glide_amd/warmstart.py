@@ -222,12 +222,16 @@ class UNet:
 
     def adam_step(self, lr: float, b1: float = 0.9, b2: float = 0.999, eps: float = 1e-8, weight_decay: float = 0.0):
         self.step_count += 1
-        st = self._stream()
-        for k, w in self.params.items():
-            _lib.call("glide_unet_adam", _p(w), _p(self.grads[k]), _p(self.m[k]), _p(self.v[k]), w.numel(),
-                      ctypes.c_float(lr), ctypes.c_float(b1), ctypes.c_float(b2), ctypes.c_float(eps),
-                      self.step_count, ctypes.c_float(weight_decay), st)
-        self.sync_weights()
+        items = (_lib.GlideAdamItem * len(self.params))()
+        for it, (k, w) in zip(items, self.params.items()):
+            it.w, it.g, it.m, it.v = (t.data_ptr() for t in (w, self.grads[k], self.m[k], self.v[k]))
+            it.n = w.numel()
+            name = k[:-2]
+            if k.endswith(".W") and name in SHAPES:   # the convolutions' working copies
+                it.wb, it.wflip = self.wb[name].data_ptr(), self.wf[name].data_ptr()
+                it.cout, it.cin = SHAPES[name]
+        _lib.call("glide_unet_adam_items", items, len(items), lr, b1, b2, eps, self.step_count, weight_decay,
+                  self._stream())
 
     # ------------------------------------------------------------ persistence
     def state_dict(self) -> dict:

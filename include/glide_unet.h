@@ -122,6 +122,20 @@ int glide_unet_mse(const float *pred, const float *target, const float *mask, lo
 int glide_unet_adam(float *w, const float *g, float *m, float *v, long n, float lr, float b1, float b2,
                     float eps, int step, float weight_decay, void *stream);
 
+/* The same step of n_items tensors (host array) in one launch per 32; a
+ * tensor with wb is a convolution's [9][cout][cin] weights, whose BF16 copies
+ * are renewed as by glide_unet_prep_weights (wflip may be NULL). */
+typedef struct GlideAdamItem {
+    float *w;
+    const float *g;
+    float *m, *v;
+    long n;
+    uint16_t *wb, *wflip;
+    int cout, cin;
+} GlideAdamItem;
+int glide_unet_adam_items(const GlideAdamItem *items, int n_items, float lr, float b1, float b2, float eps, int step,
+                          float weight_decay, void *stream);
+
 /* Network input of one domain (ny x nx cells, FP64 fields) as BF16 NHWC with
  * 32 channels: H/1000, tanh((bed + 0.917 H)/200), 100 |grad s|, log(beta) + 2,
  * B/24 - 1, 100 ds/dx, 100 ds/dy, then zeros; s = max(bed, -0.917 H) + H

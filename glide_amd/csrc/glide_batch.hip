@@ -103,14 +103,14 @@ __global__ __launch_bounds__(BTX *TY) void kb_residual(const BEntry *__restrict_
         const BEntry &B = E[e];
         if (!on[B.member]) return;
         const GlideLevel &A = CHILD ? B.C : B.L;
-        const int lt = t - pre[e], tx = cdiv(A.g.nx, BTX);   // cell tiles; edge faces by the last tiles
+        const int lt = t - pre[e], tiles_y = cdiv(A.g.ny, TY);   // cell tiles; edge faces by the last tiles
         __syncthreads();   // the previous tile's readers of S are done
         if (CHILD)
             residual_tile_lds<BTX, TY>(A.g, to_params(A.p), A.f, A.U, nullptr, A.r, A.bed, A.B, A.beta, A.mask,
-                                             A.gamma, lt % tx, lt / tx, S);
+                                             A.gamma, lt / tiles_y, lt % tiles_y, S);
         else
             residual_tile_lds<BTX, TY>(A.g, to_params(A.p), A.r, A.U, A.f, nullptr, A.bed, A.B, A.beta, A.mask,
-                                             A.gamma, lt % tx, lt / tx, S);
+                                             A.gamma, lt / tiles_y, lt % tiles_y, S);
     });
 }
 
@@ -174,11 +174,11 @@ __global__ __launch_bounds__(BTX *PTY) __attribute__((amdgpu_waves_per_eu(2))) v
     const int e = find_entry(pre, n, t);
     const GlideLevel &A = E[e].L;
     if (!on[E[e].member]) return;
-    const int lt = t - pre[e], tx = cdiv(A.g.nx, BTX);
+    const int lt = t - pre[e], tiles_y = cdiv(A.g.ny, PTY);
     vanka_fold_tile<BTX, PTY, LOCAL>(A.g, to_params(A.p), set ? A.scratch : A.U, set ? A.U : A.scratch,
                                      fold_pending<BTX, PTY>(A.scratch, A.g.ny, A.g.nx, set ^ 1),
                                      fold_pending<BTX, PTY>(A.scratch, A.g.ny, A.g.nx, set), first != 0, A.f, A.bed, A.B,
-                                     A.beta, A.gamma, A.active, A.g.nx / RB + 1, n_newton, lt % tx, lt / tx, F);
+                                     A.beta, A.gamma, A.active, A.g.nx / RB + 1, n_newton, lt / tiles_y, lt % tiles_y, F);
 }
 
 // a wave a tile

@@ -58,13 +58,13 @@ int check_geom(const GlideGeom *g)
 
 inline hipStream_t S(void *s) { return (hipStream_t)s; }
 
-// Workgroups per CU of the persistent single-level launches (Vanka sweep,
-// residual); set by glide_set_persistence.  The Vanka sweep's 64 gives one
-// tile per workgroup at every level size used here (measured fastest: the
-// hardware then balances clustered local-smoother work); the residual's 8
-// loops each workgroup over several tiles where a level has more tiles than
-// that.  Launch shapes only: results do not depend on them.
-std::atomic<int> g_wg_per_cu[2] = {{64}, {8}};
+// Workgroups per CU of the single-level launches (Vanka sweep, residual); set
+// by glide_set_persistence.  The default 64 gives one tile per workgroup at
+// every level size used here (measured fastest: the hardware then balances
+// clustered local-smoother work, and straight kernels hold fewer registers);
+// launches with more tiles loop.  Launch shapes only: results do not depend
+// on them.
+std::atomic<int> g_wg_per_cu[2] = {{64}, {64}};
 // Levels with at most g_small_max_cells cells sweep with the small-level
 // kernel: variant 0 = k_vanka compiled for one wave per SIMD (the whole
 // register file), 1 = the row split (k_vanka_rows), 2 = k_vanka_multi (up to
@@ -109,7 +109,6 @@ dim3 persistent_grid(long tiles, int per_cu)
     return dim3((unsigned)((g + NXCD - 1) / NXCD * NXCD));
 }
 dim3 vanka_grid(int ny, int nx) { return persistent_grid((long)cdiv(nx, TX) * cdiv(ny, TY), g_wg_per_cu[0]); }
-dim3 residual_grid(int ny, int nx, int ty) { return persistent_grid((long)cdiv(nx, TX) * cdiv(ny, ty), g_wg_per_cu[1]); }
 dim3 point_grid(int ny, int nx) { return dim3((nx + 1 + TX - 1) / TX, (ny + 1 + TY - 1) / TY); }
 dim3 cell_grid(int ny, int nx) { return dim3((nx + TX - 1) / TX, (ny + TY - 1) / TY); }
 inline unsigned blocks1d(size_t n, int bs = 256) { return (unsigned)((n + bs - 1) / bs); }
@@ -122,7 +121,10 @@ int glide::set_error(int code, const char *msg) { return fail(code, msg); }
 // ---------------------------------------------------------------------------
 // Residual r = F(U) - f (- sub)  (glide/cuda/residuals.cu:6-292)
 // ---------------------------------------------------------------------------
-template <int RTY>
+// LOOP: fewer workgroups than tiles (tile_loop); kept apart because the loop's
+// hoisted values took the straight kernel from 64 registers to 112, two 64 x 8
+// workgroups a CU instead of three: 1024^2 41.5 -> 34.1 us, 768^2 29.9 -> 23.8.
+template <int RTY, bool LOOP>
 __global__ __launch_bounds__(TX *RTY) void k_residual(GlideGeom g, Params p, double *__restrict__ r,
                                                       const double *__restrict__ U, const double *__restrict__ f,
                                                       const double *__restrict__ sub, const double *__restrict__ bed,
@@ -132,11 +134,17 @@ __global__ __launch_bounds__(TX *RTY) void k_residual(GlideGeom g, Params p, dou
 {
     __shared__ ResidLDS<TX, RTY> S;
     if (zero && blockIdx.x == 0 && threadIdx.x == 0 && threadIdx.y == 0) *zero = 0;   // a flag the next kernel raises
-    const int tx = cdiv(g.nx, TX), total = tx * cdiv(g.ny, RTY);   // cell tiles; edge faces by the last tiles
-    tile_loop(total, [&](int t) {
-        __syncthreads();   // the previous tile's readers of S are done
-        residual_tile_lds<TX, RTY>(g, p, r, U, f, sub, bed, B, beta, mask, gamma, t % tx, t / tx, S);
-    });
+    const int tiles_y = cdiv(g.ny, RTY), total = cdiv(g.nx, TX) * tiles_y;   // cell tiles; edge faces by the last tiles
+    if (LOOP) {
+        tile_loop(total, [&](int t) {
+            __syncthreads();   // the previous tile's readers of S are done
+            residual_tile_lds<TX, RTY>(g, p, r, U, f, sub, bed, B, beta, mask, gamma, t / tiles_y, t % tiles_y, S);
+        });
+        return;
+    }
+    const int t = chunked_tile(blockIdx.x, total);
+    if (t >= total) return;
+    residual_tile_lds<TX, RTY>(g, p, r, U, f, sub, bed, B, beta, mask, gamma, t / tiles_y, t % tiles_y, S);
 }
 
 // ---------------------------------------------------------------------------
@@ -179,10 +187,11 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void k_
     int n_newton)
 {
     __shared__ FoldLDS<TX, TY> F;
-    const int tx = cdiv(g.nx, TX);
+    const int tiles_y = cdiv(g.ny, TY), total = cdiv(g.nx, TX) * tiles_y, t = chunked_tile(blockIdx.x, total);
+    if (t >= total) return;
     vanka_fold_tile<TX, TY, LOCAL>(g, p, U, Uo, fold_pending<TX, TY>(scratch, g.ny, g.nx, set ^ 1),
                                    fold_pending<TX, TY>(scratch, g.ny, g.nx, set), first != 0, f, bed, B, beta, gamma, blk,
-                                   nbx, n_newton, blockIdx.x % tx, blockIdx.x / tx, F);
+                                   nbx, n_newton, t / tiles_y, t % tiles_y, F);
 }
 __global__ __launch_bounds__(TX) void k_fold_finish(int ny, int nx, double *__restrict__ U, double *scratch, int set)
 {
@@ -1206,15 +1215,14 @@ int launch_residual(const GlideGeom &g, const Params &p, double *r, const double
                     hipStream_t st, int *zero = nullptr)
 {
     const int ty = residual_ty();
-    if (ty == 16)
-        hipLaunchKernelGGL(k_residual<16>, residual_grid(g.ny, g.nx, 16), dim3(TX, 16), 0, st, g, p, r, U, f, sub, bed,
-                           B, beta, mask, gamma, zero);
-    else if (ty == 8)
-        hipLaunchKernelGGL(k_residual<8>, residual_grid(g.ny, g.nx, 8), dim3(TX, 8), 0, st, g, p, r, U, f, sub, bed, B,
-                           beta, mask, gamma, zero);
-    else
-        hipLaunchKernelGGL(k_residual<4>, residual_grid(g.ny, g.nx, 4), dim3(TX, 4), 0, st, g, p, r, U, f, sub, bed, B,
-                           beta, mask, gamma, zero);
+    const long tiles = (long)cdiv(g.nx, TX) * cdiv(g.ny, ty);
+    const bool loop = tiles > (long)n_cu() * g_wg_per_cu[1];
+    const dim3 grid = loop ? persistent_grid(tiles, g_wg_per_cu[1]) : dim3(chunked_grid((int)tiles));
+    auto k = ty == 16  ? (loop ? k_residual<16, true> : k_residual<16, false>)
+             : ty == 8 ? (loop ? k_residual<8, true> : k_residual<8, false>)
+                       : (loop ? k_residual<4, true> : k_residual<4, false>);
+    hipLaunchKernelGGL(k, grid, dim3(TX, ty == 16 || ty == 8 ? ty : 4), 0, st, g, p, r, U, f, sub, bed, B, beta, mask, gamma,
+                       zero);
     return check_launch("residual");
 }
 
@@ -1277,8 +1285,9 @@ int launch_sweeps(const GlideGeom &g, const Params &p, double *U, const double *
             if (n_sweeps & 1) sweep(local), s = 1;
             const dim3 tiles(cdiv(g.nx, TX) * cdiv(g.ny, TY));
             for (int k = 0; s < n_sweeps; s++, k++)
-                hipLaunchKernelGGL(k_vanka_fold<LOCAL>, tiles, block, 0, st, g, p, k & 1 ? scratch : U, k & 1 ? U : scratch,
-                                   scratch, k & 1, k == 0, f, bed, B, beta, gamma, blk, nbx, n_newton);
+                hipLaunchKernelGGL(k_vanka_fold<LOCAL>, dim3(chunked_grid((int)tiles.x)), block, 0, st, g, p,
+                                   k & 1 ? scratch : U, k & 1 ? U : scratch, scratch, k & 1, k == 0, f, bed, B, beta, gamma,
+                                   blk, nbx, n_newton);
             hipLaunchKernelGGL(k_fold_finish, tiles, dim3(TX), 0, st, g.ny, g.nx, U, scratch, 1);
         }
         for (; s < n_sweeps; s++) sweep(local);

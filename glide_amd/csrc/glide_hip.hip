@@ -59,12 +59,14 @@ int check_geom(const GlideGeom *g)
 inline hipStream_t S(void *s) { return (hipStream_t)s; }
 
 // Workgroups per CU of the single-level launches (Vanka sweep, residual); set
-// by glide_set_persistence.  The default 64 gives one tile per workgroup at
-// every level size used here (measured fastest: the hardware then balances
-// clustered local-smoother work, and straight kernels hold fewer registers);
-// launches with more tiles loop.  Launch shapes only: results do not depend
-// on them.
-std::atomic<int> g_wg_per_cu[2] = {{64}, {64}};
+// by glide_set_persistence.  The default ONE_TILE gives one tile per workgroup
+// at every level size (measured fastest: the hardware then balances clustered
+// local-smoother work, and straight kernels hold fewer registers); with fewer,
+// launches of more tiles loop.  Launch shapes only: results do not depend on
+// them.
+constexpr int ONE_TILE = 64;
+constexpr long MAX_WG = (1L << 22) - NXCD;   // a grid stays below 2^32 threads
+std::atomic<int> g_wg_per_cu[2] = {{ONE_TILE}, {ONE_TILE}};
 // Levels with at most g_small_max_cells cells sweep with the small-level
 // kernel: variant 0 = k_vanka compiled for one wave per SIMD (the whole
 // register file), 1 = the row split (k_vanka_rows), 2 = k_vanka_multi (up to
@@ -102,9 +104,10 @@ int n_cu()
     return cu[dev];
 }
 // min(tiles, CUs x per_cu) workgroups, at least 8 and a multiple of 8 (tile_loop)
+long most_wg(int per_cu) { return per_cu == ONE_TILE ? MAX_WG : (long)n_cu() * per_cu; }
 dim3 persistent_grid(long tiles, int per_cu)
 {
-    long g = tiles < (long)n_cu() * per_cu ? tiles : (long)n_cu() * per_cu;
+    long g = std::min(tiles, most_wg(per_cu));
     g = g < NXCD ? NXCD : g;
     return dim3((unsigned)((g + NXCD - 1) / NXCD * NXCD));
 }
@@ -157,8 +160,11 @@ __global__ __launch_bounds__(TX *RTY) void k_residual(GlideGeom g, Params p, dou
 // the Newton chain's latency); small levels, whose few waves each run alone
 // on a SIMD, take 1 (the whole register file: no spills, longer schedules).
 // LOOP: fewer workgroups than tiles, each looping over tiles (tile_loop); kept
-// apart because the loop's hoisted values cost the straight kernel 300 bytes
-// of spill per lane.
+// apart because the loop's hoisted values cost registers.  The tile takes its
+// parameters by way of opaque(), so that what follows from them is not among
+// those values: 16 bytes of spill a lane instead of 348, a sweep of 2304^2 cells
+// on some 16000 workgroups 1360 -> 841 us (one tile a workgroup: 802, without the
+// apply pass 723).
 template <bool LOCAL, int WPE, bool LOOP>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void k_vanka(
     GlideGeom g, Params p, const double *__restrict__ U, const double *__restrict__ f, const double *__restrict__ bed,
@@ -170,7 +176,8 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE))) void 
     if (LOOP)
         tile_loop(total, [&](int t) {
             __syncthreads();   // the previous tile's readers of L are done
-            vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, t % tx, t / tx, L);
+            vanka_tile<TX, TY, LOCAL>(opaque(g), opaque(p), U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, t % tx,
+                                      t / tx, L);
         });
     else if ((int)blockIdx.x < total)
         vanka_tile<TX, TY, LOCAL>(g, p, U, f, bed, B, beta, gamma, blk, nbx, n_newton, cd, blockIdx.x % tx,
@@ -1216,8 +1223,9 @@ int launch_residual(const GlideGeom &g, const Params &p, double *r, const double
 {
     const int ty = residual_ty();
     const long tiles = (long)cdiv(g.nx, TX) * cdiv(g.ny, ty);
-    const bool loop = tiles > (long)n_cu() * g_wg_per_cu[1];
-    const dim3 grid = loop ? persistent_grid(tiles, g_wg_per_cu[1]) : dim3(chunked_grid((int)tiles));
+    const int per_cu = g_wg_per_cu[1];
+    const bool loop = tiles > most_wg(per_cu);
+    const dim3 grid = loop ? persistent_grid(tiles, per_cu) : dim3(chunked_grid((int)tiles));
     auto k = ty == 16  ? (loop ? k_residual<16, true> : k_residual<16, false>)
              : ty == 8 ? (loop ? k_residual<8, true> : k_residual<8, false>)
                        : (loop ? k_residual<4, true> : k_residual<4, false>);

@@ -67,6 +67,23 @@ __device__ __forceinline__ void tile_loop(int total, const Body &body)
     }
 }
 
+// The same values, unknown to the compiler: a loop's body that takes them computes
+// what follows from them anew instead of holding it in registers over the loop.
+__device__ __forceinline__ GlideGeom opaque(GlideGeom g)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(g.ny), "+s"(g.nx), "+s"(g.dx), "+s"(g.dt));
+#endif
+    return g;
+}
+__device__ __forceinline__ Params opaque(Params p)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm volatile("" : "+s"(p.n), "+s"(p.eps_reg), "+s"(p.water_drag), "+s"(p.calving_rate), "+s"(p.gl_c), "+s"(p.gl_derivatives));
+#endif
+    return p;
+}
+
 // One tile per workgroup with the tiles dealt to the XCDs in chunks of up to
 // TCH consecutive tiles, as tile_loop deals them: workgroup b (on XCD b % 8)
 // takes tile (x + 8 c) tch + o for x = b % 8, c = (b / 8) / tch, o = (b / 8)

@@ -342,8 +342,8 @@ int glide_batch_time_restriction(GlideBatch *batch, int phase, int reps, double 
                                  void *stream);
 
 /* Workgroups per CU of the persistent single-level launches: kernel 0 =
- * the Vanka sweep, 1 = the residual (default 64, i.e. one tile per workgroup,
- * for both).  Each launch has
+ * the Vanka sweep, 1 = the residual.  64, the default for both, is one tile per
+ * workgroup at every level size; with 1 to 63 a launch has
  * min(tiles, CUs x wg_per_cu) workgroups looping over its tiles.  A launch
  * shape only: results do not depend on it.  Process-wide (atomic); no
  * reference counterpart. */

@@ -17,6 +17,7 @@
 // (deterministic, no atomics).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -1306,8 +1307,6 @@ int conv_nj(long P, int C)
         if (C % (16 * nj) == 0 && pw * (C / (16 * nj)) >= 2048) return nj;
     return 1;
 }
-// LDS bytes of a workgroup of nw waves
-
 void pool2(const bf16_t *x, int N, int H, int W, int C, bf16_t *y, hipStream_t st)
 {
     const long n = (long)N * (H / 2) * (W / 2) * C;
@@ -1341,29 +1340,54 @@ void conv_launch(const ConvArgs &c, hipStream_t st)
                        dim3(64 * NW * NG), 0, st, c.xa, c.CA, c.up, c.xb, c.H, c.W, tx, tiles, c.Wt, c.Cout, c.bias,
                        c.relu, c.ya, c.out, c.pool, c.ga, c.SA, c.acc_a, c.gb, c.acc_b);
 }
-// Row pairs per workgroup (tile rows / 2): the tallest tile reads the fewest
-// halo rows, so 4 where that still gives a workgroup per CU and the input fits
-// 64 KB of LDS, else 2, else 1.
+// Row pairs per workgroup (tile rows / 2), and whether the staged kernel is the
+// faster one at all.  Its time goes with the pixels of its tiles, inside the
+// image or not; the direct kernel's with the pixels that there are (twice the
+// price in its narrowest form), down to some 84000 pixels by 32 output channels
+// (56000 with 128 and more input channels), below which it waits out its loads.  A
+// staged pixel costs, in pixels of the direct kernel, 0.29 where the weights are
+// staged too, 0.4 in the taller tiles with three chunks of input channels and one
+// workgroup for all output channels, else 0.56 (measured over 1 to 4000 images of
+// 1 to 64 pixels a side and strips of 500, 32 to 192 channels).  The cheapest
+// height that still gives a workgroup per CU is taken, the taller one of two
+// (fewer halo rows), and the direct kernel where it costs less than that and the
+// tiles have no CU each.  96 -> 96 channels: 4000 images of 2 x 2 pixels 236 us
+// staged, 27 direct; 1000 of 8 x 8 62 and 45; 500 of 20 x 20 97 and 151; 256 of 32 x
+// 32 70 and 189.
 template <int NG, int NCH, int MODE>
-void conv_staged(const ConvArgs &c, hipStream_t st)
+bool conv_staged(const ConvArgs &c, hipStream_t st)
 {
-    auto wgs = [&](int nw) {
-        return (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * nw - 1) / (2 * nw)) * c.N * (c.Cout / (32 * NG));
+    constexpr bool TALL = conv_lds(4, NCH) <= 64 * 1024 || conv_wl(4, NG, NCH), MID = conv_lds(2, NCH) <= 64 * 1024;
+    const long groups = c.Cout / 32, pixels = (long)c.N * c.H * c.W;
+    int nw = 1;
+    long wgs = 0;
+    double cost = 0.0;
+    auto height = [&](int k, bool has) {
+        const long w = (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * k - 1) / (2 * k)) * c.N * (groups / NG);
+        const double each = conv_wl(k, NG, NCH) ? 0.29 : NCH == 3 && groups == NG && k > 1 ? 0.4 : 0.56;
+        const double x = each * w * (2 * k * CV_W) * NG / groups;
+        if (!has || (k > 1 && w < 256) || (wgs && x >= cost)) return;
+        nw = k, wgs = w, cost = x;
     };
-    if constexpr (conv_lds(4, NCH) <= 64 * 1024 || conv_wl(4, NG, NCH))
-        if (wgs(4) >= 256) return conv_launch<4, NG, NCH, MODE>(c, st);
-    if constexpr (conv_lds(2, NCH) <= 64 * 1024)
-        if (wgs(2) >= 256) return conv_launch<2, NG, NCH, MODE>(c, st);
-    conv_launch<1, NG, NCH, MODE>(c, st);
+    height(4, TALL);
+    height(2, MID);
+    height(1, true);
+    const double price = conv_nj(pixels, c.Cout) > 1 ? 1.0 : NCH == 3 && groups == 3 ? 1.5 : 2.0;
+    if (wgs > 256 && cost > std::max(price * pixels, (NCH < 4 ? 84e3 : 56e3) / groups)) return false;
+    if constexpr (TALL)
+        if (nw == 4) return conv_launch<4, NG, NCH, MODE>(c, st), true;
+    if constexpr (MID)
+        if (nw == 2) return conv_launch<2, NG, NCH, MODE>(c, st), true;
+    return conv_launch<1, NG, NCH, MODE>(c, st), true;
 }
 // The workgroup's waves share the staged input among up to 3 groups of 32 output channels.
 template <int NCH, int MODE>
-void conv_groups(const ConvArgs &c, hipStream_t st)
+bool conv_groups(const ConvArgs &c, hipStream_t st)
 {
     const int ng = c.Cout / 32;
     if (ng % 3 == 0) return conv_staged<3, NCH, MODE>(c, st);
     if (ng % 2 == 0) return conv_staged<2, NCH, MODE>(c, st);
-    conv_staged<1, NCH, MODE>(c, st);
+    return conv_staged<1, NCH, MODE>(c, st);
 }
 template <int NJ, int MODE>
 void conv_direct(const ConvArgs &c, hipStream_t st)
@@ -1376,19 +1400,25 @@ void conv_direct(const ConvArgs &c, hipStream_t st)
 }
 // The channel counts of the network's layers have a staged instance.  It reads
 // the bias and stores in 16-byte pieces, which the direct kernel does not: a
-// tensor off that alignment takes the direct kernel.
+// tensor off that alignment takes the direct kernel, and so do images that leave
+// most of a tile empty (conv_staged).
 template <int MODE>
 void conv(ConvArgs c, hipStream_t st)
 {
     const uintptr_t al = (uintptr_t)c.bias | (uintptr_t)c.ya | (uintptr_t)c.out | (uintptr_t)c.pool | (uintptr_t)c.ga |
                          (uintptr_t)c.gb;
-    switch ((al & 15) ? 0 : (c.CA + c.CB) / 32) {
-    case 1: return conv_groups<1, MODE>(c, st);
-    case 2: return conv_groups<2, MODE>(c, st);
-    case 3: return conv_groups<3, MODE>(c, st);
-    case 4: return conv_groups<4, MODE>(c, st);
-    case 6: return conv_groups<6, MODE>(c, st);
-    }
+    auto staged = [&] {
+        if (al & 15) return false;
+        switch ((c.CA + c.CB) / 32) {
+        case 1: return conv_groups<1, MODE>(c, st);
+        case 2: return conv_groups<2, MODE>(c, st);
+        case 3: return conv_groups<3, MODE>(c, st);
+        case 4: return conv_groups<4, MODE>(c, st);
+        case 6: return conv_groups<6, MODE>(c, st);
+        }
+        return false;
+    };
+    if (staged()) return;
     switch (conv_nj((long)c.N * c.H * c.W, c.Cout)) {
     case 4: conv_direct<4, MODE>(c, st); break;
     case 2: conv_direct<2, MODE>(c, st); break;

@@ -537,8 +537,14 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const bf16_t *__restri
     const bf16_t *lsrc = src + (long)s0 * cs + 8 * (lane & 3);
     // position in its image of the x row's first pixel; the rows above (dy = -1)
     // and below (dy = 1) the image are zero
-    long r0 = is_x ? ((p_lo + shift) % HW + HW) % HW : 0;
+    const bool in32 = P + 2 * HW < (1L << 31);   // a 64-bit remainder is a tenth of the time of a call of few pixels
+    long r0 = p_lo + shift + 2 * HW;   // shift >= -HW - 1
+    r0 = !is_x ? 0 : in32 ? (long)((uint32_t)r0 % (uint32_t)HW) : r0 % HW;
     const long bad_lo = dy < 0 ? HW - W : 0, bad_hi = dy == 0 ? 0 : bad_lo + W;
+    // k % HW for k < HW + 16 WG_NR; an image smaller than a staged row by its reciprocal (subtracting it again and
+    // again took 300 images of one pixel from 15 to 88 us)
+    const uint32_t inv = HW < 16 * WG_NR ? (uint32_t)((65535 + HW) / HW) : 0;   // exact: k (HW inv - 2^16) < 2^16
+    auto wrap = [&](long k) { return inv ? k - HW * (long)(((uint32_t)k * inv) >> 16) : (k >= HW ? k - HW : k); };
     auto load = [&](long p0, uint4(&r)[WG_NR]) {
         const long q0 = p0 + shift;
         const bool inside = is_x ? q0 >= 0 && q0 + len <= P && r0 + len <= HW && (r0 + len <= bad_lo || r0 >= bad_hi)
@@ -555,17 +561,13 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const bf16_t *__restri
                 const long q = q0 + s;
                 bool ok = s < len && q >= 0 && q < (is_x ? P : p_hi);
                 if (is_x) {
-                    long k = r0 + s;
-                    while (k >= HW) k -= HW;
+                    const long k = wrap(r0 + s);
                     ok = ok && !(k >= bad_lo && k < bad_hi);
                 }
                 r[m] = ok ? *(const uint4 *)(b + 16 * m * cs) : uint4{0u, 0u, 0u, 0u};
             }
         }
-        if (is_x) {
-            r0 += WG_PX;
-            while (r0 >= HW) r0 -= HW;
-        }
+        if (is_x) r0 = wrap(r0 + WG_PX);
     };
     f32x4 acc[3][2][2];
 #pragma unroll
@@ -576,7 +578,7 @@ __global__ __launch_bounds__(256, 2) void k_conv3x3_wgrad(const bf16_t *__restri
             for (int b = 0; b < 2; b++) acc[d][a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     float bsum = 0.0f;
     // column of the lane's first pixel (8 kq past the step's first)
-    int col = (int)((p_lo + 8 * kq) % W);
+    int col = in32 ? (int)((uint32_t)(p_lo + 8 * kq) % (uint32_t)W) : (int)((p_lo + 8 * kq) % W);
     const int cstep = 32 % W;
     // the lane's corner of a fragment at step 0: pixel 8 kq + r16 / 4, channels 4 (r16 % 4)
     const int fo = (8 * kq + (r16 >> 2)) * WG_LD + 4 * (r16 & 3);

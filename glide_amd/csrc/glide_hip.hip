@@ -79,8 +79,8 @@ std::atomic<int> g_wg_per_cu[2] = {{ONE_TILE}, {ONE_TILE}};
 std::atomic<long> g_small_max_cells{208 * 208};
 std::atomic<int> g_small_variant{2};
 // Tile heights (64 x TY cells) of the single-level residual (4, 8, 16; 0 = 8)
-// and of the JVP / VJP (0 = the per-point form, 4, 6, 8; initially by level
-// size, lin_ty); set by glide_set_tile_height.  Launch shapes only: results are
+// and of the JVP / VJP (0 = the per-point form, 4, 6, 8; -1 = by level size,
+// lin_ty); set by glide_set_tile_height.  Launch shapes only: results are
 // the same bits.  Residual, 64 x 4 / 8 / 16 tiles: 256^2 7.8 / 7.9 / 9.4 us,
 // 512^2 11.5 / 10.4 / 11.2, 768^2 24.6 / 25.4 / 32.4, 1024^2 39.1 / 35.3 /
 // 43.8, 2048^2 153 / 139 / 173.
@@ -1709,7 +1709,8 @@ int glide_set_tile_height(int kernel, int ty)
             return fail(GLIDE_E_ARG, "residual tile height must be 0 (the default), 4, 8 or 16");
         g_res_ty = ty;
     } else if (kernel == 1) {
-        if (ty != 0 && ty != 4 && ty != 6 && ty != 8) return fail(GLIDE_E_ARG, "JVP/VJP tile height must be 0, 4, 6 or 8");
+        if (ty != -1 && ty != 0 && ty != 4 && ty != 6 && ty != 8)
+            return fail(GLIDE_E_ARG, "JVP/VJP tile height must be -1 (by level size), 0, 4, 6 or 8");
         g_lin_ty = ty;
     } else {
         return fail(GLIDE_E_ARG, "kernel must be 0 (residual) or 1 (JVP/VJP)");

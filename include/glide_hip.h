@@ -351,8 +351,8 @@ int glide_set_persistence(int kernel, int wg_per_cu);
 
 /* Tile heights of the single-level stencils (tiles of 64 x ty points):
  * kernel 0 = the residual (4, 8 or 16; 0, the default, = 8), 1 = the JVP and
- * VJP (4, 6 or 8; 0 = the per-point form without LDS staging; until set, by
- * level size: 6 (JVP) or 4 (VJP) while all tiles are resident at once, 8
+ * VJP (4, 6 or 8; 0 = the per-point form without LDS staging; -1, the default,
+ * by level size: 6 (JVP) or 4 (VJP) while all tiles are resident at once, 8
  * above).  A launch shape only: results are bitwise the same.  Process-wide
  * (atomic); no reference counterpart. */
 int glide_set_tile_height(int kernel, int ty);

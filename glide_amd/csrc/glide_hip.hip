@@ -990,8 +990,9 @@ __global__ __launch_bounds__(TX *LTY, LTY == 4 ? 3 : 4) void k_jvp(GlideGeom g, 
     if (t >= total) return;
     lin_tile_lds<TX, LTY, false, TX * LTY>(g, p, jo, nullptr, U, dU, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
 }
-// WY: rows of threads; those past the tile's only stage (lin_helpers)
-template <int LTY, int WY = LTY>
+// WY: rows of threads; those past the tile's only stage (lin_helpers).  STREAM:
+// tiles row by row and stores past the caches (lin_streams).
+template <int LTY, int WY = LTY, bool STREAM = false>
 __global__ __launch_bounds__(TX *WY, WY > LTY ? 2 : LTY == 4 ? 3 : 4) void k_vjp(GlideGeom g, Params p, double *__restrict__ out,
                                                  const double *__restrict__ base, const double *__restrict__ U,
                                                  const double *__restrict__ lam, const double *__restrict__ bed,
@@ -1002,7 +1003,9 @@ __global__ __launch_bounds__(TX *WY, WY > LTY ? 2 : LTY == 4 ? 3 : 4) void k_vjp
     const int tiles_y = cdiv(g.ny, LTY), total = cdiv(g.nx, TX) * tiles_y;
     const int t = chunked_tile(blockIdx.x, total);
     if (t >= total) return;
-    lin_tile_lds<TX, LTY, true, TX * WY>(g, p, out, base, U, lam, bed, B, beta, mask, t / tiles_y, t % tiles_y, S);
+    const int tiles_x = cdiv(g.nx, TX);
+    lin_tile_lds<TX, LTY, true, TX * WY, STREAM>(g, p, out, base, U, lam, bed, B, beta, mask, STREAM ? t % tiles_x : t / tiles_y,
+                                                 STREAM ? t / tiles_x : t % tiles_y, S);
 }
 // Height of the staged JVP / VJP tiles.  While all tiles are resident at once
 // (two 64 x 6 tiles of the JVP or three 64 x 4 tiles of the VJP a CU, which is
@@ -1020,6 +1023,12 @@ __global__ __launch_bounds__(TX *WY, WY > LTY ? 2 : LTY == 4 ? 3 : 4) void k_vjp
 // With more tiles than CUs the extra waves only take the others' issue.
 inline bool lin_helpers(const GlideGeom &g) { return (long)cdiv(g.nx, TX) * cdiv(g.ny, 4) <= n_cu(); }
 inline bool lin_tall(const GlideGeom &g) { return (long)cdiv(g.nx, TX) * cdiv(g.ny, 4) > 3L * n_cu(); }
+// Levels whose VJP (13 values a cell) the last-level cache of 256 MB doesn't hold:
+// tiles dealt row by row share the lines at their sides, which then come from
+// memory, while they are near, and the output leaves the cache to the inputs.
+// 1500^2 122.9 us down the columns, 123.2 row by row; 1800^2 211 and 193; 2300^2 345
+// and 329; 3000^2 579 and 556.
+inline bool lin_streams(const GlideGeom &g) { return 13 * 8 * (long)g.ny * g.nx > 256L << 20; }
 inline int lin_ty(const GlideGeom &g, bool vjp)
 {
     const int ty = g_lin_ty;
@@ -1514,7 +1523,9 @@ int launch_vjp(const GlideGeom &g, const Params &p, double *out, const double *b
 {
     const int ty = lin_ty(g, true);
     const dim3 grid4 = lin_grid(g, 4), grid8 = lin_grid(g, 8), grid6 = lin_grid(g, 6);
-    if (ty == 8)
+    if (ty == 8 && lin_streams(g))
+        hipLaunchKernelGGL((k_vjp<8, 8, true>), grid8, dim3(TX, 8), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
+    else if (ty == 8)
         hipLaunchKernelGGL(k_vjp<8>, grid8, dim3(TX, 8), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);
     else if (ty == 6)
         hipLaunchKernelGGL(k_vjp<6>, grid6, dim3(TX, 6), 0, st, g, p, out, base, U, lam, bed, B, beta, mask);

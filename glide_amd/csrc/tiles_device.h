@@ -1459,8 +1459,9 @@ struct LinTile {
     }
 };
 
-// VJP: out = base - l when base != NULL (the adjoint residual f_adj - J^T lambda)
-template <int TX, int TY, bool VJP, int NT>
+// VJP: out = base - l when base != NULL (the adjoint residual f_adj - J^T lambda).
+// STREAM: the output bypasses the caches (a level that they don't hold).
+template <int TX, int TY, bool VJP, int NT, bool STREAM = false>
 __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p, double *__restrict__ out,
                                              const double *__restrict__ base, const double *__restrict__ U,
                                              const double *__restrict__ D, const double *__restrict__ bed,
@@ -1473,7 +1474,13 @@ __device__ __forceinline__ void lin_tile_lds(const GlideGeom &g, const Params &p
     const int ny = g.ny, nx = g.nx, i = T.i0 + threadIdx.y, j = T.j0 + threadIdx.x;
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
     if (i > ny || j > nx) return;
-    auto emit = [&](size_t k, double val) { out[k] = (VJP && base) ? base[k] - val : val; };
+    auto emit = [&](size_t k, double val) {
+        if (VJP && base) val = base[k] - val;
+        if (STREAM)
+            __builtin_nontemporal_store(val, out + k);
+        else
+            out[k] = val;
+    };
     auto urow = [&](int i, int j) { emit((size_t)i * (nx + 1) + j, T.u_row(i, j)); };
     auto vrow = [&](int i, int j) { emit(nu + (size_t)i * nx + j, T.v_row(i, j)); };
     if (i < ny) urow(i, j);

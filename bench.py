@@ -283,7 +283,7 @@ def ensemble_bench(dt=10.0, n_vcycles=3):
 
     from glide_amd import synthetic as S
     from glide_amd.autotune import tune
-    from glide_amd.ensemble import BK_RESIDUAL, BK_VANKA, Ensemble
+    from glide_amd.ensemble import BK_RESIDUAL, Ensemble
     from glide_amd.physics import IcePhysics
 
     members = S.ensemble_members()
@@ -312,8 +312,9 @@ def ensemble_bench(dt=10.0, n_vcycles=3):
         solo_ms.append((time.perf_counter() - t0) * 1e3)
     # the batched Vanka sweep with every member enabled: phase 0 holds the
     # 6-level members' finest levels (16 x 512^2 + 16 x 768^2)
-    vty = int(rec["choice"]["vanka"]["0"])
-    v_ms = ens.time_kernel(BK_VANKA, 0, vty, 0, reps=5)
+    v_ms = ens.time_sweep(0)   # in the form that the schedule's sweeps run it
+    v_form = ens.sweep_form(0)
+    v_kernel = "kb_vanka_multi" if v_form > 0 else "kb_vanka_fold" if v_form < 0 else "kb_vanka"
     v_cells = sum(d["ny"] * d["nx"] for d in members if d["n_levels"] == ens.n_phases)
     v_tf = sweep_flops(v_cells) / (v_ms * 1e-3) / 1e12
     # ensemble-wide residual on every finest level (one launch)
@@ -345,11 +346,11 @@ def ensemble_bench(dt=10.0, n_vcycles=3):
         "throughput_member_steps_per_s": round(len(members) / (batched_ms * 1e-3), 2),
         "throughput_cell_vcycles_per_s": float(f"{cells * n_vcycles / (batched_ms * 1e-3):.4e}"),
         "autotune_s": round(tune_s, 1), "tile_heights": rec["choice"],
-        "vanka_roofline": {"kernel": "kb_vanka (phase 0: 16 x 512^2 + 16 x 768^2 finest levels, one launch)",
+        "vanka_roofline": {"kernel": f"{v_kernel}<false> (phase 0: 16 x 512^2 + 16 x 768^2 finest levels, one sweep)",
                            "bound": "valu", "note": "FP64 vector arithmetic (no MFMA)", "achieved": round(v_tf, 3),
                            "peak": PEAK_FP64_TFLOPS, "unit": "TFLOP/s", "frac": round(v_tf / PEAK_FP64_TFLOPS, 4),
                            "ms_per_launch": round(v_ms, 4), "work": f"{v_cells} cells x (eta + 10 Newton x "
-                                                                    f"{FLOPS_NEWTON_ITER} flop)", "tile_height": vty},
+                                                                    f"{FLOPS_NEWTON_ITER} flop)"},
         "stencil_roofline": {"kernel": "kb_residual (every finest level, one launch)", "bound": "hbm",
                              "achieved": round(res_gbs, 1), "peak": PEAK_HBM_GBS, "unit": "GB/s",
                              "frac": round(res_gbs / PEAK_HBM_GBS, 4), "ms_per_launch": round(res_ms, 4),

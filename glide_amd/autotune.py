@@ -3,7 +3,9 @@
 For every phase of an :class:`Ensemble` plan the tuner times each tunable
 kernel over its candidate tile heights (64-wide tiles: one wave64 per tile
 row) on the plan's own members, in place, with HIP events, and keeps the
-fastest.  Timings are state-preserving (the Vanka timing writes only the
+fastest.  Phases that run several sweeps a launch, or sweeps without an apply
+pass, do so on tiles of one shape: there the smoother, which takes only single
+and odd first sweeps, keeps its default height and is not timed.  Timings are state-preserving (the Vanka timing writes only the
 per-cell update scratch, the residual timings only residual buffers), so the
 tuner may run on a live ensemble between time steps.  Tile shape never
 changes results: every shape computes the same per-point arithmetic.
@@ -26,6 +28,7 @@ CANDIDATES = {
     BK_RESIDUAL: (2, 4, 8, 16),
     BK_RESIDUAL_CHILD: (2, 4, 8, 16),
 }
+DEFAULT_VANKA = 4
 NAMES = {BK_VANKA: "vanka", BK_VANKA_LOCAL: "vanka_local", BK_RESIDUAL: "residual",
          BK_RESIDUAL_CHILD: "residual_child"}
 
@@ -80,9 +83,12 @@ def tune(ens: Ensemble, reps: int = 5, use_cache: bool = True, path: str | None 
                 continue                      # no sweeps run on the finest-level pseudo-phase
             if k == BK_RESIDUAL_CHILD and p >= ens.n_phases - 1:
                 continue                      # the coarsest phase has no child
-            t = {ty: ens.time_kernel(k, p, ty, 0, reps) for ty in cands}
-            best = min(t, key=t.get)
-            times[NAMES[k]][str(p)] = {str(ty): ms for ty, ms in t.items()}
+            if k == BK_VANKA and ens.sweep_form(p):
+                best = DEFAULT_VANKA
+            else:
+                t = {ty: ens.time_kernel(k, p, ty, 0, reps) for ty in cands}
+                best = min(t, key=t.get)
+                times[NAMES[k]][str(p)] = {str(ty): ms for ty, ms in t.items()}
             choice[NAMES[k]][str(p)] = best
             if k == BK_VANKA:
                 choice[NAMES[BK_VANKA_LOCAL]][str(p)] = best

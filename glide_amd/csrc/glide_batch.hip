@@ -509,20 +509,42 @@ int b_vanka(const GlideBatch *b, int p, bool local, int shape, int occ, int n_ne
     return bcheck("batched vanka");
 }
 
+// What repeats in a phase's sweeps: n > 0 of them a launch (kb_vanka_multi) where
+// the tiles have a CU each, -1 = one a launch without an apply pass (kb_vanka_fold)
+// where every level is wide enough for it, 0 = the smoother and its apply pass
+int sweep_form(const GlideBatch *b, int p)
+{
+    const BPhase &P = b->ph[p];
+    for (int ns = MULTI_MAX; ns >= 1; ns--)
+        if (P.total[multi_table(ns)] <= b->n_cu) return ns;
+    return P.fold ? -1 : 0;
+}
+void b_multi(const GlideBatch *b, int p, bool local, int n_newton, int ns, int to_u, hipStream_t st)
+{
+    const BPhase &P = b->ph[p];
+    hipLaunchKernelGGL((local ? kb_vanka_multi<true> : kb_vanka_multi<false>), dim3(P.total[multi_table(ns)]), dim3(MS, MS), 0,
+                       st, entries(b, p), table(b, p, multi_table(ns)), P.n, b->d_on, n_newton, ns, to_u);
+}
+void b_fold(const GlideBatch *b, int p, bool local, int n_newton, int set, int first, hipStream_t st)
+{
+    const BPhase &P = b->ph[p];
+    const int tid = table_id(0, TK_CELL, SHAPE_PTY);
+    hipLaunchKernelGGL((local ? kb_vanka_fold<true> : kb_vanka_fold<false>), dim3(chunked_grid(P.total[tid])),
+                       dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, tid), P.n, b->d_on, n_newton, set, first);
+}
+
 int b_sweeps(const GlideBatch *b, int p, bool local, int n_sweeps, int n_newton, hipStream_t st)
 {
     const BPhase &P = b->ph[p];
     const int kern = local ? BK_VANKA_LOCAL : BK_VANKA;
     const int apt = table_id(0, TK_POINT, SHAPE_PTY);
     const unsigned ga = grid_of(b, P.total[apt], 8);
-    // phases whose tiles have a CU each take several sweeps a launch, larger ones
-    // fold the apply pass into the next sweep; both alternate the state between U
-    // and the scratch: an even count of launches, or the first sweep in place (as
-    // the single-level sweeps)
-    int per = 0, launches = 0, in_place = n_sweeps;
-    for (int ns = MULTI_MAX; ns >= 1 && !per; ns--)
-        if (P.total[multi_table(ns)] <= b->n_cu) per = ns;
-    const bool fold = !per && P.fold && n_sweeps > 1;
+    // several sweeps a launch and folded ones alternate the state between U and the
+    // scratch: an even count of launches, or the first sweep in place (as the
+    // single-level sweeps)
+    const int form = sweep_form(b, p), per = form > 0 ? form : 0;
+    const bool fold = form < 0 && n_sweeps > 1;
+    int launches = 0, in_place = n_sweeps;
     if (per) {
         launches = cdiv(n_sweeps, per);
         if ((launches & 1) && launches < n_sweeps) launches++;
@@ -542,20 +564,40 @@ int b_sweeps(const GlideBatch *b, int p, bool local, int n_sweeps, int n_newton,
     }
     for (int s = in_place; launches > 0; launches--) {
         const int ns = cdiv(n_sweeps - s, launches);
-        hipLaunchKernelGGL((local ? kb_vanka_multi<true> : kb_vanka_multi<false>), dim3(P.total[multi_table(ns)]),
-                           dim3(MS, MS), 0, st, entries(b, p), table(b, p, multi_table(ns)), P.n, b->d_on, n_newton, ns,
-                           launches & 1);
+        b_multi(b, p, local, n_newton, ns, launches & 1, st);
         s += ns;
     }
     if (fold) {
         const int tid = table_id(0, TK_CELL, SHAPE_PTY), total = P.total[tid];
-        for (int s = in_place, k = 0; s < n_sweeps; s++, k++)
-            hipLaunchKernelGGL((local ? kb_vanka_fold<true> : kb_vanka_fold<false>), dim3(chunked_grid(total)),
-                               dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, tid), P.n, b->d_on, n_newton, k & 1, k == 0);
+        for (int s = in_place, k = 0; s < n_sweeps; s++, k++) b_fold(b, p, local, n_newton, k & 1, k == 0, st);
         hipLaunchKernelGGL(kb_fold_finish, dim3(cdiv(total, PTY)), dim3(BTX, PTY), 0, st, entries(b, p), table(b, p, tid), P.n,
                            b->d_on);
     }
     return bcheck("batched sweeps");
+}
+
+// mean ms of `run` over reps calls after one to warm up
+template <class Run>
+int time_launches(int reps, double *ms, hipStream_t st, const Run &run)
+{
+    hipEvent_t e0, e1;
+    hipError_t he = hipEventCreate(&e0);
+    if (he == hipSuccess) he = hipEventCreate(&e1);
+    if (he != hipSuccess) return bfail((int)he, "event creation failed");
+    int rc = run();
+    if (rc == GLIDE_OK) (void)hipEventRecord(e0, st);
+    for (int k = 0; k < reps && rc == GLIDE_OK; k++) rc = run();
+    if (rc == GLIDE_OK) {
+        (void)hipEventRecord(e1, st);
+        he = hipEventSynchronize(e1);
+        float t = 0.0f;
+        if (he == hipSuccess) he = hipEventElapsedTime(&t, e0, e1);
+        if (he != hipSuccess) rc = bfail((int)he, "event timing failed");
+        *ms = (double)t / reps;
+    }
+    (void)hipEventDestroy(e0);
+    (void)hipEventDestroy(e1);
+    return rc;
 }
 
 template <int OP>
@@ -889,6 +931,36 @@ int glide_batch_set_tiles(GlideBatch *b, int kernel, int phase, int ty, int wg_p
     return GLIDE_OK;
 }
 
+int glide_batch_sweep_form(GlideBatch *b, int phase, int *form)
+{
+    if (!b || !form) return bfail(GLIDE_E_NULL, "batch and form are required");
+    if (phase < 0 || phase > b->n_phases) return bfail(GLIDE_E_ARG, "phase out of range");
+    *form = sweep_form(b, phase);
+    return GLIDE_OK;
+}
+
+int glide_batch_time_sweep(GlideBatch *b, int phase, int local, int reps, double *ms, void *stream)
+{
+    if (!b || !ms) return bfail(GLIDE_E_NULL, "batch and ms are required");
+    if (reps < 1 || reps > 1000) return bfail(GLIDE_E_ARG, "reps out of range");
+    if (phase < 0 || phase > b->n_phases) return bfail(GLIDE_E_ARG, "phase out of range");
+    const BPhase &P = b->ph[phase];
+    const int form = sweep_form(b, phase), kern = local ? BK_VANKA_LOCAL : BK_VANKA;
+    *ms = 0.0;
+    hipStream_t st = (hipStream_t)stream;
+    // the launch that several sweeps repeat, from U into the scratch
+    const int rc = time_launches(reps, ms, st, [&]() {
+        if (form == 0) return b_vanka(b, phase, local != 0, P.shape[kern], P.occ[kern], 10, st);
+        if (form > 0)
+            b_multi(b, phase, local != 0, 10, form, 0, st);
+        else
+            b_fold(b, phase, local != 0, 10, 0, 1, st);
+        return bcheck("batched sweep");
+    });
+    if (form > 0) *ms /= form;
+    return rc;
+}
+
 int glide_batch_time_kernel(GlideBatch *b, int kernel, int phase, int ty, int wg_per_cu, int reps, double *ms,
                             void *stream)
 {
@@ -902,33 +974,15 @@ int glide_batch_time_kernel(GlideBatch *b, int kernel, int phase, int ty, int wg
     const int keep_s = P.shape[kernel], keep_o = P.occ[kernel];
     BTRY(glide_batch_set_tiles(b, kernel, phase, ty, wg_per_cu));
     hipStream_t st = (hipStream_t)stream;
-    hipEvent_t e0, e1;
-    hipError_t he = hipEventCreate(&e0);
-    if (he == hipSuccess) he = hipEventCreate(&e1);
-    if (he != hipSuccess) return bfail((int)he, "event creation failed");
     const int s = P.shape[kernel], o = P.occ[kernel];
-    int rc = GLIDE_OK;
-    auto run = [&]() {
+    const int rc = time_launches(reps, ms, st, [&]() {
         switch (kernel) {
         case BK_VANKA: return b_vanka(b, phase, false, s, o, 10, st);
         case BK_VANKA_LOCAL: return b_vanka(b, phase, true, s, o, 10, st);
         case BK_RESIDUAL: return b_residual(b, phase, false, s, o, st);
         default: return b_residual(b, phase, true, s, o, st);
         }
-    };
-    rc = run();   // warm-up
-    if (rc == GLIDE_OK) (void)hipEventRecord(e0, st);
-    for (int k = 0; k < reps && rc == GLIDE_OK; k++) rc = run();
-    if (rc == GLIDE_OK) {
-        (void)hipEventRecord(e1, st);
-        he = hipEventSynchronize(e1);
-        float t = 0.0f;
-        if (he == hipSuccess) he = hipEventElapsedTime(&t, e0, e1);
-        if (he != hipSuccess) rc = bfail((int)he, "event timing failed");
-        *ms = (double)t / reps;
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    });
     P.shape[kernel] = keep_s;
     P.occ[kernel] = keep_o;
     return rc;
@@ -952,24 +1006,7 @@ int glide_batch_time_restriction(GlideBatch *b, int phase, int reps, double *ms,
     *ms = 0.0;
     if (nb == 0.0) return GLIDE_OK;
     hipStream_t st = (hipStream_t)stream;
-    hipEvent_t e0, e1;
-    hipError_t he = hipEventCreate(&e0);
-    if (he == hipSuccess) he = hipEventCreate(&e1);
-    if (he != hipSuccess) return bfail((int)he, "event creation failed");
-    int rc = b_point<OP_RESTRICT_R>(b, phase, 1.0, st);   // warm-up
-    if (rc == GLIDE_OK) (void)hipEventRecord(e0, st);
-    for (int k = 0; k < reps && rc == GLIDE_OK; k++) rc = b_point<OP_RESTRICT_R>(b, phase, 1.0, st);
-    if (rc == GLIDE_OK) {
-        (void)hipEventRecord(e1, st);
-        he = hipEventSynchronize(e1);
-        float t = 0.0f;
-        if (he == hipSuccess) he = hipEventElapsedTime(&t, e0, e1);
-        if (he != hipSuccess) rc = bfail((int)he, "event timing failed");
-        *ms = (double)t / reps;
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    return rc;
+    return time_launches(reps, ms, st, [&]() { return b_point<OP_RESTRICT_R>(b, phase, 1.0, st); });
 }
 
 }  // extern "C"

@@ -99,6 +99,19 @@ class Ensemble:
         _lib.call("glide_batch_set_tiles", self._h, int(kernel), int(phase), int(ty), int(wg_per_cu))
         self.tiles[(int(kernel), int(phase))] = (int(ty), int(wg_per_cu))
 
+    def sweep_form(self, phase: int) -> int:
+        """How several sweeps run on ``phase``: 1 to 3 of them a launch, -1 = one a launch with
+        no apply pass, 0 = the smoother and its apply pass."""
+        form = ctypes.c_int()
+        _lib.call("glide_batch_sweep_form", self._h, int(phase), ctypes.byref(form))
+        return form.value
+
+    def time_sweep(self, phase: int, local: bool = False, reps: int = 5) -> float:
+        """Mean ms of one of several sweeps of ``phase`` in its form (form 0: without the apply pass)."""
+        ms = ctypes.c_double()
+        _lib.call("glide_batch_time_sweep", self._h, int(phase), int(local), int(reps), ctypes.byref(ms), self._stream())
+        return ms.value
+
     def time_kernel(self, kernel: int, phase: int, ty: int, wg_per_cu: int = 0, reps: int = 5) -> float:
         ms = ctypes.c_double()
         _lib.call("glide_batch_time_kernel", self._h, int(kernel), int(phase), int(ty), int(wg_per_cu), int(reps),

@@ -283,8 +283,8 @@ int glide_adjoint_residual(const GlideLevel *level, void *stream);
 typedef struct GlideBatch GlideBatch;
 
 /* Kernel ids for the tile autotuner (glide_batch_set_tiles / _time_kernel). */
-#define GLIDE_BK_VANKA 0          /* full Vanka sweep, tile height 1/2/4/8 */
-#define GLIDE_BK_VANKA_LOCAL 1    /* local Vanka sweep, tile height 1/2/4/8 */
+#define GLIDE_BK_VANKA 0          /* smoother of a full Vanka sweep, tile height 1/2/4/8 */
+#define GLIDE_BK_VANKA_LOCAL 1    /* smoother of a local Vanka sweep, tile height 1/2/4/8 */
 #define GLIDE_BK_RESIDUAL 2       /* residual, tile height 2/4/8/16 */
 #define GLIDE_BK_RESIDUAL_CHILD 3 /* FAS right-hand side on the child level */
 
@@ -325,10 +325,22 @@ int glide_batch_set_enabled(GlideBatch *batch, const unsigned char *on, void *st
  * budget default) of one kernel in one phase; _time_kernel runs it reps
  * times with those settings (state-preserving: the Vanka timing writes only
  * scratch, the residual timings only r and the child's f) and returns the
- * mean time per launch in ms, leaving the plan's settings unchanged. */
+ * mean time per launch in ms, leaving the plan's settings unchanged.  The Vanka
+ * kernels' heights are those of the smoother with an apply pass, which a phase
+ * of form 0 (glide_batch_sweep_form) runs for all sweeps and the others for a
+ * single or odd first one. */
 int glide_batch_set_tiles(GlideBatch *batch, int kernel, int phase, int ty, int wg_per_cu);
 int glide_batch_time_kernel(GlideBatch *batch, int kernel, int phase, int ty, int wg_per_cu,
                             int reps, double *ms, void *stream);
+
+/* How a call of several sweeps runs on a phase: 1 to 3 = so many a launch, -1 =
+ * one a launch with no apply pass, 0 = the smoother and its apply pass. */
+int glide_batch_sweep_form(GlideBatch *batch, int phase, int *form);
+
+/* Mean ms of one of several sweeps (10 Newton iterations; local != 0: of a local
+ * pass) of a phase in its form, form 0 without the apply pass, over reps
+ * launches.  Writes only scratch. */
+int glide_batch_time_sweep(GlideBatch *batch, int phase, int local, int reps, double *ms, void *stream);
 
 /* Times the batched restriction of the residual (r_c = R r, every member of
  * `phase` that has a child level, one launch) over reps launches on the

@@ -159,13 +159,6 @@ __host__ __device__ __forceinline__ double sigm_end(double z, double c)
 {
     return c * z > 0.0 ? 0x1.ffffffee4b79ap-1 : 0x1.1b4865556b5d5p-29;
 }
-__host__ __device__ __forceinline__ Ground ground_mid(double bed, double H, const Params &p)
-{
-    Ground o;
-    o.g = sigm_mid(fma(0.917, H, bed), p.gl_c);
-    o.gd = p.gl_derivatives ? p.gl_c * o.g * (1.0 - o.g) : 0.0;
-    return o;
-}
 
 // a value that is the same in every lane, held in scalar registers
 __host__ __device__ __forceinline__ double uniform(double x)

@@ -172,7 +172,8 @@ __global__ __launch_bounds__(64 * NW * NG, NCH == 1 ? 5 : NCH == 6 ? 2 : NCH == 
     }
 
     // The weights are not in the L2s when a layer starts, and the workgroups of an XCD walk them in step, each prefetch
-    // a miss: so every XCD's workgroups first touch all of them, a line of 128 bytes a thread
+    // a miss: so every XCD's workgroups first touch them, up to two lines of 128 bytes a thread (with few workgroups
+    // the last of the weights stay untouched)
     uint32_t touched = 0;
     if (!WL) {
         const long lines = (9 * tap + 127) / 128;

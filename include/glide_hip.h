@@ -64,8 +64,10 @@ typedef struct GlideLevel {
     double *U, *f, *r, *w, *z;                   /* n_total each */
     double *Lambda, *Lambda_out, *f_adj, *r_adj; /* n_total each (adjoint) */
     double *H_prev, *bed, *B, *beta, *smb, *gamma, *chi, *mask; /* nc each */
-    double *scratch;      /* 5 * nc doubles (Vanka per-cell updates; the small-level
-                             sweeps' alternate state) */
+    double *scratch;      /* 5 * nc doubles, overwritten by forward sweeps of every level size
+                             (per-cell updates, or the alternate state and updates pending
+                             between tiles), by adjoint sweeps (the half-updated Lambda), by
+                             V-cycles and by glide_residual_norm */
     unsigned char *active;/* (ny/14+1)*(nx/14+1) bytes: local-smoother blocks */
 } GlideLevel;
 
@@ -131,7 +133,8 @@ int glide_vjp(const GlideGeom *g, const GlideParams *p, double *l, const double 
 /* n_sweeps forward Vanka sweeps, each = per-cell damped Newton on the 5
  * local unknowns with eta frozen, then U += 0.5 * delta.  active == NULL
  * smooths every cell; otherwise only cells whose 14x14 reference block has
- * active[block] != 0 (see glide_local_activation).  scratch: 5*nc doubles.
+ * active[block] != 0 (see glide_local_activation).  scratch: 5*nc doubles,
+ * overwritten, no value of which is read before it is written.
  * Replaces kernels vanka_smooth / vanka_smooth_local
  * (glide/cuda/vanka.cu:3-439, 844-1295) and the host loops
  * Grid.vanka_sweep / vanka_sweep_local (glide/grid.py:256-317). */
@@ -142,9 +145,9 @@ int glide_vanka_sweep(const GlideGeom *g, const GlideParams *p, double *U, const
 
 /* glide_vanka_sweep without the scratch argument, for callers that cannot
  * allocate (code under HIP graph capture, tight serving loops, harnesses
- * that forbid hipMalloc): no counterpart in the reference.  The per-cell
- * updates (and the small levels' alternate state, see
- * glide_set_small_levels) go to a static device array of 5 x 2^20 doubles (40 MiB) that
+ * that forbid hipMalloc): no counterpart in the reference.  What a sweep keeps
+ * there (per-cell updates, or the alternate state and the updates pending
+ * between tiles) goes to a static device array of 5 x 2^20 doubles (40 MiB) that
  * each GPU the library runs on holds until the process ends, so levels up
  * to 2^20 cells (1024 x 1024) are accepted and larger ones fail with
  * GLIDE_E_SIZE.  Nothing is allocated; the array is shared by every call on

@@ -75,22 +75,22 @@ def parse():
 
 # HBM bytes per launch at 512^2, measured with rocprofv3 --pmc FETCH_SIZE and
 # WRITE_SIZE (one run each) and calibrated in the same program on kernels of
-# known traffic: a 256 MiB torch.sum reads 131,134 KiB of FETCH_SIZE (bytes =
+# known traffic: a 256 MiB torch.sum reads 131,135 KiB of FETCH_SIZE (bytes =
 # 2048 x FETCH_SIZE) and a 256 MiB fill writes 262,144 KiB of WRITE_SIZE
-# (bytes = 1024 x WRITE_SIZE).  Vanka sweep + apply pass: FETCH 13,209.6 + 8,710.5,
-# WRITE 10,240 + 6,248; residual (cell tiles, 64 x 16): FETCH 14,137.4, WRITE
-# 6,248; JVP / VJP (64 x 4 tiles, XCD-chunked order): FETCH 11,717.3 / 11,872.0,
-# WRITE 6,179.7 / 6,182.1.
+# (bytes = 1024 x WRITE_SIZE).  Vanka sweep, one of ten: FETCH 11,569.6, WRITE
+# 7,265.2, and a tenth of the pass that adds the last pending updates (1,029.0,
+# 620.0); residual (64 x 8 tiles): FETCH 11,586.4, WRITE 6,152.2; JVP / VJP (64 x 8):
+# FETCH 11,695.0 / 12,353.4, WRITE 8,202.5 / 10,257.1.
 # HBM bytes per launch of the batched residual restriction over phase 0 of the
 # 64-member plan (16 x 768^2 + 16 x 512^2 finest levels -> their children),
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE on bench.py --ensemble-only with the
 # calibration above: FETCH 135,703.5, WRITE 81,546.5 KiB per dispatch (the
 # compulsory 409 MB less the part of r the 256 MB last-level cache serves).
 TRAFFIC_ENSEMBLE_RESTRICT_PHASE0 = (2 * 135703.5 + 81546.5) * 1024
-TRAFFIC_512 = {"vanka": (2 * (13209.6 + 8710.5) + 10240.0 + 6248.0) * 1024,
-               "residual": (2 * 14137.4 + 6248.0) * 1024,
-               "jvp": (2 * 11717.3 + 6179.7) * 1024,
-               "vjp": (2 * 11872.0 + 6182.1) * 1024}
+TRAFFIC_512 = {"vanka": (2 * (11569.6 + 102.9) + 7265.2 + 62.0) * 1024,
+               "residual": (2 * 11586.4 + 6152.2) * 1024,
+               "jvp": (2 * 11695.0 + 8202.5) * 1024,
+               "vjp": (2 * 12353.4 + 10257.1) * 1024}
 
 
 def kernel_rooflines(ph, reps=20):

@@ -31,6 +31,11 @@ __host__ __device__ inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 // smoother's active blocks) still spreads over all XCDs.  The launch must
 // have at least 8 workgroups.
 constexpr int TCH = 8;
+__host__ __device__ inline int tile_chunk(int total)
+{
+    const int tch = total / (2 * NXCD);
+    return tch < 1 ? 1 : tch > TCH ? TCH : tch;
+}
 
 __host__ __device__ inline size_t n_u(int ny, int nx) { return (size_t)ny * (nx + 1); }
 __host__ __device__ inline size_t n_v(int ny, int nx) { return (size_t)(ny + 1) * nx; }
@@ -55,7 +60,7 @@ __device__ __forceinline__ void tile_loop(int total, const Body &body)
 {
     const int G = gridDim.x, b = blockIdx.x;
     const bool one = G >= total;   // tile b only; one loop for both cases, so that the body is compiled once
-    const int tch = max(1, min(TCH, total / (2 * NXCD)));
+    const int tch = tile_chunk(total);
     const int x = b % NXCD, lane = b / NXCD;
     const int nwg = (G - x + NXCD - 1) / NXCD;
     const int nchunks = (total + tch - 1) / tch;
@@ -93,16 +98,14 @@ __device__ __forceinline__ Params opaque(Params p)
 // one L2: against tile b row by row, local sweeps (vanka_fold_tile) of 387 x 501
 // 38.8 -> 36.7 us, of 1024^2 146 -> 140, full ones of 256^2 14.4 -> 13.8, of 512^2
 // 37.4 -> 36.6.
-__device__ __forceinline__ int chunked_tile(int b, int total)
+__host__ __device__ __forceinline__ int chunked_tile(int b, int total)
 {
-    const int tch = max(1, min(TCH, total / (2 * NXCD)));
-    const int k = b / NXCD;
+    const int tch = tile_chunk(total), k = b / NXCD;
     return (b % NXCD + NXCD * (k / tch)) * tch + k % tch;
 }
 __host__ __device__ inline int chunked_grid(int total)
 {
-    const int tch = total / (2 * NXCD) < 1 ? 1 : (total / (2 * NXCD) > TCH ? TCH : total / (2 * NXCD));
-    const int span = NXCD * tch;
+    const int span = NXCD * tile_chunk(total);
     return (total + span - 1) / span * span;
 }
 
@@ -902,6 +905,12 @@ struct MultiLDS {
 };
 // cells of a dimension of n that a workgroup owns after ns sweeps
 __host__ __device__ inline int multi_own(int n, int ns) { return n <= MS ? n : MS + 1 - 4 * ns; }
+// first cell of the tile that owns cells io ..: 2 ns more at the top and left, and inside the level where that has room
+__host__ __device__ inline int multi_origin(int io, int n, int ns)
+{
+    const int o = io - 2 * ns < n - MS ? io - 2 * ns : n - MS;
+    return o > 0 ? o : 0;
+}
 
 template <bool LOCAL>
 __device__ __forceinline__ void vanka_multi_tile(const GlideGeom &g, const Params &p, const double *U, double *Uo,
@@ -914,8 +923,7 @@ __device__ __forceinline__ void vanka_multi_tile(const GlideGeom &g, const Param
     const size_t nu = n_u(ny, nx), nv = n_v(ny, nx);
     const int oy = multi_own(ny, ns), ox = multi_own(nx, ns);
     const int io = by * oy, jo = bx * ox;   // owned cells [io, io + oy) x [jo, jo + ox)
-    // the tile: 2 ns cells more at the top and left, and inside the level where that has room
-    const int i0 = max(min(io - 2 * ns, ny - MS), 0), j0 = max(min(jo - 2 * ns, nx - MS), 0);
+    const int i0 = multi_origin(io, ny, ns), j0 = multi_origin(jo, nx, ns);
     const int tid = threadIdx.y * MS + threadIdx.x;
     const bool in = i0 + (int)threadIdx.y < ny && j0 + (int)threadIdx.x < nx;
     // threads past the level's edge run its nearest cell and drop the result (a

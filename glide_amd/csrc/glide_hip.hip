@@ -81,9 +81,9 @@ std::atomic<int> g_small_variant{2};
 // Tile heights (64 x TY cells) of the single-level residual (4, 8, 16; 0 = 8)
 // and of the JVP / VJP (0 = the per-point form, 4, 6, 8; -1 = by level size,
 // lin_ty); set by glide_set_tile_height.  Launch shapes only: results are
-// the same bits.  Residual, 64 x 4 / 8 / 16 tiles: 256^2 7.8 / 7.9 / 9.4 us,
-// 512^2 11.5 / 10.4 / 11.2, 768^2 24.6 / 25.4 / 32.4, 1024^2 39.1 / 35.3 /
-// 43.8, 2048^2 153 / 139 / 173.
+// the same bits.  Residual, 64 x 4 / 8 / 16 tiles, the same buffers each call:
+// 256^2 6.3 / 6.3 / 7.6 us, 512^2 10.3 / 8.7 / 8.8, 768^2 21.1 / 19.6 / 25.6,
+// 1024^2 35.5 / 27.4 / 34.2, 2048^2 141 / 117 / 146.
 std::atomic<int> g_res_ty{0};
 std::atomic<int> g_lin_ty{-1};
 int residual_ty()
@@ -126,7 +126,8 @@ int glide::set_error(int code, const char *msg) { return fail(code, msg); }
 // ---------------------------------------------------------------------------
 // LOOP: fewer workgroups than tiles (tile_loop); kept apart because the loop's
 // hoisted values took the straight kernel from 64 registers to 112, two 64 x 8
-// workgroups a CU instead of three: 1024^2 41.5 -> 34.1 us, 768^2 29.9 -> 23.8.
+// workgroups a CU instead of three: 1024^2 31.1 us looping, 27.4 straight (the
+// same buffers each call; 33.0 on new data).
 template <int RTY, bool LOOP>
 __global__ __launch_bounds__(TX *RTY) void k_residual(GlideGeom g, Params p, double *__restrict__ r,
                                                       const double *__restrict__ U, const double *__restrict__ f,
@@ -1011,9 +1012,9 @@ __global__ __launch_bounds__(TX *WY, WY > LTY ? 2 : LTY == 4 ? 3 : 4) void k_vjp
 // (two 64 x 6 tiles of the JVP or three 64 x 4 tiles of the VJP a CU, which is
 // what their registers allow without spills) the short tiles have the shorter
 // chain; beyond that the 64 x 8 tiles' smaller halo and four waves a SIMD pay.
-// JVP, 64 x 6 / 64 x 8: 256^2 7.9 / 8.8 us, 384^2 11.4 / 13.3, 512^2 18.0 /
-// 13.4, 1024^2 56.7 / 47.5.  VJP, 64 x 4 / 64 x 8: 256^2 8.5 / 10.0, 384^2 13.1
-// / 15.1, 512^2 18.5 / 15.5, 1024^2 59.9 / 56.9.  The adjoint colours (k_adjoint)
+// JVP, 64 x 6 / 64 x 8, the same buffers each call: 256^2 7.7 / 8.6 us, 384^2
+// 11.2 / 13.2, 512^2 17.5 / 13.5, 1024^2 57.3 / 49.2.  VJP, 64 x 4 / 64 x 8: 256^2
+// 7.1 (with helpers) / 9.8, 384^2 13.1 / 15.1, 512^2 19.9 / 15.4, 1024^2 65.9 / 57.5.  The adjoint colours (k_adjoint)
 // change over at the VJP's line: 256^2 (without helpers) 9.6 / 10.4, 384^2 18.0 / 19.3, 512^2 22.4
 // / 20.3, 1024^2 82.4 / 74.7.
 // Levels whose 64 x 4 tiles have a CU each: four more rows of threads take the

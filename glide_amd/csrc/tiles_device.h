@@ -162,8 +162,8 @@ __device__ __forceinline__ double eta2_from(int i, int j, int ny, int nx, double
 // sign of zeros.
 //
 // Bound by FP64 issue: about half of it is the power law and the sigmoid per
-// haloed cell.  512^2: 11.5 -> 9.2 us; 1024^2 on new data each pass: 47.9 ->
-// 39.7 us (3.0 TB/s of compulsory traffic; 24 us at the rate of a large copy).
+// haloed cell.  512^2: 11.5 -> 8.7 us; 1024^2 on new data each pass: 47.9 ->
+// 33.0 us (3.6 TB/s of compulsory traffic; 23 us at the rate of a large copy).
 // ---------------------------------------------------------------------------
 template <int TX, int TY>
 struct ResidLDS {
@@ -1144,9 +1144,10 @@ __device__ __forceinline__ double prol_H_at(const double *hc, const double *wc, 
 // Rounding as in the residual: every output sums its terms in the per-point
 // form's order, with powers of two on the constants, the short exp and log,
 // and a factor of 0 where a term vanishes at the domain edge, so the bits are
-// those of the per-point form up to the sign of zeros.  JVP of 512^2: 21.2 ->
-// 13.4 us, 1024^2: 71 -> 47.5; VJP of 333 x 517: 16.5 -> 14.2 (the staged form
-// before, which kept the velocities in LDS and evaluated each face's terms).
+// those of the per-point form up to the sign of zeros.  On new data each pass,
+// JVP of 512^2 21.2 -> 14.6 us, VJP of 333 x 517 16.5 -> 14.5; in the caches, JVP of
+// 1024^2 71 -> 49 (the staged form before, which kept the velocities in LDS and
+// evaluated each face's terms).
 //
 // The tiles cover the cells (cdiv(nx, TX) x cdiv(ny, TY)); the faces at j = nx
 // and i = ny go with the last tiles as in the residual.

@@ -1345,16 +1345,17 @@ void conv_launch(const ConvArgs &c, hipStream_t st)
 }
 // Row pairs per workgroup (tile rows / 2), and whether the staged kernel is the
 // faster one at all.  Its time goes with the pixels of its tiles, inside the
-// image or not; the direct kernel's with the pixels that there are (twice the
-// price in its narrowest form), down to some 84000 pixels by 32 output channels
-// (56000 with 128 and more input channels), below which it waits out its loads.  A
-// staged pixel costs, in pixels of the direct kernel, 0.29 where the weights are
-// staged too, 0.4 in the taller tiles with three chunks of input channels and one
-// workgroup for all output channels, else 0.56 (measured over 1 to 4000 images of
-// 1 to 64 pixels a side and strips of 500, 32 to 192 channels).  The cheapest
-// height that still gives a workgroup per CU is taken, the taller one of two
-// (fewer halo rows), and the direct kernel where it costs less than that and the
-// tiles have no CU each.  96 -> 96 channels: 4000 images of 2 x 2 pixels 236 us
+// image or not; the direct kernel's with the pixels that there are (at 2.2 times
+// the price in its narrowest form, 1.7 with 96 -> 96 channels), down to some 84000
+// pixels by 32 output channels (56000 with 128 and more input channels), below
+// which it waits out its loads.  A staged pixel costs, in pixels of the direct
+// kernel, 0.28 where the weights are staged too, 0.45 in the taller tiles with
+// three chunks of input channels and one workgroup for all output channels, else
+// 0.56 (measured over 1 to 4000 images of 1 to 64 pixels a side and strips of 500,
+// 32 to 192 channels: of the two kernels the faster one or within 10% of it, but for
+// some shapes near the line, up to 1.5 times).  The cheapest height that still
+// gives a workgroup per CU is taken, the taller one of two (fewer halo rows), and
+// the direct kernel where it costs less than that and the tiles have no CU each.  96 -> 96 channels: 4000 images of 2 x 2 pixels 236 us
 // staged, 27 direct; 1000 of 8 x 8 62 and 45; 500 of 20 x 20 97 and 151; 256 of 32 x
 // 32 70 and 189.
 template <int NG, int NCH, int MODE>
@@ -1367,7 +1368,7 @@ bool conv_staged(const ConvArgs &c, hipStream_t st)
     double cost = 0.0;
     auto height = [&](int k, bool has) {
         const long w = (long)((c.W + CV_W - 1) / CV_W) * ((c.H + 2 * k - 1) / (2 * k)) * c.N * (groups / NG);
-        const double each = conv_wl(k, NG, NCH) ? 0.29 : NCH == 3 && groups == NG && k > 1 ? 0.4 : 0.56;
+        const double each = conv_wl(k, NG, NCH) ? 0.28 : NCH == 3 && groups == NG && k > 1 ? 0.45 : 0.56;
         const double x = each * w * (2 * k * CV_W) * NG / groups;
         if (!has || (k > 1 && w < 256) || (wgs && x >= cost)) return;
         nw = k, wgs = w, cost = x;
@@ -1375,7 +1376,7 @@ bool conv_staged(const ConvArgs &c, hipStream_t st)
     height(4, TALL);
     height(2, MID);
     height(1, true);
-    const double price = conv_nj(pixels, c.Cout) > 1 ? 1.0 : NCH == 3 && groups == 3 ? 1.5 : 2.0;
+    const double price = conv_nj(pixels, c.Cout) > 1 ? 1.0 : NCH == 3 && groups == 3 ? 1.7 : 2.2;
     if (wgs > 256 && cost > std::max(price * pixels, (NCH < 4 ? 84e3 : 56e3) / groups)) return false;
     if constexpr (TALL)
         if (nw == 4) return conv_launch<4, NG, NCH, MODE>(c, st), true;
